@@ -102,7 +102,7 @@ def _normal(gen, shape, std=1.0, mean=0.0):
     return torch.randn(shape, generator=gen, device="cuda", dtype=torch.float32) * std + mean
 
 
-def prepare(case, seed):
+def _inputs(case, seed):
     gen = torch.Generator(device="cuda")
     gen.manual_seed(seed)
     kind = case["kind"]
@@ -138,6 +138,11 @@ def prepare(case, seed):
         state["gamma"], state["beta"] = _normal(gen, (d,), 0.1, 1.0).to(half), _normal(gen, (d,), 0.1).to(half)
         state["w1"], state["b1"] = _normal(gen, (hidden, d), 0.02).to(half), _normal(gen, (hidden,), 0.1).to(half)
         state["w2"], state["b2"] = _normal(gen, (d, hidden), 0.02).to(half), _normal(gen, (d,), 0.1).to(half)
+    return state
+
+
+def prepare(case, seed):
+    state = _inputs(case, seed)
     run(state)          # a program has its kernels compiled and loaded before it serves
     return state
 
@@ -204,3 +209,48 @@ def tolerance(case):
     if kind == "softmax":
         return {"rel": {"f32": 5e-7, "bf16": 7e-3, "f16": 9e-4}[case["dtype"]]}
     return {"rel": 1.6e-3}
+
+
+def _layernorm64(x, gamma, beta):
+    x = x.double()
+    mean = x.mean(-1, keepdim=True)
+    var = ((x - mean) ** 2).mean(-1, keepdim=True)
+    return (x - mean) / torch.sqrt(var + 1e-5) * gamma.double() + beta.double()
+
+
+def _gelu64(x):
+    """The tanh form, with the six-figure constant that the framework's operator is defined by."""
+    return 0.5 * x * (1.0 + torch.tanh(0.797884 * (x + 0.044715 * x ** 3)))
+
+
+def exact(case, seed):
+    """What `run` returns for these inputs, computed in 64 bits with plain torch."""
+    kind = case["kind"]
+    state = _inputs(case, seed)
+    if kind in ("linear", "matmul"):
+        x, w = state["x"].double(), state["w"].double()
+        if case["trans_w"]:
+            w = w.transpose(-1, -2).contiguous()
+        y = x @ w if x.dim() == 2 else torch.stack([x[i] @ w[i] for i in range(x.shape[0])])
+        return y * (state["sx"] * state["sw"]) if "sx" in state else y
+    if kind == "attention":
+        q, k, v = state["q"], state["k"], state["v"]
+        b, h, s, d = q.shape
+        out = torch.empty(q.shape, dtype=torch.float64, device=q.device)
+        future = torch.ones((s, s), dtype=torch.bool, device=q.device).triu(1) if case["causal"] else None
+        for i in range(b):
+            for j in range(h):
+                scores = q[i, j].double() @ k[i, j].double().t().contiguous() * d ** -0.5
+                if future is not None:
+                    scores.masked_fill_(future, float("-inf"))
+                out[i, j] = torch.softmax(scores, -1) @ v[i, j].double()
+        return out
+    if kind == "layernorm":
+        y = _layernorm64(state["x"], state["gamma"], state["beta"])
+        return _gelu64(y) if case["gelu"] else y
+    if kind == "softmax":
+        return torch.softmax(state["x"].double(), -1)
+    h = state["table"].double()[state["ids"]]
+    u = _layernorm64(h, state["gamma"], state["beta"])
+    u = _gelu64(u @ state["w1"].double().t().contiguous() + state["b1"].double())
+    return h + u @ state["w2"].double().t().contiguous() + state["b2"].double()
