@@ -613,9 +613,51 @@ bool chooseTailSplit(const KernelSpec& s, int64_t tiles, int64_t kt, int64_t bat
   return true;
 }
 
+// Tile, wavefronts and LDS buffers of a 16-bit GEMM with direct loads: the least modelled time of the forms below.  A
+// form's workgroups run `slots` at a time (one or two per CU, by their LDS); a round of them takes a + b * (share of the
+// slots in use), in us at K = 4096, fitted to 400 timings of both weight layouts (M 1-4001, N 1024-11008, K 1024-4096;
+// the choice is within 10 % of the best form on all but two of 28 shapes, and there within 15 %).  Examples, us:
+//   M, N, K            256x256/2  128x128/2  128x128/3  64x128/3  64x128/4  64x64/4      (tile / LDS buffers)
+//   4001, 11008, 4096     284        351                                      795
+//   1000, 11008, 4096      87         97         92       107       119       124
+//    300, 11008, 4096      75         45         55        38        40        45
+//    512,  4096, 4096      75         40         25        23        22        25
+//    128,  4096, 4096                 40         24        21        18        13
+//     16, 11008, 4096                                      21        18        15
+// A small tile has few MFMAs per k-tile to hide a load under: with two buffers (one k-tile ahead) the 128 x 4096 x 4096
+// product waits 0.45 us per k-tile, with four 0.2.
+struct Gemm16Form { int64_t bm, bn, wm, wn, nbuf; double slots, a, b; };
+static const Gemm16Form* chooseGemm16Form(int64_t m, int64_t n, int64_t k, int64_t batch) {
+  static const Gemm16Form forms[] = {
+      {256, 256, 4, 2, 2, 256, 55, 45}, {128, 128, 4, 2, 2, 512, 32, 31}, {128, 128, 4, 2, 3, 256, 14, 25},
+      {64, 128, 2, 2, 3, 512, 13, 28},  {64, 128, 2, 2, 4, 256, 18, 5},   {64, 64, 2, 2, 4, 512, 12, 12},
+  };
+  const Gemm16Form* best = nullptr;
+  double least = 0.0;
+  for (const auto& f : forms) {
+    if ((m < f.bm && (f.bm > 64 || batch != 1)) || n < f.bn || k < 64) continue;
+    if (k % 64 && f.bm == 256) continue;       // no register left for the moved-back k-tile: 1500 x 11008 x 1040 155 us against 60
+    const double tiles = (double)ceilDiv(m, f.bm) * (double)ceilDiv(n, f.bn) * (double)batch, rounds = std::ceil(tiles / f.slots);
+    if (f.bn == 128 && f.nbuf == 4 && rounds > 1) continue;     // one workgroup per CU pays in a single round only
+    const double cost = rounds * (f.a + f.b * tiles / (rounds * f.slots));
+    if (!best || cost < least) { best = &f; least = cost; }
+  }
+  return best;
+}
+
 bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err) {
   int64_t m, n, k, batch;
   if (!gemmCommon(s, err, m, n, k, batch)) return false;
+  // Where the caller has looked at the operands' addresses (ALIGN = 16) and asks for no tile or switch of its own, and every
+  // row starts on 16 bytes: one of the forms with direct loads
+  bool own = false;
+  for (const char* key : {"BM", "BN", "BK", "WM", "WN", "M16", "D2L", "BTR", "BPAD", "STAGES", "NBUF", "SK_UNITS", "INTERLEAVE", "SETPRIO"}) own = own || s.has(key);
+  const Gemm16Form* form = nullptr;
+  if (!own && s.get("ALIGN", 0) >= 16 && !s.get("TA", 0) && k % 8 == 0 && (s.get("TB", 0) || n % 8 == 0)) form = chooseGemm16Form(m, n, k, batch);
+  if (form) {
+    s.p["BM"] = form->bm; s.p["BN"] = form->bn; s.p["WM"] = form->wm; s.p["WN"] = form->wn;
+    s.p["M16"] = 1; s.p["D2L"] = 1; s.p["NBUF"] = form->nbuf;
+  }
   int64_t dm, dn;
   defaultGemmTile(m, n, batch, dm, dn);
   int64_t bm = s.get("BM", dm);
@@ -631,34 +673,53 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   // 4096 x 11008 x 4096 product with a pad of 32, none with 64)
   int64_t bpad = s.get("BPAD", (bn * 2) % 256 == 0 ? 64 : 32);
   if (bpad < 0 || bpad % 16) { err = "gemm_bf16: BPAD must be a multiple of 16 bytes"; return false; }
-  const bool edge = (m % bm) || (n % bn) || (k % bk);
+  const bool ragged = (m % bm) || (n % bn) || (k % bk);
+  // Ragged sizes without guarded loads: the last tiles are moved back to end at the edge (GB_SHIFT in the kernel).  Needs a
+  // whole tile in every dimension, rows that start on 16-byte boundaries (ALIGN = 16: the caller has looked at the
+  // operands' addresses; without it the guarded loads, which take any address, stay) and no tail split.
+  // fewer rows than one tile: the rows past the last are read from the last one (GB_CLAMP; direct loads only)
+  const bool clamp = m < bm && batch == 1 && s.get("D2L", 1) != 0;
+  const bool canShift = s.get("ALIGN", 0) >= 16 && (m >= bm || clamp) && n >= bn && k >= bk && k % 8 == 0 && (!s.get("TA", 0) || m % 8 == 0) &&
+                        (s.get("TB", 0) || n % 8 == 0) && s.get("SK_UNITS", 0) <= 0;
   // the 16x16x32 MFMA (see the kernel): whole 64-deep k-tiles, A contiguous along k, B contiguous along k or read
   // through the transposing LDS reads, loads without guards
-  const bool m16Fits = bk == 64 && !s.get("TA", 0) && (s.get("TB", 0) || s.get("BTR", 1)) && !edge && k % 8 == 0 && n % 8 == 0 &&
+  const bool m16Fits = bk == 64 && !s.get("TA", 0) && (s.get("TB", 0) || s.get("BTR", 1)) && (!ragged || canShift) &&
                        (wm * wn) % 2 == 0 && bm % (8 * wm * wn) == 0 && bn % (8 * wm * wn) == 0 && s.get("STAGES", 1) == 1 &&
                        s.get("SK_UNITS", 0) <= 0 && bm / wm % 16 == 0 && bn / wn % 16 == 0;
   // direct loads into LDS (global_load_lds_dwordx4, see the kernel): every wavefront moves a whole, even number of
   // 1 KiB blocks per operand tile; row-major weights need the 256-column tile and eight wavefronts
   const int64_t waves = wm * wn;
   const bool d2lFits = m16Fits && bm % (16 * waves) == 0 &&
-                       (s.get("TB", 0) ? bn % (16 * waves) == 0 : (bn == 256 && waves == 8));
+                       (s.get("TB", 0) ? bn % (16 * waves) == 0 : ((bn == 64 || bn == 128 || bn == 256) && (bn / 8) % waves == 0));
   // Default on the 256 x 256 tile with eight wavefronts, where it was measured: with direct loads 0.295-0.303 ms on
   // 4096 x 11008 x 4096 in either weight layout against 0.310-0.315 ms ([N][K]) and 0.338-0.346 ms ([K][N]) for the
   // 32x32x16 form; through registers 0.320-0.328 ms for [K][N] (also 4-8 % ahead on 4096^3, 8192^3 and
   // 2048 x 8192 x 2048) and level with the other form for [N][K].
-  const bool m16 = s.get("M16", m16Fits && d2lFits && bm == 256 && bn == 256 && waves == 8 && s.get("D2L", 1)) != 0;
+  const bool m16 = s.get("M16", m16Fits && d2lFits && !clamp && bm == 256 && bn == 256 && waves == 8 && s.get("D2L", 1)) != 0;
   s.p["M16"] = m16;
-  if (m16 && !m16Fits) { err = "gemm_bf16: M16 needs full 64-deep tiles, TA = 0, one staging set and no tail split"; return false; }
-  const bool d2l = m16 && s.get("D2L", d2lFits) != 0;
+  // a K that is no multiple of BK: the last k-tile is moved back as well, where the direct loads are used
+  const bool kTail = k % bk != 0 && canShift && m16 && d2lFits && s.get("D2L", 1) != 0;
+  const bool shift = ragged && canShift && (k % bk == 0 || kTail) && (!clamp || (m16 && d2lFits));
+  const bool edge = ragged && !shift;
+  s.p["SHIFT"] = shift;
+  if (m16 && (!m16Fits || edge)) { err = "gemm_bf16: M16 needs full 64-deep tiles, TA = 0, one staging set and no tail split"; return false; }
+  // row-major weights in other tiles than 256 columns of eight wavefronts: on request, and in the forms chosen above
+  const bool d2l = m16 && s.get("D2L", d2lFits && (s.get("TB", 0) || (bn == 256 && waves == 8))) != 0;
   s.p["D2L"] = d2l;
-  if (d2l && !d2lFits) { err = "gemm_bf16: D2L needs M16 and whole 1 KiB blocks per wavefront (row-major weights: BN = 256, eight wavefronts)"; return false; }
+  if (d2l && !d2lFits) { err = "gemm_bf16: D2L needs M16 and whole 1 KiB blocks per wavefront (row-major weights: BN = 64, 128 or 256)"; return false; }
+  const int64_t nbuf = s.get("NBUF", 2);
+  if (nbuf < 2 || nbuf > 6 || (nbuf > 2 && (!d2l || (nbuf - 1) * (bm / 8 + bn / 8) / waves > 63))) {
+    err = "gemm_bf16: NBUF is 2 to 6, more than two with direct loads only";
+    return false;
+  }
+  s.p["NBUF"] = nbuf;
   // the 16x16x32 form's transposing reads take eight consecutive k rows of 32 bytes together: the pitch must be an odd
   // multiple of 32 bytes (through registers; direct loads leave the rows unpadded and swizzle them instead)
   if (m16 && !s.has("BPAD")) bpad = 32;
   if (d2l) bpad = 0;
   const int64_t rowA = m16 ? bk * 2 : bk * 2 + 16;
   const int64_t ldsB = s.get("TB", 0) ? bn * rowA : bk * (bn * 2 + bpad);
-  const int64_t lds = 2 * bm * rowA + 2 * ldsB;
+  const int64_t lds = nbuf * (bm * rowA + ldsB);
   if (lds > 160 * 1024) { err = "gemm_bf16: tile needs more than 160 KiB of LDS"; return false; }
   const bool outBf16 = s.get("OUT_BF16", 0) != 0;
   // staging register sets = tiles in flight from global memory; two only fit small wave tiles
@@ -693,10 +754,14 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   if (d2l) d.add("GB_D2L", 1);
   if (m16 && s.has("M16_DEAL")) d.add("GB_M16_DEAL", s.get("M16_DEAL", 0) ? 1 : 0);
   // 16-bit results of whole 256 x 256 tiles in the 16x16x32 form leave through LDS as whole rows (see the kernel)
-  const bool stageOk = m16 && bm == 256 && bn == 256 && wm == 4 && wn == 2 && !edge && skUnits == 0;
+  const bool stageOk = m16 && bm == 256 && bn == 256 && wm == 4 && wn == 2 && !edge && skUnits == 0 && n % 8 == 0;
   const int64_t stageC = stageOk ? std::max<int64_t>(0, std::min<int64_t>(2, s.get("STAGE_C", outBf16 ? 2 : 0))) : 0;
   s.p["STAGE_C"] = stageC;
   if (stageC) d.add("GB_STAGE_C", stageC);
+  if (shift) d.add("GB_SHIFT", 1);
+  if (nbuf > 2) d.add("GB_NBUF", nbuf);
+  if (shift && clamp) d.add("GB_CLAMP", 1);
+  if (kTail) d.add("GB_KTAIL", 1);
   if (s.has("BTR") && !s.get("TB", 0)) d.add("GB_BTR", s.get("BTR", 1) ? 1 : 0);
   // start of the walk along k staggered between the XCDs: default on for two k-contiguous operands (see the kernel)
   if (s.has("KROT")) d.add("GB_KROT_ON", s.get("KROT", 0) ? 1 : 0);

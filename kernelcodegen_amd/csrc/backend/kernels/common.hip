@@ -88,8 +88,10 @@ __device__ __forceinline__ unsigned int kcg_pack_f16x2(float lo, float hi) {
 // strip touches stay L2-resident.
 __device__ __forceinline__ void kcg_tile_coords(int pid, int tiles_m, int tiles_n, int group_m,
                                                 int& tile_m, int& tile_n) {
-  const int nb = tiles_m * tiles_n;
-  if ((nb & 7) == 0) pid = (pid & 7) * (nb >> 3) + (pid >> 3);
+  // (a count that is no multiple of eight gives the first XCDs one tile more; without the renumbering there, every XCD
+  // fetched every panel: 300 x 11008 x 4096 bf16 on 258 tiles of 128 x 128 52 us, 45 us with it; on 430 of 64 x 128 71 and 38)
+  const int nb = tiles_m * tiles_n, rest = nb & 7, xcd = pid & 7;
+  pid = xcd * (nb >> 3) + (xcd < rest ? xcd : rest) + (pid >> 3);
   const int per_group = group_m * tiles_n;
   const int g = pid / per_group;
   const int first_m = g * group_m;

@@ -10,6 +10,13 @@
 //   GB_STAGES                    1 or 2 sets of staging registers = tiles in flight from global memory
 //   GB_INTERLEAVE                1: deal each k-step's memory instructions out between its MFMAs
 //   GB_EDGE                      1: ragged tiles, guard loads and stores
+//   GB_SHIFT                     1: ragged M or N without guarded loads: the last tile of a row or column of tiles is moved
+//                                back to end at the edge (see the kernel)
+//   GB_CLAMP                     1: M < GB_BM, one row of tiles: rows past the last are read from the last row and not
+//                                stored (direct loads only)
+//   GB_NBUF                      LDS buffers per operand, 2 (default) to 6; more than two with direct loads only: the loads of
+//                                k-tile kt + GB_NBUF start with k-tile kt
+//   GB_KTAIL                     1: K is no multiple of GB_BK; the last k-tile is moved back likewise (direct loads only)
 //   GB_F16                       1: the operands (and a 16-bit result) are IEEE half instead of bf16; the tiles
 //                                move as 16-bit patterns either way, only the MFMA and the result's rounding differ
 //   GB_OUT_BF16                  1: C has the operands' 16-bit type, else fp32
@@ -268,6 +275,22 @@ struct KcgTLoader {
 #define GB_KROT_ON (GB_TA == 0 && GB_TB == 1)
 #define GB_KROT_DEFAULTED
 #endif
+#ifndef GB_SHIFT
+#define GB_SHIFT 0
+#define GB_SHIFT_DEFAULTED 1
+#endif
+#ifndef GB_CLAMP
+#define GB_CLAMP 0
+#define GB_CLAMP_DEFAULTED 1
+#endif
+#ifndef GB_NBUF
+#define GB_NBUF 2
+#define GB_NBUF_DEFAULTED 1
+#endif
+#ifndef GB_KTAIL
+#define GB_KTAIL 0
+#define GB_KTAIL_DEFAULTED 1
+#endif
 #define GB_KROT (GB_KROT_ON && !GB_GUARD && GB_SK_UNITS == 0 && GB_K % GB_BK == 0)
 #define GB_GUARD ((GB_EDGE != 0) | ((GB_K % 8) != 0) | ((GB_TA != 0) & ((GB_M % 8) != 0)) | ((GB_TB == 0) & ((GB_N % 8) != 0)))
 
@@ -321,8 +344,14 @@ typedef _Float16 kcg_f16x8 __attribute__((ext_vector_type(8)));
 #if (GB_BM % (32 * GB_WM)) || (GB_BN % (32 * GB_WN)) || (GB_BK % 16)
 #error "tile shape does not divide into 32x32x16 MFMA tiles"
 #endif
-#if GB_D2L && (!GB_M16 || (GB_BTR && GB_BN != 256))
-#error "direct loads into LDS: only with the 16x16x32 form; row-major weights need 256-column tiles"
+#if GB_D2L && (!GB_M16 || (GB_BTR && GB_BN != 256 && GB_BN != 128 && GB_BN != 64))
+#error "direct loads into LDS: only with the 16x16x32 form; row-major weights need tiles of 64, 128 or 256 columns"
+#endif
+#if GB_NBUF != 2 && !GB_D2L
+#error "more than two LDS buffers: only with direct loads"
+#endif
+#if (GB_SHIFT && (GB_EDGE || GB_SK_UNITS > 0 || (GB_M < GB_BM && !GB_CLAMP) || GB_N < GB_BN)) || (GB_CLAMP && (!GB_D2L || !GB_SHIFT || GB_M >= GB_BM)) || (GB_KTAIL && (!GB_D2L || GB_K < GB_BK || GB_K % GB_BK == 0))
+#error "moved-back tiles: whole tiles must fit the operands; a moved-back k-tile needs direct loads"
 #endif
 #if GB_M16 && (GB_BK != 64 || GB_TA != 0 || (GB_TB == 0 && !GB_BTR) || GB_GUARD || GB_SK_UNITS > 0 || GB_STAGES != 1 || GB_NT % 128 || GB_BM % (GB_NT / 8) || (GB_TB == 1 && GB_BN % (GB_NT / 8)))
 #error "the 16x16x32 form needs whole 64-deep k-tiles, a k-contiguous A, unguarded loads, no tail split and one staging set"
@@ -348,12 +377,12 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
              , unsigned* __restrict__ W
 #endif
 ) {
-  __shared__ __attribute__((aligned(16))) char kcg_smem[2 * GB_BM * GB_ROWB + 2 * GB_BBUF];
+  __shared__ __attribute__((aligned(16))) char kcg_smem[GB_NBUF * (GB_BM * GB_ROWB + GB_BBUF)];
 #if GB_SK_UNITS > 0
   __shared__ unsigned kcg_sk_arrived;
 #endif
-  char* sA = kcg_smem;                                  // [2][GB_BM][GB_ROWB]
-  char* sB = kcg_smem + 2 * GB_BM * GB_ROWB;            // [2][GB_BN][GB_ROWB], or [2][GB_BK][GB_BROWB] (GB_BTR)
+  char* sA = kcg_smem;                                  // [GB_NBUF][GB_BM][GB_ROWB]
+  char* sB = kcg_smem + GB_NBUF * GB_BM * GB_ROWB;      // [GB_NBUF][GB_BN][GB_ROWB], or [GB_NBUF][GB_BK][GB_BROWB] (GB_BTR)
 
 #if GB_STAGGER
   // Out of step on purpose.  All workgroups of a launch start together and take the same time for a tile, so all of
@@ -411,8 +440,18 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
   const int len = ke - kb;
   int tile_m, tile_n;
   kcg_tile_coords(pid, tiles_m, tiles_n, GB_GROUP_M, tile_m, tile_n);
+#if GB_SHIFT
+  // Ragged M or N: the last tile is moved back so that it ends at the edge.  All loads then stay inside the operands
+  // without a guard (guarded loads go two bytes at a time and keep the direct loads out: 1000 x 11008 x 4096 with
+  // row-major weights took 687 us that way, 87 us this way); the rows and columns that the tile before it owns are
+  // computed again and not stored.
+  const int m_own = tile_m * GB_BM, n_own = tile_n * GB_BN;               // first row and column that this tile stores
+  const int m0 = GB_CLAMP || m_own + GB_BM <= GB_M ? m_own : GB_M - GB_BM;
+  const int n0 = n_own + GB_BN <= GB_N ? n_own : GB_N - GB_BN;
+#else
   const int m0 = tile_m * GB_BM;
   const int n0 = tile_n * GB_BN;
+#endif
   // Where this workgroup's walk along k starts.  At any moment all workgroups of a launch are at about the same k, and
   // with a row pitch that is a power of two (K = 4096: 8 KB rows) the lines they ask for then differ only in address
   // bits far above the ones that select the memory channel: every request of that moment goes to the same few
@@ -424,6 +463,8 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #if GB_KROT
   const int rot_k = (int)(blockIdx.x & 7) * GB_KT / 8 * GB_BK;
 #define GB_KPOS(k0) (((k0) + rot_k) % GB_K)
+#elif GB_KTAIL
+#define GB_KPOS(k0) ((k0) + GB_BK <= GB_K ? (k0) : GB_K - GB_BK)
 #else
 #define GB_KPOS(k0) (k0)
 #endif
@@ -474,9 +515,10 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
   // row, still within the row's one 128-byte line.  No staging registers, no LDS store instructions; a tile's loads
   // are issued behind the barrier that frees its buffer and awaited in front of the next barrier.
   constexpr int UA = GB_BM / 8 / (GB_NT / 64);                                     // instructions per wavefront and tile
-  constexpr int UB = GB_BTR ? GB_BK / 2 / (GB_NT / 64) : GB_BN / 8 / (GB_NT / 64);
+  constexpr int RB = 1024 / (GB_BN * 2) > 0 ? 1024 / (GB_BN * 2) : 1;              // k rows of row-major weights per instruction
+  constexpr int UB = GB_BTR ? GB_BK / RB / (GB_NT / 64) : GB_BN / 8 / (GB_NT / 64);
   static_assert(UA % 2 == 0 && GB_BM % (8 * (GB_NT / 64)) == 0, "direct loads: whole, even numbers of 8-row groups per wavefront");
-  static_assert(GB_BTR ? (UB == 4 && GB_NT == 512) : (UB % 2 == 0 && GB_BN % (8 * (GB_NT / 64)) == 0), "direct loads of B: four blocks per wavefront");
+  static_assert(GB_BTR ? UB * RB * (GB_NT / 64) == GB_BK && UB >= 1 : (UB % 2 == 0 && GB_BN % (8 * (GB_NT / 64)) == 0), "direct loads of B: whole blocks per wavefront");
   // The instruction is written out: through the builtin the compiler, which cannot tell that the transposing reads
   // that follow touch the other buffer, puts a wait for all outstanding loads in front of each of them.  Here it sees
   // neither the LDS write nor the counter; the waits are the explicit ones in front of the barriers.  The address is a
@@ -487,38 +529,103 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(lane_off), "s"(base), "s"(l) : "memory");
   };
   const unsigned d2l_lane = (unsigned)(lane >> 3) * (unsigned)(GB_K * 2) + (unsigned)(((lane & 7) ^ (lane >> 4)) * 16);
+  // odd groups of eight rows: chunk 4 further on, one address bit where rows are whole 128-byte lines
+  const unsigned d2l_lane1 = GB_K % 64 == 0 ? d2l_lane ^ 64u
+                                            : (unsigned)(lane >> 3) * (unsigned)(GB_K * 2) + (unsigned)(((lane & 7) ^ (lane >> 4) ^ 4) * 16);
+#if GB_CLAMP
+  unsigned d2l_lane_a[UA];
+#pragma unroll
+  for (int t = 0; t < UA; ++t) {
+    const int row = (wave * UA + t) * 8 + (lane >> 3);
+    d2l_lane_a[t] = (unsigned)(row < GB_M ? row : GB_M - 1) * (unsigned)(GB_K * 2) + (unsigned)(((lane & 7) ^ (lane >> 4) ^ ((t & 1) * 4)) * 16);
+  }
+  auto d2l_a = [&](int k0, char* sbuf, int t) __attribute__((always_inline)) {
+    lds_dma((const char*)(As + k0), d2l_lane_a[t], sbuf + (wave_u * UA + t) * 8 * GB_ROWB);
+  };
+#endif
   auto d2l = [&](const kcg_u16* g, int row0, int k0, char* sbuf, int t, int upw) __attribute__((always_inline)) {
     const int grp = wave_u * upw + t;                      // group of eight rows within the tile; its parity is that of t
-    lds_dma((const char*)(g + (long)(row0 + grp * 8) * GB_K + k0), d2l_lane ^ (unsigned)((t & 1) * 64), sbuf + grp * 8 * GB_ROWB);
+    lds_dma((const char*)(g + (long)(row0 + grp * 8) * GB_K + k0), (t & 1) ? d2l_lane1 : d2l_lane, sbuf + grp * 8 * GB_ROWB);
   };
 #if GB_BTR
-  // Row-major weights: a tile row is 512 bytes of consecutive n, one instruction moves two k rows.  Rows are not
-  // padded; the 32-byte granule g of row k lies at granule g ^ f(k), f(k) = k % 4 + 4 ((k / 8) % 2): the eight k rows
-  // that the transposing reads of two lane groups take together (k0 .. k0 + 3 and k0 + 8 .. k0 + 11) then fall on
-  // disjoint banks.  Block b = 4 wave + t holds rows 2 b and 2 b + 1: f = (i / 32) + 2 (t % 2) + 4 (wave % 2).
-  const unsigned d2l_lane_b = (unsigned)(lane >> 5) * (unsigned)(GB_N * 2) +
-                              (((((unsigned)(lane & 31) >> 1) ^ (unsigned)(lane >> 5) ^ (4u * (wave & 1))) << 1) | (unsigned)(lane & 1)) * 16u;
+  // Row-major weights: a tile row is 2 * GB_BN bytes of consecutive n, one instruction moves RB = 2, 4 or 8 k rows.  Rows
+  // are not padded; the 32-byte granule g of row k lies at granule g ^ f(k): the eight k rows that the transposing reads of
+  // two lane groups take together (k0 .. k0 + 3 and k0 + 8 .. k0 + 11) then fall on disjoint banks.  Rows of 256 bytes and
+  // more start on the same bank: f(k) = k % 4 + 4 ((k / 8) % 2); of rows of 128 bytes every other one does, and they have
+  // four granules: f(k) = (k / 2) % 2 + 2 ((k / 8) % 2).  Block b = UB wave + t holds rows RB b .. RB b + RB - 1.
+  unsigned d2l_lane_b[UB];
+#pragma unroll
+  for (int t = 0; t < UB; ++t) {
+    const int r = lane / (64 / RB), c = lane % (64 / RB), kr = (wave * UB + t) * RB + r;
+    const int f = GB_BN >= 128 ? (kr & 3) + 4 * ((kr >> 3) & 1) : ((kr >> 1) & 1) + 2 * ((kr >> 3) & 1);
+    d2l_lane_b[t] = (unsigned)r * (unsigned)(GB_N * 2) + (unsigned)((((c >> 1) ^ f) << 1) | (c & 1)) * 16u;
+  }
   auto d2l_b = [&](int k0, char* sbuf, int t) __attribute__((always_inline)) {
     const int blk = wave_u * UB + t;
-    lds_dma((const char*)(Bs + (long)(k0 + blk * 2) * GB_N + n0), d2l_lane_b ^ (unsigned)((t & 1) * 64), sbuf + blk * 2 * GB_BROWB);
+    lds_dma((const char*)(Bs + (long)(k0 + blk * RB) * GB_N + n0), d2l_lane_b[t], sbuf + blk * 1024);
   };
 #endif
   auto d2l_unit = [&](int u, int k0, int buf) __attribute__((always_inline)) {
+#if GB_CLAMP
+    if (u < UA) d2l_a(GB_KPOS(k0), sA + buf * (GB_BM * GB_ROWB), u);
+#else
     if (u < UA) d2l(As, m0, GB_KPOS(k0), sA + buf * (GB_BM * GB_ROWB), u, UA);
+#endif
 #if GB_BTR
     else d2l_b(GB_KPOS(k0), sB + buf * GB_BBUF, u - UA);
 #else
     else d2l(Bs, n0, GB_KPOS(k0), sB + buf * GB_BBUF, u - UA, UB);
 #endif
   };
+#if GB_KTAIL
+  // The last k-tile starts at K - GB_BK: its first KZ values of k were multiplied with the tile before it, and every lane
+  // overwrites those it fetched itself (the 16 bytes at lane * 16 of each of its blocks) with zeros, in both operands.
+  // Called once the loads have landed, in front of the barrier that publishes the tile.
+  auto zero_tail = [&](int buf) __attribute__((always_inline)) {
+    constexpr int KZ = GB_BK - GB_K % GB_BK;
+    const kcg_u32x4 zero = {0u, 0u, 0u, 0u};
+    auto rows = [&](char* sbuf, int upw) __attribute__((always_inline)) {
+      for (int t = 0; t < upw; ++t)
+        if ((((lane & 7) ^ (lane >> 4)) ^ ((t & 1) * 4)) * 8 < KZ) *(kcg_u32x4*)(sbuf + (wave_u * upw + t) * 8 * GB_ROWB + lane * 16) = zero;
+    };
+    rows(sA + buf * (GB_BM * GB_ROWB), UA);
+#if GB_BTR
+    for (int t = 0; t < UB; ++t)
+      if ((wave_u * UB + t) * RB + lane / (64 / RB) < KZ) *(kcg_u32x4*)(sB + buf * GB_BBUF + (wave_u * UB + t) * 1024 + lane * 16) = zero;
+#else
+    rows(sB + buf * GB_BBUF, UB);
+#endif
+  };
+  static_assert(GB_K % 8 == 0, "whole 16-byte chunks along k");
+#endif
+  // s_waitcnt vmcnt(n), the other counters left alone
+#define GB_VMCNT(n) (0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
+#if GB_NBUF > 2
+  static_assert((GB_NBUF - 1) * (UA + UB) <= 63, "the loads in flight fit the counter");
+  if (GB_NBUF <= GB_KT) {
+#pragma unroll
+    for (int b = 0; b < GB_NBUF; ++b)
+#pragma unroll
+      for (int u = 0; u < UA + UB; ++u) d2l_unit(u, b * GB_BK, b);
+    __builtin_amdgcn_s_waitcnt(GB_VMCNT((GB_NBUF - 1) * (UA + UB)));   // tile 0 has landed
+  } else {
+#pragma unroll
+    for (int b = 0; b < (GB_NBUF < GB_KT ? GB_NBUF : GB_KT); ++b)
+#pragma unroll
+      for (int u = 0; u < UA + UB; ++u) d2l_unit(u, b * GB_BK, b);
+    __builtin_amdgcn_s_waitcnt(GB_VMCNT(0));
+  }
+  __syncthreads();
+#else
 #pragma unroll
   for (int u = 0; u < UA + UB; ++u) d2l_unit(u, 0, 0);
-  __builtin_amdgcn_s_waitcnt(0x0F70);                       // vmcnt(0): tile 0 has landed
+  __builtin_amdgcn_s_waitcnt(GB_VMCNT(0));                  // tile 0 has landed
   __syncthreads();
   if (1 < len) {
 #pragma unroll
     for (int u = 0; u < UA + UB; ++u) d2l_unit(u, GB_BK, 1);
   }
+#endif
 #else
   // Prologue: tile 0 through set 0 into LDS buffer 0, then tiles 1..GB_STAGES
   // into their staging sets.
@@ -567,7 +674,7 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #if GB_D2L
   // natural k order (group q holds k 8 q .. 8 q + 7), unpadded rows with swizzled 32-byte granules (see d2l_b)
   const kcg_lds_ptr bT = (kcg_lds_ptr)sB + (8 * (lane >> 4) + (lane & 15) / 4) * GB_BROWB + 8 * (lane & 3);
-  const int bswz = ((lane & 15) >> 2) + 4 * ((lane >> 4) & 1);
+  const int bswz = GB_BN >= 128 ? ((lane & 15) >> 2) + 4 * ((lane >> 4) & 1) : ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1);
   int boff[GB_TN];
 #pragma unroll
   for (int j = 0; j < GB_TN; ++j) boff[j] = ((wn * GB_WTN / 16 + j) ^ bswz) * 32;
@@ -613,15 +720,15 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
   // mode_c: 1 = steady state (tile kt+1 is written to LDS, tile kt+1+GB_STAGES loaded), 2 = write only,
   // 3 = neither (the last iteration), 0 = decided at run time from the iteration count.
   auto iteration = [&](const int kt, auto par_c, auto mode_c) {
-    constexpr int buf = decltype(par_c)::v ? 1 : 0;
+    constexpr int buf = decltype(par_c)::v, nbuf = (buf + 1) % GB_NBUF;     // this tile's buffer, the next one's
     constexpr int mode = decltype(mode_c)::v;
     constexpr bool steady = mode == 1;
     constexpr int set = (buf + 1) % GB_STAGES;
     const bool feed = mode == 0 ? kt + 1 < len : mode != 3;               // tile kt+1 exists: write it to LDS
     const bool fetch = mode == 0 ? kt + 1 + GB_STAGES < len : mode == 1;  // tile kt+1+GB_STAGES exists: load it
     const char* cA = fA + buf * (GB_BM * GB_ROWB);
-    char* nA = sA + (buf ^ 1) * (GB_BM * GB_ROWB);
-    char* nB = sB + (buf ^ 1) * GB_BBUF;
+    char* nA = sA + nbuf * (GB_BM * GB_ROWB);
+    char* nB = sB + nbuf * GB_BBUF;
     const int k2 = (kt + 1 + GB_STAGES) * GB_BK;
 #if GB_M16
     // The MFMAs of a step go column by column over the wavefront's tiles: the B fragment of column j has its last use
@@ -662,13 +769,17 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
       }
       if (last) {
 #if GB_D2L
-        __builtin_amdgcn_s_waitcnt(0x0F70);                 // vmcnt(0): this wavefront's share of tile kt+1 has landed
+        // this wavefront's share of tile kt+1 has landed; in the steady state tiles kt+2 .. kt+GB_NBUF-1 are still under way
+        __builtin_amdgcn_s_waitcnt(GB_VMCNT(steady ? (GB_NBUF - 2) * (UA + UB) : 0));
+#endif
+#if GB_KTAIL
+        if (mode == 0 && kt + 2 == len) zero_tail(nbuf);
 #endif
         __syncthreads();
         if (feed) {
 #pragma unroll
           for (int i = 0; i < GB_TM; ++i)
-            fa[nxt][i] = *(const GB_FRAG*)(fA + (buf ^ 1) * (GB_BM * GB_ROWB) + i * GB_FR * GB_ROWB + GB_KOFF(0));
+            fa[nxt][i] = *(const GB_FRAG*)(fA + nbuf * (GB_BM * GB_ROWB) + i * GB_FR * GB_ROWB + GB_KOFF(0));
         }
       }
 #pragma unroll
@@ -680,12 +791,12 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
         }
         __builtin_amdgcn_sched_barrier(0);
         if (!last) fb[0][j] = read_fb(buf, ks + 1, j);
-        else if (feed) fb[0][j] = read_fb(buf ^ 1, 0, j);
+        else if (feed) fb[0][j] = read_fb(nbuf, 0, j);
 #if GB_D2L
-        if (last && kt + 2 < len) {
+        if (last && (steady || kt + GB_NBUF < len)) {
 #pragma unroll
           for (int u = 0; u < UA + UB; ++u)
-            if (u * GB_TN / (UA + UB) == j) d2l_unit(u, (kt + 2) * GB_BK, buf);
+            if (u * GB_TN / (UA + UB) == j) d2l_unit(u, (kt + GB_NBUF) * GB_BK, buf);
         }
 #else
         if (GB_M16_DEAL && ks < FS) {
@@ -728,10 +839,10 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
         if (feed) {
 #pragma unroll
           for (int i = 0; i < GB_TM; ++i)
-            fa[nxt][i] = *(const GB_FRAG*)(fA + (buf ^ 1) * (GB_BM * GB_ROWB) + i * 32 * GB_ROWB);
+            fa[nxt][i] = *(const GB_FRAG*)(fA + nbuf * (GB_BM * GB_ROWB) + i * 32 * GB_ROWB);
 #pragma unroll
           for (int j = 0; j < GB_TN; ++j)
-            fb[nxt][j] = read_fb(buf ^ 1, 0, j);
+            fb[nxt][j] = read_fb(nbuf, 0, j);
         }
       }
 #if !GB_INTERLEAVE
@@ -770,21 +881,39 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
       for (int j = 0; j < GB_TN; ++j) fb[0][j] = fb[1][j];
     }
   };
+#if GB_NBUF > 2
+  // one copy of the body per buffer; the last iterations, fewer than 2 * GB_NBUF, decide at run time what is left to load
+  int kt = 0;
+  auto steady_pass = [&](auto self, auto b_c) __attribute__((always_inline)) -> void {
+    constexpr int b = decltype(b_c)::v;
+    iteration(kt + b, KcgInt<b>{}, KcgInt<1>{});
+    if constexpr (b + 1 < GB_NBUF) self(self, KcgInt<b + 1>{});
+  };
+  auto last_pass = [&](auto self, auto b_c) __attribute__((always_inline)) -> void {
+    constexpr int b = decltype(b_c)::v;
+    if (kt + b >= len) return;
+    iteration(kt + b, KcgInt<b>{}, KcgInt<0>{});
+    if constexpr (b + 1 < GB_NBUF) self(self, KcgInt<b + 1>{});
+  };
+  for (; kt + 2 * GB_NBUF - 1 < len; kt += GB_NBUF) steady_pass(steady_pass, KcgInt<0>{});
+  for (; kt < len; kt += GB_NBUF) last_pass(last_pass, KcgInt<0>{});
+#else
   int kt = 0;                                         // counts from the segment's first k-iteration
   for (; kt + 2 + GB_STAGES < len; kt += 2) {        // both iterations of the pair feed and fetch
-    iteration(kt, KcgBool<false>{}, KcgInt<1>{});
-    iteration(kt + 1, KcgBool<true>{}, KcgInt<1>{});
+    iteration(kt, KcgInt<0>{}, KcgInt<1>{});
+    iteration(kt + 1, KcgInt<1>{}, KcgInt<1>{});
   }
 #if GB_SK_UNITS > 0
   // a split segment has an even number of iterations (and one staging set): two are left, of known kinds
-  iteration(kt, KcgBool<false>{}, KcgInt<2>{});
-  iteration(kt + 1, KcgBool<true>{}, KcgInt<3>{});
+  iteration(kt, KcgInt<0>{}, KcgInt<2>{});
+  iteration(kt + 1, KcgInt<1>{}, KcgInt<3>{});
 #else
   for (; kt < len; ++kt) {
-    if (kt & 1) iteration(kt, KcgBool<true>{}, KcgInt<0>{});
-    else iteration(kt, KcgBool<false>{}, KcgInt<0>{});
+    if (kt & 1) iteration(kt, KcgInt<1>{}, KcgInt<0>{});
+    else iteration(kt, KcgInt<0>{}, KcgInt<0>{});
   }
 #endif
+#endif   // GB_NBUF
 
 #if GB_SK_UNITS > 0
   // ---- a segment that is not a whole tile: slot, fence, count in; the last one in adds up and goes on to the stores ----
@@ -881,6 +1010,9 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
         const int col = (lane % LPR) * EPL;
         const kcg_f32x4 val = *(const kcg_f32x4*)(stage + row * 256 + (col ^ (16 * ((row >> 2) & 3))));
         const int trow = PASSES == 2 ? (row / (GB_WTM / 2)) * GB_WTM + (GB_WTM / 2) * pass + row % (GB_WTM / 2) : row;
+#if GB_SHIFT
+        if (m0 + trow < m_own || n0 + col < n_own) continue;         // stored by the tile before (whole chunks: N % 8 == 0)
+#endif
 #if GB_STAGE_C == 2
         __builtin_nontemporal_store(val, (kcg_f32x4*)(C + (long)(m0 + trow) * GB_N + n0 + col));
 #else
@@ -901,6 +1033,8 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
                                : m0 + wm * GB_WTM + i * 32 + 8 * (v / 4) + 4 * lh + (v % 4);
 #if GB_EDGE
         if (row < GB_M && col < GB_N)
+#elif GB_SHIFT
+        if (row >= m_own && col >= n_own && (!GB_CLAMP || row < GB_M))
 #endif
         {
 #if GB_OUT_BF16
@@ -932,6 +1066,23 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #ifdef GB_D2L_DEFAULTED
 #undef GB_D2L
 #undef GB_D2L_DEFAULTED
+#endif
+#ifdef GB_SHIFT_DEFAULTED
+#undef GB_SHIFT
+#undef GB_SHIFT_DEFAULTED
+#endif
+#undef GB_VMCNT
+#ifdef GB_CLAMP_DEFAULTED
+#undef GB_CLAMP
+#undef GB_CLAMP_DEFAULTED
+#endif
+#ifdef GB_NBUF_DEFAULTED
+#undef GB_NBUF
+#undef GB_NBUF_DEFAULTED
+#endif
+#ifdef GB_KTAIL_DEFAULTED
+#undef GB_KTAIL
+#undef GB_KTAIL_DEFAULTED
 #endif
 #ifdef GB_STAGE_C_DEFAULTED
 #undef GB_STAGE_C

@@ -47,6 +47,12 @@ def elementwise(x, op, inplace=False, out_dtype=None, **cfg):
     return y
 
 
+def _aligned(*ts):
+    """16 when every tensor starts on a 16-byte boundary (the kernels' ALIGN parameter): what wide loads and direct loads
+    into LDS need where a size is no multiple of the tile."""
+    return 16 if all(t.data_ptr() % 16 == 0 for t in ts) else 0
+
+
 _FAMILY = {torch.float32: "gemm_f32", torch.float64: "gemm_f64", torch.bfloat16: "gemm_bf16", torch.float16: "gemm_bf16"}
 
 
@@ -70,6 +76,7 @@ def batched_matmul(a, b, trans_a=False, trans_b=False, out_dtype=None, **cfg):
         extra["OUT_BF16"] = int(out_dtype == a.dtype)       # a 16-bit result, of the operands' type
         if a.dtype == torch.float16:
             extra["F16"] = 1
+        extra["ALIGN"] = _aligned(a, b)
     elif a.dtype == torch.float64:
         if out_dtype != torch.float64:
             raise ValueError("fp64 GEMM writes fp64")

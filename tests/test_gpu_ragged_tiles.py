@@ -1,0 +1,99 @@
+"""GEMM kernels on sizes that their tiles do not divide, and on fewer rows than a tile has: operands of small integers, so
+that every product and sum is exact in the accumulators (|sum| <= 16 k < 2^24 for the k used here) and the comparison is
+bit for bit, whatever tile and order of summation a kernel picks."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from kernelcodegen_amd import ops as _ops
+    from kernelcodegen_amd._lib import lib, check
+    check(lib().kcg_hip_init(0), "kcg_hip_init")
+    return _ops
+
+
+def _operands(m, n, k, tb, dtype, seed, batch=()):
+    rs = np.random.RandomState(seed)
+    a = rs.randint(-4, 5, size=batch + (m, k)).astype(np.float32)
+    b = rs.randint(-4, 5, size=batch + ((n, k) if tb else (k, n))).astype(np.float32)
+    want = a.astype(np.float64) @ (np.swapaxes(b, -1, -2) if tb else b).astype(np.float64)
+    return torch.from_numpy(a).cuda().to(dtype), torch.from_numpy(b).cuda().to(dtype), want
+
+
+def _shifted(t):
+    """The same values one element behind a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    out = buf[1:].view(t.shape)
+    out.copy_(t)
+    assert out.data_ptr() % 16 != 0 and out.is_contiguous()
+    return out
+
+
+# tile forms of the 16-bit kernel with direct loads
+FORMS = [dict(BM=256, BN=256, WM=4, WN=2), dict(BM=128, BN=128, WM=4, WN=2), dict(BM=128, BN=128, WM=4, WN=2, NBUF=3),
+         dict(BM=64, BN=128, WM=2, WN=2, NBUF=3), dict(BM=64, BN=128, WM=2, WN=2, NBUF=4), dict(BM=64, BN=64, WM=2, WN=2, NBUF=4)]
+
+
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("form", range(len(FORMS)))
+def test_gemm16_every_form_at_its_edges(ops, form, tb):
+    """One row or column more or less than whole tiles, a k of one tile, of a part more, of fewer tiles than buffers and of
+    more than two rounds of them."""
+    cfg = dict(FORMS[form], M16=1, D2L=1)
+    bm, bn = cfg["BM"], cfg["BN"]
+    ks = [64, 72, 64 * 3, 64 * 5 + 8, 64 * 13]
+    if bm == 256:
+        ks = [64, 64 * 3, 64 * 13]
+    for i, (m, n) in enumerate([(bm, bn), (bm + 1, bn + 8), (2 * bm - 1, 2 * bn - 8), (3 * bm, bn + 8)]):
+        for k in ks:
+            a, b, want = _operands(m, n, k, tb, torch.bfloat16, 100 * form + 10 * i + k)
+            print("form", form, (m, n, k), tb, flush=True)
+            for out in (torch.float32, torch.bfloat16):
+                c = ops.matmul(a, b, trans_b=tb, out_dtype=out, **cfg)
+                assert torch.equal(c.cpu(), torch.from_numpy(want).to(out)), (m, n, k, out)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("m,n,k", [(1, 512, 512), (15, 640, 4096), (63, 520, 136), (64, 1024, 2048), (65, 584, 1000), (300, 1000, 264),
+                                   (1000, 2056, 520), (257, 264, 64), (9, 64, 64), (64, 64, 72)])
+def test_gemm16_default_forms(ops, m, n, k, tb, dtype):
+    a, b, want = _operands(m, n, k, tb, dtype, m + n + k)
+    for out in (torch.float32, dtype):
+        c = ops.matmul(a, b, trans_b=tb, out_dtype=out)
+        assert torch.equal(c.cpu(), torch.from_numpy(want).to(out))
+    # operands off the 16-byte boundary are taken as well, and give the same numbers
+    for x, w in ((_shifted(a), b), (a, _shifted(b))):
+        assert torch.equal(ops.matmul(x, w, trans_b=tb).double().cpu(), torch.from_numpy(want))
+
+
+def test_gemm16_column_count_no_multiple_of_eight(ops):
+    for (m, n, k) in [(70, 515, 512), (5, 77, 128), (129, 257, 192)]:
+        a, b, want = _operands(m, n, k, True, torch.bfloat16, n)
+        for out in (torch.float32, torch.bfloat16):
+            assert torch.equal(ops.matmul(a, b, trans_b=True, out_dtype=out).cpu(), torch.from_numpy(want).to(out))
+
+
+def test_gemm16_batched(ops):
+    for tb in (False, True):
+        for (m, n, k) in [(65, 136, 200), (128, 64, 64), (17, 136, 200)]:
+            a, b, want = _operands(m, n, k, tb, torch.float16, m, batch=(3,))
+            assert torch.equal(ops.batched_matmul(a, b, trans_b=tb).double().cpu(), torch.from_numpy(want))
+
+
+@pytest.mark.parametrize("tb", [False, True])
+def test_gemm16_infinities_stay_in_their_rows_and_columns(ops, tb):
+    """The last k-tile is moved back over values that were multiplied already, the last tiles over rows and columns that
+    other tiles own: an infinity there reaches its own row and column only, and gives no NaN."""
+    m, n, k = 70, 136, 200
+    a, b, _ = _operands(m, n, k, tb, torch.bfloat16, 5)
+    a, b = a.abs() + 1, b.abs() + 1
+    a[3, 150], a[69, 0] = float("inf"), float("inf")
+    b[(7, 140) if tb else (140, 7)] = float("inf")
+    want = a.double().cpu() @ (b.t() if tb else b).double().cpu()
+    assert not torch.isnan(want).any()
+    assert torch.equal(ops.matmul(a, b, trans_b=tb).double().cpu(), want)
