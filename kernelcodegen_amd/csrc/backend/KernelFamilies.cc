@@ -725,6 +725,8 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   // staging register sets = tiles in flight from global memory; two only fit small wave tiles
   const int64_t stages = s.get("STAGES", 1);
   if (stages != 1 && stages != 2) { err = "gemm_bf16: STAGES must be 1 or 2"; return false; }
+  const bool fp8 = s.get("FP8_PAIRS", 0) != 0;             // from emitGemmFp8: K counts pairs of bytes
+  if (fp8 && (!d2l || edge || !s.get("TB", 0))) { err = "gemm_bf16: fp8 operands need the direct loads"; return false; }
   s.p["BM"] = bm; s.p["BN"] = bn; s.p["BK"] = bk; s.p["WM"] = wm; s.p["WN"] = wn; s.p["GROUP_M"] = gm;
   s.p["STAGES"] = stages;
   // with one wavefront per SIMD the memory instructions have to be interleaved with the MFMAs explicitly
@@ -759,6 +761,7 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   s.p["STAGE_C"] = stageC;
   if (stageC) d.add("GB_STAGE_C", stageC);
   if (shift) d.add("GB_SHIFT", 1);
+  if (fp8) d.add("GB_FP8", 1);
   if (nbuf > 2) d.add("GB_NBUF", nbuf);
   if (shift && clamp) d.add("GB_CLAMP", 1);
   if (kTail) d.add("GB_KTAIL", 1);
@@ -775,7 +778,8 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   info.grid[0] = (uint32_t)(skUnits > 0 ? skFull + skUnits : tiles);
   info.grid[1] = (uint32_t)batch;
   info.block[0] = (uint32_t)(64 * wm * wn);
-  info.numArgs = skUnits > 0 ? 4 : 3;
+  info.numArgs = fp8 ? 5 : skUnits > 0 ? 4 : 3;
+  info.numScalars = fp8 ? 2 : 0;
   if (skUnits > 0) {
     info.workspaceBytes = 4096 + skUnits * 2 * bm * bn * 4;
     info.workspaceArg = 3;
@@ -789,8 +793,33 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   int64_t m, n, k, batch;
   if (!gemmCommon(s, err, m, n, k, batch)) return false;
   const bool ta = s.get("TA", 0) != 0, tb = s.get("TB", 0) != 0;
+  // As for 16 bits: where the operands' addresses are known to be aligned and no tile or switch is asked for, one of the
+  // forms with direct loads, priced as a 16-bit product of half the depth.  256 x 256 tiles run on gemm_fp8_d2l.hip
+  // (twice the MFMA rate), smaller ones of two k-contiguous operands on the 16-bit kernel's ring of LDS buffers (us, against
+  // guarded loads: 300 x 4096 x 4096 13.9 and 17.0, 16 x 11008 x 4096 9.8 and 16.7, 700 x 2048 x 1040 7.5 and 10.5).  Whole
+  // tiles of the sizes below stay with gemm_fp8.hip: its unguarded loads on the faster MFMA are ahead of the ring
+  // (2048^3 12.4 against 14.6, 512 x 4096 x 4096 14.6 against 16.2; behind it only at M 64-256, K 4096, by 8-10 %).
+  bool own = false;
+  for (const char* key : {"BM", "BN", "BK", "WM", "WN", "D2L", "BTR", "STAGES", "PREFETCH", "ROTATE", "PINGPONG", "PERSIST", "STAGE_C", "NT_STORE", "STAGGER"}) own = own || s.has(key);
+  bool shift256 = false;
   int64_t dm, dn;
   defaultGemmTile(m, n, batch, dm, dn);
+  const bool whole = m % dm == 0 && n % dn == 0 && k % 128 == 0;
+  if (!own && !whole && s.get("ALIGN", 0) >= 16 && !ta && k % 16 == 0 && n % 16 == 0 && s.get("SCALE_PTR", 0) == 0) {
+    const Gemm16Form* form = chooseGemm16Form(m, n, k / 2, batch);
+    if (form && form->bm == 256) {
+      shift256 = true;
+    } else if (form && tb) {
+      s.p["K"] = k / 2;
+      s.p["FP8_PAIRS"] = 1;
+      const bool ok = emitGemmBf16(s, src, info, err);
+      s.p["K"] = k;
+      s.p.erase("FP8_PAIRS");
+      info.flops *= 2.0;      // two products per pair; the bytes are those of 16-bit values half as many
+      return ok;
+    }
+  }
+  if (shift256) dm = dn = 256;
   int64_t bm = s.get("BM", dm);
   int64_t bn = s.get("BN", dn);
   int64_t bk = s.get("BK", 128);
@@ -806,8 +835,8 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // the kernel); a single round is fastest without either.
   const bool legacyKnob = s.has("PREFETCH") || s.has("ROTATE") || s.has("PINGPONG") || s.has("STAGES") || (s.has("BTR") && !s.get("BTR", 1));
   const bool oneRound = ceilDiv(m, 256) * ceilDiv(n, 256) * batch <= 256;
-  if (s.get("D2L", !legacyKnob && (k <= 4096 || !oneRound)) && !ta && (tb || s.get("BTR", 1)) && n % 16 == 0 && bm == 256 && bn == 256 && bk == 128 && wm == 4 && wn == 2 &&
-      m % 256 == 0 && n % 256 == 0 && k % 128 == 0) {
+  if (s.get("D2L", !legacyKnob && (k <= 4096 || !oneRound || shift256)) && !ta && (tb || s.get("BTR", 1)) && n % 16 == 0 && bm == 256 && bn == 256 && bk == 128 && wm == 4 && wn == 2 &&
+      ((m % 256 == 0 && n % 256 == 0) || shift256) && k % 128 == 0) {
     const int64_t scalePtr = s.get("SCALE_PTR", 0);
     if (scalePtr < 0 || scalePtr > 2) { err = "gemm_fp8: SCALE_PTR is 0 (scalar arguments), 1 (A, B, C, pointers) or 2 (A, B, pointers, C)"; return false; }
     const bool outBf16 = s.get("OUT_BF16", 0) != 0;
@@ -816,7 +845,7 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     // same columns of B at the same time (4096 x 11008 x 4096, two rows: 0.160 against 0.168 ms with strips of eight,
     // 0.164 with four); four rows otherwise (level with or ahead of eight on every shape measured).
     if (!s.has("GROUP_M")) {
-      const int64_t tm = m / 256, tn = n / 256, run = tm * tn / 8;
+      const int64_t tm = ceilDiv(m, 256), tn = ceilDiv(n, 256), run = tm * tn / 8;
       gm = (tm * tn) % 8 == 0 && run % tn == 0 && run / tn >= 1 && run / tn <= 4 ? run / tn : 4;
     }
     s.p["TA"] = 0; s.p["TB"] = tb; s.p["D2L"] = 1; s.p["BTR"] = !tb;
@@ -829,11 +858,13 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     d.add("G8_RELU", s.get("RELU", 0) ? 1 : 0);
     d.add("G8_SCALE_PTR", scalePtr);
     d.add("G8_BTR", tb ? 0 : 1);
-    const int64_t tilesAll = (m / 256) * (n / 256);
-    const bool persist = s.get("PERSIST", 0) != 0 && batch == 1 && (k / 128) % 2 == 0 && tilesAll > 256;
+    const int64_t tilesAll = ceilDiv(m, 256) * ceilDiv(n, 256);
+    const bool moved = m % 256 || n % 256;
+    if (moved) d.add("G8_SHIFT", 1);
+    const bool persist = s.get("PERSIST", 0) != 0 && !moved && batch == 1 && (k / 128) % 2 == 0 && tilesAll > 256;
     s.p["PERSIST"] = persist;
     if (persist) d.add("G8_PERSIST", 1);
-    const bool rounds = (m / 256) * (n / 256) * batch > 256;                   // more than one round of tiles
+    const bool rounds = tilesAll * batch > 256;                   // more than one round of tiles
     // The results go through LDS and leave as whole rows of the tile (STAGE_C) unless the workgroups are persistent:
     // 4096 x 11008 x 4096 0.151 against 0.160 ms, 2 to 8 % on other shapes of more than one round, level on single
     // rounds.  The staggered start then does best at half its former width.  A bf16 result, of which a lane would
@@ -847,7 +878,7 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     d.add("G8_STAGE_C", stageC);
     src = d.wrap(kTpl_gemm_fp8_d2l);
     info.name = s.name;
-    info.grid[0] = (uint32_t)(persist ? 256 : (m / 256) * (n / 256));
+    info.grid[0] = (uint32_t)(persist ? 256 : tilesAll);
     info.grid[1] = (uint32_t)batch;
     info.block[0] = 512;
     info.numArgs = 5;
@@ -897,6 +928,8 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   const bool pingpong = s.get("PINGPONG", 0) != 0 && bk == 64 && wm * wn == 8 && !guarded && !prefetch && k / bk >= stages + 2;
   s.p["PINGPONG"] = pingpong;
   d.add("GF_PINGPONG", pingpong ? 1 : 0);
+  // guarded loads of whole chunks, where the caller has looked at the operands' addresses
+  if (edge && s.get("ALIGN", 0) >= 16 && k % 16 == 0 && (!ta || m % 16 == 0) && (tb || n % 16 == 0)) d.add("GF_WIDE", 1);
   d.add("GF_BTR", btr ? 1 : 0);
   // where the two per-tensor scales come from: trailing scalars, or one fp32 each in device memory (graph values)
   const int64_t scalePtr = s.get("SCALE_PTR", 0);

@@ -19,6 +19,10 @@
 //   GB_KTAIL                     1: K is no multiple of GB_BK; the last k-tile is moved back likewise (direct loads only)
 //   GB_F16                       1: the operands (and a 16-bit result) are IEEE half instead of bf16; the tiles
 //                                move as 16-bit patterns either way, only the MFMA and the result's rounding differ
+//   GB_FP8                       1: the operands are fp8 e4m3, both contiguous along k, taken in pairs: GB_K counts pairs.
+//                                A lane's 16 bytes of a fragment feed two v_mfma_f32_16x16x32_fp8_fp8, and two fp32
+//                                scales follow C.  Direct loads only: for launches too small for 256 x 256 tiles
+//                                (gemm_fp8_d2l.hip), where the loads and not the MFMAs set the pace
 //   GB_OUT_BF16                  1: C has the operands' 16-bit type, else fp32
 //   GB_RELU                      1: fused max(0, .) epilogue
 //   GB_STAGE_C                   1: results are turned round in LDS and stored as whole rows of the tile (see the
@@ -309,7 +313,25 @@ struct KcgTLoader {
 #define GB_SETPRIO 0
 #define GB_SETPRIO_DEFAULTED 1
 #endif
-#if GB_F16
+#ifndef GB_FP8
+#define GB_FP8 0
+#define GB_FP8_DEFAULTED 1
+#endif
+#if GB_FP8
+#ifndef KCG_GEMM16_FP8
+#define KCG_GEMM16_FP8
+__device__ __forceinline__ kcg_f32x4 kcg_mfma_fp8_pairs(kcg_i32x4 a, kcg_i32x4 b, kcg_f32x4 c) {
+  typedef long kcg_i64x2 __attribute__((ext_vector_type(2)));
+  const kcg_i64x2 x = __builtin_bit_cast(kcg_i64x2, a), y = __builtin_bit_cast(kcg_i64x2, b);
+  c = __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(x[0], y[0], c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_fp8_fp8(x[1], y[1], c, 0, 0, 0);
+}
+#endif
+#define GB_FRAG kcg_i32x4
+#define GB_MFMA(a, b, c, x, y, z) kcg_mfma_fp8_pairs(a, b, c)
+#define GB_TO16(x) ((kcg_u16)kcg_f32_to_bf16_bits(x))
+#define GB_SCALED(x) ((x) * scale)
+#elif GB_F16
 typedef _Float16 kcg_f16x8 __attribute__((ext_vector_type(8)));
 #define GB_FRAG kcg_f16x8
 #if GB_M16
@@ -326,6 +348,12 @@ typedef _Float16 kcg_f16x8 __attribute__((ext_vector_type(8)));
 #define GB_MFMA __builtin_amdgcn_mfma_f32_32x32x16_bf16
 #endif
 #define GB_TO16(x) ((kcg_u16)kcg_f32_to_bf16_bits(x))
+#endif
+#if !GB_FP8
+#define GB_SCALED(x) (x)
+#endif
+#if GB_FP8 && (!GB_D2L || GB_BTR)
+#error "fp8 operands: only with direct loads, both contiguous along k"
 #endif
 #ifndef GB_SK_UNITS
 #define GB_SK_UNITS 0
@@ -376,6 +404,9 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #if GB_SK_UNITS > 0
              , unsigned* __restrict__ W
 #endif
+#if GB_FP8
+             , float scale_a, float scale_b
+#endif
 ) {
   __shared__ __attribute__((aligned(16))) char kcg_smem[GB_NBUF * (GB_BM * GB_ROWB + GB_BBUF)];
 #if GB_SK_UNITS > 0
@@ -393,6 +424,9 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
     const int steps = (int)((blockIdx.x >> 3) & 7) * GB_STAGGER;
     for (int d = 0; d < steps; ++d) __builtin_amdgcn_s_sleep(64);
   }
+#endif
+#if GB_FP8
+  const float scale = scale_a * scale_b;
 #endif
   const int tiles_m = (GB_M + GB_BM - 1) / GB_BM;
   const int tiles_n = (GB_N + GB_BN - 1) / GB_BN;
@@ -995,7 +1029,7 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
             const int i = pass * (GB_TM / PASSES) + ii;
-            const float r = GB_RELU ? fmaxf(acc[i][j][v], 0.0f) : acc[i][j][v];
+            const float r = GB_RELU ? fmaxf(GB_SCALED(acc[i][j][v]), 0.0f) : GB_SCALED(acc[i][j][v]);
             const int row = wm * (GB_WTM / PASSES) + 16 * ii + 4 * lq + v, col = wn * GB_WTN + 16 * j + l16;
 #if GB_OUT_BF16
             stage[row * 256 + (col ^ (16 * lq))] = GB_TO16(r);
@@ -1038,9 +1072,9 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #endif
         {
 #if GB_OUT_BF16
-          C[(long)row * GB_N + col] = GB_TO16(GB_RELU ? fmaxf(acc[i][j][v], 0.0f) : acc[i][j][v]);
+          C[(long)row * GB_N + col] = GB_TO16(GB_RELU ? fmaxf(GB_SCALED(acc[i][j][v]), 0.0f) : GB_SCALED(acc[i][j][v]));
 #else
-          C[(long)row * GB_N + col] = GB_RELU ? fmaxf(acc[i][j][v], 0.0f) : acc[i][j][v];
+          C[(long)row * GB_N + col] = GB_RELU ? fmaxf(GB_SCALED(acc[i][j][v]), 0.0f) : GB_SCALED(acc[i][j][v]);
 #endif
         }
       }
@@ -1120,6 +1154,11 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #undef GB_FRAG
 #undef GB_MFMA
 #undef GB_TO16
+#undef GB_SCALED
+#ifdef GB_FP8_DEFAULTED
+#undef GB_FP8
+#undef GB_FP8_DEFAULTED
+#endif
 #ifdef GB_F16_DEFAULTED
 #undef GB_F16
 #undef GB_F16_DEFAULTED

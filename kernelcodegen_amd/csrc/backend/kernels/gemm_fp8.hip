@@ -9,6 +9,9 @@
 //   GF_WM GF_WN                  wavefronts along M and N; block = 64*GF_WM*GF_WN
 //   GF_GROUP_M                   tile rows per L2 strip
 //   GF_EDGE                      1: ragged tiles, guard loads and stores
+//   GF_WIDE                      1: every row of both operands is whole 16-byte chunks on 16-byte boundaries: a guarded load
+//                                takes or leaves a chunk as a whole (byte by byte otherwise: 16 x 11008 x 4096 with
+//                                row-major weights 137 us, 19 us in chunks)
 //   GF_OUT_BF16                  1: C is bf16, else fp32
 //   GF_RELU                      1: fused max(0, .) epilogue
 //   GF_STAGES                    1 or 2 sets of staging registers = tiles in flight from global memory
@@ -39,7 +42,7 @@
 template <bool B> struct KcgBool8 { static constexpr bool v = B; };
 
 // 16-byte chunks (16 fp8 values), contiguous along k in global memory.
-template <int ROWS, int BK, int NT, bool GUARD>
+template <int ROWS, int BK, int NT, int GUARD>
 struct KcgKLoader8 {
   static constexpr int CPR = BK / 16;
   static constexpr int CHUNKS = ROWS * CPR;
@@ -62,6 +65,10 @@ struct KcgKLoader8 {
       const unsigned char* p = g + (long)(row0 + rr) * ld + (k0 + c * 16);
       if (!GUARD) {
         v = *(const kcg_u32x4*)p;
+      } else if (GUARD == 2) {
+        const bool in = row0 + rr < row_lim && k0 + c * 16 < k_lim;
+        const kcg_u32x4 t = *(const kcg_u32x4*)(in ? p : g);      // the operand's first chunk in the place of one outside
+        v = in ? t : v;
       } else if (row0 + rr < row_lim) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
@@ -86,7 +93,7 @@ struct KcgKLoader8 {
 // bytes.  KR = 8 when such blocks keep at least half the lanes busy, else 4: with eight rows a wavefront's load
 // covers 64 bytes of each row instead of 32 (6 % on the 4096 x 11008 x 4096 product with operands in HBM) and
 // its 8-byte LDS stores stay conflict free, at the price of idle lanes.
-template <int COLS, int BK, int NT, bool GUARD>
+template <int COLS, int BK, int NT, int GUARD>
 struct KcgTLoader8 {
   static constexpr int KR = ((BK / 8) * (COLS / 16) * 2 >= NT) ? 8 : 4;
   static constexpr int KB = BK / KR;
@@ -105,6 +112,10 @@ struct KcgTLoader8 {
         const unsigned char* p = g + (long)k * ld + (col0 + cb * 16);
         if (!GUARD) {
           v = *(const kcg_u32x4*)p;
+        } else if (GUARD == 2) {
+          const bool in = k < k_lim && col0 + cb * 16 < col_lim;
+          const kcg_u32x4 t = *(const kcg_u32x4*)(in ? p : g);
+          v = in ? t : v;
         } else if (k < k_lim) {
 #pragma unroll
           for (int j = 0; j < 16; ++j) {
@@ -180,7 +191,15 @@ __device__ __forceinline__ kcg_i32x8 kcg_ld32(const char* p) {
 #define GF_BROWB (GF_BN + 32)
 #define GF_SB_BYTES (GF_BTR ? 2 * GF_BK * GF_BROWB : 2 * GF_BN * GF_ROWB)
 #define GF_KT ((GF_K + GF_BK - 1) / GF_BK)
-#define GF_GUARD ((GF_EDGE != 0) | ((GF_K % 16) != 0) | ((GF_TA != 0) & ((GF_M % 16) != 0)) | ((GF_TB == 0) & ((GF_N % 16) != 0)))
+#ifndef GF_WIDE
+#define GF_WIDE 0
+#define GF_WIDE_DEFAULTED
+#endif
+#if GF_WIDE && (GF_K % 16 || (GF_TA && GF_M % 16) || (!GF_TB && GF_N % 16))
+#error "gemm_fp8: guarded loads in chunks need rows of whole 16-byte chunks"
+#endif
+#define GF_GUARD ((GF_WIDE + 1) * GF_GUARDED)
+#define GF_GUARDED ((GF_EDGE != 0) | ((GF_K % 16) != 0) | ((GF_TA != 0) & ((GF_M % 16) != 0)) | ((GF_TB == 0) & ((GF_N % 16) != 0)))
 
 #if (GF_BM % (32 * GF_WM)) || (GF_BN % (32 * GF_WN)) || (GF_BK % 64)
 #error "tile shape does not divide into 32x32x64 MFMA tiles"
@@ -574,6 +593,11 @@ void GF_NAME(const unsigned char* __restrict__ A, const unsigned char* __restric
 #undef GF_BTR
 #undef GF_KT
 #undef GF_GUARD
+#undef GF_GUARDED
+#ifdef GF_WIDE_DEFAULTED
+#undef GF_WIDE
+#undef GF_WIDE_DEFAULTED
+#endif
 #undef GF_C_T
 #ifdef GF_SCALE_PTR_DEFAULTED
 #undef GF_SCALE_PTR

@@ -4,6 +4,8 @@
 // gemm_fp8.hip for every other case).  Parameters:
 //   G8_NAME                      kernel symbol
 //   G8_M G8_N G8_K G8_BATCH      problem: multiples of 256, 256 and 128
+//   G8_SHIFT                     1: M and N are at least 256 and N a multiple of 16; the last tile of a row or column of tiles
+//                                is moved back to end at the edge and stores only what the tile before it does not own
 //   G8_GROUP_M                   tile rows per L2 strip
 //   G8_OUT_BF16                  1: C is bf16, else fp32
 //   G8_RELU                      1: fused max(0, .) epilogue
@@ -48,7 +50,11 @@ template <bool B> struct KcgBool8d { static constexpr bool v = B; };
 #define G8_SCALE_PTR 0
 #define G8_SCALE_PTR_DEFAULTED
 #endif
-#if (G8_M % 256) || (G8_N % 256) || (G8_K % 128)
+#ifndef G8_SHIFT
+#define G8_SHIFT 0
+#define G8_SHIFT_DEFAULTED
+#endif
+#if (G8_SHIFT ? (G8_M < 256 || G8_N < 256 || G8_N % 16) : ((G8_M % 256) || (G8_N % 256))) || (G8_K % 128)
 #error "gemm_fp8_d2l: whole 256 x 256 x 128 tiles only"
 #endif
 #if G8_OUT_BF16
@@ -79,6 +85,9 @@ template <bool B> struct KcgBool8d { static constexpr bool v = B; };
 #ifndef G8_STAGE_C
 #define G8_STAGE_C 0
 #define G8_STAGE_C_DEFAULTED
+#endif
+#if G8_SHIFT && (G8_PERSIST || !G8_STAGE_C)
+#error "gemm_fp8_d2l: moved-back tiles store whole rows (G8_STAGE_C), one workgroup per tile"
 #endif
 #if G8_STAGE_C && G8_PERSIST
 #error "gemm_fp8_d2l: results do not go through LDS with persistent workgroups (whose LDS holds the next tile by then)"
@@ -121,12 +130,18 @@ void G8_NAME(const unsigned char* __restrict__ A, const unsigned char* __restric
     for (int d = 0; d < steps; ++d) __builtin_amdgcn_s_sleep(8);
   }
 #endif
-  const int tiles_m = G8_M / 256, tiles_n = G8_N / 256;
+  const int tiles_m = (G8_M + 255) / 256, tiles_n = (G8_N + 255) / 256;
   int tile_m, tile_n;
   kcg_tile_coords(blockIdx.x, tiles_m, tiles_n, G8_GROUP_M, tile_m, tile_n);
   // (the division in kcg_tile_coords runs on the vector unit: the tile origins go back into scalar registers here, the
   // load instructions below take their base addresses from there)
   int m0 = __builtin_amdgcn_readfirstlane(tile_m * 256), n0 = __builtin_amdgcn_readfirstlane(tile_n * 256);
+#if G8_SHIFT
+  // 2000 x 11008 x 4096, bf16 result: 272 us with guarded loads (gemm_fp8.hip), 96 us this way
+  const int m_own = m0, n_own = n0;                        // first row and column that this tile stores
+  if (m0 + 256 > G8_M) m0 = G8_M - 256;
+  if (n0 + 256 > G8_N) n0 = G8_N - 256;
+#endif
   // Persistent workgroups.  The k-tiles of a workgroup's consecutive output tiles form one stream: the loads of the next
   // output tile's first k-tiles are issued behind the barriers of this one's last two, its first fragments are read
   // under this one's last MFMAs, and only then are the results stored: the stores drain while the next tile multiplies,
@@ -155,6 +170,9 @@ void G8_NAME(const unsigned char* __restrict__ A, const unsigned char* __restric
   // sixteen rows that the transposing reads of two lane groups take together (k0 .. k0 + 7 and k0 + 16 .. k0 + 23) then
   // fall on sixteen different groups of four banks.  For lane i of block 4 wave + t: f = i / 16 + 4 (t % 2) + 8 (wave % 2).
   const unsigned dma_lane_b = (unsigned)(lane >> 4) * (unsigned)G8_N + (unsigned)((((lane & 15) ^ (lane >> 4)) ^ (8 * (wave & 1))) * 16);
+  // odd blocks: granule 4 further on, one address bit where the rows are whole 128-byte lines
+  const unsigned dma_lane_b1 = G8_N % 128 == 0 ? dma_lane_b ^ 64u
+                                               : (unsigned)(lane >> 4) * (unsigned)G8_N + (unsigned)((((lane & 15) ^ (lane >> 4)) ^ (8 * (wave & 1)) ^ 4) * 16);
   const unsigned char* rowsB = B + (long)(wave_u * 16) * G8_N + n0;
   const unsigned char* rowsBn = B + (long)(wave_u * 16) * G8_N + n0n;
 #else
@@ -171,7 +189,7 @@ void G8_NAME(const unsigned char* __restrict__ A, const unsigned char* __restric
     const unsigned char* rB = nxt ? rowsBn : rowsB;
 #if G8_BTR
     const unsigned char* base = u < 4 ? rA + (long)t * 8 * G8_K + (long)kt * 128 : rB + ((long)kt * 128 + t * 4) * G8_N;
-    const unsigned lane_off = (u < 4 ? dma_lane : dma_lane_b) ^ (unsigned)((t & 1) * 64);
+    const unsigned lane_off = u < 4 ? dma_lane ^ (unsigned)((t & 1) * 64) : (t & 1) ? dma_lane_b1 : dma_lane_b;
 #else
     const unsigned char* base = (u < 4 ? rA : rB) + (long)t * 8 * G8_K + (long)kt * 128;
     const unsigned lane_off = dma_lane ^ (unsigned)((t & 1) * 64);
@@ -353,6 +371,9 @@ void G8_NAME(const unsigned char* __restrict__ A, const unsigned char* __restric
           const int col = (lane % LPR) * EPL;
           const kcg_f32x4 val = *(const kcg_f32x4*)(stage + row * 256 + (col ^ (16 * ((row >> 2) & 3))));
           const int trow = PASSES == 2 ? (row >> 5) * 64 + 32 * pass + (row & 31) : row;
+#if G8_SHIFT
+          if (m0 + trow < m_own || n0 + col < n_own) continue;                // (N % 16 == 0: whole pieces)
+#endif
           G8_C_T* at = C + (long)(m0 + trow) * G8_N + n0 + col;
 #if G8_NT_STORE
           __builtin_nontemporal_store(val, (kcg_f32x4*)at);
@@ -394,6 +415,10 @@ void G8_NAME(const unsigned char* __restrict__ A, const unsigned char* __restric
 #ifdef G8_SCALE_PTR_DEFAULTED
 #undef G8_SCALE_PTR
 #undef G8_SCALE_PTR_DEFAULTED
+#endif
+#ifdef G8_SHIFT_DEFAULTED
+#undef G8_SHIFT
+#undef G8_SHIFT_DEFAULTED
 #endif
 #ifdef G8_BTR_DEFAULTED
 #undef G8_BTR

@@ -104,7 +104,7 @@ def matmul_fp8(a, b, scale_a, scale_b, trans_a=False, trans_b=True, out_dtype=to
     if k != k2:
         raise ValueError("incompatible K dimensions")
     kern = R.get_kernel("gemm_fp8", M=m, N=n, K=k, BATCH=batch, TA=int(trans_a), TB=int(trans_b),
-                        OUT_BF16=int(out_dtype == torch.bfloat16), **cfg)
+                        OUT_BF16=int(out_dtype == torch.bfloat16), ALIGN=_aligned(a, b), **cfg)
     c = torch.empty(tuple(a.shape[:-2]) + (m, n), dtype=out_dtype, device=a.device)
     kern.launch(a, b, c, float(scale_a), float(scale_b))
     return c

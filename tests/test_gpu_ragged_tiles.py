@@ -97,3 +97,33 @@ def test_gemm16_infinities_stay_in_their_rows_and_columns(ops, tb):
     want = a.double().cpu() @ (b.t() if tb else b).double().cpu()
     assert not torch.isnan(want).any()
     assert torch.equal(ops.matmul(a, b, trans_b=tb).double().cpu(), want)
+
+
+@pytest.mark.parametrize("tb", [True, False])
+@pytest.mark.parametrize("m,n,k", [(257, 272, 128), (511, 528, 384), (300, 5008, 256), (1000, 4112, 1040), (16, 512, 512), (1, 528, 2048),
+                                   (65, 80, 144), (130, 1040, 400), (700, 2064, 272), (64, 64, 128)])
+def test_gemm_fp8_default_forms(ops, m, n, k, tb):
+    """Moved-back 256 x 256 tiles, the ring of LDS buffers (weights contiguous along k) and guarded loads of whole chunks;
+    products up to 16 and |sum| <= 16 k < 2^16 stay exact in every MFMA's accumulator."""
+    a, b, want = _operands(m, n, k, tb, torch.float8_e4m3fn, m + n + k)
+    for out in (torch.float32, torch.bfloat16):
+        c = ops.matmul_fp8(a, b, 0.5, 2.0, trans_b=tb, out_dtype=out)
+        assert torch.equal(c.cpu(), torch.from_numpy(want).to(out))
+    for x, w in ((_shifted(a), b), (a, _shifted(b))):
+        assert torch.equal(ops.matmul_fp8(x, w, 1.0, 1.0, trans_b=tb).double().cpu(), torch.from_numpy(want))
+
+
+@pytest.mark.parametrize("ta,tb", [(True, False), (True, True)])
+def test_gemm_fp8_chunks_of_a_column_major_operand(ops, ta, tb):
+    m, n, k = 80, 96, 208
+    a, b, want = _operands(m, n, k, tb, torch.float8_e4m3fn, 9)
+    at = a.view(torch.uint8).t().contiguous().view(torch.float8_e4m3fn)
+    assert torch.equal(ops.matmul_fp8(at, b, 1.0, 1.0, trans_a=ta, trans_b=tb).double().cpu(), torch.from_numpy(want))
+
+
+def test_gemm_fp8_large_tiles_moved_back(ops):
+    for tb in (True, False):
+        for (m, n, k) in [(4001, 4128, 128), (2000, 5008, 256)]:
+            a, b, want = _operands(m, n, k, tb, torch.float8_e4m3fn, m)
+            c = ops.matmul_fp8(a, b, 1.0, 1.0, trans_b=tb, out_dtype=torch.float32)
+            assert torch.equal(c.double().cpu(), torch.from_numpy(want))
