@@ -425,6 +425,31 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     if (m < t || n < t) continue;
     if ((double)ceilDiv(m, t) * (double)ceilDiv(n, t) * (double)batch >= 256.0) { tile = t; break; }
   }
+  // Sizes that this tile does not divide, and a B contiguous along k for the direct loads, get the tile of least work instead:
+  // rounds of 256 tiles times the tile's area, weighted by the rate it reaches (4000 x 4096 x 4096: 256 912 us, 128 928, 64
+  // 971).  The last tiles are moved back (no guards), so small tiles cost little and leave little idle.  Direct loads need rows
+  // of whole 16-byte chunks and a caller who has looked at the operands' addresses (ALIGN = 16); us, against guarded 256 or 128
+  // tiles: 16 x 777 x 1000 x 500 118 and 167, 2 x 1100 x 1300 x 900 50 and 65, 1500 x 2048 x 300 19 and 24; 2048 x 1984 x
+  // 1088 takes 128: 68 and 78.  Rows of any length, through registers: 1501 x 2047 x 303 21 and 31, 777 x 1003 x 501 13 and 23.
+  // k-tiles of 32 for 64 x 64 direct-load tiles whose rows are then whole 128-byte lines (1024^3 with a k-contiguous B: 18.8
+  // us, 16 21.4), else of 16 (K 500, 777 x 1000: 16 11.8 us, 32 20.4: every row of a k-tile of 32 straddles two lines).
+  bool own = false;
+  for (const char* key : {"BM", "BN", "BK", "WM", "WN", "WK", "NBUF", "PAD"}) own = own || s.has(key);
+  const bool direct = s.get("D2L", 1) != 0 && s.get("ALIGN", 0) >= 16 && !s.get("TA", 0) && k % 4 == 0 && (s.get("TB", 0) || n % 4 == 0);
+  const bool divides = m % tile == 0 && n % tile == 0 && k % (tile <= 128 ? 32 : 16) == 0;
+  if (!own && (!divides || (direct && s.get("TB", 0))) && m >= 64 && n >= 64 && k >= 16) {
+    static const struct { int64_t t; double weight; } sizes[] = {{256, 0.985}, {128, 1.0}, {64, 1.06}};
+    double least = 0.0;
+    for (const auto& z : sizes) {
+      if (m < z.t || n < z.t) continue;
+      const double work = std::ceil((double)ceilDiv(m, z.t) * (double)ceilDiv(n, z.t) * (double)batch / 256.0) * (double)(z.t * z.t) * z.weight;
+      if (least == 0.0 || work < least) { least = work; tile = z.t; }
+    }
+    s.p["BM"] = s.p["BN"] = tile;
+    s.p["BK"] = direct ? (tile == 64 && k % 32 == 0 ? 32 : 16) : (tile == 128 ? 32 : 16);
+    s.p["WM"] = s.p["WN"] = tile == 64 ? 2 : 4;
+    if (s.get("TB", 0)) { s.p["WK"] = 1; s.p["NBUF"] = 2; }    // two wavefront groups gain nothing where B is read 16 bytes at a time (19.9 us at 1024^3)
+  }
   int64_t bm = s.get("BM", tile), bn = s.get("BN", tile);
   int64_t bk = s.get("BK", bm <= 128 && bn <= 128 ? 32 : 16);
   int64_t wm = s.get("WM", bm >= 128 ? 4 : 2), wn = s.get("WN", bn >= 128 ? 4 : 2), gm = s.get("GROUP_M", 8);
@@ -437,8 +462,10 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   s.p["BM"] = bm; s.p["BN"] = bn; s.p["BK"] = bk; s.p["WM"] = wm; s.p["WN"] = wn; s.p["GROUP_M"] = gm;
 
   // Whole tiles with BK = 16 or 32 of two row-major operands: the kernel that loads both tiles straight into LDS
-  // (kernels/gemm_f32_d2l.hip)
-  const bool d2l = s.get("D2L", 1) != 0 && !s.get("TA", 0) && !s.get("TB", 0) && (bk == 16 || bk == 32) && !edge && bm % 64 == 0 &&
+  // (kernels/gemm_f32_d2l.hip).  Where the caller has looked at the operands' addresses (ALIGN = 16) and rows are whole
+  // 16-byte chunks, also a B that is contiguous along k, and sizes that the tiles do not divide.
+  const bool aligned = s.get("ALIGN", 0) >= 16 && k % 4 == 0 && (s.get("TB", 0) || n % 4 == 0) && m >= bm && n >= bn && k >= bk;
+  const bool d2l = s.get("D2L", 1) != 0 && !s.get("TA", 0) && (!s.get("TB", 0) || aligned) && (bk == 16 || bk == 32) && (!edge || aligned) && bm % 64 == 0 &&
                    (bn == 64 || bn == 128 || bn == 256) && bm % (32 * wm) == 0 && bn % (32 * wn) == 0 && (bm + bn) * bk * 8 <= 160 * 1024;
   s.p["D2L"] = d2l;
   // WK = 2: two groups of WM x WN wavefronts split the steps of every k-tile and add their partial sums through LDS at
@@ -447,7 +474,7 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // 64 x 64 x 32 tiles of four wavefronts on a launch that gives a CU at most one workgroup: two groups and three buffers
   // (1024^3: 19.7 against 20.7-21.1 us, 512 x 512 x 2048: 35.6 against 37.8 us; either one alone is slower, 22.5 and 23.7 us;
   // with several workgroups per CU, 1536^3, the groups change nothing and the launch keeps the plain form)
-  const bool small = wkFits && bm == 64 && bn == 64 && wm * wn == 4 && (m / bm) * (n / bn) * batch <= 256;
+  const bool small = wkFits && bm == 64 && bn == 64 && wm * wn == 4 && ceilDiv(m, bm) * ceilDiv(n, bn) * batch <= 256;
   const int64_t wk = s.get("WK", small ? 2 : 1);
   if (wk != 1 && !(wk == 2 && wkFits)) { err = "gemm_f32: WK is 1 or 2; 2 needs whole tiles of two row-major operands, BK = 32, at most eight wavefronts per group and BM * BN <= 64 (BM + BN)"; return false; }
   s.p["WK"] = wk;
@@ -469,9 +496,12 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     d.add("GL_NBUF", nbuf);
     d.add("GL_GROUP_M", gm);
     d.add("GL_RELU", s.get("RELU", 0) ? 1 : 0);
+    if (m % bm || n % bn) d.add("GL_SHIFT", 1);
+    if (k % bk) d.add("GL_KTAIL", 1);
+    if (s.get("TB", 0)) d.add("GL_TB", 1);
     src = d.wrap(kTpl_gemm_f32_d2l);
     info.name = s.name;
-    info.grid[0] = (uint32_t)((m / bm) * (n / bn));
+    info.grid[0] = (uint32_t)(ceilDiv(m, bm) * ceilDiv(n, bn));
     info.grid[1] = (uint32_t)batch;
     info.block[0] = (uint32_t)(64 * wm * wn * wk);
     info.numArgs = 3;
@@ -486,7 +516,12 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   d.add("GM_TA", s.get("TA", 0) ? 1 : 0); d.add("GM_TB", s.get("TB", 0) ? 1 : 0);
   d.add("GM_BM", bm); d.add("GM_BN", bn); d.add("GM_BK", bk);
   d.add("GM_WM", wm); d.add("GM_WN", wn); d.add("GM_GROUP_M", gm);
-  d.add("GM_EDGE", edge ? 1 : 0);
+  // Ragged sizes that hold a whole tile: the last tiles are moved back (any row length: a 16-byte load of floats needs an
+  // alignment of four bytes, which every float has)
+  const bool shift = edge && m >= bm && n >= bn;
+  d.add("GM_EDGE", edge && !shift ? 1 : 0);
+  if (shift) d.add("GM_SHIFT", 1);
+  s.p["SHIFT"] = shift;
   d.add("GM_RELU", s.get("RELU", 0) ? 1 : 0);
   d.add("GM_PAD", pad);
   src = d.wrap(kTpl_gemm_f32);

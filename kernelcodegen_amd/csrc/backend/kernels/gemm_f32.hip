@@ -8,6 +8,9 @@
 //   GM_WM GM_WN                  wavefronts along M and N; block = 64*GM_WM*GM_WN
 //   GM_GROUP_M                   tile rows per L2 strip
 //   GM_EDGE                      1: some tile is ragged, guard loads and stores
+//   GM_SHIFT                     1: M or N is no multiple of the tile (but both hold a whole one): the last tile of a row or
+//                                column of tiles is moved back to end at the edge and stores only what the tile before it
+//                                does not own, so that only the last k-tile's loads are guarded (GM_EDGE is 0 then)
 //   GM_RELU                      1: fused max(0, .) epilogue
 //
 // LDS holds both operand tiles k-major, sA[k][m] and sB[k][n], double buffered.
@@ -17,6 +20,19 @@
 // spreads the transposing stores of a k-contiguous operand over the banks.
 // Lane l, accumulator register v of a 32x32 tile hold
 //   row 8*(v/4) + 4*(l/32) + v%4, column l%32.
+#ifndef GM_SHIFT
+#define GM_SHIFT 0
+#define GM_SHIFT_DEFAULTED
+#endif
+#if GM_SHIFT && (GM_EDGE || GM_M < GM_BM || GM_N < GM_BN)
+#error "gemm_f32: moved-back tiles must fit the operands"
+#endif
+// rows of any length start on 4 bytes only, which is all that a 16-byte load of floats needs; spelled out where it matters
+#ifndef KCG_GEMM32_HELPERS
+#define KCG_GEMM32_HELPERS
+typedef float kcg_f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+#endif
+#define GM_KGUARD (GM_SHIFT && GM_K % GM_BK != 0)
 #define GM_NT (64 * GM_WM * GM_WN)
 #define GM_WTM (GM_BM / GM_WM)
 #define GM_WTN (GM_BN / GM_WN)
@@ -52,8 +68,14 @@ void GM_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
   const int tiles_n = (GM_N + GM_BN - 1) / GM_BN;
   int tile_m, tile_n;
   kcg_tile_coords(blockIdx.x, tiles_m, tiles_n, GM_GROUP_M, tile_m, tile_n);
+#if GM_SHIFT
+  const int m_own = tile_m * GM_BM, n_own = tile_n * GM_BN;
+  const int m0 = m_own + GM_BM <= GM_M ? m_own : GM_M - GM_BM;
+  const int n0 = n_own + GM_BN <= GM_N ? n_own : GM_N - GM_BN;
+#else
   const int m0 = tile_m * GM_BM;
   const int n0 = tile_n * GM_BN;
+#endif
   const long batch = blockIdx.y;
   A += batch * (long)GM_M * GM_K;
   B += batch * (long)GM_K * GM_N;
@@ -63,6 +85,9 @@ void GM_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
 
   // ---- global -> registers (one k-tile of A and of B) ----
   auto load_tiles = [&](int k0) {
+#if GM_SHIFT
+    const bool tail = GM_KGUARD && k0 + GM_BK > GM_K;      // the last k-tile: values of k past the end read as zero
+#endif
 #pragma unroll
     for (int i = 0; i < GM_AV; ++i) {
       const int q = i * GM_NT + tid;
@@ -71,7 +96,14 @@ void GM_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
 #if GM_TA == 0
         const int r = q / (GM_BK / 4), kc = (q % (GM_BK / 4)) * 4;   // 4 along k
         const float* p = A + (long)(m0 + r) * GM_K + (k0 + kc);
-#if GM_EDGE || (GM_K % 4)
+#if GM_SHIFT
+        if (!tail) {
+          v = *(const kcg_f32x4_any*)p;
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) if (k0 + kc + j < GM_K) v[j] = p[j];
+        }
+#elif GM_EDGE || (GM_K % 4)
         if (m0 + r < GM_M) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) if (k0 + kc + j < GM_K) v[j] = p[j];
@@ -82,7 +114,9 @@ void GM_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
 #else
         const int kk = q / (GM_BM / 4), mc = (q % (GM_BM / 4)) * 4;   // 4 along m
         const float* p = A + (long)(k0 + kk) * GM_M + (m0 + mc);
-#if GM_EDGE || (GM_M % 4)
+#if GM_SHIFT
+        if (!tail || k0 + kk < GM_K) v = *(const kcg_f32x4_any*)p;
+#elif GM_EDGE || (GM_M % 4)
         if (k0 + kk < GM_K) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) if (m0 + mc + j < GM_M) v[j] = p[j];
@@ -102,7 +136,9 @@ void GM_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
 #if GM_TB == 0
         const int kk = q / (GM_BN / 4), nc = (q % (GM_BN / 4)) * 4;   // 4 along n
         const float* p = B + (long)(k0 + kk) * GM_N + (n0 + nc);
-#if GM_EDGE || (GM_N % 4)
+#if GM_SHIFT
+        if (!tail || k0 + kk < GM_K) v = *(const kcg_f32x4_any*)p;
+#elif GM_EDGE || (GM_N % 4)
         if (k0 + kk < GM_K) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) if (n0 + nc + j < GM_N) v[j] = p[j];
@@ -113,7 +149,14 @@ void GM_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
 #else
         const int r = q / (GM_BK / 4), kc = (q % (GM_BK / 4)) * 4;   // 4 along k
         const float* p = B + (long)(n0 + r) * GM_K + (k0 + kc);
-#if GM_EDGE || (GM_K % 4)
+#if GM_SHIFT
+        if (!tail) {
+          v = *(const kcg_f32x4_any*)p;
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) if (k0 + kc + j < GM_K) v[j] = p[j];
+        }
+#elif GM_EDGE || (GM_K % 4)
         if (n0 + r < GM_N) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) if (k0 + kc + j < GM_K) v[j] = p[j];
@@ -228,12 +271,19 @@ void GM_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
 #endif
 #if GM_EDGE
         if (row < GM_M && col < GM_N)
+#elif GM_SHIFT
+        if (row >= m_own && col >= n_own)
 #endif
           C[(long)row * GM_N + col] = o;
       }
     }
 }
 #undef GM_NT
+#undef GM_KGUARD
+#ifdef GM_SHIFT_DEFAULTED
+#undef GM_SHIFT
+#undef GM_SHIFT_DEFAULTED
+#endif
 #undef GM_WTM
 #undef GM_WTN
 #undef GM_TM

@@ -1,8 +1,14 @@
 // ---- fp32 GEMM on v_mfma_f32_32x32x2_f32, operand tiles straight from global memory into LDS ----------------------
-// C[b] = A[b] * B[b]: A [M][K], B [K][N], C [M][N], all row-major fp32; whole GL_BM x GL_BN x GL_BK tiles only (the emitter
-// falls back to gemm_f32.hip for every other case).  Parameters:
+// C[b] = A[b] * B[b]: A [M][K], B [K][N] (GL_TB: [N][K]), C [M][N], all row-major fp32; at least one whole
+// GL_BM x GL_BN x GL_BK tile (the emitter falls back to gemm_f32.hip for every other case).  Parameters:
 //   GL_NAME                      kernel symbol
-//   GL_M GL_N GL_K GL_BATCH      problem: multiples of GL_BM, GL_BN and GL_BK
+//   GL_M GL_N GL_K GL_BATCH      problem: multiples of GL_BM, GL_BN and GL_BK unless moved back:
+//   GL_SHIFT                     1: M or N is no multiple of the tile; the last tile of a row or column of tiles is moved back
+//                                to end at the edge and stores only what the tile before it does not own
+//   GL_KTAIL                     1: K is no multiple of GL_BK (but of four); the last k-tile starts at K - GL_BK, and what the
+//                                tile before it has multiplied already is overwritten with zeros in LDS
+//   GL_TB                        1: B is [N][K]; its tile lies in LDS as A's does, and a lane reads its four k with one
+//                                ds_read_b128
 //   GL_BM GL_BN GL_BK            workgroup tile: GL_BM a multiple of 64, GL_BN 64, 128 or 256, GL_BK 16 or 32
 //   GL_WM GL_WN                  wavefronts along m and n; a wavefront's part of the tile is whole 32 x 32 MFMA tiles
 //   GL_WK                        (1 or 2) groups of GL_WM x GL_WN wavefronts that share the tile's results and split the
@@ -37,10 +43,22 @@
 #define KCG_GEMM32D_HELPERS
 template <bool B> struct KcgBool32d { static constexpr bool v = B; };
 #endif
-#if (GL_M % GL_BM) || (GL_N % GL_BN) || (GL_K % GL_BK) || (GL_BK != 16 && GL_BK != 32)
-#error "gemm_f32_d2l: whole tiles only"
+#ifndef GL_SHIFT
+#define GL_SHIFT 0
+#define GL_SHIFT_DEFAULTED
 #endif
-#if (GL_BM % 64) || (GL_BN != 64 && GL_BN != 128 && GL_BN != 256) || (GL_BM % (32 * GL_WM)) || (GL_BN % (32 * GL_WN))
+#ifndef GL_KTAIL
+#define GL_KTAIL 0
+#define GL_KTAIL_DEFAULTED
+#endif
+#ifndef GL_TB
+#define GL_TB 0
+#define GL_TB_DEFAULTED
+#endif
+#if (GL_SHIFT ? (GL_M < GL_BM || GL_N < GL_BN) : ((GL_M % GL_BM) || (GL_N % GL_BN))) || (GL_KTAIL ? (GL_K < GL_BK || GL_K % GL_BK == 0 || GL_K % 4) : (GL_K % GL_BK != 0)) || (GL_BK != 16 && GL_BK != 32)
+#error "gemm_f32_d2l: whole tiles only, or moved back"
+#endif
+#if (GL_BM % 64) || (GL_BN != 64 && GL_BN != 128 && GL_BN != 256) || (GL_BM % (32 * GL_WM)) || (GL_BN % (32 * GL_WN)) || (GL_TB && GL_BN % (256 / (GL_BK / 4) ))
 #error "gemm_f32_d2l: GL_BM is a multiple of 64, GL_BN 64, 128 or 256 (a 1 KiB block is whole rows of the B tile), 32 x 32 MFMA tiles per wavefront"
 #endif
 #ifndef GL_WK
@@ -58,7 +76,7 @@ template <bool B> struct KcgBool32d { static constexpr bool v = B; };
 #define GL_NBUF 2
 #define GL_NBUF_DEFAULTED
 #endif
-#define GL_KT (GL_K / GL_BK)
+#define GL_KT ((GL_K + GL_BK - 1) / GL_BK)
 #define GL_NG (GL_WM * GL_WN)
 #define GL_NW (GL_NG * GL_WK)
 #define GL_TM (GL_BM / GL_WM / 32)
@@ -85,12 +103,14 @@ void GL_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
   const int wm = (wave % GL_NG) / GL_WN, wn = wave % GL_WN;
   const int l32 = lane & 31, lh = lane >> 5;
 
-  const int tiles_m = GL_M / GL_BM, tiles_n = GL_N / GL_BN;
+  const int tiles_m = (GL_M + GL_BM - 1) / GL_BM, tiles_n = (GL_N + GL_BN - 1) / GL_BN;
   int tile_m, tile_n;
   kcg_tile_coords(blockIdx.x, tiles_m, tiles_n, GL_GROUP_M, tile_m, tile_n);
   // (the division in kcg_tile_coords runs on the vector unit: the tile origins go back into scalar registers here, the
   // load instructions below take their base addresses from there)
-  const int m0 = __builtin_amdgcn_readfirstlane(tile_m * GL_BM), n0 = __builtin_amdgcn_readfirstlane(tile_n * GL_BN);
+  const int m_own = tile_m * GL_BM, n_own = tile_n * GL_BN;            // first row and column that this tile stores
+  const int m0 = __builtin_amdgcn_readfirstlane(!GL_SHIFT || m_own + GL_BM <= GL_M ? m_own : GL_M - GL_BM);
+  const int n0 = __builtin_amdgcn_readfirstlane(!GL_SHIFT || n_own + GL_BN <= GL_N ? n_own : GL_N - GL_BN);
   const long batch = blockIdx.y;
   A += batch * (long)GL_M * GL_K;
   B += batch * (long)GL_K * GL_N;
@@ -99,11 +119,24 @@ void GL_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
   // ---- loads: block b of a k-tile's BLK blocks of 1 KiB (A's sixteen-row groups, then B's groups of 256 / GL_BN rows)
   //      is moved by wavefront b % GL_NW ----
   const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) char*)kcg_smem;
-  // (GL_BK 32: a block is eight rows, and the rows of an odd block are swizzled with 4 more: byte offset ^ 64)
+  // (GL_BK 32: a block is eight rows, and the rows of an odd block are swizzled with 4 more: byte offset ^ 64 where the rows
+  // are whole 128-byte lines)
   const unsigned a_lane = (unsigned)(lane / CH) * (unsigned)(GL_K * 4) + (unsigned)(((lane % CH) ^ ((lane >> 4) & 3)) * 16);
+  const unsigned a_lane1 = (unsigned)(lane / CH) * (unsigned)(GL_K * 4) + (unsigned)(((lane % CH) ^ ((lane >> 4) & 3) ^ 4) * 16);
+#if GL_TB
+  const char* tileB = (const char*)(B + (long)n0 * GL_K);
+#else
   const unsigned b_lane = (unsigned)(lane / (GL_BN / 4)) * (unsigned)(GL_N * 4) + (unsigned)(lane % (GL_BN / 4)) * 16u;
-  const char* tileA = (const char*)(A + (long)m0 * GL_K);
   const char* tileB = (const char*)(B + n0);
+#endif
+  const char* tileA = (const char*)(A + (long)m0 * GL_K);
+  auto a_off = [&](int blk) __attribute__((always_inline)) -> unsigned {
+    return GL_BK == 16 ? a_lane : GL_K % 32 == 0 ? a_lane ^ (unsigned)((blk & 1) * 64) : (blk & 1) ? a_lane1 : a_lane;
+  };
+  // first k of k-tile kt
+  auto kpos = [&](int kt) __attribute__((always_inline)) -> long {
+    return GL_KTAIL && kt == GL_KT - 1 ? (long)(GL_K - GL_BK) : (long)kt * GL_BK;
+  };
   auto dma = [&](int kt, int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int x = 0; x < (BLK + GL_NW - 1) / GL_NW; ++x) {
@@ -113,14 +146,36 @@ void GL_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
         const int bb = blk - BLK_A;                        // B: rows bb * (1024 / ROW_B) .. of the k-tile
         unsigned dst = lds_base + (is_a ? (unsigned)(buf * TILE_A + blk * 1024) : (unsigned)(B_AT + buf * TILE_B + bb * 1024));
         dst = __builtin_amdgcn_readfirstlane(dst);
-        const char* src = is_a ? tileA + (long)blk * (1024 / ROW_A) * GL_K * 4 + (long)kt * ROW_A
-                               : tileB + ((long)kt * GL_BK + (long)bb * (1024 / ROW_B)) * GL_N * 4;
-        const unsigned lane_off = is_a ? (GL_BK == 32 ? a_lane ^ (unsigned)((blk & 1) * 64) : a_lane) : b_lane;
+#if GL_TB
+        const int rb = is_a ? blk : bb;                    // block within its operand
+        const char* src = (is_a ? tileA : tileB) + (long)rb * (1024 / ROW_A) * GL_K * 4 + kpos(kt) * 4;
+        const unsigned lane_off = a_off(rb);
+#else
+        const char* src = is_a ? tileA + (long)blk * (1024 / ROW_A) * GL_K * 4 + kpos(kt) * 4
+                               : tileB + (kpos(kt) + (long)bb * (1024 / ROW_B)) * GL_N * 4;
+        const unsigned lane_off = is_a ? a_off(blk) : b_lane;
+#endif
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                      :: "v"(lane_off), "s"(src), "s"(dst) : "memory");
       }
     }
   };
+
+#if GL_KTAIL
+  // the wavefront's own blocks of the last k-tile, landed: the first KZ values of k become zero, in both operands
+  auto zero_tail = [&](int buf) __attribute__((always_inline)) {
+    constexpr int KZ = GL_BK - GL_K % GL_BK;
+    const kcg_f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int blk = wave_u; blk < BLK; blk += GL_NW) {
+      const bool is_a = blk < BLK_A;
+      const int bb = blk - BLK_A, rb = is_a ? blk : bb;
+      const int chunk = (lane % CH) ^ ((lane >> 4) & 3) ^ (GL_BK == 32 ? (rb & 1) * 4 : 0);
+      const bool out = is_a || GL_TB ? chunk * 4 < KZ : bb * (1024 / ROW_B) + lane / (GL_BN / 4) < KZ;
+      char* dst = kcg_smem + (is_a ? buf * TILE_A + blk * 1024 : B_AT + buf * TILE_B + bb * 1024);
+      if (out) *(kcg_f32x4*)(dst + lane * 16) = zero;
+    }
+  };
+#endif
 
   // ---- fragments of half u of the tile in buffer buf ----
   const int ma = wm * (GL_TM * 32) + l32;                  // the lane's row of A's first block; the next are 32 further each
@@ -128,15 +183,26 @@ void GL_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
   // the swizzle term, which is exact because 2 u, 2 wk and lh occupy different bits, its eight rows of B into the base)
   const int sw = ((ma >> SW_SH) & (CH - 1)) ^ (2 * wk);    // the same for every block: 32 rows further changes nothing
   const char* fA = kcg_smem + ma * ROW_A;
+#if GL_TB
+  const char* fB = kcg_smem + B_AT + (wn * (GL_TN * 32) + l32) * ROW_A;     // row n; swizzled as A's rows are
+#else
   const char* fB = kcg_smem + B_AT + (8 * wk + lh * 4) * ROW_B + (wn * (GL_TN * 32) + l32) * 4;
+#endif
   auto read_fragments = [&](int buf, int u, kcg_f32x4 (&a)[GL_TM], float (&b)[GL_TN][4]) __attribute__((always_inline)) {
     const int pos = ((2 * u + lh) ^ sw) * 16;
 #pragma unroll
     for (int i = 0; i < GL_TM; ++i) a[i] = *(const kcg_f32x4*)(fA + buf * TILE_A + i * 32 * ROW_A + pos);
 #pragma unroll
-    for (int j = 0; j < GL_TN; ++j)
+    for (int j = 0; j < GL_TN; ++j) {
+#if GL_TB
+      const kcg_f32x4 four = *(const kcg_f32x4*)(fB + buf * TILE_B + j * 32 * ROW_A + pos);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) b[j][e] = four[e];
+#else
 #pragma unroll
       for (int e = 0; e < 4; ++e) b[j][e] = *(const float*)(fB + buf * TILE_B + (8 * u + e) * ROW_B + j * 128);
+#endif
+    }
   };
 
   kcg_f32x16 acc[GL_TM][GL_TN];
@@ -177,6 +243,9 @@ void GL_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
         read_fragments(par, (s + 1) * GL_WK, fa[(s + 1) & 1], fb[(s + 1) & 1]);
       } else {
         __builtin_amdgcn_s_waitcnt(0x0F70);                // vmcnt(0): this wavefront's blocks of tile kt+1 have landed
+#if GL_KTAIL
+        if (kt + 2 == GL_KT) zero_tail(par ^ 1);
+#endif
         __syncthreads();                                   // (its wait for LDS covers the last fragment reads of tile kt)
         if (more) read_fragments(par ^ 1, 0, fa[0], fb[0]);     // OWN is even: the step below uses set 1
       }
@@ -217,6 +286,9 @@ void GL_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
         } else {
           if (sent) __builtin_amdgcn_s_waitcnt(0x0F70 | (((GL_NBUF - 2) * PER) & 15) | ((((GL_NBUF - 2) * PER) >> 4) << 14));
           else __builtin_amdgcn_s_waitcnt(0x0F70);         // the last tiles: nothing younger is out, wait for all
+#if GL_KTAIL
+          if (kt + 2 == GL_KT) zero_tail(next);
+#endif
           __syncthreads();
           if (kt + 1 < GL_KT) read_fragments(next, 0, fa[0], fb[0]);
         }
@@ -266,11 +338,26 @@ void GL_NAME(const float* __restrict__ A, const float* __restrict__ B, float* __
 #if GL_RELU
         o = fmaxf(0.0f, o);
 #endif
-        C[(long)row * GL_N + col] = o;
+#if GL_SHIFT
+        if (row >= m_own && col >= n_own)
+#endif
+          C[(long)row * GL_N + col] = o;
       }
     }
 }
 #undef GL_KT
+#ifdef GL_SHIFT_DEFAULTED
+#undef GL_SHIFT
+#undef GL_SHIFT_DEFAULTED
+#endif
+#ifdef GL_KTAIL_DEFAULTED
+#undef GL_KTAIL
+#undef GL_KTAIL_DEFAULTED
+#endif
+#ifdef GL_TB_DEFAULTED
+#undef GL_TB
+#undef GL_TB_DEFAULTED
+#endif
 #undef GL_NW
 #undef GL_NG
 #ifdef GL_WK_DEFAULTED

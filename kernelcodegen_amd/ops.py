@@ -47,10 +47,13 @@ def elementwise(x, op, inplace=False, out_dtype=None, **cfg):
     return y
 
 
-def _aligned(*ts):
-    """16 when every tensor starts on a 16-byte boundary (the kernels' ALIGN parameter): what wide loads and direct loads
-    into LDS need where a size is no multiple of the tile."""
-    return 16 if all(t.data_ptr() % 16 == 0 for t in ts) else 0
+def _aligned(a, b):
+    """True when both operands start on a 16-byte boundary, which the direct loads into LDS need."""
+    return not (a.data_ptr() | b.data_ptr()) & 15
+
+
+def _alignment(aligned):
+    return {"ALIGN": 16} if aligned else {"D2L": 0}
 
 
 _FAMILY = {torch.float32: "gemm_f32", torch.float64: "gemm_f64", torch.bfloat16: "gemm_bf16", torch.float16: "gemm_bf16"}
@@ -76,14 +79,16 @@ def batched_matmul(a, b, trans_a=False, trans_b=False, out_dtype=None, **cfg):
         extra["OUT_BF16"] = int(out_dtype == a.dtype)       # a 16-bit result, of the operands' type
         if a.dtype == torch.float16:
             extra["F16"] = 1
-        extra["ALIGN"] = _aligned(a, b)
+        extra.update(_alignment(_aligned(a, b)))
     elif a.dtype == torch.float64:
         if out_dtype != torch.float64:
             raise ValueError("fp64 GEMM writes fp64")
     elif out_dtype != torch.float32:
         raise ValueError("fp32 GEMM writes fp32")
+    else:
+        extra.update(_alignment(_aligned(a, b)))
     kern = R.get_kernel(_FAMILY[a.dtype], M=m, N=n, K=k, BATCH=batch, TA=int(trans_a), TB=int(trans_b),
-                        **extra, **cfg)
+                        **{**extra, **cfg})
     c = torch.empty(tuple(a.shape[:-2]) + (m, n), dtype=out_dtype, device=a.device)
     kern.launch(a, b, c)
     return c
@@ -104,7 +109,7 @@ def matmul_fp8(a, b, scale_a, scale_b, trans_a=False, trans_b=True, out_dtype=to
     if k != k2:
         raise ValueError("incompatible K dimensions")
     kern = R.get_kernel("gemm_fp8", M=m, N=n, K=k, BATCH=batch, TA=int(trans_a), TB=int(trans_b),
-                        OUT_BF16=int(out_dtype == torch.bfloat16), ALIGN=_aligned(a, b), **cfg)
+                        OUT_BF16=int(out_dtype == torch.bfloat16), **{**_alignment(_aligned(a, b)), **cfg})
     c = torch.empty(tuple(a.shape[:-2]) + (m, n), dtype=out_dtype, device=a.device)
     kern.launch(a, b, c, float(scale_a), float(scale_b))
     return c

@@ -127,3 +127,50 @@ def test_gemm_fp8_large_tiles_moved_back(ops):
             a, b, want = _operands(m, n, k, tb, torch.float8_e4m3fn, m)
             c = ops.matmul_fp8(a, b, 1.0, 1.0, trans_b=tb, out_dtype=torch.float32)
             assert torch.equal(c.double().cpu(), torch.from_numpy(want))
+
+
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("m,n,k", [(64, 64, 16), (65, 68, 20), (777, 1000, 500), (300, 460, 96), (129, 252, 1028), (64, 64, 32), (127, 64, 100),
+                                   (128, 192, 64), (2000, 2000, 48), (1024, 1024, 96), (65, 67, 33), (200, 301, 99), (130, 64, 15), (257, 255, 17),
+                                   (63, 64, 64), (1, 4, 4)])
+def test_gemm_f32_default_forms(ops, m, n, k, tb):
+    """Direct loads with moved-back tiles and k-tiles (rows of whole 16-byte chunks), 16-byte loads at any row length with
+    the last k-tile guarded, and the guarded form where an operand holds no whole tile."""
+    a, b, want = _operands(m, n, k, tb, torch.float32, m + n + k)
+    assert torch.equal(ops.matmul(a, b, trans_b=tb).double().cpu(), torch.from_numpy(want))
+    for x, w in ((_shifted(a), b), (a, _shifted(b))):
+        assert torch.equal(ops.matmul(x, w, trans_b=tb).double().cpu(), torch.from_numpy(want))
+
+
+F32_FORMS = [dict(BM=256, BN=256, BK=16, WM=4, WN=4), dict(BM=128, BN=128, BK=16, WM=4, WN=4), dict(BM=64, BN=64, BK=16, WM=2, WN=2),
+             dict(BM=64, BN=64, BK=32, WM=2, WN=2), dict(BM=64, BN=64, BK=32, WM=2, WN=2, WK=2, NBUF=3), dict(BM=64, BN=64, BK=32, WM=2, WN=2, NBUF=4)]
+
+
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("form", range(len(F32_FORMS)))
+def test_gemm_f32_direct_load_forms_at_their_edges(ops, form, tb):
+    cfg = F32_FORMS[form]
+    bm, bk = cfg["BM"], cfg["BK"]
+    for i, (m, n) in enumerate([(bm, bm), (bm + 1, bm + 4), (2 * bm - 1, 2 * bm - 4)]):
+        for k in (bk, bk + 4, 3 * bk, 5 * bk - 4, 9 * bk):
+            a, b, want = _operands(m, n, k, tb, torch.float32, 100 * form + 10 * i + k, batch=(2,))
+            assert torch.equal(ops.batched_matmul(a, b, trans_b=tb, **cfg).double().cpu(), torch.from_numpy(want)), (m, n, k)
+
+
+@pytest.mark.parametrize("ta,tb", [(True, False), (True, True)])
+def test_gemm_f32_column_major_left_operand(ops, ta, tb):
+    for (m, n, k) in [(70, 75, 33), (131, 129, 50), (64, 200, 19)]:
+        a, b, want = _operands(m, n, k, tb, torch.float32, m)
+        assert torch.equal(ops.matmul(a.t().contiguous(), b, trans_a=True, trans_b=tb).double().cpu(), torch.from_numpy(want))
+
+
+@pytest.mark.parametrize("tb", [False, True])
+def test_gemm_f32_infinities_stay_in_their_rows_and_columns(ops, tb):
+    for (m, n, k) in [(70, 136, 100), (70, 135, 101)]:
+        a, b, _ = _operands(m, n, k, tb, torch.float32, 5)
+        a, b = a.abs() + 1, b.abs() + 1
+        a[3, 90], a[69, 0] = float("inf"), float("inf")
+        b[(7, 85) if tb else (85, 7)] = float("inf")
+        want = a.double().cpu() @ (b.t() if tb else b).double().cpu()
+        assert not torch.isnan(want).any()
+        assert torch.equal(ops.matmul(a, b, trans_b=tb).double().cpu(), want)
