@@ -69,28 +69,39 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
     err = "layernorm: scale/bias length must divide the normalised length";
     return false;
   }
-  int64_t vw = s.get("VW", (n % 4 == 0 && ng % 4 == 0 && nb % 4 == 0) ? 4 : 1);
-  if (vw != 1 && vw != 4) { err = "layernorm: VW must be 1 or 4"; return false; }
-  if (vw == 4 && (n % 4 || ng % 4 || nb % 4)) { err = "layernorm: VW=4 needs lengths divisible by 4"; return false; }
+  // 16 bytes per access where all lengths divide into them (16-bit types fall back to fours), and on large launches of any
+  // row length, scale and bias then being of that length.  Small odd launches keep single elements: the row's end, element by
+  // element, is a second trip to memory there (bf16 100 x 1001: 3.5 us, 4.9 in fours), and so do short rows, where most of a
+  // wavefront would idle, and rows beyond the 32 elements a lane holds.  bf16, us, single elements, fours, eights: 16384 x 4096
+  // 115, 81, 51; 12000 x 2048 47, 30, 20; 12000 x 2047 54, 41, 27; 30000 x 257 44, 22, 29.
+  const bool f16 = s.get("F16", 0) != 0;
+  auto divides = [&](int64_t w) { return n % w == 0 && ng % w == 0 && nb % w == 0; };
+  const bool anyLength = ng == n && nb == n && n >= 256 && n <= 1024 * 32 && (double)rows * (double)n >= 1048576.0;
+  const int64_t wide = f16 ? 8 : 4;
+  int64_t vw = s.get("VW", divides(wide) && n >= 512 ? wide : anyLength ? (n >= 1024 ? wide : 4) : divides(4) ? 4 : 1);
+  if (vw != 1 && vw != 4 && vw != 8) { err = "layernorm: VW must be 1, 4 or 8"; return false; }
+  if (vw > 1 && s.has("VW") && !divides(vw)) { err = "layernorm: VW=4 needs lengths divisible by 4"; return false; }
   int64_t tpr = s.get("TPR", 0);
   if (rows > 0xFFFFFFFFLL) { err = "layernorm: too many rows"; return false; }
   if (tpr == 0) {
-    // four vectors per lane measured best for 4096-float rows, with and without the GELU
-    tpr = nextPow2(ceilDiv(n, vw * 4));
+    // four vectors per lane measured best for 4096-float rows, with and without the GELU; of 16-bit values, eight to a vector,
+    // two beyond 4096 (bf16 16384 x 8192: 90 us against 116; 16384 x 4096: 62 against 51)
+    tpr = nextPow2(ceilDiv(n, vw * (vw == 8 && n > 4096 ? 2 : 4)));
     if (tpr < 64) tpr = 64;
     if (tpr > 512) tpr = 512;
   }
   if (tpr < 64 || tpr > 1024 || (tpr & (tpr - 1))) { err = "layernorm: TPR must be a power of two in [64,1024]"; return false; }
   int64_t vpt = ceilDiv(n, tpr * vw);
-  if (vpt > 8 && !s.has("TPR")) {  // widen the team: up to 8 vectors per lane leave room for gamma, beta and a prefetched row
+  const int64_t few = vw == 8 ? 4 : 8;     // vectors per lane that leave room for gamma, beta and a second row in registers
+  if (vpt > few && !s.has("TPR")) {  // widen the team: up to 8 vectors per lane leave room for gamma, beta and a prefetched row
     tpr = 1024;
     vpt = ceilDiv(n, tpr * vw);
   }
-  const bool f16 = s.get("F16", 0) != 0;
   const double esize = f16 ? 2.0 : 4.0;
-  if (vpt > 32) {
+  if (vpt > (vw == 8 ? 16 : 32)) {
     // the group does not fit the register file of one workgroup: three streamed passes
     const int64_t block = 1024;
+    if (!divides(vw)) vw = divides(4) ? 4 : 1;
     s.p["VW"] = vw; s.p["TPR"] = block; s.p["RPB"] = 1; s.p["VPT"] = 0; s.p["NG"] = ng; s.p["NB"] = nb;
     Defines d;
     d.add("LS_NAME", s.name);
@@ -135,13 +146,14 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   // workgroup per row; a plain copy reaches 6.3-6.4 TB/s under the same conditions.
   const int64_t groups = ceilDiv(rows, rpb);
   int64_t grid = s.get("GRID", 0);
-  if (grid <= 0) grid = vpt <= 8 ? 512 : groups;      // rows too long to prefetch keep one workgroup per group
+  // (four per CU where a lane's share of a row is two vectors of eight: bf16 16384 x 1000 13.3 us against 16.9)
+  if (grid <= 0) grid = vpt <= few ? (vw == 8 && vpt <= 2 ? 1024 : 512) : groups;      // rows too long to prefetch keep one workgroup per group
   if (grid > groups) grid = groups;
   if (grid > 0x7FFFFFFFLL) grid = 0x7FFFFFFFLL;
   s.p["GRID"] = grid;
   d.add("LN_GRID", grid);
   d.add("LN_STREAM", s.get("STREAM", 1) ? 1 : 0);
-  d.add("LN_LEAN", s.get("LEAN", vpt > 8 ? 1 : 0) ? 1 : 0);
+  d.add("LN_LEAN", s.get("LEAN", vpt > few ? 1 : 0) ? 1 : 0);
   // one reduction per row (merged means and sums of squared deviations) where every lane holds the same number of values
   const bool onePass = s.get("ONEPASS", 0) != 0 && n % (tpr * vw) == 0;
   s.p["ONEPASS"] = onePass;
@@ -248,9 +260,14 @@ bool emitBinary(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::st
 bool emitSoftmax(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err) {
   if (!need(s, {"ROWS", "N"}, err) || !positive(s, {"ROWS", "N"}, err)) return false;
   const int64_t rows = s.p["ROWS"], n = s.p["N"];
-  int64_t vw = s.get("VW", n % 4 == 0 ? 4 : 1);
-  if (vw != 1 && vw != 4) { err = "softmax: VW must be 1 or 4"; return false; }
-  if (vw == 4 && n % 4) { err = "softmax: VW=4 needs a row length divisible by 4"; return false; }
+  // As for LayerNorm: 16 bytes per access where the length divides into them, and on large launches of any length (us, single
+  // elements, fours, 16 bytes: bf16 12000 x 2048 41.7, 18.7, 16.5; 4096 x 4096 29.9, 13.5, 9.6; 2000 x 32000 138, 68, 47;
+  // 12000 x 2047 42.9, 22.6, 20.6; 30000 x 257 20.3, 12.1, 14.6; 100 x 1001 3.3, 3.9).
+  const int64_t wide = s.get("F16", 0) ? 8 : 4;
+  const bool anyLength = n >= 256 && n <= 1024 * 32 && (double)rows * (double)n >= 1048576.0;
+  int64_t vw = s.get("VW", n % wide == 0 && n >= 512 ? wide : anyLength ? (n >= 1024 ? wide : 4) : n % 4 == 0 ? 4 : 1);
+  if (vw != 1 && vw != 4 && vw != 8) { err = "softmax: VW must be 1, 4 or 8"; return false; }
+  if (vw > 1 && s.has("VW") && n % vw) { err = "softmax: VW=4 needs a row length divisible by 4"; return false; }
   int64_t tpr = s.get("TPR", 0);
   if (tpr == 0) {
     tpr = nextPow2(ceilDiv(n, vw * 4));      // about four vectors per lane
@@ -259,7 +276,8 @@ bool emitSoftmax(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   }
   if (tpr < 64 || tpr > 1024 || (tpr & (tpr - 1))) { err = "softmax: TPR must be a power of two in [64,1024]"; return false; }
   const int64_t vpt = ceilDiv(n, tpr * vw);
-  if (vpt > 32) {
+  if (vpt > (vw == 8 ? 16 : 32)) {
+    if (n % vw) vw = n % 4 == 0 ? 4 : 1;
     // rows too long for registers (a vocabulary of 150 000 logits, say): one workgroup per row, two streamed passes
     if (rows > 0x7FFFFFFFLL) { err = "softmax: too many rows"; return false; }
     const bool inplaceLong = s.get("INPLACE", 1) != 0;

@@ -174,3 +174,37 @@ def test_gemm_f32_infinities_stay_in_their_rows_and_columns(ops, tb):
         want = a.double().cpu() @ (b.t() if tb else b).double().cpu()
         assert not torch.isnan(want).any()
         assert torch.equal(ops.matmul(a, b, trans_b=tb).double().cpu(), want)
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-6), (torch.float16, 2 ** -10), (torch.bfloat16, 2 ** -7)])
+@pytest.mark.parametrize("rows,n", [(1, 257), (3, 259), (5, 511), (129, 2047), (7, 4097), (2, 32767), (3, 256), (4, 255), (9, 1001), (1200, 1003),
+                                    (4200, 257), (600, 2050), (2050, 512), (600, 8192), (300, 4100), (40, 31999), (70, 16000)])
+def test_rows_of_any_length(ops, rows, n, dtype, tol):
+    """Softmax and LayerNorm over rows that start anywhere: results within one rounding of the type (2^-10 and 2^-7: one ulp
+    above 1, relative; fp32 sums of n <= 2^15 terms in trees stay below 1e-6), and nothing written behind the result."""
+    gen = torch.Generator(device="cuda").manual_seed(rows * n)
+    x = torch.randn((rows, n), generator=gen, device="cuda").to(dtype)
+    g = (torch.rand((n,), generator=gen, device="cuda") + 0.5).to(dtype)
+    b = torch.randn((n,), generator=gen, device="cuda").to(dtype)
+    x64 = x.double()
+    want = torch.softmax(x64, -1)
+    y = ops.softmax(x)
+    assert ((y.double() - want).abs() <= tol * want + (2.0 ** -24 if dtype == torch.float16 else 0.0)).all()
+    z = x.clone()
+    assert torch.equal(ops.softmax(z, inplace=True), y)
+    c = x64 - x64.mean(-1, keepdim=True)
+    want = c / torch.sqrt((c * c).mean(-1, keepdim=True) + 1e-5) * g.double() + b.double()
+    for out in (None, torch.full((rows + 1, n), 7.0, device="cuda", dtype=dtype)):
+        got = ops.layernorm(x, g, b, -1, out=None if out is None else out[:rows])
+        assert ((got.double() - want).norm() <= tol * want.norm()).all()
+        assert out is None or (out[rows:] == 7.0).all()
+
+
+def test_softmax_rows_of_infinities_and_nan(ops):
+    x = torch.randn((4, 1001), device="cuda")
+    x[0, 500:] = float("-inf")
+    x[1, 1000] = float("nan")
+    x[2, :1000] = float("-inf")
+    y, want = ops.softmax(x), torch.softmax(x.double(), -1)
+    assert torch.equal(torch.isnan(y), torch.isnan(want))
+    assert ((y.double() - want).abs()[[0, 2, 3]] <= 1e-6).all()
