@@ -112,6 +112,11 @@ int kcg_hip_get_kernel(kcg_module_t module, const char *name, kcg_kernel_t *out)
 int kcg_hip_launch(kcg_kernel_t kernel, const uint32_t grid[3], const uint32_t block[3],
                    uint32_t lds_bytes, void *stream, void **args);
 
+/* kcg_hip_launch with the argument values themselves: `slots` is `num_args` (at most 16) consecutive 8-byte slots, each
+ * holding one argument from its first byte on (a pointer, or a 4-byte float in the slot's low half).  `dims` is grid x, y, z,
+ * block x, y, z and the LDS bytes.  For callers to whom building arrays of pointers is dear (an interpreted language). */
+int kcg_hip_launch_packed(kcg_kernel_t kernel, const uint32_t dims[7], void *stream, const void *slots, int num_args);
+
 /* Average duration of `iters` back-to-back launches after `warmup` untimed
  * ones, measured with HIP events recorded on `stream`. */
 int kcg_hip_time_launches(kcg_kernel_t kernel, const uint32_t grid[3], const uint32_t block[3],

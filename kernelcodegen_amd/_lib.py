@@ -84,6 +84,7 @@ def _declare(L):
     L.kcg_hip_compile.argtypes = [C.c_char_p, cpp, C.c_int, C.POINTER(vp), C.c_char_p, sz]
     L.kcg_hip_get_kernel.argtypes = [vp, C.c_char_p, C.POINTER(vp)]
     L.kcg_hip_launch.argtypes = [vp, u32p, u32p, C.c_uint32, vp, C.POINTER(vp)]
+    L.kcg_hip_launch_packed.argtypes = [vp, vp, vp, vp, C.c_int]
     L.kcg_hip_time_launches.argtypes = [vp, u32p, u32p, C.c_uint32, vp, C.POINTER(vp), C.c_int, C.c_int,
                                         C.POINTER(C.c_float)]
     L.kcg_hip_module_destroy.argtypes = [vp]

@@ -409,6 +409,16 @@ int kcg_hip_launch(kcg_kernel_t kernel, const uint32_t grid[3], const uint32_t b
                                       lds_bytes, (hipStream_t)stream, args, nullptr));
 }
 
+int kcg_hip_launch_packed(kcg_kernel_t kernel, const uint32_t dims[7], void *stream, const void *slots, int num_args) {
+  if (!kernel || !dims || !slots || num_args < 1 || num_args > 16) return KCG_ERR_INVALID_ARGUMENT;
+  int rc = checkDims(dims, dims + 3);
+  if (rc) return rc;
+  void *args[16];
+  for (int i = 0; i < num_args; ++i) args[i] = (char *)slots + 8 * i;
+  return hipErr(hipModuleLaunchKernel(kernel->fn, dims[0], dims[1], dims[2], dims[3], dims[4], dims[5], dims[6],
+                                      (hipStream_t)stream, args, nullptr));
+}
+
 int kcg_hip_time_launches(kcg_kernel_t kernel, const uint32_t grid[3], const uint32_t block[3],
                           uint32_t lds_bytes, void *stream, void **args,
                           int warmup, int iters, float *avg_ms) {

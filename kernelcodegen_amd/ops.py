@@ -15,35 +15,61 @@ def _need_cuda(*ts):
             raise ValueError("operands must be contiguous device tensors")
 
 
+# (operator, every property of the operands that the kernel depends on) -> the bound launch of that kernel.  Nothing in a
+# key or a value belongs to one tensor: shapes, types, options and whether the operands are aligned.  A call with kernel
+# parameters of its own (cfg) goes through get_kernel each time.
+_bound = {}
+
+
+def _bind(key, cfg, kern, scalars=0):
+    run = kern.bind(scalars)
+    if key is not None and not cfg:
+        _bound[key] = run
+    return run
+
+
 # storage type of the row kernels (their arithmetic is fp32 throughout): the kernels' F16 parameter
 _STORAGE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
 
 def layernorm(x, gamma, beta, axis, eps=1e-5, gelu=False, out=None, **cfg):
     _need_cuda(x, gamma, beta)
+    eps, gelu = float(eps), int(gelu)          # plain numbers: a key must not hold an object that can change
+    key = ("layernorm", x.shape, x.dtype, gamma.shape, gamma.dtype, beta.shape, beta.dtype, axis, eps, gelu)
+    run = None if cfg else _bound.get(key)
+    if run is None:
+        run = _bind(key, cfg, _layernorm_kernel(x, gamma, beta, axis, eps, gelu, cfg))
+    y = torch.empty_like(x) if out is None else out
+    run(x.data_ptr(), gamma.data_ptr(), beta.data_ptr(), y.data_ptr())
+    return y
+
+
+def _layernorm_kernel(x, gamma, beta, axis, eps, gelu, cfg):
     axis = axis + x.dim() if axis < 0 else axis
     rows = int(math.prod(x.shape[:axis])) if axis > 0 else 1
     n = x.numel() // rows
     if x.dtype not in _STORAGE or gamma.dtype != x.dtype or beta.dtype != x.dtype:
         raise ValueError("the LayerNorm kernel takes fp32, IEEE half or bfloat16 tensors of one type")
-    k = R.get_kernel("layernorm", ROWS=rows, N=n, NG=gamma.numel(), NB=beta.numel(), EPS=float(eps),
-                     GELU=int(gelu), F16=_STORAGE[x.dtype], **cfg)
-    y = torch.empty_like(x) if out is None else out
-    k.launch(x, gamma, beta, y)
-    return y
+    return R.get_kernel("layernorm", ROWS=rows, N=n, NG=gamma.numel(), NB=beta.numel(), EPS=float(eps),
+                        GELU=int(gelu), F16=_STORAGE[x.dtype], **cfg)
+
+
+_CTYPE = {torch.float32: "float", torch.int32: "int", torch.float16: "_Float16", torch.bfloat16: "__bf16"}
 
 
 def elementwise(x, op, inplace=False, out_dtype=None, **cfg):
     _need_cuda(x)
-    ctype = {torch.float32: "float", torch.int32: "int", torch.float16: "_Float16", torch.bfloat16: "__bf16"}
-    out_dtype = out_dtype or x.dtype
-    k = R.get_kernel("elementwise", N=x.numel(), OP=op, INPLACE=int(inplace), IN_T=ctype[x.dtype],
-                     OUT_T=ctype[out_dtype], **cfg)
+    out_dtype, inplace = out_dtype or x.dtype, int(inplace)
+    key = ("elementwise", x.numel(), op, inplace, x.dtype, out_dtype)
+    run = None if cfg else _bound.get(key)
+    if run is None:
+        run = _bind(key, cfg, R.get_kernel("elementwise", N=x.numel(), OP=op, INPLACE=int(inplace), IN_T=_CTYPE[x.dtype],
+                                           OUT_T=_CTYPE[out_dtype], **cfg))
     if inplace:
-        k.launch(x)
+        run(x.data_ptr())
         return x.view(out_dtype)
     y = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    k.launch(x, y)
+    run(x.data_ptr(), y.data_ptr())
     return y
 
 
@@ -63,6 +89,21 @@ def batched_matmul(a, b, trans_a=False, trans_b=False, out_dtype=None, **cfg):
     """a: [..., m, k] (or [..., k, m] when trans_a), b: [..., k, n] (or [..., n, k]).  out_dtype None: fp64 for fp64
     operands, fp32 for all others; a type the operands' kernel family does not write raises."""
     _need_cuda(a, b)
+    trans_a, trans_b = bool(trans_a), bool(trans_b)
+    key = ("matmul", a.shape, b.shape, a.dtype, b.dtype, trans_a, trans_b, out_dtype, _aligned(a, b))
+    hit = None if cfg else _bound.get(key)
+    if hit is None:
+        hit = _matmul_launch(a, b, trans_a, trans_b, out_dtype, cfg)
+        if not cfg:
+            _bound[key] = hit
+    run, shape, out_dtype = hit
+    c = torch.empty(shape, dtype=out_dtype, device=a.device)
+    run(a.data_ptr(), b.data_ptr(), c.data_ptr())
+    return c
+
+
+def _matmul_launch(a, b, trans_a, trans_b, out_dtype, cfg):
+    """The bound kernel, shape and type of the result."""
     if a.dtype != b.dtype or a.dtype not in _FAMILY:
         raise ValueError("unsupported operand dtypes")
     batch = int(math.prod(a.shape[:-2])) if a.dim() > 2 else 1
@@ -89,9 +130,9 @@ def batched_matmul(a, b, trans_a=False, trans_b=False, out_dtype=None, **cfg):
         extra.update(_alignment(_aligned(a, b)))
     kern = R.get_kernel(_FAMILY[a.dtype], M=m, N=n, K=k, BATCH=batch, TA=int(trans_a), TB=int(trans_b),
                         **{**extra, **cfg})
-    c = torch.empty(tuple(a.shape[:-2]) + (m, n), dtype=out_dtype, device=a.device)
-    kern.launch(a, b, c)
-    return c
+    if kern.info["workspace_bytes"]:
+        return (lambda *p: kern.launch(*p)), tuple(a.shape[:-2]) + (m, n), out_dtype
+    return kern.bind(), tuple(a.shape[:-2]) + (m, n), out_dtype
 
 
 def matmul_fp8(a, b, scale_a, scale_b, trans_a=False, trans_b=True, out_dtype=torch.float32, **cfg):
@@ -99,6 +140,20 @@ def matmul_fp8(a, b, scale_a, scale_b, trans_a=False, trans_b=True, out_dtype=to
     accumulation.  a: [..., m, k] (or [..., k, m] when trans_a), b: [..., k, n] (or [..., n, k] when
     trans_b, the default: both operands k-contiguous, no transposition on the way into LDS)."""
     _need_cuda(a, b)
+    trans_a, trans_b = bool(trans_a), bool(trans_b)
+    key = ("matmul_fp8", a.shape, b.shape, a.dtype, b.dtype, trans_a, trans_b, out_dtype, _aligned(a, b))
+    hit = None if cfg else _bound.get(key)
+    if hit is None:
+        hit = _matmul_fp8_launch(a, b, trans_a, trans_b, out_dtype, cfg)
+        if not cfg:
+            _bound[key] = hit
+    run, shape = hit
+    c = torch.empty(shape, dtype=out_dtype, device=a.device)
+    run(a.data_ptr(), b.data_ptr(), c.data_ptr(), float(scale_a), float(scale_b))
+    return c
+
+
+def _matmul_fp8_launch(a, b, trans_a, trans_b, out_dtype, cfg):
     if a.dtype != torch.float8_e4m3fn or b.dtype != torch.float8_e4m3fn:
         raise ValueError("operands must be float8_e4m3fn")
     if out_dtype not in (torch.float32, torch.bfloat16):
@@ -110,9 +165,7 @@ def matmul_fp8(a, b, scale_a, scale_b, trans_a=False, trans_b=True, out_dtype=to
         raise ValueError("incompatible K dimensions")
     kern = R.get_kernel("gemm_fp8", M=m, N=n, K=k, BATCH=batch, TA=int(trans_a), TB=int(trans_b),
                         OUT_BF16=int(out_dtype == torch.bfloat16), **{**_alignment(_aligned(a, b)), **cfg})
-    c = torch.empty(tuple(a.shape[:-2]) + (m, n), dtype=out_dtype, device=a.device)
-    kern.launch(a, b, c, float(scale_a), float(scale_b))
-    return c
+    return kern.bind(scalars=2), tuple(a.shape[:-2]) + (m, n)
 
 
 def matmul(a, b, **cfg):
@@ -130,17 +183,20 @@ def fmha(q, k, v, scale=None, causal=False, out_dtype=None, **cfg):
     out_dtype = q.dtype if out_dtype is None else out_dtype
     if out_dtype not in (q.dtype, torch.float32):
         raise ValueError("output must have the operands' type or be fp32")
-    b, h, s, d = q.shape
-    scale = d ** -0.5 if scale is None else float(scale)
-    if q.dtype == torch.float32:
-        kern = R.get_kernel("fmha_f32", B=b, H=h, S=s, D=d, CAUSAL=int(causal), SCALE=scale, **cfg)
-        o = torch.empty(q.shape, dtype=torch.float32, device=q.device)
-        kern.launch(q, k, v, o)
-        return o
-    kern = R.get_kernel("fmha_bf16", B=b, H=h, S=s, D=d, CAUSAL=int(causal), SCALE=scale,
-                        OUT_BF16=int(out_dtype == q.dtype), F16=int(q.dtype == torch.float16), **cfg)
+    scale, causal = (None if scale is None else float(scale)), int(causal)
+    key = ("fmha", q.shape, q.dtype, scale, causal, out_dtype)
+    run = None if cfg else _bound.get(key)
+    if run is None:
+        b, h, s, d = q.shape
+        scale = d ** -0.5 if scale is None else scale
+        if q.dtype == torch.float32:
+            kern = R.get_kernel("fmha_f32", B=b, H=h, S=s, D=d, CAUSAL=int(causal), SCALE=scale, **cfg)
+        else:
+            kern = R.get_kernel("fmha_bf16", B=b, H=h, S=s, D=d, CAUSAL=int(causal), SCALE=scale,
+                                OUT_BF16=int(out_dtype == q.dtype), F16=int(q.dtype == torch.float16), **cfg)
+        run = _bind(key, cfg, kern)
     o = torch.empty(q.shape, dtype=out_dtype, device=q.device)
-    kern.launch(q, k, v, o)
+    run(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr())
     return o
 
 
@@ -150,6 +206,23 @@ def binary(x, y, op, inplace=False, **cfg):
     _need_cuda(x, y)
     if x.dtype not in (torch.float32, torch.float16) or y.dtype != x.dtype:
         raise ValueError("the binary kernel takes two fp32 or two IEEE half operands")
+    inplace = int(inplace)
+    key = ("binary", x.shape, y.shape, x.dtype, op, inplace)
+    hit = None if cfg else _bound.get(key)
+    if hit is None:
+        hit = _binary_launch(x, y, op, inplace, cfg)
+        if not cfg:
+            _bound[key] = hit
+    run, shape = hit
+    if inplace:
+        run(x.data_ptr(), y.data_ptr())
+        return x
+    z = torch.empty(shape, dtype=torch.bool if op in ("Equal", "Greater") else x.dtype, device=x.device)
+    run(x.data_ptr(), y.data_ptr(), z.data_ptr())
+    return z
+
+
+def _binary_launch(x, y, op, inplace, cfg):
     shape = torch.broadcast_shapes(x.shape, y.shape)
 
     def strides(t):
@@ -163,12 +236,7 @@ def binary(x, y, op, inplace=False, **cfg):
 
     k = R.get_kernel("binary", OP=op, DIMS=",".join(map(str, shape)), SA=strides(x), SB=strides(y), INPLACE=int(inplace),
                      F16=int(x.dtype == torch.float16), **cfg)
-    if inplace:
-        k.launch(x, y)
-        return x
-    z = torch.empty(shape, dtype=torch.bool if op in ("Equal", "Greater") else x.dtype, device=x.device)
-    k.launch(x, y, z)
-    return z
+    return k.bind(), shape
 
 
 def gather(x, indices, axis=0, **cfg):
@@ -180,8 +248,20 @@ def gather(x, indices, axis=0, **cfg):
         raise ValueError("gather indices must be int64")
     if not -x.dim() <= axis < x.dim():
         raise ValueError("axis out of range")
+    key = ("gather", x.shape, x.dtype, indices.shape, axis)
+    hit = None if cfg else _bound.get(key)
+    if hit is None:
+        hit = _gather_launch(x, indices, axis, cfg)
+        if not cfg:
+            _bound[key] = hit
+    run, shape = hit
+    out = torch.empty(shape, dtype=x.dtype, device=x.device)
+    run(x.data_ptr(), indices.data_ptr(), out.data_ptr())
+    return out
+
+
+def _gather_launch(x, indices, axis, cfg):
     axis %= x.dim()
-    x, indices = x.contiguous(), indices.contiguous()
     outer = 1
     for d in x.shape[:axis]:
         outer *= d
@@ -191,9 +271,7 @@ def gather(x, indices, axis=0, **cfg):
     single = tuple(indices.shape) == (1,)
     shape = tuple(x.shape[:axis]) + (() if single else tuple(indices.shape)) + tuple(x.shape[axis + 1:])
     kern = R.get_kernel("gather", OUTER=outer, AXIS=x.shape[axis], NIDX=indices.numel(), INNER=inner, ESIZE=x.element_size(), **cfg)
-    out = torch.empty(shape, dtype=x.dtype, device=x.device)
-    kern.launch(x, indices, out)
-    return out
+    return kern.bind(), shape
 
 
 def softmax(x, inplace=False):
@@ -201,15 +279,16 @@ def softmax(x, inplace=False):
     _need_cuda(x)
     if x.dtype not in _STORAGE:
         raise ValueError("the softmax kernel takes fp32, IEEE half or bfloat16 operands")
-    x = x if inplace else x.contiguous()
-    if not x.is_contiguous():
-        raise ValueError("an in-place softmax needs a contiguous tensor")
-    n = x.shape[-1]
-    kern = R.get_kernel("softmax", ROWS=x.numel() // n, N=n, INPLACE=int(inplace), F16=_STORAGE[x.dtype])
+    inplace = int(inplace)
+    key = ("softmax", x.shape, x.dtype, inplace)
+    run = _bound.get(key)
+    if run is None:
+        n = x.shape[-1]
+        run = _bind(key, None, R.get_kernel("softmax", ROWS=x.numel() // n, N=n, INPLACE=int(inplace), F16=_STORAGE[x.dtype]))
     if inplace:
-        kern.launch(x)
+        run(x.data_ptr())
         return x
     y = torch.empty_like(x)
-    kern.launch(x, y)
+    run(x.data_ptr(), y.data_ptr())
     return y
 

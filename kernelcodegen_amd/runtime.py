@@ -3,6 +3,7 @@ pick up a code object built ahead of time), load it, launch it on torch's
 current stream.  torch supplies device memory and the stream handle only."""
 import ctypes as C
 import os
+import struct
 
 from . import _lib
 from ._lib import LaunchInfo, check, lib
@@ -127,6 +128,17 @@ def compile_to_code(src, opts=(), use_cache=True, refresh=False):
         lib().kcg_hip_free_code(code)
 
 
+def _current_stream():
+    """A function that returns the handle of torch's current stream on the current device (without the Stream object that
+    torch.cuda.current_stream() builds, where this torch offers it)."""
+    import torch
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return lambda: torch.cuda.current_stream().cuda_stream
+    device = torch.cuda.current_device
+    return lambda: raw(device())
+
+
 class Kernel:
     def __init__(self, module, handle, info=None):
         self.module, self.handle, self.info = module, handle, info
@@ -179,6 +191,24 @@ class Kernel:
         lds = self.info["lds_bytes"] if lds_bytes is None else lds_bytes
         holders, arr = self._pack(self._complete(args))
         check(lib().kcg_hip_launch(self.handle, g, b, lds, self._stream(stream), arr), "kcg_hip_launch")
+
+    def bind(self, scalars=0):
+        """launch() on the current stream for a kernel without a workspace, as a function of the arguments' values: device
+        pointers as integers, then `scalars` fp32 numbers.  Everything that is the same for all launches is prepared here:
+        the general launch() spends most of a small call on ctypes objects (an eight-call block 148 us, 41 this way)."""
+        info = self.info
+        if info["workspace_bytes"]:
+            raise ValueError("the kernel takes a workspace")
+        n = info["num_args"]
+        pack = struct.Struct("<" + "Q" * (n - scalars) + "f4x" * scalars).pack
+        dims = (C.c_uint32 * 7)(*info["grid"], *info["block"], info["lds_bytes"])
+        address, handle, entry, stream = C.addressof(dims), self.handle, lib().kcg_hip_launch_packed, _current_stream()
+
+        def run(*values, _keep=(dims, self)):
+            rc = entry(handle, address, stream(), pack(*values), n)
+            if rc:
+                check(rc, "kcg_hip_launch_packed")
+        return run
 
     def arg_sets(self, sets):
         """Packs several argument lists for launch_sequence / time_rotating; keep the result alive while in use."""

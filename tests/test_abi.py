@@ -77,6 +77,17 @@ def test_null_arguments_are_rejected():
     assert lib.kcg_hip_graph_destroy(None) == 1
 
 
+def test_launch_packed_rejects_bad_arguments():
+    lib = _lib.lib()
+    dims = (C.c_uint32 * 7)(1, 1, 1, 64, 1, 1, 0)
+    at = C.addressof(dims)
+    assert lib.kcg_hip_launch_packed(None, at, None, b"\0" * 8, 1) == 1
+    for nargs in (0, 17, -1):
+        assert lib.kcg_hip_launch_packed(at, at, None, b"\0" * 8, nargs) == 1
+    assert lib.kcg_hip_launch_packed(at, None, None, b"\0" * 8, 1) == 1
+    assert lib.kcg_hip_launch_packed(at, at, None, None, 1) == 1
+
+
 def test_emitter_reports_bad_parameters():
     with pytest.raises(_lib.KcgError, match="unknown kernel family"):
         R.emit_kernel("conv2d", "kernel0", N=1)
