@@ -1017,6 +1017,21 @@ bool emitFmhaBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
     else if (sl % 64 == 0 && sl <= 512) br = 64;
     else br = sl > 128 ? 256 : (sl > 64 ? 128 : (sl > 32 ? 64 : 32));
   }
+  // Launches that leave half the compute units or more without a workgroup of 256 queries (under the mask: without a pair of
+  // query tiles) take 128 queries per workgroup instead, and under the mask pairs only where enough of them are left for every
+  // CU: the pairs balance the work of a full part, on an emptier one they halve its parallelism (us, before and now: B2 H16
+  // S777 D64 19.4 and 15.4, causal 29.7 and 16.0; B1 H8 S2048 D64 36.0 and 25.6, causal 44.7 and 26.5; B3 H12 S1300 D64 causal
+  // 38.8 and 26.9; B1 H32 S2048 D128 causal 69.3 and 57.3, with pairs).  Above that 256 stays ahead: B3 H12 S1300 D64 with 216
+  // workgroups 28.5 against 31.4; causal with 192 pairs B4 H32 S600 D128 41 against 64, B4 H12 S2048 D64 46 against 61.
+  const bool masked = s.get("CAUSAL", 0) != 0;
+  bool own = s.get("BR", 0) > 0 || s.get("BC", 0) > 0 || s.get("QW", 0) > 0;
+  for (const char* key : {"D2L", "PAIR", "PERSIST", "OCC", "STAGE_O"}) own = own || s.has(key);
+  const double heads = (double)b * (double)h, jobs = (double)ceilDiv(sl, br) * heads / (masked && ((b * h) % 2 == 0 || ceilDiv(sl, br) % 2 == 0) ? 2.0 : 1.0);
+  bool noPair = false;
+  if (!own && jobs <= 128.0) {
+    if (br == 256) br = 128;
+    noPair = masked && (double)ceilDiv(sl, br) * heads / 2.0 < 256.0;
+  }
   if (bc <= 0) {
     bc = sl > 32 ? 64 : 32;
     if (2 * bc * (dh * 2 + 16) + 3 * bc * (dh * 2 + 32) > 160 * 1024) bc = 32;   // head dim 256: 64-key tiles do not fit the LDS
@@ -1062,7 +1077,7 @@ bool emitFmhaBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   // causal: a workgroup takes a pair of query tiles with the same total number of key tiles, unless asked not to:
   // PAIR = 1 of one head (an even number of query tiles), PAIR = 2 of two heads (an even number of heads; see the kernel)
   // (across two heads by default: the same speed as within one head, 641 against 763 MB of HBM traffic at B8 H32 S2048 D128)
-  int64_t pairMode = causal ? s.get("PAIR", (b * h) % 2 == 0 ? 2 : 1) : 0;
+  int64_t pairMode = causal ? s.get("PAIR", noPair ? 0 : (b * h) % 2 == 0 ? 2 : 1) : 0;
   if (pairMode == 2 && (b * h) % 2) pairMode = 1;
   if (pairMode == 1 && ceilDiv(sl, br) % 2) pairMode = 0;
   if (pairMode < 0 || pairMode > 2) { err = "fmha_bf16: PAIR is 0, 1 or 2"; return false; }
@@ -1107,7 +1122,14 @@ bool emitFmhaF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   if (dh % 32 || dh > 256) { err = "fmha_f32: head dim must be a multiple of 32, at most 256"; return false; }
   // queries per workgroup (32 per wavefront): four wavefronts, fewer for short sequences
   int64_t br = s.get("BR", 0);
-  if (br <= 0) br = sl >= 128 ? 128 : (sl > 64 ? 128 : (sl > 32 ? 64 : 32));
+  if (br <= 0) {
+    br = sl >= 128 ? 128 : (sl > 64 ? 128 : (sl > 32 ? 64 : 32));
+    // Under the mask at head dims above 64, whose workgroups have a CU to themselves, two rounds of them end as late as the
+    // longest query tiles: half the tile evens that out (B4 H32 S512 D128 139 and 103 us, B1 H32 S2048 D128 520 and 341;
+    // one round loses, B1 H32 S1024 D128 146 and 166, more gain nothing, B8 H32 S640 D128 342 and 350).
+    const double tiles = (double)ceilDiv(sl, 128) * (double)b * (double)h;
+    if (s.get("CAUSAL", 0) && dh > 64 && br == 128 && !s.has("PAIR") && !s.has("D2L") && tiles > 256.0 && tiles <= 512.0) br = 64;
+  }
   if (br % 32 || br > 512) { err = "fmha_f32: BR must be a multiple of 32, at most 512"; return false; }
   // keys per LDS tile: 64 for head dims above 64 while two workgroups' tiles fit the LDS together, else 32 (measured at
   // B8 H32 S2048: head dim 64 135 against 131 TFLOP/s with 32-key tiles, head dim 128 the same either way)

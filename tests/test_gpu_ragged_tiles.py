@@ -208,3 +208,21 @@ def test_softmax_rows_of_infinities_and_nan(ops):
     y, want = ops.softmax(x), torch.softmax(x.double(), -1)
     assert torch.equal(torch.isnan(y), torch.isnan(want))
     assert ((y.double() - want).abs()[[0, 2, 3]] <= 1e-6).all()
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 1e-2), (torch.float16, 2e-3), (torch.float32, 4e-6)])
+@pytest.mark.parametrize("b,h,s,d", [(1, 8, 333, 64), (2, 16, 777, 64), (1, 3, 64, 64), (1, 3, 65, 128), (1, 3, 129, 64), (1, 5, 256, 128),
+                                     (1, 32, 1100, 128), (4, 32, 260, 64), (3, 12, 1300, 64), (2, 64, 512, 128)])
+def test_attention_on_small_launches(ops, b, h, s, d, dtype, tol, causal):
+    """128 queries per workgroup and no pairs of query tiles where the launch leaves compute units empty, 64 for fp32 under
+    the mask; the tolerances are those of the other attention tests (16-bit probabilities, fp32 sums)."""
+    gen = torch.Generator(device="cuda").manual_seed(s + d)
+    q, k, v = (torch.randn((b, h, s, d), generator=gen, device="cuda").to(dtype) for _ in range(3))
+    got = ops.fmha(q, k, v, causal=causal).double()
+    for i in range(b):
+        scores = (q[i].double() @ k[i].double().transpose(-1, -2).contiguous()) * d ** -0.5
+        if causal:
+            scores.masked_fill_(torch.ones((s, s), dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+        want = torch.softmax(scores, -1) @ v[i].double()
+        assert ((got[i] - want).norm() <= tol * want.norm()).item()
