@@ -685,6 +685,10 @@ static const Gemm16Form* chooseGemm16Form(int64_t m, int64_t n, int64_t k, int64
       {256, 256, 4, 2, 2, 256, 55, 45}, {128, 128, 4, 2, 2, 512, 32, 31}, {128, 128, 4, 2, 3, 256, 14, 25},
       {64, 128, 2, 2, 3, 512, 13, 28},  {64, 128, 2, 2, 4, 256, 18, 5},   {64, 64, 2, 2, 4, 512, 12, 12},
   };
+  // few rows: tiles of 32 x 64 (us, against 64 x 64: 8 x 1024 x 4096 9.2 and 11.6, 16 x 11008 x 4096 14.6 and 15.0, 32 x 4096 x
+  // 4096 12.1 and 13.2, 1 x 4096 x 4096 11.4 and 12.3)
+  static const Gemm16Form few = {32, 64, 1, 4, 4, 512, 0, 0};
+  if (m <= 32 && batch == 1 && n >= 64 && k >= 64) return &few;
   const Gemm16Form* best = nullptr;
   double least = 0.0;
   for (const auto& f : forms) {
@@ -719,30 +723,32 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   // 256x256 tiles run as 8 wavefronts (two per SIMD, 64x128 each) so that one wavefront's
   // LDS and global-memory instructions issue under the other's MFMAs
   int64_t wm = s.get("WM", bm >= 256 && bn >= 256 ? 4 : 2), wn = s.get("WN", 2), gm = s.get("GROUP_M", 8);
-  if (!checkTile(s, bm, bn, bk, wm, wn, 16, err)) return false;
+  // an A tile of 32 rows, four wavefronts side by side: direct loads of at most so many rows only (checked below)
+  const bool fewRows = bm == 32 && bn == 64 && wm == 1 && wn == 4 && bk == 64 && m <= bm && batch == 1 && s.get("M16", 0) && s.get("D2L", 1);
+  if (!fewRows && !checkTile(s, bm, bn, bk, wm, wn, 16, err)) return false;
   // A tiles k-contiguous with 16 bytes of padding a row; B tiles the same, or [k][n] rows with 32 bytes of padding
   // pad of an sB[k][n] row: the 32 lanes that a transposing read serves together take four k rows of 64 bytes, which fall
   // on disjoint banks when the row pitch is 64 modulo 256 (SQ_LDS_BANK_CONFLICT: 22.5 M cycles per launch of the
   // 4096 x 11008 x 4096 product with a pad of 32, none with 64)
   int64_t bpad = s.get("BPAD", (bn * 2) % 256 == 0 ? 64 : 32);
   if (bpad < 0 || bpad % 16) { err = "gemm_bf16: BPAD must be a multiple of 16 bytes"; return false; }
-  const bool ragged = (m % bm) || (n % bn) || (k % bk);
+  const bool ragged = (m % bm) || (n % bn) || (k % bk) || fewRows;
   // Ragged sizes without guarded loads: the last tiles are moved back to end at the edge (GB_SHIFT in the kernel).  Needs a
   // whole tile in every dimension, rows that start on 16-byte boundaries (ALIGN = 16: the caller has looked at the
   // operands' addresses; without it the guarded loads, which take any address, stay) and no tail split.
   // fewer rows than one tile: the rows past the last are read from the last one (GB_CLAMP; direct loads only)
-  const bool clamp = m < bm && batch == 1 && s.get("D2L", 1) != 0;
+  const bool clamp = (m < bm || fewRows) && batch == 1 && s.get("D2L", 1) != 0;
   const bool canShift = s.get("ALIGN", 0) >= 16 && (m >= bm || clamp) && n >= bn && k >= bk && k % 8 == 0 && (!s.get("TA", 0) || m % 8 == 0) &&
                         (s.get("TB", 0) || n % 8 == 0) && s.get("SK_UNITS", 0) <= 0;
   // the 16x16x32 MFMA (see the kernel): whole 64-deep k-tiles, A contiguous along k, B contiguous along k or read
   // through the transposing LDS reads, loads without guards
   const bool m16Fits = bk == 64 && !s.get("TA", 0) && (s.get("TB", 0) || s.get("BTR", 1)) && (!ragged || canShift) &&
-                       (wm * wn) % 2 == 0 && bm % (8 * wm * wn) == 0 && bn % (8 * wm * wn) == 0 && s.get("STAGES", 1) == 1 &&
+                       (wm * wn) % 2 == 0 && (fewRows || bm % (8 * wm * wn) == 0) && bn % (8 * wm * wn) == 0 && s.get("STAGES", 1) == 1 &&
                        s.get("SK_UNITS", 0) <= 0 && bm / wm % 16 == 0 && bn / wn % 16 == 0;
   // direct loads into LDS (global_load_lds_dwordx4, see the kernel): every wavefront moves a whole, even number of
   // 1 KiB blocks per operand tile; row-major weights need the 256-column tile and eight wavefronts
   const int64_t waves = wm * wn;
-  const bool d2lFits = m16Fits && bm % (16 * waves) == 0 &&
+  const bool d2lFits = m16Fits && (fewRows ? canShift : bm % (16 * waves) == 0) &&
                        (s.get("TB", 0) ? bn % (16 * waves) == 0 : ((bn == 64 || bn == 128 || bn == 256) && (bn / 8) % waves == 0));
   // Default on the 256 x 256 tile with eight wavefronts, where it was measured: with direct loads 0.295-0.303 ms on
   // 4096 x 11008 x 4096 in either weight layout against 0.310-0.315 ms ([N][K]) and 0.338-0.346 ms ([K][N]) for the
@@ -759,6 +765,7 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   // row-major weights in other tiles than 256 columns of eight wavefronts: on request, and in the forms chosen above
   const bool d2l = m16 && s.get("D2L", d2lFits && (s.get("TB", 0) || (bn == 256 && waves == 8))) != 0;
   s.p["D2L"] = d2l;
+  if (fewRows && !(shift && clamp && d2l)) { err = "gemm_bf16: tiles of 32 rows need aligned operands and direct loads"; return false; }
   if (d2l && !d2lFits) { err = "gemm_bf16: D2L needs M16 and whole 1 KiB blocks per wavefront (row-major weights: BN = 64, 128 or 256)"; return false; }
   const int64_t nbuf = s.get("NBUF", 2);
   if (nbuf < 2 || nbuf > 6 || (nbuf > 2 && (!d2l || (nbuf - 1) * (bm / 8 + bn / 8) / waves > 63))) {

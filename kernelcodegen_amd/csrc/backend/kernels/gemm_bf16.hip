@@ -12,8 +12,8 @@
 //   GB_EDGE                      1: ragged tiles, guard loads and stores
 //   GB_SHIFT                     1: ragged M or N without guarded loads: the last tile of a row or column of tiles is moved
 //                                back to end at the edge (see the kernel)
-//   GB_CLAMP                     1: M < GB_BM, one row of tiles: rows past the last are read from the last row and not
-//                                stored (direct loads only)
+//   GB_CLAMP                     1: M <= GB_BM, one row of tiles: rows past the last are read from the last row and not
+//                                stored (direct loads only; GB_BM may be 32 then)
 //   GB_NBUF                      LDS buffers per operand, 2 (default) to 6; more than two with direct loads only: the loads of
 //                                k-tile kt + GB_NBUF start with k-tile kt
 //   GB_KTAIL                     1: K is no multiple of GB_BK; the last k-tile is moved back likewise (direct loads only)
@@ -369,7 +369,7 @@ typedef _Float16 kcg_f16x8 __attribute__((ext_vector_type(8)));
 #define GB_SK_PER0 ((GB_SK_GTILES * GB_KT + GB_SK_GUNITS - 1) / (GB_SK_GUNITS > 0 ? GB_SK_GUNITS : 1))
 #define GB_SK_PER (GB_SK_PER0 + (GB_SK_PER0 & 1))                    // k-iterations per unit, even
 
-#if (GB_BM % (32 * GB_WM)) || (GB_BN % (32 * GB_WN)) || (GB_BK % 16)
+#if (GB_BM % (32 * GB_WM)) || (GB_BN % (GB_FR * GB_WN)) || (GB_BK % 16)
 #error "tile shape does not divide into 32x32x16 MFMA tiles"
 #endif
 #if GB_D2L && (!GB_M16 || (GB_BTR && GB_BN != 256 && GB_BN != 128 && GB_BN != 64))
@@ -378,10 +378,10 @@ typedef _Float16 kcg_f16x8 __attribute__((ext_vector_type(8)));
 #if GB_NBUF != 2 && !GB_D2L
 #error "more than two LDS buffers: only with direct loads"
 #endif
-#if (GB_SHIFT && (GB_EDGE || GB_SK_UNITS > 0 || (GB_M < GB_BM && !GB_CLAMP) || GB_N < GB_BN)) || (GB_CLAMP && (!GB_D2L || !GB_SHIFT || GB_M >= GB_BM)) || (GB_KTAIL && (!GB_D2L || GB_K < GB_BK || GB_K % GB_BK == 0))
+#if (GB_SHIFT && (GB_EDGE || GB_SK_UNITS > 0 || (GB_M < GB_BM && !GB_CLAMP) || GB_N < GB_BN)) || (GB_CLAMP && (!GB_D2L || !GB_SHIFT || GB_M > GB_BM)) || (GB_BM == 32 && GB_D2L && !GB_CLAMP) || (GB_KTAIL && (!GB_D2L || GB_K < GB_BK || GB_K % GB_BK == 0))
 #error "moved-back tiles: whole tiles must fit the operands; a moved-back k-tile needs direct loads"
 #endif
-#if GB_M16 && (GB_BK != 64 || GB_TA != 0 || (GB_TB == 0 && !GB_BTR) || GB_GUARD || GB_SK_UNITS > 0 || GB_STAGES != 1 || GB_NT % 128 || GB_BM % (GB_NT / 8) || (GB_TB == 1 && GB_BN % (GB_NT / 8)))
+#if GB_M16 && (GB_BK != 64 || GB_TA != 0 || (GB_TB == 0 && !GB_BTR) || GB_GUARD || GB_SK_UNITS > 0 || GB_STAGES != 1 || GB_NT % 128 || (GB_BM % (GB_NT / 8) && !GB_CLAMP) || (GB_TB == 1 && GB_BN % (GB_NT / 8)))
 #error "the 16x16x32 form needs whole 64-deep k-tiles, a k-contiguous A, unguarded loads, no tail split and one staging set"
 #endif
 #if GB_SK_UNITS > 0 && (GB_BATCH != 1 || GB_SK_TAIL <= 0 || GB_SK_TAIL > 1024 || GB_SK_PER > GB_KT || GB_SK_PER < 2)
@@ -548,10 +548,13 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
   // is applied on the source side: the lane that fills position p of row r fetches chunk p ^ ((r / 2) % 8) of that
   // row, still within the row's one 128-byte line.  No staging registers, no LDS store instructions; a tile's loads
   // are issued behind the barrier that frees its buffer and awaited in front of the next barrier.
+  // Few rows: an A tile of 32 rows.  What a launch of few tiles waits for is a CU's intake, 16 KB per k-tile in 0.18 us with
+  // 64 rows of each operand, so half the rows that are not there are not loaded (8 x 1024 x 4096: 11.6 us with 64 rows, 9.2
+  // with 32; 16 rows, which leave half the wavefronts without a load of their own, 9.9).
   constexpr int UA = GB_BM / 8 / (GB_NT / 64);                                     // instructions per wavefront and tile
   constexpr int RB = 1024 / (GB_BN * 2) > 0 ? 1024 / (GB_BN * 2) : 1;              // k rows of row-major weights per instruction
   constexpr int UB = GB_BTR ? GB_BK / RB / (GB_NT / 64) : GB_BN / 8 / (GB_NT / 64);
-  static_assert(UA % 2 == 0 && GB_BM % (8 * (GB_NT / 64)) == 0, "direct loads: whole, even numbers of 8-row groups per wavefront");
+  static_assert((GB_CLAMP || UA % 2 == 0) && UA > 0 && GB_BM % (8 * (GB_NT / 64)) == 0, "direct loads: whole, even numbers of 8-row groups per wavefront");
   static_assert(GB_BTR ? UB * RB * (GB_NT / 64) == GB_BK && UB >= 1 : (UB % 2 == 0 && GB_BN % (8 * (GB_NT / 64)) == 0), "direct loads of B: whole blocks per wavefront");
   // The instruction is written out: through the builtin the compiler, which cannot tell that the transposing reads
   // that follow touch the other buffer, puts a wait for all outstanding loads in front of each of them.  Here it sees
@@ -570,8 +573,8 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
   unsigned d2l_lane_a[UA];
 #pragma unroll
   for (int t = 0; t < UA; ++t) {
-    const int row = (wave * UA + t) * 8 + (lane >> 3);
-    d2l_lane_a[t] = (unsigned)(row < GB_M ? row : GB_M - 1) * (unsigned)(GB_K * 2) + (unsigned)(((lane & 7) ^ (lane >> 4) ^ ((t & 1) * 4)) * 16);
+    const int grp = wave * UA + t, row = grp * 8 + (lane >> 3);
+    d2l_lane_a[t] = (unsigned)(row < GB_M ? row : GB_M - 1) * (unsigned)(GB_K * 2) + (unsigned)(((lane & 7) ^ (lane >> 4) ^ ((grp & 1) * 4)) * 16);
   }
   auto d2l_a = [&](int k0, char* sbuf, int t) __attribute__((always_inline)) {
     lds_dma((const char*)(As + k0), d2l_lane_a[t], sbuf + (wave_u * UA + t) * 8 * GB_ROWB);
@@ -618,16 +621,16 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
   auto zero_tail = [&](int buf) __attribute__((always_inline)) {
     constexpr int KZ = GB_BK - GB_K % GB_BK;
     const kcg_u32x4 zero = {0u, 0u, 0u, 0u};
-    auto rows = [&](char* sbuf, int upw) __attribute__((always_inline)) {
+    auto zero_rows = [&](char* sbuf, int upw) __attribute__((always_inline)) {
       for (int t = 0; t < upw; ++t)
-        if ((((lane & 7) ^ (lane >> 4)) ^ ((t & 1) * 4)) * 8 < KZ) *(kcg_u32x4*)(sbuf + (wave_u * upw + t) * 8 * GB_ROWB + lane * 16) = zero;
+        if ((((lane & 7) ^ (lane >> 4)) ^ (((wave_u * upw + t) & 1) * 4)) * 8 < KZ) *(kcg_u32x4*)(sbuf + (wave_u * upw + t) * 8 * GB_ROWB + lane * 16) = zero;
     };
-    rows(sA + buf * (GB_BM * GB_ROWB), UA);
+    zero_rows(sA + buf * (GB_BM * GB_ROWB), UA);
 #if GB_BTR
     for (int t = 0; t < UB; ++t)
       if ((wave_u * UB + t) * RB + lane / (64 / RB) < KZ) *(kcg_u32x4*)(sB + buf * GB_BBUF + (wave_u * UB + t) * 1024 + lane * 16) = zero;
 #else
-    rows(sB + buf * GB_BBUF, UB);
+    zero_rows(sB + buf * GB_BBUF, UB);
 #endif
   };
   static_assert(GB_K % 8 == 0, "whole 16-byte chunks along k");
@@ -778,6 +781,7 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #define GB_M16_DEAL 1
 #endif
     static_assert(KS % 2 == 0, "the A fragment sets alternate per k-step");
+#if !GB_D2L
     auto feed_unit = [&](int u) __attribute__((always_inline)) {
       if (u < PA) {
         if (feed) la[set].store_unit(u, nA, GB_ROWB, tid);
@@ -787,6 +791,7 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
         if (fetch) GB_LOAD_B(set, u - PA, k2);
       }
     };
+#endif
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int cur = ks & 1, nxt = cur ^ 1;
@@ -796,11 +801,13 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #pragma unroll
         for (int i = 0; i < GB_TM; ++i) fa[nxt][i] = *(const GB_FRAG*)(cA + i * GB_FR * GB_ROWB + GB_KOFF(ks + 1));
       }
-      if (!GB_D2L && !GB_M16_DEAL && ks < FS) {
+#if !GB_D2L
+      if (!GB_M16_DEAL && ks < FS) {
 #pragma unroll
         for (int u = 0; u < UNITS; ++u)
           if ((u < PA ? u * WA : PA * WA + (u - PA) * WB) * FS / WORK == ks) feed_unit(u);
       }
+#endif
       if (last) {
 #if GB_D2L
         // this wavefront's share of tile kt+1 has landed; in the steady state tiles kt+2 .. kt+GB_NBUF-1 are still under way

@@ -60,7 +60,8 @@ def test_gemm16_every_form_at_its_edges(ops, form, tb):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("tb", [False, True])
 @pytest.mark.parametrize("m,n,k", [(1, 512, 512), (15, 640, 4096), (63, 520, 136), (64, 1024, 2048), (65, 584, 1000), (300, 1000, 264),
-                                   (1000, 2056, 520), (257, 264, 64), (9, 64, 64), (64, 64, 72)])
+                                   (1000, 2056, 520), (257, 264, 64), (9, 64, 64), (64, 64, 72),
+                                   (16, 128, 64), (16, 72, 64 * 13), (17, 136, 72), (31, 64, 320), (32, 192, 64 * 7 + 8), (33, 64, 128)])
 def test_gemm16_default_forms(ops, m, n, k, tb, dtype):
     a, b, want = _operands(m, n, k, tb, dtype, m + n + k)
     for out in (torch.float32, dtype):
