@@ -433,6 +433,10 @@ bool checkTile(const KernelSpec& s, int64_t bm, int64_t bn, int64_t bk, int64_t 
   return true;
 }
 
+// Rows short enough that a lane's offset within the rows of one direct load (at most 64 rows where rows are clamped) stays
+// in 32 bits: where more than the whole tiles of the direct-load kernels is taken, longer ones keep the other kernels.
+static bool shortRows(int64_t n, int64_t k) { return n <= (1 << 23) && k <= (1 << 23); }
+
 bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err) {
   int64_t m, n, k, batch;
   if (!gemmCommon(s, err, m, n, k, batch)) return false;
@@ -453,7 +457,7 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // us, 16 21.4), else of 16 (K 500, 777 x 1000: 16 11.8 us, 32 20.4: every row of a k-tile of 32 straddles two lines).
   bool own = false;
   for (const char* key : {"BM", "BN", "BK", "WM", "WN", "WK", "NBUF", "PAD"}) own = own || s.has(key);
-  const bool direct = s.get("D2L", 1) != 0 && s.get("ALIGN", 0) >= 16 && !s.get("TA", 0) && k % 4 == 0 && (s.get("TB", 0) || n % 4 == 0);
+  const bool direct = s.get("D2L", 1) != 0 && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !s.get("TA", 0) && k % 4 == 0 && (s.get("TB", 0) || n % 4 == 0);
   const bool divides = m % tile == 0 && n % tile == 0 && k % (tile <= 128 ? 32 : 16) == 0;
   if (!own && (!divides || (direct && s.get("TB", 0))) && m >= 64 && n >= 64 && k >= 16) {
     static const struct { int64_t t; double weight; } sizes[] = {{256, 0.985}, {128, 1.0}, {64, 1.06}};
@@ -482,7 +486,7 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // Whole tiles with BK = 16 or 32 of two row-major operands: the kernel that loads both tiles straight into LDS
   // (kernels/gemm_f32_d2l.hip).  Where the caller has looked at the operands' addresses (ALIGN = 16) and rows are whole
   // 16-byte chunks, also a B that is contiguous along k, and sizes that the tiles do not divide.
-  const bool aligned = s.get("ALIGN", 0) >= 16 && k % 4 == 0 && (s.get("TB", 0) || n % 4 == 0) && m >= bm && n >= bn && k >= bk;
+  const bool aligned = s.get("ALIGN", 0) >= 16 && shortRows(n, k) && k % 4 == 0 && (s.get("TB", 0) || n % 4 == 0) && m >= bm && n >= bn && k >= bk;
   const bool d2l = s.get("D2L", 1) != 0 && !s.get("TA", 0) && (!s.get("TB", 0) || aligned) && (bk == 16 || bk == 32) && (!edge || aligned) && bm % 64 == 0 &&
                    (bn == 64 || bn == 128 || bn == 256) && bm % (32 * wm) == 0 && bn % (32 * wn) == 0 && (bm + bn) * bk * 8 <= 160 * 1024;
   s.p["D2L"] = d2l;
@@ -710,7 +714,7 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   bool own = false;
   for (const char* key : {"BM", "BN", "BK", "WM", "WN", "M16", "D2L", "BTR", "BPAD", "STAGES", "NBUF", "SK_UNITS", "INTERLEAVE", "SETPRIO"}) own = own || s.has(key);
   const Gemm16Form* form = nullptr;
-  if (!own && s.get("ALIGN", 0) >= 16 && !s.get("TA", 0) && k % 8 == 0 && (s.get("TB", 0) || n % 8 == 0)) form = chooseGemm16Form(m, n, k, batch);
+  if (!own && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !s.get("TA", 0) && k % 8 == 0 && (s.get("TB", 0) || n % 8 == 0)) form = chooseGemm16Form(m, n, k, batch);
   if (form) {
     s.p["BM"] = form->bm; s.p["BN"] = form->bn; s.p["WM"] = form->wm; s.p["WN"] = form->wn;
     s.p["M16"] = 1; s.p["D2L"] = 1; s.p["NBUF"] = form->nbuf;
@@ -738,7 +742,7 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   // operands' addresses; without it the guarded loads, which take any address, stay) and no tail split.
   // fewer rows than one tile: the rows past the last are read from the last one (GB_CLAMP; direct loads only)
   const bool clamp = (m < bm || fewRows) && batch == 1 && s.get("D2L", 1) != 0;
-  const bool canShift = s.get("ALIGN", 0) >= 16 && (m >= bm || clamp) && n >= bn && k >= bk && k % 8 == 0 && (!s.get("TA", 0) || m % 8 == 0) &&
+  const bool canShift = s.get("ALIGN", 0) >= 16 && shortRows(n, k) && (m >= bm || clamp) && n >= bn && k >= bk && k % 8 == 0 && (!s.get("TA", 0) || m % 8 == 0) &&
                         (s.get("TB", 0) || n % 8 == 0) && s.get("SK_UNITS", 0) <= 0;
   // the 16x16x32 MFMA (see the kernel): whole 64-deep k-tiles, A contiguous along k, B contiguous along k or read
   // through the transposing LDS reads, loads without guards
@@ -865,7 +869,7 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   int64_t dm, dn;
   defaultGemmTile(m, n, batch, dm, dn);
   const bool whole = m % dm == 0 && n % dn == 0 && k % 128 == 0;
-  if (!own && !whole && s.get("ALIGN", 0) >= 16 && !ta && k % 16 == 0 && n % 16 == 0 && s.get("SCALE_PTR", 0) == 0) {
+  if (!own && !whole && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !ta && k % 16 == 0 && n % 16 == 0 && s.get("SCALE_PTR", 0) == 0) {
     const Gemm16Form* form = chooseGemm16Form(m, n, k / 2, batch);
     if (form && form->bm == 256) {
       shift256 = true;
