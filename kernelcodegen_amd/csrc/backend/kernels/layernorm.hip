@@ -65,17 +65,16 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
     for (int j = 0; j < LN_VW; ++j) r[j] = (float)x[j];
     return r;
   };
-  // elements idx .. of p, a run of LN_N (gamma, beta: periods of `period`); zeros behind its end
-  auto load_vec = [&](const LN_IO* __restrict__ p, int idx, int period, auto once) __attribute__((always_inline)) -> vec_t {
+#if LN_N % LN_VW
+  // elements idx .. of p, LN_N in all; zeros behind its end
+  auto load_any = [&](const LN_IO* __restrict__ p, int idx, auto once) __attribute__((always_inline)) -> vec_t {
     vec_t r;
-    if (idx + LN_VW <= LN_N) {
-      const io_vec_t* at = (const io_vec_t*)(p + idx % period);
-      return widen(kcg_stream_load<decltype(once)::v>(at));
-    }
+    if (idx + LN_VW <= LN_N) return widen(kcg_stream_load<decltype(once)::v>((const io_vec_t*)(p + idx)));
 #pragma unroll
-    for (int j = 0; j < LN_VW; ++j) r[j] = LN_N % LN_VW != 0 && idx + j < LN_N ? (float)p[idx + j] : 0.0f;
+    for (int j = 0; j < LN_VW; ++j) r[j] = idx + j < LN_N ? (float)p[idx + j] : 0.0f;
     return r;
   };
+#endif
   const int tid = threadIdx.x;
   const int tr = tid % LN_TPR;               // position inside the row team
   const int rb = tid / LN_TPR;               // row inside the block
@@ -98,8 +97,18 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
 #pragma unroll
   for (int i = 0; i < LN_VPT; ++i) {
     const int idx = (i * LN_TPR + tr) * LN_VW;
-    g[i] = load_vec(G, idx, LN_NG, KcgLnOnce<false>{});
-    b[i] = load_vec(Bt, idx, LN_NB, KcgLnOnce<false>{});
+#if LN_N % LN_VW
+    g[i] = load_any(G, idx, KcgLnOnce<false>{});
+    b[i] = load_any(Bt, idx, KcgLnOnce<false>{});
+#else
+    if (idx < LN_N) {
+      g[i] = widen(*(const io_vec_t*)(G + (idx % LN_NG)));
+      b[i] = widen(*(const io_vec_t*)(Bt + (idx % LN_NB)));
+    } else {
+#pragma unroll
+      for (int j = 0; j < LN_VW; ++j) { g[i][j] = 0.0f; b[i][j] = 0.0f; }
+    }
+#endif
   }
 #endif
 
@@ -109,8 +118,12 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
 #pragma unroll
     for (int i = 0; i < LN_VPT; ++i) {
       const int idx = (i * LN_TPR + tr) * LN_VW;
-      if (live) {
-        dst[i] = load_vec(x, idx, LN_N, KcgLnOnce<LN_STREAM != 0>{});   // read once: 3-4 % faster from HBM with the hint, 10 % slower when the input is still in the last-level cache
+      if (live && idx < LN_N) {
+#if LN_N % LN_VW
+        dst[i] = load_any(x, idx, KcgLnOnce<LN_STREAM != 0>{});
+#else
+        dst[i] = widen(kcg_stream_load<LN_STREAM != 0>((const io_vec_t*)(x + idx)));   // read once: 3-4 % faster from HBM with the hint, 10 % slower when the input is still in the last-level cache
+#endif
       } else {
 #pragma unroll
         for (int j = 0; j < LN_VW; ++j) dst[i][j] = 0.0f;
@@ -226,7 +239,11 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
       if (live && idx < LN_N) {
         io_vec_t o;
 #if LN_LEAN
-        const vec_t gi = load_vec(G, idx, LN_NG, KcgLnOnce<false>{}), bi = load_vec(Bt, idx, LN_NB, KcgLnOnce<false>{});
+#if LN_N % LN_VW
+        const vec_t gi = load_any(G, idx, KcgLnOnce<false>{}), bi = load_any(Bt, idx, KcgLnOnce<false>{});
+#else
+        const vec_t gi = widen(*(const io_vec_t*)(G + (idx % LN_NG))), bi = widen(*(const io_vec_t*)(Bt + (idx % LN_NB)));
+#endif
 #else
         const vec_t gi = g[i], bi = b[i];
 #endif
@@ -238,13 +255,14 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
 #endif
           o[j] = (LN_IO)t;
         }
-        if (LN_N % LN_VW == 0 || idx + LN_VW <= LN_N) {
-          __builtin_nontemporal_store(o, (io_vec_t*)(y + idx));
-        } else {
+#if LN_N % LN_VW
+        if (idx + LN_VW > LN_N) {
 #pragma unroll
           for (int j = 0; j + 1 < LN_VW; ++j)
             if (idx + j < LN_N) y[idx + j] = o[j];
-        }
+        } else
+#endif
+        __builtin_nontemporal_store(o, (io_vec_t*)(y + idx));
       }
     }
 #if !LN_LEAN
