@@ -1035,7 +1035,7 @@ bool emitFmhaBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   // 38.8 and 26.9; B1 H32 S2048 D128 causal 69.3 and 57.3, with pairs).  Above that 256 stays ahead: B3 H12 S1300 D64 with 216
   // workgroups 28.5 against 31.4; causal with 192 pairs B4 H32 S600 D128 41 against 64, B4 H12 S2048 D64 46 against 61.
   const bool masked = s.get("CAUSAL", 0) != 0;
-  bool own = s.get("BR", 0) > 0 || s.get("BC", 0) > 0 || s.get("QW", 0) > 0;
+  bool own = !s.get("FILL", 0) || s.get("BR", 0) > 0 || s.get("BC", 0) > 0 || s.get("QW", 0) > 0;    // (on request: FILL)
   for (const char* key : {"D2L", "PAIR", "PERSIST", "OCC", "STAGE_O"}) own = own || s.has(key);
   const double heads = (double)b * (double)h, jobs = (double)ceilDiv(sl, br) * heads / (masked && ((b * h) % 2 == 0 || ceilDiv(sl, br) % 2 == 0) ? 2.0 : 1.0);
   bool noPair = false;
@@ -1139,7 +1139,7 @@ bool emitFmhaF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     // longest query tiles: half the tile evens that out (B4 H32 S512 D128 139 and 103 us, B1 H32 S2048 D128 520 and 341;
     // one round loses, B1 H32 S1024 D128 146 and 166, more gain nothing, B8 H32 S640 D128 342 and 350).
     const double tiles = (double)ceilDiv(sl, 128) * (double)b * (double)h;
-    if (s.get("CAUSAL", 0) && dh > 64 && br == 128 && !s.has("PAIR") && !s.has("D2L") && tiles > 256.0 && tiles <= 512.0) br = 64;
+    if (s.get("FILL", 0) && s.get("CAUSAL", 0) && dh > 64 && br == 128 && !s.has("PAIR") && !s.has("D2L") && tiles > 256.0 && tiles <= 512.0) br = 64;
   }
   if (br % 32 || br > 512) { err = "fmha_f32: BR must be a multiple of 32, at most 512"; return false; }
   // keys per LDS tile: 64 for head dims above 64 while two workgroups' tiles fit the LDS together, else 32 (measured at

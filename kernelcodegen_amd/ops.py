@@ -190,10 +190,10 @@ def fmha(q, k, v, scale=None, causal=False, out_dtype=None, **cfg):
         b, h, s, d = q.shape
         scale = d ** -0.5 if scale is None else scale
         if q.dtype == torch.float32:
-            kern = R.get_kernel("fmha_f32", B=b, H=h, S=s, D=d, CAUSAL=int(causal), SCALE=scale, **cfg)
+            kern = R.get_kernel("fmha_f32", B=b, H=h, S=s, D=d, CAUSAL=int(causal), SCALE=scale, **{"FILL": 1, **cfg})
         else:
             kern = R.get_kernel("fmha_bf16", B=b, H=h, S=s, D=d, CAUSAL=int(causal), SCALE=scale,
-                                OUT_BF16=int(out_dtype == q.dtype), F16=int(q.dtype == torch.float16), **cfg)
+                                OUT_BF16=int(out_dtype == q.dtype), F16=int(q.dtype == torch.float16), **{"FILL": 1, **cfg})
         run = _bind(key, cfg, kern)
     o = torch.empty(q.shape, dtype=out_dtype, device=q.device)
     run(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr())
