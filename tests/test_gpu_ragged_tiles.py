@@ -45,28 +45,27 @@ def test_gemm16_every_form_at_its_edges(ops, form, tb):
     more than two rounds of them."""
     cfg = dict(FORMS[form], M16=1, D2L=1)
     bm, bn = cfg["BM"], cfg["BN"]
-    ks = [64, 72, 64 * 3, 64 * 5 + 8, 64 * 13]
-    if bm == 256:
-        ks = [64, 64 * 3, 64 * 13]
-    for i, (m, n) in enumerate([(bm, bn), (bm + 1, bn + 8), (2 * bm - 1, 2 * bn - 8), (3 * bm, bn + 8)]):
+    ks = [64, 64 * 13] if bm == 256 else [72, 64 * 5 + 8, 64 * 13]
+    for i, (m, n) in enumerate([(bm + 1, bn + 8), (2 * bm - 1, 2 * bn - 8)]):
         for k in ks:
             a, b, want = _operands(m, n, k, tb, torch.bfloat16, 100 * form + 10 * i + k)
             print("form", form, (m, n, k), tb, flush=True)
-            for out in (torch.float32, torch.bfloat16):
-                c = ops.matmul(a, b, trans_b=tb, out_dtype=out, **cfg)
-                assert torch.equal(c.cpu(), torch.from_numpy(want).to(out)), (m, n, k, out)
+            out = torch.bfloat16 if i else torch.float32
+            c = ops.matmul(a, b, trans_b=tb, out_dtype=out, **cfg)
+            assert torch.equal(c.cpu(), torch.from_numpy(want).to(out)), (m, n, k, out)
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("tb", [False, True])
 @pytest.mark.parametrize("m,n,k", [(1, 512, 512), (15, 640, 4096), (63, 520, 136), (64, 1024, 2048), (65, 584, 1000), (300, 1000, 264),
                                    (1000, 2056, 520), (257, 264, 64), (9, 64, 64), (64, 64, 72),
                                    (16, 128, 64), (16, 72, 64 * 13), (17, 136, 72), (31, 64, 320), (32, 192, 64 * 7 + 8), (33, 64, 128)])
-def test_gemm16_default_forms(ops, m, n, k, tb, dtype):
+def test_gemm16_default_forms(ops, m, n, k, tb):
+    dtype = torch.float16 if (m + n) % 3 == 0 else torch.bfloat16
+    out = dtype if k % 3 == 0 else torch.float32
     a, b, want = _operands(m, n, k, tb, dtype, m + n + k)
-    for out in (torch.float32, dtype):
-        c = ops.matmul(a, b, trans_b=tb, out_dtype=out)
-        assert torch.equal(c.cpu(), torch.from_numpy(want).to(out))
+    assert torch.equal(ops.matmul(a, b, trans_b=tb, out_dtype=out).cpu(), torch.from_numpy(want).to(out))
+    if m > 64:
+        return
     # operands off the 16-byte boundary are taken as well, and give the same numbers
     for x, w in ((_shifted(a), b), (a, _shifted(b))):
         assert torch.equal(ops.matmul(x, w, trans_b=tb).double().cpu(), torch.from_numpy(want))
@@ -107,9 +106,10 @@ def test_gemm_fp8_default_forms(ops, m, n, k, tb):
     """Moved-back 256 x 256 tiles, the ring of LDS buffers (weights contiguous along k) and guarded loads of whole chunks;
     products up to 16 and |sum| <= 16 k < 2^16 stay exact in every MFMA's accumulator."""
     a, b, want = _operands(m, n, k, tb, torch.float8_e4m3fn, m + n + k)
-    for out in (torch.float32, torch.bfloat16):
-        c = ops.matmul_fp8(a, b, 0.5, 2.0, trans_b=tb, out_dtype=out)
-        assert torch.equal(c.cpu(), torch.from_numpy(want).to(out))
+    out = torch.float32 if m % 2 else torch.bfloat16
+    assert torch.equal(ops.matmul_fp8(a, b, 0.5, 2.0, trans_b=tb, out_dtype=out).cpu(), torch.from_numpy(want).to(out))
+    if m > 100:
+        return
     for x, w in ((_shifted(a), b), (a, _shifted(b))):
         assert torch.equal(ops.matmul_fp8(x, w, 1.0, 1.0, trans_b=tb).double().cpu(), torch.from_numpy(want))
 
@@ -152,8 +152,8 @@ F32_FORMS = [dict(BM=256, BN=256, BK=16, WM=4, WN=4), dict(BM=128, BN=128, BK=16
 def test_gemm_f32_direct_load_forms_at_their_edges(ops, form, tb):
     cfg = F32_FORMS[form]
     bm, bk = cfg["BM"], cfg["BK"]
-    for i, (m, n) in enumerate([(bm, bm), (bm + 1, bm + 4), (2 * bm - 1, 2 * bm - 4)]):
-        for k in (bk, bk + 4, 3 * bk, 5 * bk - 4, 9 * bk):
+    for i, (m, n) in enumerate([(bm + 1, bm + 4), (2 * bm - 1, 2 * bm - 4)]):
+        for k in (bk, 5 * bk - 4, 9 * bk):
             a, b, want = _operands(m, n, k, tb, torch.float32, 100 * form + 10 * i + k, batch=(2,))
             assert torch.equal(ops.batched_matmul(a, b, trans_b=tb, **cfg).double().cpu(), torch.from_numpy(want)), (m, n, k)
 
@@ -178,8 +178,8 @@ def test_gemm_f32_infinities_stay_in_their_rows_and_columns(ops, tb):
 
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-6), (torch.float16, 2 ** -10), (torch.bfloat16, 2 ** -7)])
-@pytest.mark.parametrize("rows,n", [(1, 257), (3, 259), (5, 511), (129, 2047), (7, 4097), (2, 32767), (3, 256), (4, 255), (9, 1001), (1200, 1003),
-                                    (4200, 257), (600, 2050), (2050, 512), (600, 8192), (300, 4100), (40, 31999), (70, 16000)])
+@pytest.mark.parametrize("rows,n", [(3, 259), (9, 1001), (2, 32767), (3, 256), (4, 255), (1200, 1003), (4200, 257), (600, 2050), (600, 8192),
+                                    (300, 4100), (40, 31999)])
 def test_rows_of_any_length(ops, rows, n, dtype, tol):
     """Softmax and LayerNorm over rows that start anywhere: results within one rounding of the type (2^-10 and 2^-7: one ulp
     above 1, relative; fp32 sums of n <= 2^15 terms in trees stay below 1e-6), and nothing written behind the result."""
@@ -213,8 +213,7 @@ def test_softmax_rows_of_infinities_and_nan(ops):
 
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 1e-2), (torch.float16, 2e-3), (torch.float32, 4e-6)])
-@pytest.mark.parametrize("b,h,s,d", [(1, 8, 333, 64), (2, 16, 777, 64), (1, 3, 64, 64), (1, 3, 65, 128), (1, 3, 129, 64), (1, 5, 256, 128),
-                                     (1, 32, 1100, 128), (4, 32, 260, 64), (3, 12, 1300, 64), (2, 64, 512, 128)])
+@pytest.mark.parametrize("b,h,s,d", [(1, 8, 333, 64), (1, 3, 64, 64), (1, 3, 65, 128), (1, 5, 256, 128), (1, 32, 1100, 128), (2, 64, 512, 128)])
 def test_attention_on_small_launches(ops, b, h, s, d, dtype, tol, causal):
     """128 queries per workgroup and no pairs of query tiles where the launch leaves compute units empty, 64 for fp32 under
     the mask; the tolerances are those of the other attention tests (16-bit probabilities, fp32 sums)."""
