@@ -741,7 +741,9 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   // whole tile in every dimension, rows that start on 16-byte boundaries (ALIGN = 16: the caller has looked at the
   // operands' addresses; without it the guarded loads, which take any address, stay) and no tail split.
   // fewer rows than one tile: the rows past the last are read from the last one (GB_CLAMP; direct loads only)
-  const bool clamp = (m < bm || fewRows) && batch == 1 && s.get("D2L", 1) != 0;
+  // (tiles of at most 64 rows: a lane's 32-bit offset spans the rows of the tile, and the whole-row epilogue of the 256 x 256
+  // tile stores every row that it holds)
+  const bool clamp = ((m < bm && bm <= 64) || fewRows) && batch == 1 && s.get("D2L", 1) != 0;
   const bool canShift = s.get("ALIGN", 0) >= 16 && shortRows(n, k) && (m >= bm || clamp) && n >= bn && k >= bk && k % 8 == 0 && (!s.get("TA", 0) || m % 8 == 0) &&
                         (s.get("TB", 0) || n % 8 == 0) && s.get("SK_UNITS", 0) <= 0;
   // the 16x16x32 MFMA (see the kernel): whole 64-deep k-tiles, A contiguous along k, B contiguous along k or read

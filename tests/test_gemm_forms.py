@@ -1,0 +1,32 @@
+"""Which form of the GEMM kernels a set of parameters gets, and that every set the emitter accepts compiles (no GPU needed)."""
+import pytest
+
+from kernelcodegen_amd import _lib, runtime as R
+
+TILE256 = dict(BM=256, BN=256, WM=4, WN=2)
+TILE128 = dict(BM=128, BN=128, WM=4, WN=2)
+
+
+def defines(family, **params):
+    """The parameters in front of the emitted kernel (its leading #define lines) as a dict."""
+    text, _ = R.emit_kernel(family, "kernel0", **params)
+    out = {}
+    for line in text.splitlines():
+        if not line.startswith("#define "):
+            break
+        out.update([line.split(None, 2)[1:]])
+    return out
+
+
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("tile", [TILE256, TILE128])
+@pytest.mark.parametrize("extra", [dict(OUT_BF16=1), dict(STAGE_C=1), dict(OUT_BF16=1, D2L=1), dict(K=520)])
+def test_rows_are_clamped_in_tiles_of_at_most_64_rows_only(tile, tb, extra):
+    """A 256-row tile leaves through LDS as whole rows, those past the last included: fewer rows than such a tile must not
+    reach the 16x16x32 form (its stores would run past the end of C)."""
+    params = dict(dict(M=100, N=512, K=512, TB=tb, ALIGN=16, **tile), **extra)
+    with pytest.raises(_lib.KcgError):
+        R.emit_kernel("gemm_bf16", "kernel0", M16=1, **params)
+    params.pop("D2L", None)
+    d = defines("gemm_bf16", **params)
+    assert d["GB_EDGE"] == "1" and "GB_CLAMP" not in d and "GB_SHIFT" not in d and "GB_STAGE_C" not in d
