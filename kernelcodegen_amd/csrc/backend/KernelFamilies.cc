@@ -762,14 +762,14 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   // 2048 x 8192 x 2048) and level with the other form for [N][K].
   const bool m16 = s.get("M16", m16Fits && d2lFits && !clamp && bm == 256 && bn == 256 && waves == 8 && s.get("D2L", 1)) != 0;
   s.p["M16"] = m16;
+  // row-major weights in other tiles than 256 columns of eight wavefronts: on request, and in the forms chosen above
+  const bool d2l = m16 && s.get("D2L", d2lFits && (s.get("TB", 0) || (bn == 256 && waves == 8))) != 0;
   // a K that is no multiple of BK: the last k-tile is moved back as well, where the direct loads are used
-  const bool kTail = k % bk != 0 && canShift && m16 && d2lFits && s.get("D2L", 1) != 0;
-  const bool shift = ragged && canShift && (k % bk == 0 || kTail) && (!clamp || (m16 && d2lFits));
+  const bool kTail = k % bk != 0 && canShift && d2l && d2lFits;
+  const bool shift = ragged && canShift && (k % bk == 0 || kTail) && (!clamp || (d2l && d2lFits));
   const bool edge = ragged && !shift;
   s.p["SHIFT"] = shift;
   if (m16 && (!m16Fits || edge)) { err = "gemm_bf16: M16 needs full 64-deep tiles, TA = 0, one staging set and no tail split"; return false; }
-  // row-major weights in other tiles than 256 columns of eight wavefronts: on request, and in the forms chosen above
-  const bool d2l = m16 && s.get("D2L", d2lFits && (s.get("TB", 0) || (bn == 256 && waves == 8))) != 0;
   s.p["D2L"] = d2l;
   if (fewRows && !(shift && clamp && d2l)) { err = "gemm_bf16: tiles of 32 rows need aligned operands and direct loads"; return false; }
   if (d2l && !d2lFits) { err = "gemm_bf16: D2L needs M16 and whole 1 KiB blocks per wavefront (row-major weights: BN = 64, 128 or 256)"; return false; }

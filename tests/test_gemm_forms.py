@@ -30,3 +30,22 @@ def test_rows_are_clamped_in_tiles_of_at_most_64_rows_only(tile, tb, extra):
     params.pop("D2L", None)
     d = defines("gemm_bf16", **params)
     assert d["GB_EDGE"] == "1" and "GB_CLAMP" not in d and "GB_SHIFT" not in d and "GB_STAGE_C" not in d
+
+
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("m,n,k", [(300, 512, 520), (100, 512, 512), (40, 512, 512), (300, 520, 576), (256, 512, 520), (300, 512, 512)])
+@pytest.mark.parametrize("tile", [TILE128, TILE256, dict(BM=64, BN=64, WM=2, WN=2), dict(BM=64, BN=128, WM=2, WN=2), dict(BM=128, BN=256, WM=2, WN=4)])
+def test_tiles_asked_for_without_direct_loads_are_refused_or_compile(tile, m, n, k, tb):
+    """M16 without D2L: row-major weights in tiles of fewer than 256 columns go through registers then, which can move tiles
+    back but neither a k-tile nor clamp rows; the emitter says so, or what it emits compiles."""
+    for extra in (dict(), dict(D2L=0)):
+        params = dict(M=m, N=n, K=k, TB=tb, ALIGN=16, M16=1, **dict(tile, **extra))
+        try:
+            text, _ = R.emit_kernel("gemm_bf16", "kernel0", **params)
+        except _lib.KcgError:
+            continue
+        d = defines("gemm_bf16", **params)
+        if "GB_D2L" not in d:
+            assert "GB_KTAIL" not in d and "GB_CLAMP" not in d, params
+        if m + k < 900 and n == 512:          # every branch above with few kernels to compile
+            assert R.compile_to_code(R.prelude() + text)
