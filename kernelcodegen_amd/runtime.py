@@ -205,7 +205,12 @@ class Kernel:
         address, handle, entry, stream = C.addressof(dims), self.handle, lib().kcg_hip_launch_packed, _current_stream()
 
         def run(*values, _keep=(dims, self)):
-            rc = entry(handle, address, stream(), pack(*values), n)
+            try:
+                slots = pack(*values)
+            except OverflowError:       # struct refuses a number above the fp32 range; as a C float it is infinity
+                at = n - scalars
+                slots = pack(*values[:at], *(C.c_float(v).value for v in values[at:]))
+            rc = entry(handle, address, stream(), slots, n)
             if rc:
                 check(rc, "kcg_hip_launch_packed")
         return run

@@ -1,0 +1,41 @@
+"""What a bound launch passes on, and what the operators' keys keep apart, without a GPU: the entry points that would launch are
+replaced by recorders."""
+import ctypes as C
+import struct
+
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from kernelcodegen_amd import ops, runtime as R
+
+
+class Recorder:
+    """Stands for the library: keeps what kcg_hip_launch_packed was given."""
+
+    def __init__(self):
+        self.calls = []
+
+    def kcg_hip_launch_packed(self, handle, dims, stream, slots, n):
+        self.calls.append((list((C.c_uint32 * 7).from_address(dims)), stream, bytes(slots), n))
+        return 0
+
+
+@pytest.fixture
+def recorder(monkeypatch):
+    r = Recorder()
+    monkeypatch.setattr(R, "lib", lambda: r)
+    monkeypatch.setattr(R, "_current_stream", lambda: lambda: 77)
+    return r
+
+
+def test_scalars_beyond_fp32_become_infinity(recorder):
+    """As a C float argument: a finite number above the fp32 range is not an error."""
+    kern = R.Kernel(None, 5, dict(grid=(1, 2, 3), block=(64, 1, 1), lds_bytes=9, num_args=5, workspace_bytes=0))
+    run = kern.bind(scalars=2)
+    for value in (0.5, -2.0, 1e39, -1e39, 3.4028235677973366e38, 1e-46, float("inf"), float("-inf"), 0.1, float("nan")):
+        run(1, 2, 3, value, 0.25)
+        dims, stream, slots, n = recorder.calls[-1]
+        assert dims == [1, 2, 3, 64, 1, 1, 9] and stream == 77 and n == 5
+        assert slots[:24] == struct.pack("<3Q", 1, 2, 3)
+        assert slots[24:28] == bytes(C.c_float(value)) and slots[32:36] == bytes(C.c_float(0.25))
