@@ -111,7 +111,7 @@ def _matmul_launch(a, b, trans_a, trans_b, out_dtype, cfg):
     n, k2 = (b.shape[-2], b.shape[-1]) if trans_b else (b.shape[-1], b.shape[-2])
     if k != k2:
         raise ValueError("incompatible K dimensions")
-    extra = {}
+    extra, align = {}, {}
     if out_dtype is None:
         out_dtype = torch.float64 if a.dtype == torch.float64 else torch.float32
     if a.dtype in (torch.bfloat16, torch.float16):
@@ -120,16 +120,17 @@ def _matmul_launch(a, b, trans_a, trans_b, out_dtype, cfg):
         extra["OUT_BF16"] = int(out_dtype == a.dtype)       # a 16-bit result, of the operands' type
         if a.dtype == torch.float16:
             extra["F16"] = 1
-        extra.update(_alignment(_aligned(a, b)))
+        align = _alignment(_aligned(a, b))
     elif a.dtype == torch.float64:
         if out_dtype != torch.float64:
             raise ValueError("fp64 GEMM writes fp64")
     elif out_dtype != torch.float32:
         raise ValueError("fp32 GEMM writes fp32")
     else:
-        extra.update(_alignment(_aligned(a, b)))
+        align = _alignment(_aligned(a, b))
+    # (the caller's parameters go before the alignment's, and may not name any other)
     kern = R.get_kernel(_FAMILY[a.dtype], M=m, N=n, K=k, BATCH=batch, TA=int(trans_a), TB=int(trans_b),
-                        **{**extra, **cfg})
+                        **extra, **{**align, **cfg})
     if kern.info["workspace_bytes"]:
         return (lambda *p: kern.launch(*p)), tuple(a.shape[:-2]) + (m, n), out_dtype
     return kern.bind(), tuple(a.shape[:-2]) + (m, n), out_dtype

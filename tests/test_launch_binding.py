@@ -39,3 +39,38 @@ def test_scalars_beyond_fp32_become_infinity(recorder):
         assert dims == [1, 2, 3, 64, 1, 1, 9] and stream == 77 and n == 5
         assert slots[:24] == struct.pack("<3Q", 1, 2, 3)
         assert slots[24:28] == bytes(C.c_float(value)) and slots[32:36] == bytes(C.c_float(0.25))
+
+
+@pytest.fixture
+def kernels(monkeypatch):
+    """The parameters that the operators ask kernels for; every kernel's bound launch does nothing."""
+    asked = []
+
+    class Kern:
+        info = dict(workspace_bytes=0)
+
+        def bind(self, scalars=0):
+            return lambda *values: None
+
+    def get_kernel(family, **params):
+        asked.append((family, params))
+        return Kern()
+
+    monkeypatch.setattr(R, "get_kernel", get_kernel)
+    monkeypatch.setattr(ops, "_need_cuda", lambda *ts: None)
+    monkeypatch.setattr(ops, "_bound", {})
+    return asked
+
+
+def test_parameters_that_follow_from_the_operands_cannot_be_overridden(kernels):
+    """The result's tensor is allocated from out_dtype and the operands: a kernel told otherwise would write another size."""
+    a, b = torch.zeros(64, 64, dtype=torch.float16), torch.zeros(64, 64, dtype=torch.float16)
+    for key in ("OUT_BF16", "F16", "M", "N", "K", "BATCH", "TA", "TB"):
+        with pytest.raises(TypeError):
+            ops.batched_matmul(a, b, **{key: 1})
+    f8 = a.to(torch.float8_e4m3fn)
+    with pytest.raises(TypeError):
+        ops.matmul_fp8(f8, f8, 1.0, 1.0, OUT_BF16=1)
+    assert not kernels
+    ops.batched_matmul(a, b, ALIGN=0, D2L=0)
+    assert kernels[0][1]["ALIGN"] == 0 and kernels[0][1]["D2L"] == 0
