@@ -3,6 +3,7 @@ operator instance, compile it once, launch it on torch device tensors.
 Shapes are static (baked into the kernel), like every kernel the generator
 emits."""
 import math
+import operator
 
 import torch
 
@@ -34,7 +35,8 @@ _STORAGE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
 def layernorm(x, gamma, beta, axis, eps=1e-5, gelu=False, out=None, **cfg):
     _need_cuda(x, gamma, beta)
-    eps, gelu = float(eps), int(gelu)          # plain numbers: a key must not hold an object that can change
+    # plain numbers: a key must not hold an object that can change, nor find 1 for a refused 1.0
+    axis, eps, gelu = operator.index(axis), float(eps), int(gelu)
     key = ("layernorm", x.shape, x.dtype, gamma.shape, gamma.dtype, beta.shape, beta.dtype, axis, eps, gelu)
     run = None if cfg else _bound.get(key)
     if run is None:
@@ -247,6 +249,7 @@ def gather(x, indices, axis=0, **cfg):
     _need_cuda(x, indices)
     if indices.dtype != torch.int64:
         raise ValueError("gather indices must be int64")
+    axis = operator.index(axis)
     if not -x.dim() <= axis < x.dim():
         raise ValueError("axis out of range")
     key = ("gather", x.shape, x.dtype, indices.shape, axis)

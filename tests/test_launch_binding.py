@@ -74,3 +74,15 @@ def test_parameters_that_follow_from_the_operands_cannot_be_overridden(kernels):
     assert not kernels
     ops.batched_matmul(a, b, ALIGN=0, D2L=0)
     assert kernels[0][1]["ALIGN"] == 0 and kernels[0][1]["D2L"] == 0
+
+
+def test_an_axis_is_a_whole_number_on_every_call(kernels):
+    """1.0 == 1 as a dictionary key: a call that is refused must not find the launch that an accepted one has bound."""
+    x, g = torch.zeros(4, 8), torch.zeros(8)
+    ops.layernorm(x, g, g, 1)
+    with pytest.raises(TypeError):
+        ops.layernorm(x, g, g, 1.0)
+    ids = torch.zeros(3, dtype=torch.int64)
+    ops.gather(x, ids, 1)
+    with pytest.raises(TypeError):
+        ops.gather(x, ids, 1.0)
