@@ -76,12 +76,17 @@ def elementwise(x, op, inplace=False, out_dtype=None, **cfg):
 
 
 def _aligned(a, b):
-    """True when both operands start on a 16-byte boundary, which the direct loads into LDS need."""
-    return not (a.data_ptr() | b.data_ptr()) & 15
+    """What both operands' addresses are multiples of: 16, 4, or less (1)."""
+    low = a.data_ptr() | b.data_ptr()
+    return 1 if low & 3 else 4 if low & 15 else 16
 
 
 def _alignment(aligned):
-    return {"ALIGN": 16} if aligned else {"D2L": 0}
+    """The kernel parameters for it.  Direct loads into LDS take any address that is a multiple of four bytes, so those give
+    the kernels that whole tiles get without looking (fp32 1024^3 off a 16-byte boundary: 21 us, 26 through registers; bf16
+    4096^3 with row-major weights: 112 and 129); the forms for all sizes split rows into 16-byte chunks and are for ALIGN = 16.
+    Other addresses go through registers."""
+    return {"ALIGN": 16} if aligned == 16 else {} if aligned == 4 else {"D2L": 0}
 
 
 _FAMILY = {torch.float32: "gemm_f32", torch.float64: "gemm_f64", torch.bfloat16: "gemm_bf16", torch.float16: "gemm_bf16"}

@@ -24,10 +24,10 @@ def _operands(m, n, k, tb, dtype, seed, batch=()):
     return torch.from_numpy(a).cuda().to(dtype), torch.from_numpy(b).cuda().to(dtype), want
 
 
-def _shifted(t):
-    """The same values one element behind a 16-byte boundary."""
-    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
-    out = buf[1:].view(t.shape)
+def _shifted(t, elements=1):
+    """The same values `elements` (one) behind a 16-byte boundary."""
+    buf = torch.empty(t.numel() + elements, dtype=t.dtype, device=t.device)
+    out = buf[elements:].view(t.shape)
     out.copy_(t)
     assert out.data_ptr() % 16 != 0 and out.is_contiguous()
     return out
@@ -69,6 +69,21 @@ def test_gemm16_default_forms(ops, m, n, k, tb):
     # operands off the 16-byte boundary are taken as well, and give the same numbers
     for x, w in ((_shifted(a), b), (a, _shifted(b))):
         assert torch.equal(ops.matmul(x, w, trans_b=tb).double().cpu(), torch.from_numpy(want))
+
+
+@pytest.mark.parametrize("tb", [False, True])
+def test_whole_tiles_off_a_16_byte_boundary(ops, tb):
+    """Operands on a multiple of four bytes keep the direct loads of whole tiles, others go through registers: the same numbers."""
+    for dtype, tile in ((torch.float32, 128), (torch.bfloat16, 512), (torch.float8_e4m3fn, 512)):
+        a, b, want = _operands(tile, 512, 256, tb, dtype, tile)
+        run = ops.matmul if dtype != torch.float8_e4m3fn else lambda x, w, **kw: ops.matmul_fp8(x, w, 1.0, 1.0, **kw)
+        cfg = {} if dtype == torch.float32 else dict(BM=256, BN=256, WM=4, WN=2)
+        step = max(1, 4 // a.element_size())
+        for x, w in ((_shifted(a, step), b), (a, _shifted(b, 3 * step)), (_shifted(a, 2 * step), _shifted(b, step)), (_shifted(a), _shifted(b))):
+            assert torch.equal(run(x, w, trans_b=tb, **cfg).double().cpu(), torch.from_numpy(want))
+    a, b, want = _operands(128, 192, 256, False, torch.float32, 3)
+    cfg = dict(BM=64, BN=64, BK=32, WM=2, WN=2, WK=2, NBUF=3)
+    assert torch.equal(ops.matmul(_shifted(a), _shifted(b, 2), **cfg).double().cpu(), torch.from_numpy(want))
 
 
 def test_gemm16_column_count_no_multiple_of_eight(ops):

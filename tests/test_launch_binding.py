@@ -86,3 +86,31 @@ def test_an_axis_is_a_whole_number_on_every_call(kernels):
     ops.gather(x, ids, 1)
     with pytest.raises(TypeError):
         ops.gather(x, ids, 1.0)
+
+
+def _off(t, elements):
+    """The same shape `elements` behind a 64-byte boundary."""
+    buf = torch.zeros(t.numel() + elements + 64, dtype=t.dtype)
+    skip = -(buf.data_ptr() // t.element_size()) % (64 // t.element_size()) + elements
+    return buf[skip:skip + t.numel()].view(t.shape)
+
+
+def test_operands_off_a_16_byte_boundary_keep_the_direct_loads(kernels):
+    """Whole tiles of operands on multiples of four bytes keep the kernels that they get without a look at the addresses, and
+    what is asked of those kernels; ragged sizes keep the loads that take any address."""
+    a, h, f8 = torch.zeros(256, 256), torch.zeros(512, 512, dtype=torch.bfloat16), torch.zeros(256, 256).to(torch.float8_e4m3fn)
+    for off in (0, 1, 3):
+        ops.matmul(_off(a, off), a)
+        ops.matmul(a, _off(a, off), BM=64, BN=64, BK=32, WM=2, WN=2, WK=2, NBUF=3)
+        ops.matmul(_off(h, 2 * off), h, BM=256, BN=256)
+        ops.matmul_fp8(_off(f8, 4 * off), f8, 1.0, 1.0, BM=256, BN=256, WM=4)
+    assert len(kernels) == 11          # (the first, bound by its key, is asked for once per alignment)
+    for family, params in kernels:
+        text, _ = R.emit_kernel(family, "kernel0", **params)
+        assert "global_load_lds" in text and ("#define GL_" in text or "#define G8_" in text or "#define GB_D2L 1\n" in text), (family, params)
+    del kernels[:]
+    ops.matmul(_off(h, 1), h)
+    ops.matmul(_off(h[:300], 2), h)
+    for family, params in kernels:
+        text, _ = R.emit_kernel(family, "kernel0", **params)
+        assert "#define GB_D2L 1\n" not in text and "#define GB_SHIFT 1\n" not in text, params
