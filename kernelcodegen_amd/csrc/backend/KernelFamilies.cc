@@ -697,7 +697,9 @@ static const Gemm16Form* chooseGemm16Form(int64_t m, int64_t n, int64_t k, int64
   double least = 0.0;
   for (const auto& f : forms) {
     if ((m < f.bm && (f.bm > 64 || batch != 1)) || n < f.bn || k < 64) continue;
-    if (k % 64 && f.bm == 256) continue;       // no register left for the moved-back k-tile: 1500 x 11008 x 1040 155 us against 60
+    // a moved-back k-tile costs this form up to 128 bytes of scratch a lane: 1500 x 11008 x 1040 70 us against 61 in 128 x 128 tiles,
+    // x 1104 68 against 65, x 4080 198 against 195; many rounds would gain all the same, 4001 x 11008 x 4072 492 against 325
+    if (k % 64 && f.bm == 256) continue;
     const double tiles = (double)ceilDiv(m, f.bm) * (double)ceilDiv(n, f.bn) * (double)batch, rounds = std::ceil(tiles / f.slots);
     if (f.bn == 128 && f.nbuf == 4 && rounds > 1) continue;     // one workgroup per CU pays in a single round only
     const double cost = rounds * (f.a + f.b * tiles / (rounds * f.slots));

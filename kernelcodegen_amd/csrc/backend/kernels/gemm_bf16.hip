@@ -13,7 +13,7 @@
 //   GB_SHIFT                     1: ragged M or N without guarded loads: the last tile of a row or column of tiles is moved
 //                                back to end at the edge (see the kernel)
 //   GB_CLAMP                     1: M <= GB_BM, one row of tiles: rows past the last are read from the last row and not
-//                                stored (direct loads only; GB_BM may be 32 then)
+//                                stored (direct loads and GB_BM <= 64 only; GB_BM may be 32 then)
 //   GB_NBUF                      LDS buffers per operand, 2 (default) to 6; more than two with direct loads only: the loads of
 //                                k-tile kt + GB_NBUF start with k-tile kt
 //   GB_KTAIL                     1: K is no multiple of GB_BK; the last k-tile is moved back likewise (direct loads only)
@@ -378,7 +378,7 @@ typedef _Float16 kcg_f16x8 __attribute__((ext_vector_type(8)));
 #if GB_NBUF != 2 && !GB_D2L
 #error "more than two LDS buffers: only with direct loads"
 #endif
-#if (GB_SHIFT && (GB_EDGE || GB_SK_UNITS > 0 || (GB_M < GB_BM && !GB_CLAMP) || GB_N < GB_BN)) || (GB_CLAMP && (!GB_D2L || !GB_SHIFT || GB_M > GB_BM)) || (GB_BM == 32 && GB_D2L && !GB_CLAMP) || (GB_KTAIL && (!GB_D2L || GB_K < GB_BK || GB_K % GB_BK == 0))
+#if (GB_SHIFT && (GB_EDGE || GB_SK_UNITS > 0 || (GB_M < GB_BM && !GB_CLAMP) || GB_N < GB_BN)) || (GB_CLAMP && (!GB_D2L || !GB_SHIFT || GB_M > GB_BM || GB_BM > 64)) || (GB_BM == 32 && GB_D2L && !GB_CLAMP) || (GB_KTAIL && (!GB_D2L || GB_K < GB_BK || GB_K % GB_BK == 0))
 #error "moved-back tiles: whole tiles must fit the operands; a moved-back k-tile needs direct loads"
 #endif
 #if GB_M16 && (GB_BK != 64 || GB_TA != 0 || (GB_TB == 0 && !GB_BTR) || GB_GUARD || GB_SK_UNITS > 0 || GB_STAGES != 1 || GB_NT % 128 || (GB_BM % (GB_NT / 8) && !GB_CLAMP) || (GB_TB == 1 && GB_BN % (GB_NT / 8)))
@@ -814,7 +814,7 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
         __builtin_amdgcn_s_waitcnt(GB_VMCNT(steady ? (GB_NBUF - 2) * (UA + UB) : 0));
 #endif
 #if GB_KTAIL
-        if (mode == 0 && kt + 2 == len) zero_tail(nbuf);
+        if (mode == 2 || (mode == 0 && kt + 2 == len)) zero_tail(nbuf);
 #endif
         __syncthreads();
         if (feed) {
@@ -834,7 +834,7 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
         if (!last) fb[0][j] = read_fb(buf, ks + 1, j);
         else if (feed) fb[0][j] = read_fb(nbuf, 0, j);
 #if GB_D2L
-        if (last && (steady || kt + GB_NBUF < len)) {
+        if (last && (steady || (mode == 0 && kt + GB_NBUF < len))) {
 #pragma unroll
           for (int u = 0; u < UA + UB; ++u)
             if (u * GB_TN / (UA + UB) == j) d2l_unit(u, (kt + GB_NBUF) * GB_BK, buf);
@@ -948,6 +948,18 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
   // a split segment has an even number of iterations (and one staging set): two are left, of known kinds
   iteration(kt, KcgInt<0>{}, KcgInt<2>{});
   iteration(kt + 1, KcgInt<1>{}, KcgInt<3>{});
+#elif GB_STAGES == 1 && GB_KT == 1
+  iteration(0, KcgInt<0>{}, KcgInt<3>{});
+#elif GB_STAGES == 1
+  // Two iterations are left, three of an odd count: all of known kinds.  Deciding buffer and kind at run time instead keeps two
+  // whole bodies' registers alive around a loop; 256 x 256 tiles on an odd count of k-tiles then held 596-708 bytes of scratch
+  // a lane (bf16, us: 1024 x 11008 x 4032 149 and now 90, 4096 x 4096 x 576 68 and 24, 4096 x 11008 x 4032 436 and 287, which is
+  // what 4096 x 11008 x 4096 takes).
+#if GB_KT % 2
+  iteration(GB_KT - 3, KcgInt<0>{}, KcgInt<1>{});
+#endif
+  iteration(GB_KT - 2, KcgInt<GB_KT % 2>{}, KcgInt<2>{});
+  iteration(GB_KT - 1, KcgInt<1 - GB_KT % 2>{}, KcgInt<3>{});
 #else
   for (; kt < len; ++kt) {
     if (kt & 1) iteration(kt, KcgInt<1>{}, KcgInt<0>{});

@@ -49,3 +49,31 @@ def test_tiles_asked_for_without_direct_loads_are_refused_or_compile(tile, m, n,
             assert "GB_KTAIL" not in d and "GB_CLAMP" not in d, params
         if m + k < 900 and n == 512:          # every branch above with few kernels to compile
             assert R.compile_to_code(R.prelude() + text)
+
+
+def scratch_bytes(code):
+    """Private segment size in a code object's metadata (one kernel): scratch memory per lane."""
+    at = code.index(b".private_segment_fixed_size") + len(b".private_segment_fixed_size")
+    size = {0xcc: 1, 0xcd: 2, 0xce: 4}.get(code[at], 0)          # MessagePack: uint8, uint16, uint32, else the number itself
+    return int.from_bytes(code[at + 1:at + 1 + size], "big") if size else code[at]
+
+
+# a size for each form of the 16-bit kernel that is chosen by itself: 256 x 256 tiles whole and moved back, 128 x 128 with two
+# and three buffers, 64 x 128 with three and four, 64 x 64, 32 x 64
+SIZES = [(4096, 4096), (1000, 11008), (2048, 4096), (1000, 2048), (300, 11008), (512, 4096), (128, 4096), (16, 4096)]
+
+
+@pytest.mark.parametrize("k", [64, 128, 192, 320, 384, 1088, 1152, 72, 136, 200, 584, 1040, 1104])
+def test_no_form_of_the_16_bit_gemm_keeps_registers_in_scratch_memory(k):
+    """Any count of k-tiles, odd or even, whole or with a moved-back last one; 32 bytes are the few address registers that a
+    16-bit result's row stores cost."""
+    seen = set()
+    for m, n in SIZES:
+        for tb, out in ((0, 1), (1, 0)):
+            params = dict(M=m, N=n, K=k, TB=tb, OUT_BF16=out, ALIGN=16)
+            text, _ = R.emit_kernel("gemm_bf16", "kernel0", **params)
+            d = defines("gemm_bf16", **params)
+            seen.add((d["GB_BM"], d["GB_BN"], d.get("GB_NBUF", "2")))
+            scratch = scratch_bytes(R.compile_to_code(R.prelude() + text))
+            assert d["GB_D2L"] == "1" and scratch <= 32, params
+    assert {("64", "64", "4"), ("32", "64", "4")} <= seen and (k % 64 or ("256", "256", "2") in seen), seen

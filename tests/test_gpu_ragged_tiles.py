@@ -41,15 +41,14 @@ FORMS = [dict(BM=256, BN=256, WM=4, WN=2), dict(BM=128, BN=128, WM=4, WN=2), dic
 @pytest.mark.parametrize("tb", [False, True])
 @pytest.mark.parametrize("form", range(len(FORMS)))
 def test_gemm16_every_form_at_its_edges(ops, form, tb):
-    """One row or column more or less than whole tiles, a k of one tile, of a part more, of fewer tiles than buffers and of
-    more than two rounds of them."""
+    """One row or column more or less than whole tiles; a k of one tile, of a part more, of fewer tiles than buffers, of more than
+    two rounds of them; odd and even counts of k-tiles, whose last iterations differ."""
     cfg = dict(FORMS[form], M16=1, D2L=1)
     bm, bn = cfg["BM"], cfg["BN"]
-    ks = [64, 64 * 13] if bm == 256 else [72, 64 * 5 + 8, 64 * 13]
+    ks = [64, 128, 192, 136, 200, 64 * 12, 64 * 13] if bm == 256 else [72, 136, 64 * 4, 64 * 5 + 8, 64 * 13]
     for i, (m, n) in enumerate([(bm + 1, bn + 8), (2 * bm - 1, 2 * bn - 8)]):
         for k in ks:
             a, b, want = _operands(m, n, k, tb, torch.bfloat16, 100 * form + 10 * i + k)
-            print("form", form, (m, n, k), tb, flush=True)
             out = torch.bfloat16 if i else torch.float32
             c = ops.matmul(a, b, trans_b=tb, out_dtype=out, **cfg)
             assert torch.equal(c.cpu(), torch.from_numpy(want).to(out)), (m, n, k, out)
