@@ -57,7 +57,7 @@ void SM_NAME(const SM_IO* __restrict__ X, SM_IO* __restrict__ Y) {
       for (int j = 0; j < SM_VW; ++j) v[i][j] = (float)in[j];
     } else {
 #pragma unroll
-      for (int j = 0; j < SM_VW; ++j) v[i][j] = live && idx + j < SM_N ? (float)x[idx + j] : -__builtin_inff();   // exp gives 0: no effect on maximum or sum
+      for (int j = 0; j < SM_VW; ++j) v[i][j] = SM_N % SM_VW != 0 && live && idx + j < SM_N ? (float)x[idx + j] : -__builtin_inff();   // exp gives 0: no effect on maximum or sum
     }
   }
   float m = -__builtin_inff();

@@ -1,0 +1,31 @@
+"""The forms that LayerNorm and softmax kernels get for a row length, seen in the emitted parameters and the compiled code (no GPU
+needed)."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from kernelcodegen_amd import runtime as R
+from test_gemm_forms import defines, scratch_bytes
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+TYPES = {"f32": 0, "f16": 1, "bf16": 2}
+
+
+def code_object(family, **params):
+    text, _ = R.emit_kernel(family, "kernel0", **params)
+    return R.compile_to_code(R.prelude() + text)
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
+@pytest.mark.parametrize("n,vw", [(320, 4), (448, 4), (768, 8), (1000, 8), (2048, 8), (5120, 8)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_whole_rows_of_softmax_are_loaded_as_vectors_only(tmp_path, dtype, n, vw):
+    """A row length that the vector width divides needs no load of single elements, also where the last vectors of the team
+    lie behind the row."""
+    path = tmp_path / "kernel.hsaco"
+    path.write_bytes(code_object("softmax", ROWS=1255, N=n, INPLACE=0, F16=TYPES[dtype], VW=vw))
+    listing = subprocess.run([OBJDUMP, "-d", str(path)], capture_output=True, text=True, check=True).stdout
+    loads = set(re.findall(r"global_load_\w+", listing))
+    assert loads == {"global_load_dwordx%d" % (vw // 2)}, loads
