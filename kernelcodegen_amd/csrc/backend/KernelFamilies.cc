@@ -72,11 +72,12 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   // 16 bytes per access where all lengths divide into them (16-bit types fall back to fours), and on large launches of any
   // row length, scale and bias then being of that length.  Small odd launches keep single elements: the row's end, element by
   // element, is a second trip to memory there (bf16 100 x 1001: 3.5 us, 4.9 in fours), and so do short rows, where most of a
-  // wavefront would idle, and rows beyond the 32 elements a lane holds.  bf16, us, single elements, fours, eights: 16384 x 4096
+  // wavefront would idle, and rows beyond the 32 elements a lane holds, in 16 bits beyond 8192, where the eights of the lane
+  // that holds a row's end take too many registers (bf16 2100 x 16381: eights 53 us, single elements 42).  bf16, us, single elements, fours, eights: 16384 x 4096
   // 115, 81, 51; 12000 x 2048 47, 30, 20; 12000 x 2047 54, 41, 27; 30000 x 257 44, 22, 29.
   const bool f16 = s.get("F16", 0) != 0;
   auto divides = [&](int64_t w) { return n % w == 0 && ng % w == 0 && nb % w == 0; };
-  const bool anyLength = ng == n && nb == n && n >= 256 && n <= 1024 * 32 && (double)rows * (double)n >= 1048576.0;
+  const bool anyLength = ng == n && nb == n && n >= 256 && n <= (f16 ? 8192 : 1024 * 32) && (double)rows * (double)n >= 1048576.0;
   const int64_t wide = f16 ? 8 : 4;
   int64_t vw = s.get("VW", divides(wide) && n >= 512 ? wide : anyLength ? (n >= 1024 ? wide : 4) : divides(4) ? 4 : 1);
   if (vw != 1 && vw != 4 && vw != 8) { err = "layernorm: VW must be 1, 4 or 8"; return false; }
@@ -147,13 +148,16 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   const int64_t groups = ceilDiv(rows, rpb);
   int64_t grid = s.get("GRID", 0);
   // (four per CU where a lane's share of a row is two vectors of eight: bf16 16384 x 1000 13.3 us against 16.9)
-  if (grid <= 0) grid = vpt <= few ? (vw == 8 && vpt <= 2 ? 1024 : 512) : groups;      // rows too long to prefetch keep one workgroup per group
+  // A lane of 1024, which has 128 registers, has no room for gamma, beta and a second row beside more than 24 values of its row
+  // either: 88-212 bytes of scratch (bf16 2000 x 25600 87 us, 44 without the prefetch; fp32 1000 x 28135 70 and 47)
+  const bool crowded = vpt > few || (tpr == 1024 && vpt * vw > 24);
+  if (grid <= 0) grid = !crowded ? (vw == 8 && vpt <= 2 ? 1024 : 512) : groups;      // rows too long to prefetch keep one workgroup per group
   if (grid > groups) grid = groups;
   if (grid > 0x7FFFFFFFLL) grid = 0x7FFFFFFFLL;
   s.p["GRID"] = grid;
   d.add("LN_GRID", grid);
   d.add("LN_STREAM", s.get("STREAM", 1) ? 1 : 0);
-  d.add("LN_LEAN", s.get("LEAN", vpt > few ? 1 : 0) ? 1 : 0);
+  d.add("LN_LEAN", s.get("LEAN", crowded ? 1 : 0) ? 1 : 0);
   // one reduction per row (merged means and sums of squared deviations) where every lane holds the same number of values
   const bool onePass = s.get("ONEPASS", 0) != 0 && n % (tpr * vw) == 0;
   s.p["ONEPASS"] = onePass;

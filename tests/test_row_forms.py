@@ -29,3 +29,13 @@ def test_whole_rows_of_softmax_are_loaded_as_vectors_only(tmp_path, dtype, n, vw
     listing = subprocess.run([OBJDUMP, "-d", str(path)], capture_output=True, text=True, check=True).stdout
     loads = set(re.findall(r"global_load_\w+", listing))
     assert loads == {"global_load_dwordx%d" % (vw // 2)}, loads
+
+
+@pytest.mark.parametrize("dtype", sorted(TYPES))
+@pytest.mark.parametrize("n", [1001, 4096, 8191, 8192, 12001, 16381, 16384, 20001, 24576, 24584, 26565, 28135, 28136, 32001, 32768])
+def test_layernorm_keeps_its_rows_in_registers(n, dtype):
+    """Row, prefetched row, gamma and beta: whatever does not fit a lane's registers is read again, not kept in scratch memory (32
+    bytes: a few addresses)."""
+    for gelu in (0, 1):
+        scratch = scratch_bytes(code_object("layernorm", ROWS=2000, N=n, NG=n, NB=n, EPS=1e-5, GELU=gelu, F16=TYPES[dtype]))
+        assert scratch <= 32, (n, dtype, scratch)
