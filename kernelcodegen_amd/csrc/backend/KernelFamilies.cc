@@ -72,22 +72,32 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   // 16 bytes per access where all lengths divide into them (16-bit types fall back to fours), and on large launches of any
   // row length, scale and bias then being of that length.  Small odd launches keep single elements: the row's end, element by
   // element, is a second trip to memory there (bf16 100 x 1001: 3.5 us, 4.9 in fours), and so do short rows, where most of a
-  // wavefront would idle, and rows beyond the 32 elements a lane holds, in 16 bits beyond 8192, where the eights of the lane
-  // that holds a row's end take too many registers (bf16 2100 x 16381: eights 53 us, single elements 42).  bf16, us, single elements, fours, eights: 16384 x 4096
-  // 115, 81, 51; 12000 x 2048 47, 30, 20; 12000 x 2047 54, 41, 27; 30000 x 257 44, 22, 29.
+  // wavefront would idle, and in 16 bits lengths that leave most lanes' second eight empty (4096 to 6144, on launches of over 8 M
+  // elements) or where the eights take too many registers (beyond 8192; fp32 in fours stays ahead to the 32 elements a lane
+  // holds): bf16 us, eights and single elements, 2000 x 5555 21.8 and 18.2, 2100 x 16381 53 and 42, but 1000 x 8191 9.8 and 12.8.
+  // 16-bit rows that fours divide and eights do not go in fours, aligned as they are, while those leave a lane half a vector free
+  // (7168), on up to 4096 elements by 1024 workgroups (eights with a ragged end and fours: 300 x 3892 5.8 and 4.3, 16384 x 3892 85
+  // and 66, 4000 x 5004 35 and 27, 2000 x 7004 23 and 18; 1000 x 8188 9.2 and 11.5).
   const bool f16 = s.get("F16", 0) != 0;
+  const double elements = (double)rows * (double)n;
   auto divides = [&](int64_t w) { return n % w == 0 && ng % w == 0 && nb % w == 0; };
-  const bool anyLength = ng == n && nb == n && n >= 256 && n <= (f16 ? 8192 : 1024 * 32) && (double)rows * (double)n >= 1048576.0;
+  const bool anyLength = ng == n && nb == n && n >= 256 && n <= (f16 ? 8192 : 1024 * 32) && elements >= 1048576.0 &&
+                         !(f16 && n > 4096 && n <= 6144 && elements > 8388608.0);
   const int64_t wide = f16 ? 8 : 4;
-  int64_t vw = s.get("VW", divides(wide) && n >= 512 ? wide : anyLength ? (n >= 1024 ? wide : 4) : divides(4) ? 4 : 1);
+  // (a wavefront that fours fill and eights do not, 768 elements: fours on small launches, 300 x 768 3.2 us and 3.0)
+  const bool unfilled = f16 && n < 1024 && n % 256 == 0 && n % 512 != 0 && elements <= 2097152.0;
+  const bool fours = divides(4) && f16 && n >= 1024 && n <= 7168;
+  int64_t vw = s.get("VW", divides(wide) && n >= 512 && !unfilled ? wide : anyLength && !fours ? (n >= 1024 ? wide : 4) : divides(4) ? 4 : 1);
   if (vw != 1 && vw != 4 && vw != 8) { err = "layernorm: VW must be 1, 4 or 8"; return false; }
-  if (vw > 1 && s.has("VW") && !divides(vw)) { err = "layernorm: VW=4 needs lengths divisible by 4"; return false; }
+  if (vw > 1 && s.has("VW") && !divides(vw)) { err = "layernorm: VW=" + std::to_string(vw) + " needs lengths divisible by " + std::to_string(vw); return false; }
   int64_t tpr = s.get("TPR", 0);
   if (rows > 0xFFFFFFFFLL) { err = "layernorm: too many rows"; return false; }
   if (tpr == 0) {
-    // four vectors per lane measured best for 4096-float rows, with and without the GELU; of 16-bit values, eight to a vector,
-    // two beyond 4096 (bf16 16384 x 8192: 90 us against 116; 16384 x 4096: 62 against 51)
-    tpr = nextPow2(ceilDiv(n, vw * (vw == 8 && n > 4096 ? 2 : 4)));
+    // Four vectors per lane measured best for 4096-float rows, with and without the GELU; of 16-bit values, eight to a vector,
+    // two (so as many lanes as with fours: half of them made small launches slower than fours, bf16 us with four vectors, two,
+    // and in fours: 1 x 4096 3.24, 2.76, 3.11; 64 x 2048 3.44, 2.89, 3.34; 4000 x 4096 17.9, 14.7, 18.7; 16384 x 4096 68, 50, 66),
+    // but three where one wavefront then holds the row (64 x 1536 3.14 us, 3.33 on two).
+    tpr = nextPow2(ceilDiv(n, vw * (vw == 8 && (n > 4096 || (n > 1536 && divides(8))) ? 2 : 4)));
     if (tpr < 64) tpr = 64;
     if (tpr > 512) tpr = 512;
   }
@@ -147,11 +157,13 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   // workgroup per row; a plain copy reaches 6.3-6.4 TB/s under the same conditions.
   const int64_t groups = ceilDiv(rows, rpb);
   int64_t grid = s.get("GRID", 0);
-  // (four per CU where a lane's share of a row is two vectors of eight: bf16 16384 x 1000 13.3 us against 16.9)
+  // (four per CU where a lane's share of a row is two vectors of eight: bf16 16384 x 1000 13.3 us against 16.9; or four of
+  // four: 16384 x 3892 66 against 85)
   // A lane of 1024, which has 128 registers, has no room for gamma, beta and a second row beside more than 24 values of its row
   // either: 88-212 bytes of scratch (bf16 2000 x 25600 87 us, 44 without the prefetch; fp32 1000 x 28135 70 and 47)
   const bool crowded = vpt > few || (tpr == 1024 && vpt * vw > 24);
-  if (grid <= 0) grid = !crowded ? (vw == 8 && vpt <= 2 ? 1024 : 512) : groups;      // rows too long to prefetch keep one workgroup per group
+  const bool wideGrid = f16 && ((vw == 8 && vpt <= 2) || (vw == 4 && n >= 1024 && n <= 4096));
+  if (grid <= 0) grid = crowded ? groups : wideGrid ? 1024 : 512;      // rows too long to prefetch keep one workgroup per group
   if (grid > groups) grid = groups;
   if (grid > 0x7FFFFFFFLL) grid = 0x7FFFFFFFLL;
   s.p["GRID"] = grid;

@@ -39,3 +39,27 @@ def test_layernorm_keeps_its_rows_in_registers(n, dtype):
     for gelu in (0, 1):
         scratch = scratch_bytes(code_object("layernorm", ROWS=2000, N=n, NG=n, NB=n, EPS=1e-5, GELU=gelu, F16=TYPES[dtype]))
         assert scratch <= 32, (n, dtype, scratch)
+
+
+def lanes_in_fours(n, most):
+    """Lanes that share a row when each takes four vectors of four."""
+    lanes = 64
+    while lanes * 16 < n and lanes < most:
+        lanes *= 2
+    return lanes
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rows", [1, 64, 300, 1000])
+def test_layernorm_of_16_bit_rows_keeps_its_lanes_and_its_alignment(rows, dtype):
+    """Wider vectors take fewer loads of each lane and not fewer lanes: a small launch lasts as long as a lane's chain.  Rows that
+    fours divide and eights do not stay aligned in fours; 768 elements fill a wavefront in fours only."""
+    def form(n):
+        return defines("layernorm", ROWS=rows, N=n, NG=n, NB=n, EPS=1e-5, F16=TYPES[dtype])
+    for n in (1024, 2048, 3000, 3072, 4096, 5120, 8192):
+        d = form(n)
+        assert d["LN_VW"] == "8" and int(d["LN_TPR"]) >= lanes_in_fours(n, 512), n
+    for n in (1028, 1500, 2044, 3892, 5004, 7004):
+        d = form(n)
+        assert d["LN_VW"] == "4" and int(d["LN_TPR"]) == lanes_in_fours(n, 512), n
+    assert form(768)["LN_VW"] == "4" and form(1000)["LN_VW"] == "8"
