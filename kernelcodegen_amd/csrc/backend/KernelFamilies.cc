@@ -278,15 +278,24 @@ bool emitSoftmax(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   const int64_t rows = s.p["ROWS"], n = s.p["N"];
   // As for LayerNorm: 16 bytes per access where the length divides into them, and on large launches of any length (us, single
   // elements, fours, 16 bytes: bf16 12000 x 2048 41.7, 18.7, 16.5; 4096 x 4096 29.9, 13.5, 9.6; 2000 x 32000 138, 68, 47;
-  // 12000 x 2047 42.9, 22.6, 20.6; 30000 x 257 20.3, 12.1, 14.6; 100 x 1001 3.3, 3.9).
-  const int64_t wide = s.get("F16", 0) ? 8 : 4;
-  const bool anyLength = n >= 256 && n <= 1024 * 32 && (double)rows * (double)n >= 1048576.0;
-  int64_t vw = s.get("VW", n % wide == 0 && n >= 512 ? wide : anyLength ? (n >= 1024 ? wide : 4) : n % 4 == 0 ? 4 : 1);
+  // 12000 x 2047 42.9, 22.6, 20.6; 30000 x 257 20.3, 12.1, 14.6; 100 x 1001 3.3, 3.9).  16-bit rows
+  // that fours divide and eights do not go in fours on rows of up to 2048 elements (16384 x 1500 21.3, 22.3 in eights with a ragged
+  // end) and on launches of up to 8 M elements (300 x 3892 4.0, 4.7; 1000 x 8188 7.2, 7.7); on larger ones of longer rows eights are
+  // ahead or within 6 % (4000 x 3892 13.9 and 12.2, 16384 x 3892 48.9 and 51.8).
+  const bool f16 = s.get("F16", 0) != 0;
+  const int64_t wide = f16 ? 8 : 4;
+  const double elements = (double)rows * (double)n;
+  const bool small = elements <= 4194304.0;
+  const bool anyLength = n >= 256 && n <= 1024 * 32 && elements >= 1048576.0;
+  const bool fours = n % 4 == 0 && f16 && n >= 1024 && (n <= 2048 || elements <= 8388608.0);
+  int64_t vw = s.get("VW", n % wide == 0 && n >= 512 ? wide : anyLength && !fours ? (n >= 1024 ? wide : 4) : n % 4 == 0 ? 4 : 1);
   if (vw != 1 && vw != 4 && vw != 8) { err = "softmax: VW must be 1, 4 or 8"; return false; }
-  if (vw > 1 && s.has("VW") && n % vw) { err = "softmax: VW=4 needs a row length divisible by 4"; return false; }
+  if (vw > 1 && s.has("VW") && n % vw) { err = "softmax: VW=" + std::to_string(vw) + " needs a row length divisible by " + std::to_string(vw); return false; }
   int64_t tpr = s.get("TPR", 0);
   if (tpr == 0) {
-    tpr = nextPow2(ceilDiv(n, vw * 4));      // about four vectors per lane
+    // About four vectors per lane; on small launches of whole eights two, as many lanes as fours have (bf16 us with four vectors,
+    // two, and in fours: 1 x 4096 3.09, 2.65, 2.91; 300 x 2048 3.35, 2.99, 3.22; 1000 x 4096 5.2, 4.35, 4.5; but 4000 x 4096 10.6, 12.5)
+    tpr = nextPow2(ceilDiv(n, vw * (vw == 8 && n > 1536 && n <= 8192 && n % 8 == 0 && small ? 2 : 4)));
     if (tpr < 64) tpr = 64;
     if (tpr > 1024) tpr = 1024;
   }

@@ -63,3 +63,17 @@ def test_layernorm_of_16_bit_rows_keeps_its_lanes_and_its_alignment(rows, dtype)
         d = form(n)
         assert d["LN_VW"] == "4" and int(d["LN_TPR"]) == lanes_in_fours(n, 512), n
     assert form(768)["LN_VW"] == "4" and form(1000)["LN_VW"] == "8"
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rows", [1, 64, 500])
+def test_softmax_of_16_bit_rows_keeps_its_lanes_and_its_alignment_on_small_launches(rows, dtype):
+    def form(n, r=rows):
+        return defines("softmax", ROWS=r, N=n, INPLACE=0, F16=TYPES[dtype])
+    for n in (1024, 2048, 3000, 3072, 4096, 5120, 8192):
+        d = form(n)
+        assert d["SM_VW"] == "8" and int(d["SM_TPR"]) >= lanes_in_fours(n, 1024), n
+    for n in (1028, 1500, 2044, 3892, 5004, 8188):
+        d = form(n)
+        assert d["SM_VW"] == "4" and int(d["SM_TPR"]) == lanes_in_fours(n, 1024), n
+    assert int(form(4096, 16384)["SM_TPR"]) == 128 and form(3892, 16384)["SM_VW"] == "8" and form(1500, 16384)["SM_VW"] == "4"
