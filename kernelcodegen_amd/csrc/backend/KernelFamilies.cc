@@ -1162,13 +1162,21 @@ bool emitFmhaF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   if (dh % 32 || dh > 256) { err = "fmha_f32: head dim must be a multiple of 32, at most 256"; return false; }
   // queries per workgroup (32 per wavefront): four wavefronts, fewer for short sequences
   int64_t br = s.get("BR", 0);
+  bool halved = false;
   if (br <= 0) {
     br = sl >= 128 ? 128 : (sl > 64 ? 128 : (sl > 32 ? 64 : 32));
-    // Under the mask at head dims above 64, whose workgroups have a CU to themselves, two rounds of them end as late as the
-    // longest query tiles: half the tile evens that out (B4 H32 S512 D128 139 and 103 us, B1 H32 S2048 D128 520 and 341;
-    // one round loses, B1 H32 S1024 D128 146 and 166, more gain nothing, B8 H32 S640 D128 342 and 350).
+    // Under the mask at head dims above 64, a launch of 256 to 512 workgroups is one round that lasts as long as the longest query
+    // tile of a head.  Tiles of half the size in pairs, the longest with the shortest, all last the same (heads x S, D 128, us
+    // with tiles of 128, of 64 by themselves and in pairs: 112 x 512 138, 168, 102; 32 x 2048 520, -, 340; 90 x 384 89, 89, 80).  An
+    // odd number of them has no pairs and gains while they fill the part once and two thirds (80 x 448 123, 78; 40 x 1344 346, 287;
+    // 100 x 576 152, 162); a last tile partly filled loses (80 x 600 134, 205).  One round of 128 or less loses, B1 H32 S1024 D128
+    // 146 and 166, more gain nothing, B8 H32 S640 D128 342 and 350.
     const double tiles = (double)ceilDiv(sl, 128) * (double)b * (double)h;
-    if (s.get("FILL", 0) && s.get("CAUSAL", 0) && dh > 64 && br == 128 && !s.has("PAIR") && !s.has("D2L") && tiles > 256.0 && tiles <= 512.0) br = 64;
+    if (s.get("FILL", 0) && s.get("CAUSAL", 0) && dh > 64 && br == 128 && !s.has("PAIR") && !s.has("D2L") && tiles > 256.0 && tiles <= 512.0 && sl % 64 == 0 &&
+        (sl % 128 == 0 || (double)(sl / 64) * (double)b * (double)h <= 853.0)) {
+      br = 64;
+      halved = sl % 128 == 0;
+    }
   }
   if (br % 32 || br > 512) { err = "fmha_f32: BR must be a multiple of 32, at most 512"; return false; }
   // keys per LDS tile: 64 for head dims above 64 while two workgroups' tiles fit the LDS together, else 32 (measured at
@@ -1198,7 +1206,7 @@ bool emitFmhaF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // the default once the halved grid still gives every CU its two workgroups (B8 H32 S2048 causal: head dim 128 2.19
   // against 2.70 ms, head dim 64 1.18 against 1.45 ms; on grids smaller than the part it costs parallelism: 20 workgroups
   // instead of 40 at B1 H5 S1024 take 0.129 against 0.114 ms)
-  const bool pair = s.get("PAIR", pairFits && (nq / 2) * b * h >= 512 ? 1 : 0) != 0;
+  const bool pair = s.get("PAIR", pairFits && (halved || (nq / 2) * b * h >= 512) ? 1 : 0) != 0;
   if (pair && !pairFits) { err = "fmha_f32: PAIR needs the causal mask and an even number of query tiles"; return false; }
   s.p["BR"] = br; s.p["BC"] = bc; s.p["CAUSAL"] = causal; s.p["OCC"] = occ; s.p["D2L"] = d2l; s.p["PAIR"] = pair;
   s.f["SCALE"] = scale;
