@@ -77,3 +77,12 @@ def test_no_form_of_the_16_bit_gemm_keeps_registers_in_scratch_memory(k):
             scratch = scratch_bytes(R.compile_to_code(R.prelude() + text))
             assert d["GB_D2L"] == "1" and scratch <= 32, params
     assert {("64", "64", "4"), ("32", "64", "4")} <= seen and (k % 64 or ("256", "256", "2") in seen), seen
+
+
+
+def test_guarded_fp8_loads_in_chunks():
+    """Every aligned ragged tile but the 128 x 128 ones of two k-contiguous operands in whole k-tiles."""
+    def wide(**params):
+        return defines("gemm_fp8", **dict(dict(M=700, N=816, K=512, TB=1, ALIGN=16, D2L=0, BM=128, BN=128), **params)).get("GF_WIDE")
+    assert wide() is None and wide(ALIGN=0, K=528) is None
+    assert wide(K=528) == "1" and wide(TB=0) == "1" and wide(BM=256, BN=256) == "1" and wide(M=704, TA=1) == "1"
