@@ -900,6 +900,12 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   const bool whole = m % dm == 0 && n % dn == 0 && k % 128 == 0;
   if (!own && !whole && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !ta && k % 16 == 0 && n % 16 == 0 && s.get("SCALE_PTR", 0) == 0) {
     const Gemm16Form* form = chooseGemm16Form(m, n, k / 2, batch);
+    // Shallow products of two k-contiguous operands lose little to guarded loads, and those run on gemm_fp8.hip's larger MFMA:
+    // ahead where the choice would be 128 x 128 tiles, or 256 x 256 ones on under three quarters of the CUs (us, these and
+    // guarded 128 x 128 tiles: 2000 x 5504 x 512 16.1 and 13.3, 1000 x 11008 x 1024 21.0 and 18.7, 2000 x 2816 x 1024 13.9 and 12.3;
+    // x 2048 21.9 and 22.4, 2447 x 5504 x 1024 22.1 and 24.8 on 220 CUs, 700 x 5504 x 512 8.5 and 9.3 in 64 x 128)
+    const bool shallow = tb && k <= 1024 && k % 128 == 0 && dm == 128 && dn == 128;
+    if (form && shallow && (form->bm == 128 || (form->bm == 256 && (double)ceilDiv(m, 256) * (double)ceilDiv(n, 256) * (double)batch < 192.0))) form = nullptr;
     if (form && form->bm == 256) {
       shift256 = true;
     } else if (form && tb) {

@@ -86,3 +86,15 @@ def test_guarded_fp8_loads_in_chunks():
         return defines("gemm_fp8", **dict(dict(M=700, N=816, K=512, TB=1, ALIGN=16, D2L=0, BM=128, BN=128), **params)).get("GF_WIDE")
     assert wide() is None and wide(ALIGN=0, K=528) is None
     assert wide(K=528) == "1" and wide(TB=0) == "1" and wide(BM=256, BN=256) == "1" and wide(M=704, TA=1) == "1"
+
+
+@pytest.mark.parametrize("m,n,k,guarded", [(2000, 5504, 512, 1), (1000, 11008, 1024, 1), (2000, 2816, 1024, 1), (1000, 5504, 256, 1),
+                                           (2000, 2816, 2048, 0), (2447, 5504, 1024, 0), (700, 5504, 512, 0), (300, 11008, 512, 0), (2447, 2816, 528, 0)])
+def test_shallow_fp8_products_keep_the_guarded_tiles(m, n, k, guarded):
+    """Which kernel a ragged product of two k-contiguous operands takes by its depth and by how much of the part its tiles fill."""
+    d = defines("gemm_fp8", M=m, N=n, K=k, TB=1, ALIGN=16)
+    assert ("GF_M" in d) == bool(guarded), d
+    if guarded:
+        assert d["GF_BM"] == d["GF_BN"] == "128" and "GF_WIDE" not in d
+    d = defines("gemm_fp8", M=m, N=n, K=k, TB=0, ALIGN=16)
+    assert d.get("G8_SHIFT", d.get("GF_WIDE")) == "1"

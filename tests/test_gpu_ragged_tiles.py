@@ -115,7 +115,7 @@ def test_gemm16_infinities_stay_in_their_rows_and_columns(ops, tb):
 
 @pytest.mark.parametrize("tb", [True, False])
 @pytest.mark.parametrize("m,n,k", [(257, 272, 128), (511, 528, 384), (300, 5008, 256), (1000, 4112, 1040), (16, 512, 512), (1, 528, 2048),
-                                   (65, 80, 144), (130, 1040, 400), (700, 2064, 272), (64, 64, 128)])
+                                   (65, 80, 144), (130, 1040, 400), (700, 2064, 272), (64, 64, 128), (1100, 4112, 256)])
 def test_gemm_fp8_default_forms(ops, m, n, k, tb):
     """Moved-back 256 x 256 tiles, the ring of LDS buffers (weights contiguous along k) and guarded loads of whole chunks;
     products up to 16 and |sum| <= 16 k < 2^16 stay exact in every MFMA's accumulator."""
