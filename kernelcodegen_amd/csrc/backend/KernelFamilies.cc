@@ -1027,11 +1027,11 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   const bool pingpong = s.get("PINGPONG", 0) != 0 && bk == 64 && wm * wn == 8 && !guarded && !prefetch && k / bk >= stages + 2;
   s.p["PINGPONG"] = pingpong;
   d.add("GF_PINGPONG", pingpong ? 1 : 0);
-  // Guarded loads of whole chunks, where the caller has looked at the operands' addresses.  In 128 x 128 tiles of two operands
-  // that are contiguous along k, in whole k-tiles, the compiler joins a chunk's sixteen guarded bytes by itself, behind one branch
-  // for the row (1000 x 5504 x 512 9.4 us, 12.4 in chunks that are loaded in any case and then selected; 256 x 256 tiles 2000 x
+  // Guarded loads of whole chunks, where the caller has looked at the operands' addresses.  In tiles of up to 128 x 128 of two
+  // operands that are contiguous along k, in whole k-tiles, the compiler joins a chunk's sixteen guarded bytes by itself, behind one branch
+  // for the row (1000 x 5504 x 512 9.4 us, 12.4 in chunks that are loaded in any case and then selected; 5 x 1 x 496 x 1024 3.7 and 4.0; but 256 x 256 tiles 2000 x
   // 2816 x 2048 71 and 46, a partial k-tile 2447 x 2816 x 528 16.5 and 13.3).
-  const bool joined = !ta && tb && bm == 128 && bn == 128 && k % bk == 0;
+  const bool joined = !ta && tb && bm <= 128 && bn <= 128 && k % bk == 0;
   if (edge && !joined && s.get("ALIGN", 0) >= 16 && k % 16 == 0 && (!ta || m % 16 == 0) && (tb || n % 16 == 0)) d.add("GF_WIDE", 1);
   d.add("GF_BTR", btr ? 1 : 0);
   // where the two per-tensor scales come from: trailing scalars, or one fp32 each in device memory (graph values)
