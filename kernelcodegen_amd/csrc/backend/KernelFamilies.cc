@@ -1028,9 +1028,9 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   s.p["PINGPONG"] = pingpong;
   d.add("GF_PINGPONG", pingpong ? 1 : 0);
   // Guarded loads of whole chunks, where the caller has looked at the operands' addresses.  In tiles of up to 128 x 128 of two
-  // operands that are contiguous along k, in whole k-tiles, the compiler joins a chunk's sixteen guarded bytes by itself, behind one branch
-  // for the row (1000 x 5504 x 512 9.4 us, 12.4 in chunks that are loaded in any case and then selected; 5 x 1 x 496 x 1024 3.7 and 4.0; but 256 x 256 tiles 2000 x
-  // 2816 x 2048 71 and 46, a partial k-tile 2447 x 2816 x 528 16.5 and 13.3).
+  // operands that are contiguous along k, in whole k-tiles, the compiler joins a chunk's sixteen guarded bytes by itself, behind
+  // one branch for the row (1000 x 5504 x 512 9.4 us, 12.4 in chunks that are loaded in any case and then selected; 5 x 1 x 496 x
+  // 1024 3.7 and 4.0; but 256 x 256 tiles 2000 x 2816 x 2048 71 and 46, a partial k-tile 2447 x 2816 x 528 16.5 and 13.3).
   const bool joined = !ta && tb && bm <= 128 && bn <= 128 && k % bk == 0;
   if (edge && !joined && s.get("ALIGN", 0) >= 16 && k % 16 == 0 && (!ta || m % 16 == 0) && (tb || n % 16 == 0)) d.add("GF_WIDE", 1);
   d.add("GF_BTR", btr ? 1 : 0);
@@ -1078,9 +1078,14 @@ bool emitFmhaBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   for (const char* key : {"D2L", "PAIR", "PERSIST", "OCC", "STAGE_O"}) own = own || s.has(key);
   const double heads = (double)b * (double)h, jobs = (double)ceilDiv(sl, br) * heads / (masked && ((b * h) % 2 == 0 || ceilDiv(sl, br) % 2 == 0) ? 2.0 : 1.0);
   bool noPair = false;
+  // Under the mask at head dims above 96, whose workgroups have a CU to themselves, more than 256 of 128 queries are a second round
+  // while those of 256 by themselves are still one: heads x S, D 128, us, pairs of 256, 128 and 256 by themselves, 60 x 1024 46.9,
+  // 56.2, 37.8; 80 x 768 41.4, 44.0, 30.4; 64 x 600 40.3, 30.7, 25.2; but 16 x 2048, 256 of 128, 67.1, 46.8, 55.9.
   if (!own && jobs <= 128.0) {
-    if (br == 256) br = 128;
-    noPair = masked && (double)ceilDiv(sl, br) * heads / 2.0 < 256.0;
+    const double small = (double)ceilDiv(sl, 128) * heads;
+    const bool oneRound = masked && dh > 96 && br == 256 && small > 256.0 && small < 512.0;
+    if (br == 256 && !oneRound) br = 128;
+    noPair = masked && (oneRound || (double)ceilDiv(sl, br) * heads / 2.0 < 256.0);
   }
   if (bc <= 0) {
     bc = sl > 32 ? 64 : 32;

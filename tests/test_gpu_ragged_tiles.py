@@ -228,7 +228,7 @@ def test_softmax_rows_of_infinities_and_nan(ops):
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 1e-2), (torch.float16, 2e-3), (torch.float32, 4e-6)])
 @pytest.mark.parametrize("b,h,s,d", [(1, 8, 333, 64), (1, 3, 64, 64), (1, 3, 65, 128), (1, 5, 256, 128), (1, 32, 1100, 128), (2, 64, 512, 128),
-                                     (1, 80, 448, 128), (1, 90, 384, 128)])
+                                     (1, 80, 448, 128), (1, 90, 384, 128), (1, 64, 600, 128), (1, 80, 768, 128)])
 def test_attention_on_small_launches(ops, b, h, s, d, dtype, tol, causal):
     """128 queries per workgroup and no pairs of query tiles where the launch leaves compute units empty, 64 for fp32 under
     the mask; the tolerances are those of the other attention tests (16-bit probabilities, fp32 sums)."""
