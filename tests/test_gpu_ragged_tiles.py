@@ -167,7 +167,7 @@ def test_gemm_f32_direct_load_forms_at_their_edges(ops, form, tb):
     cfg = F32_FORMS[form]
     bm, bk = cfg["BM"], cfg["BK"]
     for i, (m, n) in enumerate([(bm + 1, bm + 4), (2 * bm - 1, 2 * bm - 4)]):
-        for k in (bk, 5 * bk - 4, 9 * bk):
+        for k in (bk, bk + 4, 3 * bk - 4, 5 * bk - 4, 9 * bk):      # (one and two k-tiles, fewer than there are buffers, too)
             a, b, want = _operands(m, n, k, tb, torch.float32, 100 * form + 10 * i + k, batch=(2,))
             assert torch.equal(ops.batched_matmul(a, b, trans_b=tb, **cfg).double().cpu(), torch.from_numpy(want)), (m, n, k)
 

@@ -114,3 +114,20 @@ def test_operands_off_a_16_byte_boundary_keep_the_direct_loads(kernels):
     for family, params in kernels:
         text, _ = R.emit_kernel(family, "kernel0", **params)
         assert "#define GB_D2L 1\n" not in text and "#define GB_SHIFT 1\n" not in text, params
+
+
+def test_options_that_change_the_kernel_are_kept_apart(kernels):
+    """Calls on the same shapes that differ in one option each, twice over: every option asks for a kernel of its own, once."""
+    x, g = torch.zeros(4, 8), torch.zeros(8)
+    q = torch.zeros(1, 2, 64, 64, dtype=torch.float16)
+    calls = [lambda: ops.layernorm(x, g, g, 1), lambda: ops.layernorm(x, g, g, 1, eps=1e-6), lambda: ops.layernorm(x, g, g, 1, gelu=True),
+             lambda: ops.layernorm(x, g, g[:4], 1), lambda: ops.fmha(q, q, q), lambda: ops.fmha(q, q, q, causal=True),
+             lambda: ops.fmha(q, q, q, scale=0.5), lambda: ops.fmha(q, q, q, scale=0.25), lambda: ops.fmha(q, q, q, out_dtype=torch.float32),
+             lambda: ops.softmax(x), lambda: ops.softmax(x.clone(), inplace=True), lambda: ops.elementwise(x, "Gelu"),
+             lambda: ops.elementwise(x, "Relu"), lambda: ops.elementwise(x, "Relu", inplace=True), lambda: ops.binary(x, x, "Add"),
+             lambda: ops.binary(x, x, "Sub"), lambda: ops.binary(x, g, "Add"), lambda: ops.matmul(x, x.t().contiguous()),
+             lambda: ops.matmul(x, x, trans_b=True), lambda: ops.matmul(x.t().contiguous(), x.t().contiguous(), trans_a=True)]
+    for call in calls + calls:
+        call()
+    assert len(kernels) == len(calls)
+    assert len({(f, tuple(sorted(p.items()))) for f, p in kernels}) == len(calls)
