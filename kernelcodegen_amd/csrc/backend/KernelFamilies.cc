@@ -523,14 +523,14 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // with several workgroups per CU, 1536^3, the groups change nothing and the launch keeps the plain form)
   const bool small = wkFits && bm == 64 && bn == 64 && wm * wn == 4 && ceilDiv(m, bm) * ceilDiv(n, bn) * batch <= 256;
   const int64_t wk = s.get("WK", small ? 2 : 1);
-  if (wk != 1 && !(wk == 2 && wkFits)) { err = "gemm_f32: WK is 1 or 2; 2 needs whole tiles of two row-major operands, BK = 32, at most eight wavefronts per group and BM * BN <= 64 (BM + BN)"; return false; }
+  if (wk != 1 && !(wk == 2 && wkFits)) { err = "gemm_f32: WK is 1 or 2; 2 needs the direct loads into LDS (D2L), BK = 32, at most eight wavefronts per group and BM * BN <= 64 (BM + BN)"; return false; }
   s.p["WK"] = wk;
   // NBUF LDS buffers per operand (the loads of k-tile kt + NBUF - 1 start with k-tile kt): more than two where a k-tile is
   // shorter than a load's way from the L2; every wavefront must then issue the same number of loads per k-tile
   const int64_t nbuf = s.get("NBUF", small && wk == 2 ? 3 : 2);
   const int64_t blocks = (bm + bn) * bk * 4 / 1024;
   if (nbuf != 2 && !(d2l && (nbuf == 3 || nbuf == 4) && blocks % (wm * wn * wk) == 0 && nbuf * (bm + bn) * bk * 4 <= 160 * 1024)) {
-    err = "gemm_f32: NBUF is 2, or 3 or 4 for whole tiles of two row-major operands whose k-tile is a whole number of 1 KiB blocks per wavefront and fits the LDS that many times";
+    err = "gemm_f32: NBUF is 2, or 3 or 4 with the direct loads into LDS (D2L) where a k-tile is a whole number of 1 KiB blocks per wavefront and fits the LDS that many times";
     return false;
   }
   s.p["NBUF"] = nbuf;

@@ -3,7 +3,7 @@
 // (sum, centred sum of squares, normalise), each a coalesced stride loop.  The
 // second and third pass re-read x, which for groups up to a few MiB is served by
 // the L2 / Infinity Cache.
-// Parameters: LS_NAME, LS_ROWS, LS_N, LS_NG, LS_NB, LS_EPS, LS_BLOCK, LS_VW (4 or 1), LS_GELU,
+// Parameters: LS_NAME, LS_ROWS, LS_N, LS_NG, LS_NB, LS_EPS, LS_BLOCK, LS_VW (8, 4 or 1), LS_GELU,
 // LS_F16 (1: IEEE half, 2: bfloat16 in memory; the arithmetic is fp32 either way).
 #ifndef LS_F16
 #define LS_F16 0
