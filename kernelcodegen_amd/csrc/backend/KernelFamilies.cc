@@ -73,8 +73,9 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   // row length, scale and bias then being of that length.  Small odd launches keep single elements: the row's end, element by
   // element, is a second trip to memory there (bf16 100 x 1001: 3.5 us, 4.9 in fours), and so do short rows, where most of a
   // wavefront would idle, and in 16 bits lengths that leave most lanes' second eight empty (4096 to 6144, on launches of over 8 M
-  // elements) or where the eights take too many registers (beyond 8192; fp32 in fours stays ahead to the 32 elements a lane
-  // holds): bf16 us, eights and single elements, 2000 x 5555 21.8 and 18.2, 2100 x 16381 53 and 42, but 1000 x 8191 9.8 and 12.8.
+  // elements), 2048 to 4096 while every row has a workgroup to itself (512), and those where the eights take too many registers
+  // (beyond 8192; fp32 in fours stays ahead to the 32 elements a lane holds): bf16 us, eights and single elements, 2000 x 5555 21.8
+  // and 18.2, 500 x 2503 6.0 and 4.5, 2100 x 16381 53 and 42, but 520 x 3001 5.1 and 5.9, 1000 x 8191 9.8 and 12.8.
   // 16-bit rows that fours divide and eights do not go in fours, aligned as they are, while those leave a lane half a vector free
   // (7168), on up to 4096 elements by 1024 workgroups (eights with a ragged end and fours: 300 x 3892 5.8 and 4.3, 16384 x 3892 85
   // and 66, 4000 x 5004 35 and 27, 2000 x 7004 23 and 18; 1000 x 8188 9.2 and 11.5).
@@ -82,7 +83,7 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   const double elements = (double)rows * (double)n;
   auto divides = [&](int64_t w) { return n % w == 0 && ng % w == 0 && nb % w == 0; };
   const bool anyLength = ng == n && nb == n && n >= 256 && n <= (f16 ? 8192 : 1024 * 32) && elements >= 1048576.0 &&
-                         !(f16 && n > 4096 && n <= 6144 && elements > 8388608.0);
+                         !(f16 && ((n > 4096 && n <= 6144 && elements > 8388608.0) || (n > 2048 && n <= 4096 && rows <= 512)));
   const int64_t wide = f16 ? 8 : 4;
   // (a wavefront that fours fill and eights do not, 768 elements: fours on small launches, 300 x 768 3.2 us and 3.0)
   const bool unfilled = f16 && n < 1024 && n % 256 == 0 && n % 512 != 0 && elements <= 2097152.0;
@@ -95,9 +96,9 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   if (tpr == 0) {
     // Four vectors per lane measured best for 4096-float rows, with and without the GELU; of 16-bit values, eight to a vector,
     // two (so as many lanes as with fours: half of them made small launches slower than fours, bf16 us with four vectors, two,
-    // and in fours: 1 x 4096 3.24, 2.76, 3.11; 64 x 2048 3.44, 2.89, 3.34; 4000 x 4096 17.9, 14.7, 18.7; 16384 x 4096 68, 50, 66),
+    // and in fours: 1 x 4096 3.24, 2.76, 3.11; 64 x 2048 3.44, 2.89, 3.34; 4000 x 4096 17.9, 14.7, 18.7; 16384 x 4096 68, 50, 66; 12000 x 3333 66, 55),
     // but three where one wavefront then holds the row (64 x 1536 3.14 us, 3.33 on two).
-    tpr = nextPow2(ceilDiv(n, vw * (vw == 8 && (n > 4096 || (n > 1536 && divides(8))) ? 2 : 4)));
+    tpr = nextPow2(ceilDiv(n, vw * (vw == 8 && n > 1536 ? 2 : 4)));
     if (tpr < 64) tpr = 64;
     if (tpr > 512) tpr = 512;
   }
@@ -279,23 +280,23 @@ bool emitSoftmax(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // As for LayerNorm: 16 bytes per access where the length divides into them, and on large launches of any length (us, single
   // elements, fours, 16 bytes: bf16 12000 x 2048 41.7, 18.7, 16.5; 4096 x 4096 29.9, 13.5, 9.6; 2000 x 32000 138, 68, 47;
   // 12000 x 2047 42.9, 22.6, 20.6; 30000 x 257 20.3, 12.1, 14.6; 100 x 1001 3.3, 3.9).  16-bit rows
-  // that fours divide and eights do not go in fours on rows of up to 2048 elements (16384 x 1500 21.3, 22.3 in eights with a ragged
-  // end) and on launches of up to 8 M elements (300 x 3892 4.0, 4.7; 1000 x 8188 7.2, 7.7); on larger ones of longer rows eights are
-  // ahead or within 6 % (4000 x 3892 13.9 and 12.2, 16384 x 3892 48.9 and 51.8).
+  // that fours divide and eights do not go in fours on launches of up to 8 M elements (eights with a ragged end and fours: 300 x
+  // 3892 4.7 and 4.0, 1000 x 8188 7.7 and 7.2); on larger ones eights are ahead or within 6 % (4000 x 3892 12.2 and 13.9, 8000 x 2044
+  // 13.2 and 13.9, 16384 x 1500 22.3 and 21.3, 16384 x 3892 51.8 and 48.9).
   const bool f16 = s.get("F16", 0) != 0;
   const int64_t wide = f16 ? 8 : 4;
   const double elements = (double)rows * (double)n;
   const bool small = elements <= 4194304.0;
   const bool anyLength = n >= 256 && n <= 1024 * 32 && elements >= 1048576.0;
-  const bool fours = n % 4 == 0 && f16 && n >= 1024 && (n <= 2048 || elements <= 8388608.0);
+  const bool fours = n % 4 == 0 && f16 && n >= 1024 && elements <= 8388608.0;
   int64_t vw = s.get("VW", n % wide == 0 && n >= 512 ? wide : anyLength && !fours ? (n >= 1024 ? wide : 4) : n % 4 == 0 ? 4 : 1);
   if (vw != 1 && vw != 4 && vw != 8) { err = "softmax: VW must be 1, 4 or 8"; return false; }
   if (vw > 1 && s.has("VW") && n % vw) { err = "softmax: VW=" + std::to_string(vw) + " needs a row length divisible by " + std::to_string(vw); return false; }
   int64_t tpr = s.get("TPR", 0);
   if (tpr == 0) {
-    // About four vectors per lane; on small launches of whole eights two, as many lanes as fours have (bf16 us with four vectors,
-    // two, and in fours: 1 x 4096 3.09, 2.65, 2.91; 300 x 2048 3.35, 2.99, 3.22; 1000 x 4096 5.2, 4.35, 4.5; but 4000 x 4096 10.6, 12.5)
-    tpr = nextPow2(ceilDiv(n, vw * (vw == 8 && n > 1536 && n <= 8192 && n % 8 == 0 && small ? 2 : 4)));
+    // About four vectors per lane; on small launches two of eights, as many lanes as fours have (bf16 us with four vectors,
+    // two, and in fours: 1 x 4096 3.09, 2.65, 2.91; 300 x 2048 3.35, 2.99, 3.22; 1000 x 4096 5.2, 4.35, 4.5; 1000 x 3893 7.2, 6.5; but 4000 x 4096 10.6, 12.5)
+    tpr = nextPow2(ceilDiv(n, vw * (vw == 8 && n > 1536 && n <= (n % 8 ? 4096 : 8192) && small ? 2 : 4)));
     if (tpr < 64) tpr = 64;
     if (tpr > 1024) tpr = 1024;
   }

@@ -63,6 +63,9 @@ def test_layernorm_of_16_bit_rows_keeps_its_lanes_and_its_alignment(rows, dtype)
         d = form(n)
         assert d["LN_VW"] == "4" and int(d["LN_TPR"]) == lanes_in_fours(n, 512), n
     assert form(768)["LN_VW"] == "4" and form(1000)["LN_VW"] == "8"
+    for n in (2503, 3893):          # single elements while every row has a workgroup of its own, then eights on as many lanes
+        d = form(n)
+        assert d["LN_VW"] == ("8" if rows > 512 else "1") and (rows <= 512 or int(d["LN_TPR"]) == lanes_in_fours(n, 512)), n
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
@@ -76,4 +79,5 @@ def test_softmax_of_16_bit_rows_keeps_its_lanes_and_its_alignment_on_small_launc
     for n in (1028, 1500, 2044, 3892, 5004, 8188):
         d = form(n)
         assert d["SM_VW"] == "4" and int(d["SM_TPR"]) == lanes_in_fours(n, 1024), n
-    assert int(form(4096, 16384)["SM_TPR"]) == 128 and form(3892, 16384)["SM_VW"] == "8" and form(1500, 16384)["SM_VW"] == "4"
+    assert int(form(4096, 16384)["SM_TPR"]) == 128 and form(3892, 16384)["SM_VW"] == "8" and form(1500, 4000)["SM_VW"] == "4"
+    assert int(form(3893, 1000)["SM_TPR"]) == lanes_in_fours(3893, 1024) and form(3893, 1000)["SM_VW"] == "8"
