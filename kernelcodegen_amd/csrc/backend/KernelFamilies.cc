@@ -463,9 +463,118 @@ bool checkTile(const KernelSpec& s, int64_t bm, int64_t bn, int64_t bk, int64_t 
 // in 32 bits: where more than the whole tiles of the direct-load kernels is taken, longer ones keep the other kernels.
 static bool shortRows(int64_t n, int64_t k) { return n <= (1 << 23) && k <= (1 << 23); }
 
+// GEMM whose wavefronts split k (kernels/gemm_wavek.hip).  type: 0 fp32, 1 bf16, 2 IEEE half, 3 fp8 e4m3.
+struct WavekForm { int64_t tm, tn, vw, wk, depth; };
+
+// Rows of whole 16-byte chunks (fp32: of four values and more; a 16-byte load of floats needs no more alignment than a float)
+// whose offsets within a tile stay in 32 bits, and whole loads of a row-major B.
+static bool wavekFits(const KernelSpec& s, int type, int64_t n, int64_t k) {
+  const int64_t es = type == 0 ? 4 : type == 3 ? 1 : 2;
+  return s.get("ALIGN", 0) >= 16 && shortRows(n, k) && k * es <= (1 << 24) && (type == 0 ? k >= 4 : k * es % 16 == 0) && !s.get("TA", 0) &&
+         (type == 0 || s.get("TB", 0) || n * es % 16 == 0) && s.get("SCALE_PTR", 0) == 0;
+}
+
+bool emitGemmWavek(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err, int type, const WavekForm& f,
+                   int64_t m, int64_t n, int64_t k, int64_t batch) {
+  const int64_t es = type == 0 ? 4 : type == 3 ? 1 : 2;
+  const bool tb = s.get("TB", 0) != 0;
+  if (!wavekFits(s, type, n, k)) { err = s.family + ": WAVEK needs aligned operands (ALIGN = 16) in rows of whole 16-byte chunks, A contiguous along k"; return false; }
+  if (f.tm < 1 || f.tm > 8 || f.tn < 1 || f.tn > 16 || f.wk < 1 || f.wk > 16 || f.depth < 1 || f.depth > 16 ||
+      (!tb && (f.vw * es < 2 || f.vw * es > 16 || (f.vw & (f.vw - 1)) || f.tn % f.vw || n % f.vw))) {
+    err = s.family + ": WAVEK is 1 to 16, TM 1 to 8, TN 1 to 16, DEPTH 1 to 16, and row-major weights need VW columns of 2 to 16 bytes that divide TN and N";
+    return false;
+  }
+  // (every wavefront needs a k-step of its own)
+  if (f.wk > ceilDiv(k * es, 128)) { err = s.family + ": WAVEK is at most the number of 128-byte steps along k"; return false; }
+  if (f.wk * std::max((16 * f.tm + (tb ? 16 * f.tn : 0)) * 128, 16 * f.tm * (16 * f.tn + 4) * 4) > 160 * 1024) { err = s.family + ": the wavefronts' rows and partial sums need more than 160 KiB of LDS"; return false; }
+  const bool out16 = s.get("OUT_BF16", 0) != 0;
+  s.p["WAVEK"] = f.wk; s.p["TM"] = f.tm; s.p["TN"] = f.tn; s.p["DEPTH"] = f.depth;
+  if (!tb) s.p["VW"] = f.vw;
+  Defines d;
+  d.add("GW_NAME", s.name);
+  d.add("GW_M", m); d.add("GW_N", n); d.add("GW_K", k); d.add("GW_BATCH", batch);
+  d.add("GW_TYPE", type);
+  d.add("GW_OUT16", out16 ? 1 : 0);
+  d.add("GW_TB", tb ? 1 : 0);
+  d.add("GW_TM", f.tm); d.add("GW_TN", f.tn);
+  if (!tb) d.add("GW_VW", f.vw);
+  d.add("GW_WK", f.wk);
+  d.add("GW_DEPTH", f.depth);
+  d.add("GW_RELU", s.get("RELU", 0) ? 1 : 0);
+  src = d.wrap(kTpl_gemm_wavek);
+  info.name = s.name;
+  info.grid[0] = (uint32_t)(ceilDiv(m, 16 * f.tm) * ceilDiv(n, 16 * f.tn));
+  info.grid[1] = (uint32_t)batch;
+  info.block[0] = (uint32_t)(64 * f.wk);
+  info.numArgs = type == 3 ? 5 : 3;
+  info.numScalars = type == 3 ? 2 : 0;
+  info.flops = 2.0 * (double)batch * (double)m * (double)n * (double)k;
+  info.bytes = (double)batch * ((double)es * ((double)m * k + (double)k * n) + (out16 ? 2.0 : 4.0) * (double)m * n);
+  return true;
+}
+
+static WavekForm wavekAsked(const KernelSpec& s, int type) {
+  return {s.get("TM", 1), s.get("TN", 4), s.get("VW", s.get("N", 0) % 4 || s.get("TN", 4) % 4 ? (type == 3 ? 2 : 1) : 4), s.get("WAVEK", 0), s.get("DEPTH", 2)};
+}
+
+// Time in us of a form whose wavefronts split k: a launch and the fixed parts of the kernel, then what is slowest of a compute
+// unit's intake (MB), the card's (MB from memory, MB through the L2s) and the MFMAs, and on top the partial sums (tiles x
+// wavefronts) and the steps that a wavefront waits for one after the other.  Fitted to 7000 timings of 200 products of the sizes
+// that launches of few tiles have (linear layers of 1 to 700 rows, 512 to 11008 columns, K 512 to 4096; fp32 256 to 2048 a
+// side, 1 to 16 of them): the form of least modelled time is within 3 % (k-contiguous B) to 7 % of the best on average.
+struct WavekRates { double fixed, cu, hbm, sums, wait, l2, mfma, odd; };
+static double wavekTime(int type, bool tb, bool out16, const WavekForm& f, int64_t m, int64_t n, int64_t k, int64_t batch) {
+  static const WavekRates rates[3][2] = {      // row-major B, k-contiguous B; `odd`: fp32 rows that start off 16 bytes, intake
+      {{2.35, 13.1, 0.41, 0.112, 0.024, 0.045, 1.55, 0.85}, {2.60, 8.25, 0.53, 0.131, 0.065, 0.018, 1.45, 1.24}},
+      {{2.23, 12.5, 0.21, 0.227, 0.103, 0.052, 3.42, 0.0}, {1.95, 8.82, 0.153, 0.408, 0.106, 0.041, 3.15, 0.0}},
+      {{2.40, 12.8, 0.267, 0.074, 0.127, 0.099, 2.97, 0.0}, {2.15, 10.2, 0.168, 0.220, 0.066, 0.047, 2.59, 0.0}}};
+  const WavekRates& r = rates[type == 0 ? 0 : type == 3 ? 2 : 1][tb ? 1 : 0];
+  const double es = type == 0 ? 4 : type == 3 ? 1 : 2, kb = (double)k * es;
+  const double tiles = (double)ceilDiv(m, 16 * f.tm) * (double)ceilDiv(n, 16 * f.tn) * (double)batch, per = std::ceil(tiles / 256.0);
+  const double rows = (double)std::min<int64_t>(16 * f.tm, ceilDiv(m, 8) * 8), bytes = (rows + 16.0 * f.tn) * kb;
+  const double steps = std::ceil(std::ceil(kb / 128.0) / (double)f.wk);
+  const double hbm = (kb * (double)(m + n) + (double)m * (double)n * (out16 ? 2.0 : 4.0)) * (double)batch;
+  const double mfma = (type == 0 ? 256.0 : type == 3 ? 64.0 : 32.0) * f.tm * f.tn * steps * per * std::max(1.0, f.wk / 4.0) / 2400.0;
+  // workgroups that a CU holds at a time: by LDS, and by registers (the slots, the sums, a set of fragments, addresses)
+  const int64_t lds = f.wk * std::max((16 * f.tm + (tb ? 16 * f.tn : 0)) * 128, 16 * f.tm * (16 * f.tn + 4) * 4);
+  const int64_t regs = ceilDiv(8 * f.depth * (f.tm + f.tn) + 4 * f.tm * f.tn + 8 * f.tm + 40, 8) * 8;
+  const int64_t waves = std::max<int64_t>(1, std::min<int64_t>(8, 512 / regs)) * 4;
+  const double held = (double)std::max<int64_t>(1, std::min<int64_t>(160 * 1024 / lds, waves / f.wk));
+  const double wait = std::ceil(tiles / (256.0 * held)) * steps / std::min<double>((double)f.depth, std::max(1.0, steps));
+  const double odd = type == 0 && k % 4 ? 1.0 + r.odd : 1.0;
+  auto p4 = [](double x) { return x * x * x * x; };
+  const double most = std::pow(p4(odd * r.cu * bytes * per / 1e6) + p4(odd * r.hbm * hbm / 1e6) + p4(odd * r.l2 * bytes * tiles / 1e6) + p4(r.mfma * mfma), 0.25);
+  return r.fixed + most + r.sums * per * f.tm * f.tn * f.wk / 16.0 + r.wait * wait;
+}
+
+// The form of least modelled time, if there is one and the caller asks for launches that fill the part (FILL); `us`: that time.
+static bool chooseWavek(const KernelSpec& s, int type, int64_t m, int64_t n, int64_t k, int64_t batch, WavekForm& best, double& us) {
+  if (!s.get("FILL", 0) || s.has("WAVEK") || !wavekFits(s, type, n, k)) return false;
+  static const int64_t tiles[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {1, 4}, {2, 4}, {4, 2}, {4, 4}, {3, 4}, {4, 3}};
+  const bool tb = s.get("TB", 0) != 0, out16 = s.get("OUT_BF16", 0) != 0;
+  const int64_t es = type == 0 ? 4 : type == 3 ? 1 : 2, steps = ceilDiv(k * es, 128);
+  us = 0.0;
+  for (const auto& t : tiles) {
+    const bool thirds = t[0] == 3 || t[1] == 3;
+    if ((thirds && type != 0) || (t[0] > 1 && 8 * t[0] >= m)) continue;
+    if (!tb && type == 3 && t[1] < 2) continue;                                    // loads of two columns and more
+    if (t[0] == 1 && t[1] == 4 && (tb || type != 3)) continue;
+    if (t[1] == 1 && t[0] == 2 && !tb) continue;
+    for (int64_t wk : {4, 8})
+      for (int64_t depth : {1, 2}) {
+        if (wk > steps || (depth > 1 && steps <= wk)) continue;
+        const WavekForm f = {t[0], t[1], tb ? 1 : n % 4 || t[1] % 2 ? 1 : std::min<int64_t>(t[1], 4), wk, depth};
+        const double time = wavekTime(type, tb, out16, f, m, n, k, batch);
+        if (us == 0.0 || time < us) { us = time; best = f; }
+      }
+  }
+  return us > 0.0;
+}
+
 bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err) {
   int64_t m, n, k, batch;
   if (!gemmCommon(s, err, m, n, k, batch)) return false;
+  if (s.get("WAVEK", 0) > 0) return emitGemmWavek(s, src, info, err, 0, wavekAsked(s, 0), m, n, k, batch);
   // The largest square tile that still gives every CU a workgroup (measured on 4096^3, 2048^3, 1024^3 and
   // 16 x 1024^3: 256^2 with 16 wavefronts, 128^2 with 16 and a deeper k-tile, 64^2 with 4 and a deeper k-tile).
   int64_t tile = 64;
@@ -484,6 +593,7 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   bool own = false;
   for (const char* key : {"BM", "BN", "BK", "WM", "WN", "WK", "NBUF", "PAD"}) own = own || s.has(key);
   const bool direct = s.get("D2L", 1) != 0 && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !s.get("TA", 0) && k % 4 == 0 && (s.get("TB", 0) || n % 4 == 0);
+  const bool any = own;
   const bool divides = m % tile == 0 && n % tile == 0 && k % (tile <= 128 ? 32 : 16) == 0;
   if (!own && (!divides || (direct && s.get("TB", 0))) && m >= 64 && n >= 64 && k >= 16) {
     static const struct { int64_t t; double weight; } sizes[] = {{256, 0.985}, {128, 1.0}, {64, 1.06}};
@@ -497,6 +607,21 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     s.p["BK"] = direct ? (tile == 64 && k % 32 == 0 ? 32 : 16) : (tile == 128 ? 32 : 16);
     s.p["WM"] = s.p["WN"] = tile == 64 ? 2 : 4;
     if (s.get("TB", 0)) { s.p["WK"] = 1; s.p["NBUF"] = 2; }    // two wavefront groups gain nothing where B is read 16 bytes at a time (19.9 us at 1024^3)
+  }
+  // Few tiles: wavefronts that split k, where the models say so clearly.  This kernel's time (fitted to the same products, within 12 %
+  // on average): rounds of tiles and the part of them in use, and on few 64 x 64 tiles a k-tile's way from memory.  us, this and
+  // that: 256^3 6.6 and 2.5, 256 x 256 x 2048 36 and 7.1, 2 x 700 x 300 x 1500 47 and 20; 1500 x 400 x 1100 34 and 22; level at
+  // 1024^3 (20); 4 x 1024^3 70 and 75.
+  if (!any && s.get("D2L", 1) != 0 && m >= 64 && n >= 64 && k >= 16) {
+    WavekForm form;
+    double us;
+    if (chooseWavek(s, 0, m, n, k, batch, form, us)) {
+      const double groups = (double)ceilDiv(m, tile) * (double)ceilDiv(n, tile) * (double)batch, rounds = std::ceil(groups / 256.0);
+      const double area = (double)(tile * tile) / 4096.0, used = std::max(0.3, groups / 256.0), sparse = tile == 64 ? std::max(0.0, 1.0 - groups / 512.0) : 0.0;
+      const double tiled = s.get("TB", 0) ? 2.95 + 0.01 * k * (area * (1.044 * rounds + 0.681 * used) * (direct ? 1.0 : 1.33) + 0.68 * sparse)
+                                          : 3.07 + 0.01 * k * (area * (1.454 * rounds + 0.239 * used) * (direct ? 1.0 : 1.26) + 0.32 * sparse);
+      if (us < 0.9 * tiled) return emitGemmWavek(s, src, info, err, 0, form, m, n, k, batch);
+    }
   }
   int64_t bm = s.get("BM", tile), bn = s.get("BN", tile);
   int64_t bk = s.get("BK", bm <= 128 && bn <= 128 ? 32 : 16);
@@ -710,7 +835,7 @@ bool chooseTailSplit(const KernelSpec& s, int64_t tiles, int64_t kt, int64_t bat
 // A small tile has few MFMAs per k-tile to hide a load under: with two buffers (one k-tile ahead) the 128 x 4096 x 4096
 // product waits 0.45 us per k-tile, with four 0.2.
 struct Gemm16Form { int64_t bm, bn, wm, wn, nbuf; double slots, a, b; };
-static const Gemm16Form* chooseGemm16Form(int64_t m, int64_t n, int64_t k, int64_t batch) {
+static const Gemm16Form* chooseGemm16Form(int64_t m, int64_t n, int64_t k, int64_t batch, double* modelled = nullptr) {
   static const Gemm16Form forms[] = {
       {256, 256, 4, 2, 2, 256, 55, 45}, {128, 128, 4, 2, 2, 512, 32, 31}, {128, 128, 4, 2, 3, 256, 14, 25},
       {64, 128, 2, 2, 3, 512, 13, 28},  {64, 128, 2, 2, 4, 256, 18, 5},   {64, 64, 2, 2, 4, 512, 12, 12},
@@ -718,6 +843,7 @@ static const Gemm16Form* chooseGemm16Form(int64_t m, int64_t n, int64_t k, int64
   // few rows: tiles of 32 x 64 (us, against 64 x 64: 8 x 1024 x 4096 9.2 and 11.6, 16 x 11008 x 4096 14.6 and 15.0, 32 x 4096 x
   // 4096 12.1 and 13.2, 1 x 4096 x 4096 11.4 and 12.3)
   static const Gemm16Form few = {32, 64, 1, 4, 4, 512, 0, 0};
+  if (modelled) *modelled = 0.0;
   if (m <= 32 && batch == 1 && n >= 64 && k >= 64) return &few;
   const Gemm16Form* best = nullptr;
   double least = 0.0;
@@ -731,18 +857,48 @@ static const Gemm16Form* chooseGemm16Form(int64_t m, int64_t n, int64_t k, int64
     const double cost = rounds * (f.a + f.b * tiles / (rounds * f.slots));
     if (!best || cost < least) { best = &f; least = cost; }
   }
+  if (modelled) *modelled = least;
   return best;
+}
+
+// Whether wavefronts that split k take less time than `tiled`, the form chosen above with `cost`: its time, fitted to the same
+// products as wavekTime (within 8 to 14 %), from that cost, or for 32-row tiles from their number.  us, this and that: bf16
+// k-contiguous 8 x 1024 x 4096 8.9 and 4.1, 16 x 2048 x 2048 5.6 and 3.3, 16 x 4096 x 4096 11.5 and 7.2, 64 x 1024 x 4096 12.8 and
+// 5.4, 200 x 1024 x 4096 13.3 and 8.7; but 64 x 11008 x 4096 22.1 against 21.3, 200 x 4096 x 1024 6.2 against 7.1.  fp8 row-major
+// 16 x 4096 x 4096 17.9 and 8.8.
+static bool wavekAhead(const KernelSpec& s, int type, const Gemm16Form* tiled, double cost, int64_t m, int64_t n, int64_t k, int64_t batch, WavekForm& form) {
+  double us;
+  if (!tiled || !chooseWavek(s, type, m, n, k, batch, form, us)) return false;
+  static const struct { double few0, few1, few2, hbm, many0, many1; } fits[2][2] = {     // 16 bits, fp8; row-major B, k-contiguous
+      {{1.95, 8.75, 0.0326, 0.0, 2.61, 1.124}, {2.13, 6.60, 0.0447, 0.0, 3.0, 0.897}},
+      {{1.55, 19.0, 0.141, 0.0, 2.88, 1.914}, {2.17, 9.54, 0.0145, 0.197, 2.44, 1.31}}};
+  const auto& c = fits[type == 3][s.get("TB", 0) ? 1 : 0];
+  const double es = type == 3 ? 1 : 2, depth = (double)k * es / 8192.0, hbm = c.hbm * (double)(m + n) * (double)k * es / 1e6;
+  const double chain = depth * (c.few1 + c.few2 * (double)ceilDiv(n, 64));
+  const double time = tiled->bm == 32 ? c.few0 + std::pow(chain * chain * chain * chain + hbm * hbm * hbm * hbm, 0.25) : c.many0 + c.many1 * depth * cost;
+  // What is asked of the models: 10 % for small tiles; 20 % for large ones, which near a full round of 256 are up to 18 % slower
+  // than modelled (1000 x 1024 x 4096 bf16 16.9, tiles 14.5); 30 % against whole fp8 tiles, which are faster than modelled.
+  // Over 560 products of 1 to 1500 rows the choice is then 1.22 times as fast as tiles alone, and 7 % slower at worst.
+  const bool wholeFp8 = type == 3 && m % 64 == 0 && n % 64 == 0 && k % 128 == 0;
+  return us < (wholeFp8 ? 0.7 : form.tm * form.tn >= 8 ? 0.8 : 0.9) * time;
 }
 
 bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err) {
   int64_t m, n, k, batch;
   if (!gemmCommon(s, err, m, n, k, batch)) return false;
+  if (s.get("WAVEK", 0) > 0) return emitGemmWavek(s, src, info, err, s.get("F16", 0) ? 2 : 1, wavekAsked(s, s.get("F16", 0) ? 2 : 1), m, n, k, batch);
   // Where the caller has looked at the operands' addresses (ALIGN = 16) and asks for no tile or switch of its own, and every
   // row starts on 16 bytes: one of the forms with direct loads
   bool own = false;
   for (const char* key : {"BM", "BN", "BK", "WM", "WN", "M16", "D2L", "BTR", "BPAD", "STAGES", "NBUF", "SK_UNITS", "INTERLEAVE", "SETPRIO"}) own = own || s.has(key);
   const Gemm16Form* form = nullptr;
-  if (!own && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !s.get("TA", 0) && k % 8 == 0 && (s.get("TB", 0) || n % 8 == 0)) form = chooseGemm16Form(m, n, k, batch);
+  if (!own && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !s.get("TA", 0) && k % 8 == 0 && (s.get("TB", 0) || n % 8 == 0)) {
+    double cost;
+    form = chooseGemm16Form(m, n, k, batch, &cost);
+    WavekForm split;
+    const int type = s.get("F16", 0) ? 2 : 1;
+    if (!s.get("FP8_PAIRS", 0) && wavekAhead(s, type, form, cost, m, n, k, batch, split)) return emitGemmWavek(s, src, info, err, type, split, m, n, k, batch);
+  }
   if (form) {
     s.p["BM"] = form->bm; s.p["BN"] = form->bn; s.p["WM"] = form->wm; s.p["WN"] = form->wn;
     s.p["M16"] = 1; s.p["D2L"] = 1; s.p["NBUF"] = form->nbuf;
@@ -886,6 +1042,7 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
 bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err) {
   int64_t m, n, k, batch;
   if (!gemmCommon(s, err, m, n, k, batch)) return false;
+  if (s.get("WAVEK", 0) > 0) return emitGemmWavek(s, src, info, err, 3, wavekAsked(s, 3), m, n, k, batch);
   const bool ta = s.get("TA", 0) != 0, tb = s.get("TB", 0) != 0;
   // As for 16 bits: where the operands' addresses are known to be aligned and no tile or switch is asked for, one of the
   // forms with direct loads, priced as a 16-bit product of half the depth.  256 x 256 tiles run on gemm_fp8_d2l.hip
@@ -899,6 +1056,12 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   int64_t dm, dn;
   defaultGemmTile(m, n, batch, dm, dn);
   const bool whole = m % dm == 0 && n % dn == 0 && k % 128 == 0;
+  if (!own && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !ta && k % 16 == 0 && n % 16 == 0 && s.get("SCALE_PTR", 0) == 0) {
+    double cost;
+    const Gemm16Form* tiled = chooseGemm16Form(m, n, k / 2, batch, &cost);
+    WavekForm split;
+    if (wavekAhead(s, 3, tiled, cost, m, n, k, batch, split)) return emitGemmWavek(s, src, info, err, 3, split, m, n, k, batch);
+  }
   if (!own && !whole && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !ta && k % 16 == 0 && n % 16 == 0 && s.get("SCALE_PTR", 0) == 0) {
     const Gemm16Form* form = chooseGemm16Form(m, n, k / 2, batch);
     // Shallow products of two k-contiguous operands lose little to guarded loads, and those run on gemm_fp8.hip's larger MFMA:

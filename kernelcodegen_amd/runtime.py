@@ -355,8 +355,21 @@ def compile_source(src, infos=None, opts=()):
 _kernel_cache = {}
 
 
+_GEMMS = ("gemm_f32", "gemm_bf16", "gemm_fp8")
+
+
+def launch_params(family, params):
+    """The parameters of a kernel that is compiled to be launched from here: a product whose caller has looked at the operands'
+    addresses (ALIGN = 16) and asks for nothing else may take the form that fills the part best (FILL), whose wavefronts split k.
+    Text that is emitted for others to keep has the tiles that its parameters name."""
+    if family in _GEMMS and params.get("ALIGN", 0) >= 16:
+        return {"FILL": 1, **params}
+    return params
+
+
 def get_kernel(family, **params):
     """Emit + compile + load one kernel of a family; memoised per process."""
+    params = launch_params(family, params)
     key = (family, tuple(sorted(params.items())))
     if key not in _kernel_cache:
         text, info = emit_kernel(family, "kernel0", **params)

@@ -1,0 +1,52 @@
+"""When a product takes the form whose wavefronts split k, and that every form compiles into registers (no GPU needed)."""
+import pytest
+
+from kernelcodegen_amd import _lib, runtime as R
+from test_gemm_forms import scratch_bytes
+
+
+def text_of(family, **params):
+    return R.emit_kernel(family, "kernel0", **R.launch_params(family, params))[0]
+
+
+SPLIT = "#define GW_WK"
+
+
+def test_only_aligned_products_without_wishes_split_k():
+    """Launched from here, on operands known to be aligned, in rows of whole chunks, A contiguous along k; all else keeps its kernel."""
+    small = dict(M=8, N=1024, K=4096, TB=1, ALIGN=16)
+    assert SPLIT in text_of("gemm_bf16", **small) and SPLIT in text_of("gemm_fp8", **small)
+    assert SPLIT not in R.emit_kernel("gemm_bf16", "kernel0", **small)[0]
+    for other in (dict(ALIGN=0), dict(K=4097), dict(K=4100), dict(TB=0, N=1020), dict(M=4096, N=4096), dict(BM=64, BN=64), dict(D2L=0), dict(WAVEK=0), dict(TA=1)):
+        assert SPLIT not in text_of("gemm_bf16", **dict(small, **other)), other
+    for other in (dict(ALIGN=0), dict(K=4104), dict(N=1032, TB=0), dict(SCALE_PTR=1), dict(BM=64, BN=64), dict(WAVEK=0)):
+        assert SPLIT not in text_of("gemm_fp8", **dict(small, **other)), other
+    single = dict(M=256, N=256, K=1024, ALIGN=16)
+    for same in (dict(), dict(TB=1), dict(K=1023), dict(N=255), dict(BATCH=3)):
+        assert SPLIT in text_of("gemm_f32", **dict(single, **same)), same
+    for other in (dict(ALIGN=0), dict(M=4096, N=4096), dict(M=60), dict(TA=1), dict(WK=2), dict(D2L=0), dict(WAVEK=0)):
+        assert SPLIT not in text_of("gemm_f32", **dict(single, **other)), other
+
+
+@pytest.mark.parametrize("bad", [dict(WAVEK=17), dict(TM=9), dict(TN=17), dict(DEPTH=17), dict(WAVEK=16, K=64), dict(TM=8, TN=8, WAVEK=8), dict(TB=0, VW=16),
+                                 dict(TB=0, TN=2, VW=4), dict(ALIGN=0), dict(K=1001), dict(TA=1)])
+def test_what_is_asked_for_and_does_not_fit_is_refused(bad):
+    with pytest.raises(_lib.KcgError):
+        R.emit_kernel("gemm_bf16", "kernel0", **dict(dict(M=100, N=512, K=1024, TB=1, ALIGN=16, WAVEK=4), **bad))
+
+
+@pytest.mark.parametrize("family,extra", [("gemm_bf16", dict(OUT_BF16=1)), ("gemm_bf16", dict(F16=1, RELU=1)), ("gemm_fp8", dict(OUT_BF16=1)), ("gemm_f32", dict())])
+@pytest.mark.parametrize("tb", [0, 1])
+def test_every_chosen_form_stays_in_registers(family, extra, tb):
+    seen = set()
+    for m, n, k in [(1, 512, 528), (8, 1024, 4096), (16, 4096, 4096), (64, 1024, 4096), (100, 1024, 4096), (200, 1024, 4096), (300, 640, 1216), (256, 256, 2048),
+                    (300, 300, 1002), (500, 500, 500), (914, 752, 1227)]:
+        if family != "gemm_f32" and (k % 16 or n % 16):
+            continue
+        text = text_of(family, M=m, N=n, K=k, TB=tb, ALIGN=16, **extra)
+        if SPLIT in text:
+            form = tuple(l.split()[2] for l in text.splitlines() if l.startswith(("#define GW_TM", "#define GW_TN", "#define GW_WK", "#define GW_DEPTH")))
+            if form not in seen:
+                seen.add(form)
+                assert scratch_bytes(R.compile_to_code(R.prelude() + text)) == 0, (m, n, k, form)
+    assert len(seen) >= 3, seen
