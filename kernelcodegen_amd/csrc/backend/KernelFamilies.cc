@@ -547,9 +547,9 @@ static double wavekTime(int type, bool tb, bool out16, const WavekForm& f, int64
   return r.fixed + most + r.sums * per * f.tm * f.tn * f.wk / 16.0 + r.wait * wait;
 }
 
-// The form of least modelled time, if there is one and the caller asks for launches that fill the part (FILL); `us`: that time.
+// The form of least modelled time, if there is one and the caller asks for it (FILL = 2); `us`: that time.
 static bool chooseWavek(const KernelSpec& s, int type, int64_t m, int64_t n, int64_t k, int64_t batch, WavekForm& best, double& us) {
-  if (!s.get("FILL", 0) || s.has("WAVEK") || !wavekFits(s, type, n, k)) return false;
+  if (s.get("FILL", 0) < 2 || s.has("WAVEK") || !wavekFits(s, type, n, k)) return false;
   static const int64_t tiles[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {1, 4}, {2, 4}, {4, 2}, {4, 4}, {3, 4}, {4, 3}};
   const bool tb = s.get("TB", 0) != 0, out16 = s.get("OUT_BF16", 0) != 0;
   const int64_t es = type == 0 ? 4 : type == 3 ? 1 : 2, steps = ceilDiv(k * es, 128);
@@ -1216,9 +1216,91 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   return true;
 }
 
+// Attention whose wavefronts split the keys (kernels/fmha_wavek.hip).  type: 0 fp32, 1 bf16, 2 IEEE half.
+static int64_t fmhaWavekLds(int type, int64_t d, int64_t qb, int64_t wk) {
+  const int64_t row = d * (type == 0 ? 4 : 2);
+  return wk * (std::max(32 * (2 * row + 48), 32 * (d * 4 + 16)) + 32 * qb * 8);
+}
+
+// Wavefronts per SIMD that the registers of a form leave room for (130 to 190 of them in 16 bits, 174 to 361 in fp32).
+static int64_t fmhaWavekEu(int type, int64_t d, int64_t qb) { return type != 0 ? (d <= 64 && qb == 1 ? 4 : qb == 2 && d > 64 ? 1 : 2) : d <= 64 && qb == 1 ? 2 : 1; }
+
+bool emitFmhaWavek(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err, int type, int64_t qb, int64_t wk) {
+  const int64_t b = s.p["B"], h = s.p["H"], sl = s.p["S"], dh = s.p["D"];
+  const int64_t es = type == 0 ? 4 : 2;
+  if ((dh != 32 && dh != 64 && dh != 128) || qb < 1 || qb > 2 || wk < 1 || wk > 16 || fmhaWavekLds(type, dh, qb, wk) > 160 * 1024 ||
+      (double)sl * (double)dh * (double)es >= 2147483648.0 || (double)ceilDiv(sl, 32 * qb) * (double)b * (double)h > 2147483647.0) {
+    err = s.family + ": WAVEK needs a head dim of 32, 64 or 128, QB 1 or 2, at most 16 wavefronts whose tiles fit 160 KiB of LDS, and heads below 2 GiB";
+    return false;
+  }
+  if (s.f.count("SCALE") && !(s.f["SCALE"] > 0.0)) { err = s.family + ": the softmax scale must be positive"; return false; }
+  const bool causal = s.get("CAUSAL", 0) != 0, out16 = type != 0 && s.get("OUT_BF16", 1) != 0;
+  const double scale = s.f.count("SCALE") ? s.f["SCALE"] : 1.0;
+  s.p["WAVEK"] = wk; s.p["QB"] = qb; s.p["CAUSAL"] = causal;
+  s.f["SCALE"] = scale;
+  Defines d;
+  d.add("FW_NAME", s.name);
+  d.add("FW_B", b); d.add("FW_H", h); d.add("FW_S", sl); d.add("FW_D", dh);
+  d.add("FW_TYPE", type);
+  d.add("FW_OUT16", out16 ? 1 : 0);
+  d.add("FW_QB", qb); d.add("FW_WK", wk);
+  d.add("FW_EU", std::max<int64_t>(1, s.get("EU", std::max(fmhaWavekEu(type, dh, qb), wk / 4))));
+  d.add("FW_CAUSAL", causal ? 1 : 0);
+  d.add("FW_C", floatLiteral(scale * 1.4426950408889634));
+  src = d.wrap(kTpl_fmha_wavek);
+  info.name = s.name;
+  info.grid[0] = (uint32_t)(ceilDiv(sl, 32 * qb) * b * h);
+  info.block[0] = (uint32_t)(64 * wk);
+  info.numArgs = 4;
+  info.flops = 4.0 * (double)b * h * (double)sl * sl * dh * (causal ? 0.5 : 1.0);
+  info.bytes = (double)b * h * sl * dh * (3.0 * es + (out16 ? 2.0 : 4.0));
+  return true;
+}
+
+// Whether wavefronts that split the keys take less time than workgroups of `br` queries that walk them (`items` of them, two query
+// tiles each if `paired`, `held` by a compute unit at a time), for callers who ask for it (FILL = 2; 1: tiles that fill the part); the
+// form in qb, wk.  Both times are modelled, in us: a launch, then the longer of the walk of one workgroup, in 32-key tiles times rounds, and the work
+// of a compute unit; for the split also the merge and the bytes out of the L2s.  Fitted to 2600 timings of 460 launches (8 to
+// 256 heads, S 64 to 2048), 10 to 22 % off on average, hence the margin: the choice is then 1.2 (bf16, head dim 64), 1.27 (128), 1.6 (fp32, 64)
+// and 1.47 (128) times as fast as walks alone and no more than 5 % slower on all but one of them.  us, walk and split, D 64: bf16
+// heads x S 8 x 333 7.8 and 4.7, 8 x 1024 14.5 and 7.8, 32 x 512 9.3 and 7.6; but 32 x 1024 15.8 and 17.2, 128 x 512 15.5 and 18.3; fp32
+// 8 x 1024 78 and 23, 32 x 512 44 and 23, 48 x 1024 133 and 113, but 128 x 512 76 and 84.
+static bool fmhaWavekAhead(const KernelSpec& s, int type, int64_t br, bool paired, double items, int64_t held, int64_t& qb, int64_t& wk) {
+  const int64_t sl = s.get("S", 0), dh = s.get("D", 0);
+  const double heads = (double)s.get("B", 0) * (double)s.get("H", 0);
+  if (s.get("FILL", 0) < 2 || s.has("WAVEK") || (dh != 64 && dh != 128) || (double)sl * (double)dh * 4.0 >= 2147483648.0) return false;
+  struct Rates { double fixed, walk, work, merge, l2, tiled, tiledWalk, tiledWork, ragged, margin; };
+  static const Rates rates[2][2] = {      // 16 bits, fp32; head dim 64, 128
+      {{1.94, 0.745, 0.415, 3.71, 0.0186, 2.90, 0.449, 0.104, 0.097, 0.85}, {1.87, 1.01, 0.714, 8.07, 0.0436, 3.93, 0.837, 0.179, 0.091, 0.78}},
+      {{0.89, 3.07, 2.25, 8.94, 0.0007, 2.66, 2.61, 0.664, 0.017, 0.8}, {0.88, 4.94, 0.449, 18.3, 0.115, 5.70, 4.24, 1.32, 0.017, 0.78}}};
+  const Rates& r = rates[type == 0][dh == 128];
+  const bool causal = s.get("CAUSAL", 0) != 0;
+  const double tiles = (double)ceilDiv(sl, 32), mean = causal ? (tiles + 1.0) / 2.0 : tiles;
+  auto longer = [](double a, double b, double c) { return std::pow(a * a * a * a + b * b * b * b + c * c * c * c, 0.25); };
+  const double each = paired ? tiles + br / 32 : causal ? (tiles + br / 32) / 2.0 : tiles;
+  const double rounds = std::ceil(items / (256.0 * (double)held)), longest = causal && !paired ? tiles : each;
+  const bool ragged = sl % br != 0 || sl % 64 != 0;
+  const double walk = r.tiled + (1.0 + (ragged ? r.ragged : 0.0)) * longer(r.tiledWalk * rounds * longest, r.tiledWork * each * items / 256.0 * (br / 32), 0.0);
+  double least = 0.0;
+  const int64_t row = dh * (type == 0 ? 4 : 2);
+  for (int64_t q : {1, 2})
+    for (int64_t w : {2, 4, 8}) {
+      if ((double)w > tiles || (q == 2 && (dh == 128 || (type == 0 && w != 4))) || fmhaWavekLds(type, dh, q, w) > 160 * 1024) continue;
+      const double groups = (double)ceilDiv(sl, 32 * q) * heads, per = std::ceil(groups / 256.0);
+      const int64_t fit = std::max<int64_t>(1, std::min<int64_t>(160 * 1024 / fmhaWavekLds(type, dh, q, w), fmhaWavekEu(type, dh, q) * 4 / w));
+      const double turns = std::ceil(groups / (256.0 * (double)fit));
+      const double chain = turns * std::ceil((turns == 1.0 ? tiles : mean) / (double)w);
+      const double work = (causal ? std::max(groups / 256.0, 1.0) * 1.15 : per) * mean * (double)q / 4.0;
+      const double us = r.fixed + longer(r.walk * chain, r.work * work, r.l2 * groups * mean * (double)row * 64.0 / 1e6) + r.merge * (double)(w * q) * per / 16.0;
+      if (least == 0.0 || us < least) { least = us; qb = q; wk = w; }
+    }
+  return least > 0.0 && least < r.margin * walk;
+}
+
 bool emitFmhaBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err) {
   if (!need(s, {"B", "H", "S", "D"}, err) || !positive(s, {"B", "H", "S", "D"}, err)) return false;
   const int64_t b = s.p["B"], h = s.p["H"], sl = s.p["S"], dh = s.p["D"];
+  if (s.get("WAVEK", 0) > 0) return emitFmhaWavek(s, src, info, err, s.get("F16", 0) ? 2 : 1, s.get("QB", 1), s.get("WAVEK", 0));
   if (dh % 32 || dh > 256) { err = "fmha_bf16: head dim must be a multiple of 32, at most 256"; return false; }
   int64_t br = s.get("BR", 0), bc = s.get("BC", 0);
   // A sequence length that the tiles do not divide is taken too (the kernel guards its last query and key tiles); the
@@ -1274,6 +1356,12 @@ bool emitFmhaBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   if (lds > 160 * 1024) { err = "fmha_bf16: tile needs more than 160 KiB of LDS"; return false; }
   const bool causal = s.get("CAUSAL", 0) != 0, outBf16 = s.get("OUT_BF16", 1) != 0;
   const double scale = s.f.count("SCALE") ? s.f["SCALE"] : 1.0;
+  if (!own) {
+    const bool two = causal && !noPair && ((b * h) % 2 == 0 || ceilDiv(sl, br) % 2 == 0);
+    int64_t splitQb, splitWk;
+    if (fmhaWavekAhead(s, s.get("F16", 0) ? 2 : 1, br, two, (double)ceilDiv(sl, br) * heads / (two ? 2.0 : 1.0), std::max<int64_t>(1, 8 / (br / 32)), splitQb, splitWk))
+      return emitFmhaWavek(s, src, info, err, s.get("F16", 0) ? 2 : 1, splitQb, splitWk);
+  }
   s.p["BR"] = br; s.p["BC"] = bc; s.p["QW"] = qw; s.p["CAUSAL"] = causal; s.p["OUT_BF16"] = outBf16;
   s.f["SCALE"] = scale;
 
@@ -1338,7 +1426,10 @@ bool emitFmhaBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
 bool emitFmhaF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err) {
   if (!need(s, {"B", "H", "S", "D"}, err) || !positive(s, {"B", "H", "S", "D"}, err)) return false;
   const int64_t b = s.p["B"], h = s.p["H"], sl = s.p["S"], dh = s.p["D"];
+  if (s.get("WAVEK", 0) > 0) return emitFmhaWavek(s, src, info, err, 0, s.get("QB", 1), s.get("WAVEK", 0));
   if (dh % 32 || dh > 256) { err = "fmha_f32: head dim must be a multiple of 32, at most 256"; return false; }
+  bool own = false;
+  for (const char* key : {"BR", "BC", "D2L", "OCC", "PAIR"}) own = own || s.has(key);
   // queries per workgroup (32 per wavefront): four wavefronts, fewer for short sequences
   int64_t br = s.get("BR", 0);
   bool halved = false;
@@ -1387,6 +1478,11 @@ bool emitFmhaF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // instead of 40 at B1 H5 S1024 take 0.129 against 0.114 ms)
   const bool pair = s.get("PAIR", pairFits && (halved || (nq / 2) * b * h >= 512) ? 1 : 0) != 0;
   if (pair && !pairFits) { err = "fmha_f32: PAIR needs the causal mask and an even number of query tiles"; return false; }
+  if (!own) {
+    int64_t splitQb, splitWk;
+    if (fmhaWavekAhead(s, 0, br, pair, (double)((pair ? nq / 2 : nq) * b * h), std::max<int64_t>(1, 4 * occ / (br / 32)), splitQb, splitWk))
+      return emitFmhaWavek(s, src, info, err, 0, splitQb, splitWk);
+  }
   s.p["BR"] = br; s.p["BC"] = bc; s.p["CAUSAL"] = causal; s.p["OCC"] = occ; s.p["D2L"] = d2l; s.p["PAIR"] = pair;
   s.f["SCALE"] = scale;
 

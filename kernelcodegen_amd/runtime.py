@@ -355,15 +355,12 @@ def compile_source(src, infos=None, opts=()):
 _kernel_cache = {}
 
 
-_GEMMS = ("gemm_f32", "gemm_bf16", "gemm_fp8")
-
-
 def launch_params(family, params):
-    """The parameters of a kernel that is compiled to be launched from here: a product whose caller has looked at the operands'
-    addresses (ALIGN = 16) and asks for nothing else may take the form that fills the part best (FILL), whose wavefronts split k.
-    Text that is emitted for others to keep has the tiles that its parameters name."""
-    if family in _GEMMS and params.get("ALIGN", 0) >= 16:
-        return {"FILL": 1, **params}
+    """The parameters of a kernel that is compiled to be launched from here.  A product whose caller has looked at the operands'
+    addresses (ALIGN = 16) and attention that is to fill the part (FILL = 1) may also take the forms whose wavefronts split k or
+    the keys (FILL = 2).  Text that is emitted for others to keep has the tiles that its parameters name."""
+    if (family.startswith("gemm_") and params.get("ALIGN", 0) >= 16 and "FILL" not in params) or (family.startswith("fmha_") and params.get("FILL") == 1):
+        return {**params, "FILL": 2}
     return params
 
 

@@ -1,0 +1,42 @@
+"""When attention takes the form whose wavefronts split the keys, and that every form compiles into registers (no GPU needed)."""
+import pytest
+
+from kernelcodegen_amd import _lib, runtime as R
+from test_gemm_forms import scratch_bytes
+
+SPLIT = "#define FW_WK"
+
+
+def text_of(family, **params):
+    return R.emit_kernel(family, "kernel0", **R.launch_params(family, params))[0]
+
+
+@pytest.mark.parametrize("family", ["fmha_bf16", "fmha_f32"])
+def test_only_small_launches_without_wishes_split_the_keys(family):
+    small = dict(B=1, H=8, S=333, D=64, SCALE=0.1, FILL=1)
+    assert SPLIT in text_of(family, **small) and SPLIT in text_of(family, **dict(small, D=128, CAUSAL=1))
+    assert SPLIT not in R.emit_kernel(family, "kernel0", **small)[0]
+    for other in (dict(FILL=0), dict(B=8, H=32, S=2048), dict(D=96), dict(D=32), dict(BR=64), dict(BC=32), dict(WAVEK=0)):
+        assert SPLIT not in text_of(family, **dict(small, **other)), other
+
+
+@pytest.mark.parametrize("bad", [dict(WAVEK=17), dict(QB=3), dict(D=96), dict(D=256), dict(SCALE=-1.0), dict(WAVEK=16, D=128), dict(B=0)])
+def test_what_is_asked_for_and_does_not_fit_is_refused(bad):
+    with pytest.raises(_lib.KcgError):
+        R.emit_kernel("fmha_bf16", "kernel0", **dict(dict(B=1, H=8, S=333, D=64, WAVEK=4), **bad))
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("family,extra", [("fmha_bf16", dict()), ("fmha_bf16", dict(F16=1)), ("fmha_bf16", dict(OUT_BF16=0)), ("fmha_f32", dict())])
+def test_every_chosen_form_stays_in_registers(family, extra, causal):
+    seen = set()
+    for heads in (8, 32, 64):
+        for s in (33, 64, 100, 333, 777, 2048):
+            for d in (64, 128):
+                text = text_of(family, B=1, H=heads, S=s, D=d, CAUSAL=causal, SCALE=0.1, FILL=1, **extra)
+                if SPLIT in text:
+                    form = (d, s % 32 == 0) + tuple(l.split()[2] for l in text.splitlines() if l.startswith(("#define FW_WK", "#define FW_QB", "#define FW_EU")))
+                    if form not in seen:
+                        seen.add(form)
+                        assert scratch_bytes(R.compile_to_code(R.prelude() + text)) == 0, (heads, s, form)
+    assert len(seen) >= 5, seen
