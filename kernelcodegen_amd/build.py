@@ -20,6 +20,7 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 KDIR = os.path.join(CSRC, "backend", "kernels")
 LIB = os.path.join(PKG, "libkcg_hip.so")
+LAUNCH = os.path.join(PKG, "_launch.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 CXX = os.environ.get("CXX", "g++")
@@ -61,7 +62,36 @@ def _stamp():
     return h.hexdigest()
 
 
+def build_launch(force=False, verbose=False):
+    """The bound launches of the Python operators (csrc/python/launch.cc), an extension module on torch's own libraries."""
+    import sysconfig
+    import torch
+    src = os.path.join(CSRC, "python", "launch.cc")
+    base = os.path.join(os.path.dirname(torch.__file__))
+    inc = os.path.join(base, "include")
+    cmd = [CXX, "-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", inc, "-I", os.path.join(inc, "torch", "csrc", "api", "include"),
+           "-I", os.path.join(ROCM, "include"), "-I", sysconfig.get_paths()["include"], src, "-o", LAUNCH, "-L", os.path.join(base, "lib"),
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    stamp_file = LAUNCH + ".stamp"
+    stamp = hashlib.sha256((open(src).read() + " ".join(cmd) + torch.__version__).encode()).hexdigest()
+    if not force and os.path.exists(LAUNCH) and os.path.exists(stamp_file) and open(stamp_file).read() == stamp:
+        return LAUNCH
+    if verbose:
+        print(" ".join(cmd))
+    subprocess.check_call(cmd, stderr=None if verbose else subprocess.DEVNULL)
+    with open(stamp_file, "w") as f:
+        f.write(stamp)
+    return LAUNCH
+
+
 def build(force=False, verbose=False):
+    """libkcg_hip.so and the native launches; returns the library."""
+    build_launch(force, verbose)
+    return build_library(force, verbose)
+
+
+def build_library(force=False, verbose=False):
     gen_templates()
     stamp_file = LIB + ".stamp"
     stamp = _stamp()

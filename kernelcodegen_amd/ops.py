@@ -22,11 +22,20 @@ def _need_cuda(*ts):
 _bound = {}
 
 
-def _bind(key, cfg, kern, scalars=0):
-    run = kern.bind(scalars)
-    if key is not None and not cfg:
-        _bound[key] = run
-    return run
+def _into(run, shape=None, dtype=None):
+    """A bound launch whose last pointer is the result: a function of the operand tensors (and numbers) that allocates the result,
+    of that shape and type on the first operand's device, or like the first operand, launches and returns it."""
+    native = getattr(run, "result", None)
+    if native is not None:
+        return native(shape, dtype)
+
+    def call(*operands):
+        first = operands[0]
+        out = torch.empty_like(first) if shape is None else torch.empty(shape, dtype=dtype, device=first.device)
+        pointers = [t.data_ptr() for t in operands if isinstance(t, torch.Tensor)]
+        run(*pointers, out.data_ptr(), *operands[len(pointers):])
+        return out
+    return call
 
 
 # storage type of the row kernels (their arithmetic is fp32 throughout): the kernels' F16 parameter
@@ -38,12 +47,16 @@ def layernorm(x, gamma, beta, axis, eps=1e-5, gelu=False, out=None, **cfg):
     # plain numbers: a key must not hold an object that can change, nor find 1 for a refused 1.0
     axis, eps, gelu = operator.index(axis), float(eps), int(gelu)
     key = ("layernorm", x.shape, x.dtype, gamma.shape, gamma.dtype, beta.shape, beta.dtype, axis, eps, gelu)
-    run = None if cfg else _bound.get(key)
-    if run is None:
-        run = _bind(key, cfg, _layernorm_kernel(x, gamma, beta, axis, eps, gelu, cfg))
-    y = torch.empty_like(x) if out is None else out
-    run(x.data_ptr(), gamma.data_ptr(), beta.data_ptr(), y.data_ptr())
-    return y
+    hit = None if cfg else _bound.get(key)
+    if hit is None:
+        run = _layernorm_kernel(x, gamma, beta, axis, eps, gelu, cfg).bind()
+        hit = run, _into(run)
+        if not cfg:
+            _bound[key] = hit
+    if out is None:
+        return hit[1](x, gamma, beta)
+    hit[0](x.data_ptr(), gamma.data_ptr(), beta.data_ptr(), out.data_ptr())
+    return out
 
 
 def _layernorm_kernel(x, gamma, beta, axis, eps, gelu, cfg):
@@ -63,13 +76,19 @@ def elementwise(x, op, inplace=False, out_dtype=None, **cfg):
     _need_cuda(x)
     out_dtype, inplace = out_dtype or x.dtype, int(inplace)
     key = ("elementwise", x.numel(), op, inplace, x.dtype, out_dtype)
-    run = None if cfg else _bound.get(key)
-    if run is None:
-        run = _bind(key, cfg, R.get_kernel("elementwise", N=x.numel(), OP=op, INPLACE=int(inplace), IN_T=_CTYPE[x.dtype],
-                                           OUT_T=_CTYPE[out_dtype], **cfg))
+    hit = None if cfg else _bound.get(key)
+    if hit is None:
+        run = R.get_kernel("elementwise", N=x.numel(), OP=op, INPLACE=int(inplace), IN_T=_CTYPE[x.dtype],
+                           OUT_T=_CTYPE[out_dtype], **cfg).bind()
+        hit = run, None if inplace or out_dtype != x.dtype else _into(run)
+        if not cfg:
+            _bound[key] = hit
+    run, into = hit
     if inplace:
         run(x.data_ptr())
-        return x.view(out_dtype)
+        return x if out_dtype == x.dtype else x.view(out_dtype)
+    if into is not None:
+        return into(x)
     y = torch.empty(x.shape, dtype=out_dtype, device=x.device)
     run(x.data_ptr(), y.data_ptr())
     return y
@@ -103,14 +122,11 @@ def batched_matmul(a, b, trans_a=False, trans_b=False, out_dtype=None, **cfg):
         hit = _matmul_launch(a, b, trans_a, trans_b, out_dtype, cfg)
         if not cfg:
             _bound[key] = hit
-    run, shape, out_dtype = hit
-    c = torch.empty(shape, dtype=out_dtype, device=a.device)
-    run(a.data_ptr(), b.data_ptr(), c.data_ptr())
-    return c
+    return hit(a, b)
 
 
 def _matmul_launch(a, b, trans_a, trans_b, out_dtype, cfg):
-    """The bound kernel, shape and type of the result."""
+    """The bound kernel, which allocates its result."""
     if a.dtype != b.dtype or a.dtype not in _FAMILY:
         raise ValueError("unsupported operand dtypes")
     batch = int(math.prod(a.shape[:-2])) if a.dim() > 2 else 1
@@ -138,9 +154,8 @@ def _matmul_launch(a, b, trans_a, trans_b, out_dtype, cfg):
     # (the caller's parameters go before the alignment's, and may not name any other)
     kern = R.get_kernel(_FAMILY[a.dtype], M=m, N=n, K=k, BATCH=batch, TA=int(trans_a), TB=int(trans_b),
                         **extra, **{**align, **cfg})
-    if kern.info["workspace_bytes"]:
-        return (lambda *p: kern.launch(*p)), tuple(a.shape[:-2]) + (m, n), out_dtype
-    return kern.bind(), tuple(a.shape[:-2]) + (m, n), out_dtype
+    run = (lambda *p: kern.launch(*p)) if kern.info["workspace_bytes"] else kern.bind()
+    return _into(run, tuple(a.shape[:-2]) + (m, n), out_dtype)
 
 
 def matmul_fp8(a, b, scale_a, scale_b, trans_a=False, trans_b=True, out_dtype=torch.float32, **cfg):
@@ -155,10 +170,7 @@ def matmul_fp8(a, b, scale_a, scale_b, trans_a=False, trans_b=True, out_dtype=to
         hit = _matmul_fp8_launch(a, b, trans_a, trans_b, out_dtype, cfg)
         if not cfg:
             _bound[key] = hit
-    run, shape = hit
-    c = torch.empty(shape, dtype=out_dtype, device=a.device)
-    run(a.data_ptr(), b.data_ptr(), c.data_ptr(), float(scale_a), float(scale_b))
-    return c
+    return hit(a, b, float(scale_a), float(scale_b))
 
 
 def _matmul_fp8_launch(a, b, trans_a, trans_b, out_dtype, cfg):
@@ -173,7 +185,7 @@ def _matmul_fp8_launch(a, b, trans_a, trans_b, out_dtype, cfg):
         raise ValueError("incompatible K dimensions")
     kern = R.get_kernel("gemm_fp8", M=m, N=n, K=k, BATCH=batch, TA=int(trans_a), TB=int(trans_b),
                         OUT_BF16=int(out_dtype == torch.bfloat16), **{**_alignment(_aligned(a, b)), **cfg})
-    return kern.bind(scalars=2), tuple(a.shape[:-2]) + (m, n)
+    return _into(kern.bind(scalars=2), tuple(a.shape[:-2]) + (m, n), out_dtype)
 
 
 def matmul(a, b, **cfg):
@@ -202,10 +214,10 @@ def fmha(q, k, v, scale=None, causal=False, out_dtype=None, **cfg):
         else:
             kern = R.get_kernel("fmha_bf16", B=b, H=h, S=s, D=d, CAUSAL=int(causal), SCALE=scale,
                                 OUT_BF16=int(out_dtype == q.dtype), F16=int(q.dtype == torch.float16), **{"FILL": 1, **cfg})
-        run = _bind(key, cfg, kern)
-    o = torch.empty(q.shape, dtype=out_dtype, device=q.device)
-    run(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr())
-    return o
+        run = _into(kern.bind(), tuple(q.shape), out_dtype)
+        if not cfg:
+            _bound[key] = run
+    return run(q, k, v)
 
 
 def binary(x, y, op, inplace=False, **cfg):
@@ -221,13 +233,10 @@ def binary(x, y, op, inplace=False, **cfg):
         hit = _binary_launch(x, y, op, inplace, cfg)
         if not cfg:
             _bound[key] = hit
-    run, shape = hit
     if inplace:
-        run(x.data_ptr(), y.data_ptr())
+        hit(x.data_ptr(), y.data_ptr())
         return x
-    z = torch.empty(shape, dtype=torch.bool if op in ("Equal", "Greater") else x.dtype, device=x.device)
-    run(x.data_ptr(), y.data_ptr(), z.data_ptr())
-    return z
+    return hit(x, y)
 
 
 def _binary_launch(x, y, op, inplace, cfg):
@@ -244,7 +253,7 @@ def _binary_launch(x, y, op, inplace, cfg):
 
     k = R.get_kernel("binary", OP=op, DIMS=",".join(map(str, shape)), SA=strides(x), SB=strides(y), INPLACE=int(inplace),
                      F16=int(x.dtype == torch.float16), **cfg)
-    return k.bind(), shape
+    return k.bind() if inplace else _into(k.bind(), tuple(shape), torch.bool if op in ("Equal", "Greater") else x.dtype)
 
 
 def gather(x, indices, axis=0, **cfg):
@@ -263,10 +272,7 @@ def gather(x, indices, axis=0, **cfg):
         hit = _gather_launch(x, indices, axis, cfg)
         if not cfg:
             _bound[key] = hit
-    run, shape = hit
-    out = torch.empty(shape, dtype=x.dtype, device=x.device)
-    run(x.data_ptr(), indices.data_ptr(), out.data_ptr())
-    return out
+    return hit(x, indices)
 
 
 def _gather_launch(x, indices, axis, cfg):
@@ -280,7 +286,7 @@ def _gather_launch(x, indices, axis, cfg):
     single = tuple(indices.shape) == (1,)
     shape = tuple(x.shape[:axis]) + (() if single else tuple(indices.shape)) + tuple(x.shape[axis + 1:])
     kern = R.get_kernel("gather", OUTER=outer, AXIS=x.shape[axis], NIDX=indices.numel(), INNER=inner, ESIZE=x.element_size(), **cfg)
-    return kern.bind(), shape
+    return _into(kern.bind(), shape, x.dtype)
 
 
 def softmax(x, inplace=False):
@@ -293,11 +299,10 @@ def softmax(x, inplace=False):
     run = _bound.get(key)
     if run is None:
         n = x.shape[-1]
-        run = _bind(key, None, R.get_kernel("softmax", ROWS=x.numel() // n, N=n, INPLACE=int(inplace), F16=_STORAGE[x.dtype]))
+        run = R.get_kernel("softmax", ROWS=x.numel() // n, N=n, INPLACE=int(inplace), F16=_STORAGE[x.dtype]).bind()
+        _bound[key] = run = run if inplace else _into(run)
     if inplace:
         run(x.data_ptr())
         return x
-    y = torch.empty_like(x)
-    run(x.data_ptr(), y.data_ptr())
-    return y
+    return run(x)
 

@@ -139,6 +139,23 @@ def _current_stream():
     return lambda: raw(device())
 
 
+_launch_type = None
+
+
+def _native_launch():
+    """The type of native bound launches (csrc/python/launch.cc), None where it has not been built."""
+    global _launch_type
+    if _launch_type is None:
+        import torch  # noqa: F401  (the extension's libraries)
+        try:
+            from . import _launch
+        except ModuleNotFoundError:
+            _launch_type = False
+        else:
+            _launch_type = _launch.Launch
+    return _launch_type or None
+
+
 class Kernel:
     def __init__(self, module, handle, info=None):
         self.module, self.handle, self.info = module, handle, info
@@ -195,11 +212,17 @@ class Kernel:
     def bind(self, scalars=0):
         """launch() on the current stream for a kernel without a workspace, as a function of the arguments' values: device
         pointers as integers, then `scalars` fp32 numbers.  Everything that is the same for all launches is prepared here:
-        the general launch() spends most of a small call on ctypes objects (an eight-call block 148 us, 41 this way)."""
+        the general launch() spends most of a small call on ctypes objects (an eight-call block 148 us, 41 this way).
+        Where the native launches are built, this is one of them, whose result() also allocates the output."""
         info = self.info
         if info["workspace_bytes"]:
             raise ValueError("the kernel takes a workspace")
         n = info["num_args"]
+        native = _native_launch() if isinstance(lib(), C.CDLL) else None
+        if native is not None:
+            return native(C.cast(lib().kcg_hip_launch_packed, C.c_void_p).value, self.handle.value,
+                          (*info["grid"], *info["block"], info["lds_bytes"]), n - scalars, scalars,
+                          lambda rc: check(rc, "kcg_hip_launch_packed"), self)
         pack = struct.Struct("<" + "Q" * (n - scalars) + "f4x" * scalars).pack
         dims = (C.c_uint32 * 7)(*info["grid"], *info["block"], info["lds_bytes"])
         address, handle, entry, stream = C.addressof(dims), self.handle, lib().kcg_hip_launch_packed, _current_stream()
