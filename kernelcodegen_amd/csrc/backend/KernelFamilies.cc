@@ -861,6 +861,30 @@ static const Gemm16Form* chooseGemm16Form(int64_t m, int64_t n, int64_t k, int64
   return best;
 }
 
+// Tiles with a side of 192: where 256 or 128 a side leave the last round of workgroups nearly empty, the sizes between them fill it.
+// The form of least modelled time among them if it is ahead of all the tiles above, else `form`.  Modelled as above, all forms
+// fitted anew to 1000 timings of 93 products of 128 to 4096 rows (10 to 16 % off each): of those the choice takes 28, 12 % faster on
+// average and 4 % slower at worst.  us, without and with: 1000 x 11008 x 4096 103 and 89, row-major 90 and 83; 400 x 11008 x 4096 69
+// and 51; 1500 x 11008 x 4096 172 and 148; 3000 x 5504 x 1536 72 and 55; 4096 x 11008 x 4096 stays, 298 against 338.
+static const Gemm16Form* chooseThirds(const Gemm16Form* form, int64_t m, int64_t n, int64_t k, int64_t batch) {
+  static const Gemm16Form forms[] = {
+      {256, 192, 4, 2, 2, 256, 68.6, 17.0}, {192, 256, 2, 4, 2, 256, 68.7, 18.5}, {128, 192, 4, 2, 2, 512, 46.9, 45.7},
+      {128, 192, 4, 2, 3, 256, 37.1, 12.4}, {192, 128, 2, 4, 2, 512, 49.4, 43.9}, {192, 128, 2, 4, 3, 256, 40.3, 9.3},
+      {256, 256, 4, 2, 2, 256, 81.5, 20.8}, {128, 128, 4, 2, 2, 512, 39.2, 27.0}, {128, 128, 4, 2, 3, 256, 26.8, 9.5},
+      {64, 128, 2, 2, 3, 512, 17.8, 25.8},  {64, 128, 2, 2, 4, 256, 21.6, 3.6}};
+  // (a moved-back k-tile among few: 3116 x 6032 x 528 39 and 45)
+  if (!form || form->bm < 64 || m < 128 || (k % 64 && k < 1024)) return form;
+  const Gemm16Form* best = nullptr;
+  double least = 0.0;
+  for (const auto& f : forms) {
+    if (m < f.bm || n < f.bn || (k % 64 && f.bm == 256)) continue;
+    const double tiles = (double)ceilDiv(m, f.bm) * (double)ceilDiv(n, f.bn) * (double)batch;
+    const double us = 2.5 + (double)k / 4096.0 * (std::ceil(tiles / f.slots) * f.a + tiles / f.slots * f.b);
+    if (!best || us < least) { best = &f; least = us; }
+  }
+  return best && (best->bm == 192 || best->bn == 192) ? best : form;
+}
+
 // Whether wavefronts that split k take less time than `tiled`, the form chosen above with `cost`: its time, fitted to the same
 // products as wavekTime (within 8 to 14 %), from that cost, or for 32-row tiles from their number.  us, this and that: bf16
 // k-contiguous 8 x 1024 x 4096 8.9 and 4.1, 16 x 2048 x 2048 5.6 and 3.3, 16 x 4096 x 4096 11.5 and 7.2, 64 x 1024 x 4096 12.8 and
@@ -898,6 +922,7 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
     WavekForm split;
     const int type = s.get("F16", 0) ? 2 : 1;
     if (!s.get("FP8_PAIRS", 0) && wavekAhead(s, type, form, cost, m, n, k, batch, split)) return emitGemmWavek(s, src, info, err, type, split, m, n, k, batch);
+    if (!s.get("FP8_PAIRS", 0)) form = chooseThirds(form, m, n, k, batch);
   }
   if (form) {
     s.p["BM"] = form->bm; s.p["BN"] = form->bn; s.p["WM"] = form->wm; s.p["WN"] = form->wn;
@@ -938,8 +963,9 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   // direct loads into LDS (global_load_lds_dwordx4, see the kernel): every wavefront moves a whole, even number of
   // 1 KiB blocks per operand tile; row-major weights need the 256-column tile and eight wavefronts
   const int64_t waves = wm * wn;
-  const bool d2lFits = m16Fits && (fewRows ? canShift : bm % (16 * waves) == 0) &&
-                       (s.get("TB", 0) ? bn % (16 * waves) == 0 : ((bn == 64 || bn == 128 || bn == 256) && (bn / 8) % waves == 0));
+  auto evenBlocks = [&](int64_t side) { return side % (16 * waves) == 0 || (side == 192 && waves == 8); };   // (192: three blocks each)
+  const bool d2lFits = m16Fits && (fewRows ? canShift : evenBlocks(bm)) &&
+                       (s.get("TB", 0) ? evenBlocks(bn) : ((bn == 64 || bn == 128 || bn == 192 || bn == 256) && (bn / 8) % waves == 0));
   // Default on the 256 x 256 tile with eight wavefronts, where it was measured: with direct loads 0.295-0.303 ms on
   // 4096 x 11008 x 4096 in either weight layout against 0.310-0.315 ms ([N][K]) and 0.338-0.346 ms ([K][N]) for the
   // 32x32x16 form; through registers 0.320-0.328 ms for [K][N] (also 4-8 % ahead on 4096^3, 8192^3 and
@@ -1006,7 +1032,8 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   if (d2l) d.add("GB_D2L", 1);
   if (m16 && s.has("M16_DEAL")) d.add("GB_M16_DEAL", s.get("M16_DEAL", 0) ? 1 : 0);
   // 16-bit results of whole 256 x 256 tiles in the 16x16x32 form leave through LDS as whole rows (see the kernel)
-  const bool stageOk = m16 && bm == 256 && bn == 256 && wm == 4 && wn == 2 && !edge && skUnits == 0 && n % 8 == 0;
+  const bool stageOk = m16 && (bm == 256 || bm == 192) && (bn == 256 || bn == 192) && wm * wn == 8 && bm / wm / 16 % 2 == 0 && (d2l || (bm == 256 && bn == 256 && wm == 4)) && !edge &&
+                       skUnits == 0 && n % 8 == 0;
   const int64_t stageC = stageOk ? std::max<int64_t>(0, std::min<int64_t>(2, s.get("STAGE_C", outBf16 ? 2 : 0))) : 0;
   s.p["STAGE_C"] = stageC;
   if (stageC) d.add("GB_STAGE_C", stageC);
@@ -1083,6 +1110,18 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     }
   }
   if (shift256) dm = dn = 256;
+  // Tiles of 192 columns where they make less of the last round idle: rounds and the part of them in use, in us at K = 4096, fitted to
+  // 81 products (us, 256 and 192 columns: 2000 x 11008 x 4096 99 and 89, 1500 x 11008 x 4096 94 and 77, 3000 x 11008 x 4096 147 and 129,
+  // 1500 x 4096 x 4096 row-major 53 and 41; but 4096 x 11008 x 4096 162 and 167, 2407 x 5440 x 2048 34 and 46): 23 of the 29 products
+  // on 256 x 256 tiles gain 11 % on average, none loses more than 2 %.
+  if (!own && dm == 256 && dn == 256 && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !ta && n % 16 == 0 && k % 128 == 0 && m >= 256 && s.get("SCALE_PTR", 0) == 0 &&
+      (shift256 || k <= 4096)) {
+    auto time = [&](int64_t cols, double a, double b) {
+      const double tiles = (double)ceilDiv(m, 256) * (double)ceilDiv(n, cols) * (double)batch / 256.0;
+      return 2.5 + (double)k / 4096.0 * (std::ceil(tiles) * a + tiles * b);
+    };
+    if (time(192, 41.3, 5.8) < time(256, 47.6, 11.1)) dn = 192;
+  }
   int64_t bm = s.get("BM", dm);
   int64_t bn = s.get("BN", dn);
   int64_t bk = s.get("BK", 128);
@@ -1098,8 +1137,11 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // the kernel); a single round is fastest without either.
   const bool legacyKnob = s.has("PREFETCH") || s.has("ROTATE") || s.has("PINGPONG") || s.has("STAGES") || (s.has("BTR") && !s.get("BTR", 1));
   const bool oneRound = ceilDiv(m, 256) * ceilDiv(n, 256) * batch <= 256;
-  if (s.get("D2L", !legacyKnob && (k <= 4096 || !oneRound || shift256)) && !ta && (tb || s.get("BTR", 1)) && n % 16 == 0 && bm == 256 && bn == 256 && bk == 128 && wm == 4 && wn == 2 &&
-      ((m % 256 == 0 && n % 256 == 0) || shift256) && k % 128 == 0) {
+  // (tiles of 192 columns, asked for or chosen above: moved back where they are ragged, so aligned operands are needed)
+  const bool thirds = bm == 256 && bn == 192 && bk == 128 && wm == 4 && wn == 2 && m >= 256 && n >= 192 && (m % 256 == 0 || s.get("ALIGN", 0) >= 16) && (n % 192 == 0 || s.get("ALIGN", 0) >= 16) &&
+                      shortRows(n, k) && s.get("PERSIST", 0) == 0 && s.get("STAGE_C", 1) != 0;
+  if (s.get("D2L", !legacyKnob && (k <= 4096 || !oneRound || shift256)) && !ta && (tb || s.get("BTR", 1)) && n % 16 == 0 && bm == 256 && (bn == 256 || thirds) && bk == 128 && wm == 4 && wn == 2 &&
+      (thirds || (m % 256 == 0 && n % 256 == 0) || shift256) && k % 128 == 0) {
     const int64_t scalePtr = s.get("SCALE_PTR", 0);
     if (scalePtr < 0 || scalePtr > 2) { err = "gemm_fp8: SCALE_PTR is 0 (scalar arguments), 1 (A, B, C, pointers) or 2 (A, B, pointers, C)"; return false; }
     const bool outBf16 = s.get("OUT_BF16", 0) != 0;
@@ -1108,7 +1150,7 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     // same columns of B at the same time (4096 x 11008 x 4096, two rows: 0.160 against 0.168 ms with strips of eight,
     // 0.164 with four); four rows otherwise (level with or ahead of eight on every shape measured).
     if (!s.has("GROUP_M")) {
-      const int64_t tm = ceilDiv(m, 256), tn = ceilDiv(n, 256), run = tm * tn / 8;
+      const int64_t tm = ceilDiv(m, 256), tn = ceilDiv(n, bn), run = tm * tn / 8;
       gm = (tm * tn) % 8 == 0 && run % tn == 0 && run / tn >= 1 && run / tn <= 4 ? run / tn : 4;
     }
     s.p["TA"] = 0; s.p["TB"] = tb; s.p["D2L"] = 1; s.p["BTR"] = !tb;
@@ -1121,8 +1163,9 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     d.add("G8_RELU", s.get("RELU", 0) ? 1 : 0);
     d.add("G8_SCALE_PTR", scalePtr);
     d.add("G8_BTR", tb ? 0 : 1);
-    const int64_t tilesAll = ceilDiv(m, 256) * ceilDiv(n, 256);
-    const bool moved = m % 256 || n % 256;
+    const int64_t tilesAll = ceilDiv(m, 256) * ceilDiv(n, bn);
+    const bool moved = m % 256 || n % bn;
+    if (bn != 256) d.add("G8_BN", bn);
     if (moved) d.add("G8_SHIFT", 1);
     const bool persist = s.get("PERSIST", 0) != 0 && !moved && batch == 1 && (k / 128) % 2 == 0 && tilesAll > 256;
     s.p["PERSIST"] = persist;
@@ -1478,7 +1521,8 @@ bool emitFmhaF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // instead of 40 at B1 H5 S1024 take 0.129 against 0.114 ms)
   const bool pair = s.get("PAIR", pairFits && (halved || (nq / 2) * b * h >= 512) ? 1 : 0) != 0;
   if (pair && !pairFits) { err = "fmha_f32: PAIR needs the causal mask and an even number of query tiles"; return false; }
-  if (!own) {
+  // (not where the direct loads are the default: with and without them the kernel gives the same bits, which a split would not)
+  if (!own && !d2l) {
     int64_t splitQb, splitWk;
     if (fmhaWavekAhead(s, 0, br, pair, (double)((pair ? nq / 2 : nq) * b * h), std::max<int64_t>(1, 4 * occ / (br / 32)), splitQb, splitWk))
       return emitFmhaWavek(s, src, info, err, 0, splitQb, splitWk);

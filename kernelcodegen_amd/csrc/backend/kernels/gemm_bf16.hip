@@ -25,6 +25,7 @@
 //                                (gemm_fp8_d2l.hip), where the loads and not the MFMAs set the pace
 //   GB_OUT_BF16                  1: C has the operands' 16-bit type, else fp32
 //   GB_RELU                      1: fused max(0, .) epilogue
+//                                (tiles of 192 rows or columns: eight wavefronts, direct loads)
 //   GB_STAGE_C                   1: results are turned round in LDS and stored as whole rows of the tile (see the
 //                                epilogue); 2: with the non-temporal hint
 //   GB_SK_UNITS                  0: one workgroup per tile.  > 0: the tiles that do not fill a whole round of
@@ -372,8 +373,8 @@ typedef _Float16 kcg_f16x8 __attribute__((ext_vector_type(8)));
 #if (GB_BM % (32 * GB_WM)) || (GB_BN % (GB_FR * GB_WN)) || (GB_BK % 16)
 #error "tile shape does not divide into 32x32x16 MFMA tiles"
 #endif
-#if GB_D2L && (!GB_M16 || (GB_BTR && GB_BN != 256 && GB_BN != 128 && GB_BN != 64))
-#error "direct loads into LDS: only with the 16x16x32 form; row-major weights need tiles of 64, 128 or 256 columns"
+#if GB_D2L && (!GB_M16 || (GB_BTR && GB_BN != 256 && GB_BN != 192 && GB_BN != 128 && GB_BN != 64))
+#error "direct loads into LDS: only with the 16x16x32 form; row-major weights need tiles of 64, 128, 192 or 256 columns"
 #endif
 #if GB_NBUF != 2 && !GB_D2L
 #error "more than two LDS buffers: only with direct loads"
@@ -391,8 +392,8 @@ typedef _Float16 kcg_f16x8 __attribute__((ext_vector_type(8)));
 #error "tail split: needs an even number of whole k-tiles per tile and per unit, and one staging set"
 #endif
 
-#if GB_STAGE_C && (!GB_M16 || GB_BM != 256 || GB_BN != 256 || GB_WM != 4 || GB_WN != 2 || GB_EDGE || GB_SK_UNITS > 0)
-#error "gemm_bf16: results go through LDS (GB_STAGE_C) only from whole 256 x 256 tiles of the 16x16x32 form, 4 x 2 wavefronts"
+#if GB_STAGE_C && (!GB_M16 || (GB_BM != 256 && GB_BM != 192) || (GB_BN != 256 && GB_BN != 192) || GB_WM * GB_WN != 8 || GB_TM % 2 || GB_EDGE || GB_SK_UNITS > 0)
+#error "gemm_bf16: results go through LDS (GB_STAGE_C) only from whole tiles of 192 or 256 a side of the 16x16x32 form, eight wavefronts"
 #endif
 extern "C" __global__ __launch_bounds__(GB_NT)
 void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
@@ -552,10 +553,13 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
   // 64 rows of each operand, so half the rows that are not there are not loaded (8 x 1024 x 4096: 11.6 us with 64 rows, 9.2
   // with 32; 16 rows, which leave half the wavefronts without a load of their own, 9.9).
   constexpr int UA = GB_BM / 8 / (GB_NT / 64);                                     // instructions per wavefront and tile
-  constexpr int RB = 1024 / (GB_BN * 2) > 0 ? 1024 / (GB_BN * 2) : 1;              // k rows of row-major weights per instruction
-  constexpr int UB = GB_BTR ? GB_BK / RB / (GB_NT / 64) : GB_BN / 8 / (GB_NT / 64);
-  static_assert((GB_CLAMP || UA % 2 == 0) && UA > 0 && GB_BM % (8 * (GB_NT / 64)) == 0, "direct loads: whole, even numbers of 8-row groups per wavefront");
-  static_assert(GB_BTR ? UB * RB * (GB_NT / 64) == GB_BK && UB >= 1 : (UB % 2 == 0 && GB_BN % (8 * (GB_NT / 64)) == 0), "direct loads of B: whole blocks per wavefront");
+  // k rows of row-major weights per instruction (192 columns: eight rows in three instructions, a wavefront's share of a tile)
+  constexpr bool THIRDS = GB_BN == 192;
+  constexpr int RB = 1024 / (GB_BN * 2) > 0 ? 1024 / (GB_BN * 2) : 1;
+  constexpr int UB = !GB_BTR ? GB_BN / 8 / (GB_NT / 64) : THIRDS ? 3 : GB_BK / RB / (GB_NT / 64);
+  static_assert((GB_CLAMP || UA % 2 == 0 || GB_BM == 192) && UA > 0 && GB_BM % (8 * (GB_NT / 64)) == 0, "direct loads: whole numbers of 8-row groups per wavefront");
+  static_assert(GB_BTR ? (THIRDS ? GB_NT == 512 && GB_BK == 64 : UB * RB * (GB_NT / 64) == GB_BK && UB >= 1)
+                       : ((UB % 2 == 0 || GB_BN == 192) && GB_BN % (8 * (GB_NT / 64)) == 0), "direct loads of B: whole blocks per wavefront");
   // The instruction is written out: through the builtin the compiler, which cannot tell that the transposing reads
   // that follow touch the other buffer, puts a wait for all outstanding loads in front of each of them.  Here it sees
   // neither the LDS write nor the counter; the waits are the explicit ones in front of the barriers.  The address is a
@@ -580,38 +584,43 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
     lds_dma((const char*)(As + k0), d2l_lane_a[t], sbuf + (wave_u * UA + t) * 8 * GB_ROWB);
   };
 #endif
-  auto d2l = [&](const kcg_u16* g, int row0, int k0, char* sbuf, int t, int upw) __attribute__((always_inline)) {
-    const int grp = wave_u * upw + t;                      // group of eight rows within the tile; its parity is that of t
-    lds_dma((const char*)(g + (long)(row0 + grp * 8) * GB_K + k0), (t & 1) ? d2l_lane1 : d2l_lane, sbuf + grp * 8 * GB_ROWB);
+  // group of eight rows within the tile: its parity is that of t, with an odd number of them per wavefront that of wave + t
+  const unsigned d2l_swap0 = (wave_u & 1) ? d2l_lane1 : d2l_lane, d2l_swap1 = (wave_u & 1) ? d2l_lane : d2l_lane1;
+  auto d2l = [&](const kcg_u16* g, int row0, int k0, char* sbuf, int t, auto upw_c) __attribute__((always_inline)) {
+    constexpr int upw = decltype(upw_c)::v;
+    const int grp = wave_u * upw + t;
+    const unsigned at = upw % 2 ? ((t & 1) ? d2l_swap1 : d2l_swap0) : (t & 1) ? d2l_lane1 : d2l_lane;
+    lds_dma((const char*)(g + (long)(row0 + grp * 8) * GB_K + k0), at, sbuf + grp * 8 * GB_ROWB);
   };
 #if GB_BTR
   // Row-major weights: a tile row is 2 * GB_BN bytes of consecutive n, one instruction moves RB = 2, 4 or 8 k rows.  Rows
   // are not padded; the 32-byte granule g of row k lies at granule g ^ f(k): the eight k rows that the transposing reads of
-  // two lane groups take together (k0 .. k0 + 3 and k0 + 8 .. k0 + 11) then fall on disjoint banks.  Rows of 256 bytes and
-  // more start on the same bank: f(k) = k % 4 + 4 ((k / 8) % 2); of rows of 128 bytes every other one does, and they have
-  // four granules: f(k) = (k / 2) % 2 + 2 ((k / 8) % 2).  Block b = UB wave + t holds rows RB b .. RB b + RB - 1.
+  // two lane groups take together (k0 .. k0 + 3 and k0 + 8 .. k0 + 11) then fall on disjoint banks.  Rows of 256 and 512
+  // bytes start on the same bank: f(k) = k % 4 + 4 ((k / 8) % 2); of rows of 128 and 384 bytes every other one does, and their
+  // granules come in fours: f(k) = (k / 2) % 2 + 2 ((k / 8) % 2).  Block b = UB wave + t holds rows RB b .. RB b + RB - 1.
   unsigned d2l_lane_b[UB];
 #pragma unroll
   for (int t = 0; t < UB; ++t) {
-    const int r = lane / (64 / RB), c = lane % (64 / RB), kr = (wave * UB + t) * RB + r;
-    const int f = GB_BN >= 128 ? (kr & 3) + 4 * ((kr >> 3) & 1) : ((kr >> 1) & 1) + 2 * ((kr >> 3) & 1);
+    const int r = THIRDS ? (t * 64 + lane) / 24 : lane / (64 / RB), c = THIRDS ? (t * 64 + lane) % 24 : lane % (64 / RB);
+    const int kr = THIRDS ? wave * 8 + r : (wave * UB + t) * RB + r;
+    const int f = GB_BN % 128 == 0 ? (kr & 3) + 4 * ((kr >> 3) & 1) : ((kr >> 1) & 1) + 2 * ((kr >> 3) & 1);
     d2l_lane_b[t] = (unsigned)r * (unsigned)(GB_N * 2) + (unsigned)((((c >> 1) ^ f) << 1) | (c & 1)) * 16u;
   }
   auto d2l_b = [&](int k0, char* sbuf, int t) __attribute__((always_inline)) {
     const int blk = wave_u * UB + t;
-    lds_dma((const char*)(Bs + (long)(k0 + blk * RB) * GB_N + n0), d2l_lane_b[t], sbuf + blk * 1024);
+    lds_dma((const char*)(Bs + (long)(k0 + (THIRDS ? wave_u * 8 : blk * RB)) * GB_N + n0), d2l_lane_b[t], sbuf + blk * 1024);
   };
 #endif
   auto d2l_unit = [&](int u, int k0, int buf) __attribute__((always_inline)) {
 #if GB_CLAMP
     if (u < UA) d2l_a(GB_KPOS(k0), sA + buf * (GB_BM * GB_ROWB), u);
 #else
-    if (u < UA) d2l(As, m0, GB_KPOS(k0), sA + buf * (GB_BM * GB_ROWB), u, UA);
+    if (u < UA) d2l(As, m0, GB_KPOS(k0), sA + buf * (GB_BM * GB_ROWB), u, KcgInt<UA>{});
 #endif
 #if GB_BTR
     else d2l_b(GB_KPOS(k0), sB + buf * GB_BBUF, u - UA);
 #else
-    else d2l(Bs, n0, GB_KPOS(k0), sB + buf * GB_BBUF, u - UA, UB);
+    else d2l(Bs, n0, GB_KPOS(k0), sB + buf * GB_BBUF, u - UA, KcgInt<UB>{});
 #endif
   };
 #if GB_KTAIL
@@ -628,7 +637,7 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
     zero_rows(sA + buf * (GB_BM * GB_ROWB), UA);
 #if GB_BTR
     for (int t = 0; t < UB; ++t)
-      if ((wave_u * UB + t) * RB + lane / (64 / RB) < KZ) *(kcg_u32x4*)(sB + buf * GB_BBUF + (wave_u * UB + t) * 1024 + lane * 16) = zero;
+      if ((THIRDS ? wave_u * 8 + (t * 64 + lane) / 24 : (wave_u * UB + t) * RB + lane / (64 / RB)) < KZ) *(kcg_u32x4*)(sB + buf * GB_BBUF + (wave_u * UB + t) * 1024 + lane * 16) = zero;
 #else
     zero_rows(sB + buf * GB_BBUF, UB);
 #endif
@@ -711,7 +720,7 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #if GB_D2L
   // natural k order (group q holds k 8 q .. 8 q + 7), unpadded rows with swizzled 32-byte granules (see d2l_b)
   const kcg_lds_ptr bT = (kcg_lds_ptr)sB + (8 * (lane >> 4) + (lane & 15) / 4) * GB_BROWB + 8 * (lane & 3);
-  const int bswz = GB_BN >= 128 ? ((lane & 15) >> 2) + 4 * ((lane >> 4) & 1) : ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1);
+  const int bswz = GB_BN % 128 == 0 ? ((lane & 15) >> 2) + 4 * ((lane >> 4) & 1) : ((lane >> 3) & 1) + 2 * ((lane >> 4) & 1);
   int boff[GB_TN];
 #pragma unroll
   for (int j = 0; j < GB_TN; ++j) boff[j] = ((wn * GB_WTN / 16 + j) ^ bswz) * 32;
@@ -1022,9 +1031,9 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #if GB_STAGE_C
   // Whole rows.  Out of the 16 x 16 accumulator tiles a store instruction writes 16 values of each of four rows (64
   // bytes in fp32, 32 in a 16-bit type: two bytes a lane), and the pieces of a 128-byte line leave at different times.
-  // Here the 256 x 256 tile goes through LDS, the k loop's 128 KiB: in two halves of 128 rows as fp32 (the wavefront's
+  // Here the tile (256 x 256, or 192 a side) goes through LDS, the k loop's 128 KiB: in two halves of 128 rows as fp32 (the wavefront's
   // tile rows 0-1, then 2-3: every wavefront takes part in both), at once in a 16-bit type.  Row r of the staged part is
-  // 256 values, its chunk c of 16 values at chunk c ^ ((r / 4) % 4), so that the four rows a wavefront writes at a time
+  // GB_BN values, its chunk c of 16 values at chunk c ^ ((r / 4) % 4), so that the four rows a wavefront writes at a time
   // fall on different banks; then every lane stores 16 bytes of a row, a wavefront one or two whole rows at a time
   // (GB_STAGE_C 2: with the non-temporal hint).  16-bit results gain 2-3 % (4096 x 11008 x 4096: 0.280 against 0.287 ms);
   // fp32 results, whose pieces are 64 bytes already, gain nothing in this kernel and keep the plain epilogue.
@@ -1034,8 +1043,9 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
 #else
     typedef float stage_t;
 #endif
-    constexpr int ES = (int)sizeof(stage_t), PASSES = ES == 4 ? 2 : 1, RP = 256 / PASSES;    // rows per pass
-    constexpr int LPR = 256 * ES / 16, RPI = 64 / LPR, EPL = 16 / ES;                        // lanes per row, rows per instruction, values per lane
+    constexpr int ES = (int)sizeof(stage_t), PASSES = ES == 4 ? 2 : 1, RP = GB_BM / PASSES;  // rows per pass
+    constexpr int LPR = GB_BN * ES / 16, EPL = 16 / ES;                                      // lanes per row, values per lane
+    static_assert(RP * LPR % GB_NT == 0, "whole turns of the workgroup");
     stage_t* stage = (stage_t*)kcg_smem;
     const int lq = lane >> 4, l16 = lane & 15;
 #pragma unroll
@@ -1051,17 +1061,19 @@ void GB_NAME(const kcg_u16* __restrict__ A, const kcg_u16* __restrict__ B,
             const float r = GB_RELU ? fmaxf(GB_SCALED(acc[i][j][v]), 0.0f) : GB_SCALED(acc[i][j][v]);
             const int row = wm * (GB_WTM / PASSES) + 16 * ii + 4 * lq + v, col = wn * GB_WTN + 16 * j + l16;
 #if GB_OUT_BF16
-            stage[row * 256 + (col ^ (16 * lq))] = GB_TO16(r);
+            stage[row * GB_BN + (col ^ (16 * lq))] = GB_TO16(r);
 #else
-            stage[row * 256 + (col ^ (16 * lq))] = r;
+            stage[row * GB_BN + (col ^ (16 * lq))] = r;
 #endif
           }
       __syncthreads();
 #pragma unroll
-      for (int x = 0; x < RP / 8 / RPI; ++x) {
-        const int row = wave * (RP / 8) + x * RPI + lane / LPR;
-        const int col = (lane % LPR) * EPL;
-        const kcg_f32x4 val = *(const kcg_f32x4*)(stage + row * 256 + (col ^ (16 * ((row >> 2) & 3))));
+      for (int x = 0; x < RP * LPR / GB_NT; ++x) {
+        // a wavefront's rows one after the other (192 columns: its run of chunks, rows end inside an instruction)
+        const int chunk = wave * (RP * LPR / (GB_NT / 64)) + x * 64 + lane;
+        const int row = chunk / LPR;
+        const int col = (chunk % LPR) * EPL;
+        const kcg_f32x4 val = *(const kcg_f32x4*)(stage + row * GB_BN + (col ^ (16 * ((row >> 2) & 3))));
         const int trow = PASSES == 2 ? (row / (GB_WTM / 2)) * GB_WTM + (GB_WTM / 2) * pass + row % (GB_WTM / 2) : row;
 #if GB_SHIFT
         if (m0 + trow < m_own || n0 + col < n_own) continue;         // stored by the tile before (whole chunks: N % 8 == 0)
