@@ -620,7 +620,8 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
       const double area = (double)(tile * tile) / 4096.0, used = std::max(0.3, groups / 256.0), sparse = tile == 64 ? std::max(0.0, 1.0 - groups / 512.0) : 0.0;
       const double tiled = s.get("TB", 0) ? 2.95 + 0.01 * k * (area * (1.044 * rounds + 0.681 * used) * (direct ? 1.0 : 1.33) + 0.68 * sparse)
                                           : 3.07 + 0.01 * k * (area * (1.454 * rounds + 0.239 * used) * (direct ? 1.0 : 1.26) + 0.32 * sparse);
-      if (us < 0.9 * tiled) return emitGemmWavek(s, src, info, err, 0, form, m, n, k, batch);
+      // (k-contiguous B on whole k-tiles of 32 is faster than modelled: 3 x 532 x 388 x 1184 22.2 us, split 23.6)
+      if (us < (s.get("TB", 0) && direct && k % 32 == 0 ? 0.8 : 0.88) * tiled) return emitGemmWavek(s, src, info, err, 0, form, m, n, k, batch);
     }
   }
   int64_t bm = s.get("BM", tile), bn = s.get("BN", tile);
