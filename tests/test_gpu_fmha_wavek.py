@@ -2,7 +2,8 @@
 tiles, query blocks and the wavefronts do not divide, one tile, wavefronts without a tile, both masks, every operand type.
 
 The reference is fp64.  Tolerances, relative in the 2-norm: fp32 4e-6, a sum of up to 300 fp32 products with the hardware's exp2
-(2e-7 each); 16 bits: half a unit in the last place of the probabilities and of the result, 2^-9 (bf16) or 2^-12 (half) each, times 2."""
+(2e-7 each); 16 bits: half a unit in the last place of the probabilities and of the result, at most 2^-8 of a value (bf16)
+or 2^-11 (half): both together 7.8e-3 and 9.8e-4."""
 import pytest
 import torch
 
