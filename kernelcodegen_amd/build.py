@@ -63,10 +63,10 @@ def _stamp():
 
 
 def build_launch(force=False, verbose=False):
-    """The bound launches of the Python operators (csrc/python/launch.cc), an extension module on torch's own libraries."""
+    """The bound launches of the Python operators (launch.cc), an extension module on torch's own libraries."""
     import sysconfig
     import torch
-    src = os.path.join(CSRC, "python", "launch.cc")
+    src = os.path.join(os.path.dirname(CSRC), "launch.cc")
     base = os.path.join(os.path.dirname(torch.__file__))
     inc = os.path.join(base, "include")
     cmd = [CXX, "-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",

@@ -1,4 +1,4 @@
-"""The native bound launches (csrc/python/launch.cc): what they refuse without a GPU, and what they pass on and return with one."""
+"""The native bound launches (launch.cc): what they refuse without a GPU, and what they pass on and return with one."""
 import ctypes as C
 
 import pytest
