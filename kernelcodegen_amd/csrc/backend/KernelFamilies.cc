@@ -69,28 +69,49 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
     err = "layernorm: scale/bias length must divide the normalised length";
     return false;
   }
-  // 16 bytes per access where all lengths divide into them (16-bit types fall back to fours), and on large launches of any
-  // row length, scale and bias then being of that length.  Small odd launches keep single elements: the row's end, element by
-  // element, is a second trip to memory there (bf16 100 x 1001: 3.5 us, 4.9 in fours), and so do short rows, where most of a
-  // wavefront would idle, and in 16 bits lengths that leave most lanes' second eight empty (4096 to 6144, on launches of over 8 M
-  // elements), 2048 to 4096 while every row has a workgroup to itself (512), and those where the eights take too many registers
-  // (beyond 8192; fp32 in fours stays ahead to the 32 elements a lane holds): bf16 us, eights and single elements, 2000 x 5555 21.8
-  // and 18.2, 500 x 2503 6.0 and 4.5, 2100 x 16381 53 and 42, but 520 x 3001 5.1 and 5.9, 1000 x 8191 9.8 and 12.8.
-  // 16-bit rows that fours divide and eights do not go in fours, aligned as they are, while those leave a lane half a vector free
-  // (7168), on up to 4096 elements by 1024 workgroups (eights with a ragged end and fours: 300 x 3892 5.8 and 4.3, 16384 x 3892 85
-  // and 66, 4000 x 5004 35 and 27, 2000 x 7004 23 and 18; 1000 x 8188 9.2 and 11.5).
   const bool f16 = s.get("F16", 0) != 0;
   const double elements = (double)rows * (double)n;
   auto divides = [&](int64_t w) { return n % w == 0 && ng % w == 0 && nb % w == 0; };
-  const bool anyLength = ng == n && nb == n && n >= 256 && n <= (f16 ? 8192 : 1024 * 32) && elements >= 1048576.0 &&
-                         !(f16 && ((n > 4096 && n <= 6144 && elements > 8388608.0) || (n > 2048 && n <= 4096 && rows <= 512)));
+  // Rows of 512 to 8192 elements, for callers who ask for it (FILL = 2) and on more than 1024 rows: 16 bytes per access whatever the
+  // length, and the fewest lanes that hold a row in `most` vectors each, since a lane past the row's end idles as long as the others
+  // work (bf16, 640 vectors a row: 128 lanes of five against 512 of which 320 take two).  Up to 256 rows the launch is one row's chain,
+  // which more lanes shorten; up to 2048 the part is not full yet.  Scale and bias are then read again by every row (they come out of
+  // the caches) and rows have a workgroup each, without a next row under way: more wavefronts fit a CU that way than the held
+  // values' registers leave.  Where rows fill the registers all the same, and in fp32, large launches stay with 512 workgroups that
+  // hold and prefetch.  us, before and now, bf16: 16384 x 5120 89 and 58, 4000 x 2560 12.7 and 6.6, 1100 x 6144 10.4 and 5.1, 100 x 1280
+  // 3.15 and 2.43, 16384 x 4096 49.7 and 45.8, odd lengths 16384 x 1001 31.7 and 14.2, 4000 x 2503 21.8 and 8.5, 16384 x 7777 138 and 106;
+  // fp32 16384 x 1280 34.7 and 28.6, 1100 x 4096 8.4 and 6.3, 16384 x 3333 81 and 74.  Held and prefetched, and neither: bf16 16384 x 8192
+  // 86 and 95, 4000 x 7777 28.8 and 30.4, but 4000 x 7168 24.1 and 22.9; fp32 4000 x 2560 15.8 and 16.9, but 4000 x 1280 7.5 and 6.7,
+  // 16384 x 640 17.0 and 15.7 (but 9208 x 948 13.0 and 14.9).
   const int64_t wide = f16 ? 8 : 4;
+  bool tuned = (s.get("FILL", 0) >= 2 || rows > 1024) && n >= 512 && n <= 8192 && ((ng == n && nb == n) || divides(wide));
+  for (const char* key : {"VW", "TPR", "RPB", "GRID", "LEAN", "ONEPASS"}) tuned = tuned && !s.has(key);
+  if (tuned) {
+    const bool hold = rows <= 256 || (f16 ? n > 6144 && elements > 24e6 : n > 768 && elements > (n <= 1024 ? 6e6 : 8e6));
+    // (fp32: a wavefront by itself up to 1024, 1 x 576 2.03 us and 2.11; held rows beyond 4096 on 512 lanes, 16384 x 5120 111 and 114)
+    const int64_t most = f16 ? (rows <= 256 ? 1 : rows <= 2048 ? 3 : 6) : rows > 256 ? 5 : n > 1024 ? 1 : 4;
+    int64_t lanes = 64;
+    while (lanes * most * wide < n && lanes < 256) lanes *= 2;
+    if (lanes * 6 * wide < n || (!f16 && rows > 256 && hold && n > 4096)) lanes = 512;
+    s.p["VW"] = wide; s.p["TPR"] = lanes;
+    s.p["LEAN"] = !hold;
+    s.p["GRID"] = hold && rows > 256 ? (n <= 1024 ? 768 : 512) : rows;       // (fp32 16384 x 832 19.5 us and 21.0, 9208 x 948 13.0 and 13.6)
+  }
+  // Else 16 bytes per access where all lengths divide into them (16-bit types fall back to fours), and on launches of at least a
+  // million elements of any row length, scale and bias then being of that length; smaller odd launches and short rows, where most of
+  // a wavefront would idle, keep single elements, and so do 16-bit rows of 2048 to 4096 while every row has a workgroup to itself
+  // (512), and those where the eights take too many registers (beyond 8192; fp32 in fours stays ahead to the 32 elements a lane holds):
+  // bf16 us, eights and single elements, 2100 x 16381 53 and 42, but 1000 x 8191 9.8 and 12.8.
+  // 16-bit rows that fours divide and eights do not go in fours, aligned as they are, while those leave a lane half a vector free
+  // (7168), on up to 4096 elements by 1024 workgroups.
+  const bool anyLength = ng == n && nb == n && n >= 256 && n <= (f16 ? 8192 : 1024 * 32) && elements >= 1048576.0 &&
+                         !(f16 && n > 2048 && n <= 4096 && rows <= 512);
   // (a wavefront that fours fill and eights do not, 768 elements: fours on small launches, 300 x 768 3.2 us and 3.0)
   const bool unfilled = f16 && n < 1024 && n % 256 == 0 && n % 512 != 0 && elements <= 2097152.0;
   const bool fours = divides(4) && f16 && n >= 1024 && n <= 7168;
   int64_t vw = s.get("VW", divides(wide) && n >= 512 && !unfilled ? wide : anyLength && !fours ? (n >= 1024 ? wide : 4) : divides(4) ? 4 : 1);
   if (vw != 1 && vw != 4 && vw != 8) { err = "layernorm: VW must be 1, 4 or 8"; return false; }
-  if (vw > 1 && s.has("VW") && !divides(vw)) { err = "layernorm: VW=" + std::to_string(vw) + " needs lengths divisible by " + std::to_string(vw); return false; }
+  if (vw > 1 && s.has("VW") && !tuned && !divides(vw)) { err = "layernorm: VW=" + std::to_string(vw) + " needs lengths divisible by " + std::to_string(vw); return false; }
   int64_t tpr = s.get("TPR", 0);
   if (rows > 0xFFFFFFFFLL) { err = "layernorm: too many rows"; return false; }
   if (tpr == 0) {

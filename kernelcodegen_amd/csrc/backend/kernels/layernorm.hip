@@ -16,29 +16,29 @@
 // the reference nest's formulation (centre first, biased variance of the
 // centred values, scale by 1/sqrt(var + eps)); only the summation order differs.
 //
-// The grid is persistent: LN_GRID workgroups walk the row groups with stride
-// LN_GRID.  A lane always owns the same columns, so gamma and beta are loaded
-// once, and the loads of the next row group are issued before the current one
-// is reduced: the reductions and the stores run under memory latency instead
-// of adding to it.
+// LN_GRID workgroups walk the row groups with stride LN_GRID.  A lane always owns the same columns, so gamma and beta are loaded
+// once, and where there is a next row group its loads are issued before the current one is reduced: the reductions and the
+// stores run under memory latency instead of adding to it.  What is held for later (gamma, beta, the next row) stays in the type
+// it has in memory, half the registers in 16 bits.
 //   LN_GRID      number of workgroups
 //   LN_STREAM    1: the rows are read with the non-temporal hint (they are read once); 0: plain loads
 //                (a row length that LN_VW does not divide is taken too, with gamma and beta of the whole length: rows then
-//                start anywhere, the accesses ask for element alignment only, and the lane that holds the row's end goes
-//                element by element; fp32, 12000 x 2047: 52 us one element at a time, 37 us this way)
-//   LN_LEAN      1: rows too long to hold gamma, beta and a second row in
-//                registers: re-read gamma/beta per row and do not prefetch
+//                start anywhere, the accesses ask for element alignment only, and the row's last vector is moved back to its
+//                end: two lanes then hold some values, which count once and are stored twice, alike.  No lane goes element
+//                by element.  us, fp32 12000 x 2047: 52 one element at a time, 37 with
+//                the end element by element; bf16 4000 x 7777 37.8 that way, 28.8 this way, both with 512 workgroups; fp32 16384 x 3333
+//                81 and 74)
+//   LN_LEAN      1: gamma and beta are read again for every row and there is no prefetch: rows too long to hold them, and
+//                those where the wavefronts that the registers then leave room for hide more (bf16 1100 x 6144: 5.1 us, holding
+//                them 6.8, and the next row 8.0)
 //   LN_ONEPASS   1: mean and centred sum of squares from ONE reduction: every lane forms the mean and the sum of
 //                squared deviations of its own values, and lanes (then wavefronts) merge their (mean, M2) pairs
 //                pairwise, M2 = M2a + M2b + (mean_b - mean_a)^2 n / 2 for two parts of n values each (Chan, Golub,
 //                LeVeque) -- the same centred, biased variance, one exchange through LDS and one barrier per row
 //                instead of two.  Needs every lane to hold the same number of values (LN_N a multiple of
 //                LN_TPR * LN_VW); the emitter asks for it only then.
-#ifndef KCG_LN_HELPERS
-#define KCG_LN_HELPERS
-template <bool B> struct KcgLnOnce { static constexpr bool v = B; };      // read once: with the non-temporal hint
-#endif
 #define LN_GROUPS ((LN_ROWS + LN_RPB - 1) / LN_RPB)
+#define LN_WALKS (LN_GRID < LN_GROUPS)
 #ifndef LN_F16
 #define LN_F16 0
 #define LN_F16_DEFAULTED
@@ -65,16 +65,6 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
     for (int j = 0; j < LN_VW; ++j) r[j] = (float)x[j];
     return r;
   };
-#if LN_N % LN_VW
-  // elements idx .. of p, LN_N in all; zeros behind its end
-  auto load_any = [&](const LN_IO* __restrict__ p, int idx, auto once) __attribute__((always_inline)) -> vec_t {
-    vec_t r;
-    if (idx + LN_VW <= LN_N) return widen(kcg_stream_load<decltype(once)::v>((const io_vec_t*)(p + idx)));
-#pragma unroll
-    for (int j = 0; j < LN_VW; ++j) r[j] = idx + j < LN_N ? (float)p[idx + j] : 0.0f;
-    return r;
-  };
-#endif
   const int tid = threadIdx.x;
   const int tr = tid % LN_TPR;               // position inside the row team
   const int rb = tid / LN_TPR;               // row inside the block
@@ -92,58 +82,60 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
   const int wv = tr / KCG_WAVE;
 #endif
 
-#if !LN_LEAN
-  vec_t g[LN_VPT], b[LN_VPT];
-#pragma unroll
-  for (int i = 0; i < LN_VPT; ++i) {
-    const int idx = (i * LN_TPR + tr) * LN_VW;
-#if LN_N % LN_VW
-    g[i] = load_any(G, idx, KcgLnOnce<false>{});
-    b[i] = load_any(Bt, idx, KcgLnOnce<false>{});
-#else
-    if (idx < LN_N) {
-      g[i] = widen(*(const io_vec_t*)(G + (idx % LN_NG)));
-      b[i] = widen(*(const io_vec_t*)(Bt + (idx % LN_NB)));
-    } else {
-#pragma unroll
-      for (int j = 0; j < LN_VW; ++j) { g[i][j] = 0.0f; b[i][j] = 0.0f; }
-    }
-#endif
-  }
-#endif
+  // a lane's i-th vector: where it would begin, where it does, and which of its values are the lane's own.  `apart` is 0 in a way that
+  // the compiler takes to differ between lanes: where no lane's i-th vector is whole (2049 elements on 256 lanes of eights) it would
+  // otherwise load that one address into scalar registers, and a scalar load ignores the two lowest bits of an address.
+  int apart = 0;
+  asm("" : "+v"(apart));
+  auto begin = [&](int i) __attribute__((always_inline)) { return (i * LN_TPR + tr) * LN_VW; };
+  auto column = [&](int i) __attribute__((always_inline)) {
+    return (i + 1) * LN_TPR * LN_VW <= LN_N || begin(i) + LN_VW <= LN_N ? begin(i) : LN_N - LN_VW + apart;
+  };
+  auto place = [&](int i) __attribute__((always_inline)) { return LN_N % LN_VW == 0 ? begin(i) : column(i); };      // where begin(i) < LN_N
+  auto counts = [&](int i, int j) __attribute__((always_inline)) {
+    return (i + 1) * LN_TPR * LN_VW <= LN_N || (begin(i) < LN_N && (LN_N % LN_VW == 0 || column(i) + j >= begin(i)));
+  };
 
-  auto load_row = [&](long row, vec_t (&dst)[LN_VPT]) {
+  // Workgroups that walk the rows load each vector behind a branch of its own, which waits for the row before the next one is
+  // reduced; without the branches a row's loads stay in flight over the reductions of the one before, and the time goes up (fp32
+  // 16384 x 8192 180 us and 190, 16384 x 4096 87.2 and 88.5): the memory is faster with fewer requests at a time.
+  auto load_row = [&](long row, io_vec_t (&dst)[LN_VPT]) __attribute__((always_inline)) {
     const bool live = row < LN_ROWS;
     const LN_IO* __restrict__ x = X + (live ? row : 0) * (long)LN_N;
 #pragma unroll
-    for (int i = 0; i < LN_VPT; ++i) {
-      const int idx = (i * LN_TPR + tr) * LN_VW;
-      if (live && idx < LN_N) {
-#if LN_N % LN_VW
-        dst[i] = load_any(x, idx, KcgLnOnce<LN_STREAM != 0>{});
-#else
-        dst[i] = widen(kcg_stream_load<LN_STREAM != 0>((const io_vec_t*)(x + idx)));   // read once: 3-4 % faster from HBM with the hint, 10 % slower when the input is still in the last-level cache
-#endif
-      } else {
+    for (int i = 0; i < LN_VPT; ++i)
+      if (LN_WALKS && !(live && begin(i) < LN_N)) {
 #pragma unroll
-        for (int j = 0; j < LN_VW; ++j) dst[i][j] = 0.0f;
+        for (int j = 0; j < LN_VW; ++j) dst[i][j] = (LN_IO)0.0f;
+      } else {
+        dst[i] = kcg_stream_load<LN_STREAM != 0>((const io_vec_t*)(x + (LN_WALKS ? place(i) : column(i))));   // read once: 3-4 % faster from HBM with the hint, 10 % slower when the input is still in the last-level cache
       }
-    }
   };
 
-  vec_t v[LN_VPT];
 #if !LN_LEAN
-  vec_t vn[LN_VPT];
-  load_row((long)blockIdx.x * LN_RPB + rb, v);
+  io_vec_t g[LN_VPT], b[LN_VPT];
+#pragma unroll
+  for (int i = 0; i < LN_VPT; ++i) {
+    g[i] = *(const io_vec_t*)(G + (column(i) % LN_NG));
+    b[i] = *(const io_vec_t*)(Bt + (column(i) % LN_NB));
+  }
+#endif
+  io_vec_t in[LN_VPT];
+#if !LN_LEAN
+  load_row((long)blockIdx.x * LN_RPB + rb, in);
 #endif
   for (long grp = blockIdx.x; grp < LN_GROUPS; grp += LN_GRID) {
     const long row = grp * LN_RPB + rb;
     const bool live = row < LN_ROWS;
 #if LN_LEAN
-    load_row(row, v);
-#else
-    if (grp + LN_GRID < LN_GROUPS) load_row((grp + LN_GRID) * LN_RPB + rb, vn);
+    load_row(row, in);
+#elif LN_WALKS
+    io_vec_t next[LN_VPT];
+    if (grp + LN_GRID < LN_GROUPS) load_row((grp + LN_GRID) * LN_RPB + rb, next);
 #endif
+    vec_t v[LN_VPT];
+#pragma unroll
+    for (int i = 0; i < LN_VPT; ++i) v[i] = widen(in[i]);
 
 #if LN_ONEPASS
     // the lane's own LN_VPT * LN_VW values
@@ -197,7 +189,7 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
 #pragma unroll
     for (int i = 0; i < LN_VPT; ++i)
 #pragma unroll
-      for (int j = 0; j < LN_VW; ++j) s += v[i][j];
+      for (int j = 0; j < LN_VW; ++j) s += (LN_WALKS && LN_N % LN_VW == 0) || counts(i, j) ? v[i][j] : 0.0f;
     s = kcg_wave_sum(s);
 #if LN_TPR > KCG_WAVE
     if ((tr % KCG_WAVE) == 0) red[0][rb][wv] = s;
@@ -210,15 +202,13 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
 
     float q = 0.0f;
 #pragma unroll
-    for (int i = 0; i < LN_VPT; ++i) {
-      const int idx = (i * LN_TPR + tr) * LN_VW;
+    for (int i = 0; i < LN_VPT; ++i)
 #pragma unroll
       for (int j = 0; j < LN_VW; ++j) {
-        const float d = (idx + j < LN_N) ? v[i][j] - mean : 0.0f;
+        const float d = v[i][j] - mean;
         v[i][j] = d;
-        q += d * d;
+        q += counts(i, j) ? d * d : 0.0f;
       }
-    }
     q = kcg_wave_sum(q);
 #if LN_TPR > KCG_WAVE
     // red[0] is rewritten only after this barrier, red[1] only after the next
@@ -235,17 +225,12 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
     LN_IO* __restrict__ y = Y + (live ? row : 0) * (long)LN_N;
 #pragma unroll
     for (int i = 0; i < LN_VPT; ++i) {
-      const int idx = (i * LN_TPR + tr) * LN_VW;
-      if (live && idx < LN_N) {
+      if (live && begin(i) < LN_N) {
         io_vec_t o;
 #if LN_LEAN
-#if LN_N % LN_VW
-        const vec_t gi = load_any(G, idx, KcgLnOnce<false>{}), bi = load_any(Bt, idx, KcgLnOnce<false>{});
+        const vec_t gi = widen(*(const io_vec_t*)(G + (column(i) % LN_NG))), bi = widen(*(const io_vec_t*)(Bt + (column(i) % LN_NB)));
 #else
-        const vec_t gi = widen(*(const io_vec_t*)(G + (idx % LN_NG))), bi = widen(*(const io_vec_t*)(Bt + (idx % LN_NB)));
-#endif
-#else
-        const vec_t gi = g[i], bi = b[i];
+        const vec_t gi = widen(g[i]), bi = widen(b[i]);
 #endif
 #pragma unroll
         for (int j = 0; j < LN_VW; ++j) {
@@ -255,23 +240,17 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
 #endif
           o[j] = (LN_IO)t;
         }
-#if LN_N % LN_VW
-        if (idx + LN_VW > LN_N) {
-#pragma unroll
-          for (int j = 0; j + 1 < LN_VW; ++j)
-            if (idx + j < LN_N) y[idx + j] = o[j];
-        } else
-#endif
-        __builtin_nontemporal_store(o, (io_vec_t*)(y + idx));
+        __builtin_nontemporal_store(o, (io_vec_t*)(y + place(i)));
       }
     }
-#if !LN_LEAN
+#if !LN_LEAN && LN_WALKS
 #pragma unroll
-    for (int i = 0; i < LN_VPT; ++i) v[i] = vn[i];
+    for (int i = 0; i < LN_VPT; ++i) in[i] = next[i];
 #endif
   }
 }
 #undef LN_GROUPS
+#undef LN_WALKS
 #undef LN_IO
 #ifdef LN_ONEPASS_DEFAULTED
 #undef LN_ONEPASS

@@ -143,7 +143,7 @@ _launch_type = None
 
 
 def _native_launch():
-    """The type of native bound launches (csrc/python/launch.cc), None where it has not been built."""
+    """The type of native bound launches (launch.cc), None where it has not been built."""
     global _launch_type
     if _launch_type is None:
         import torch  # noqa: F401  (the extension's libraries)
@@ -379,10 +379,10 @@ _kernel_cache = {}
 
 
 def launch_params(family, params):
-    """The parameters of a kernel that is compiled to be launched from here.  Attention, and a product whose caller has looked at
-    the operands' addresses (ALIGN = 16), may take the forms that fill the part, those whose wavefronts split k or the keys included
-    (FILL = 2), unless the caller names another FILL than 1.  Text that is emitted for others to keep has the tiles that its parameters name."""
-    if (family.startswith("fmha_") or (family.startswith("gemm_") and params.get("ALIGN", 0) >= 16)) and params.get("FILL", 1) == 1:
+    """The parameters of a kernel that is compiled to be launched from here.  Attention, LayerNorm, and a product whose caller has
+    looked at the operands' addresses (ALIGN = 16), may take the forms that fill the part, those whose wavefronts split k or the keys
+    included (FILL = 2), unless the caller names another FILL than 1.  Text that is emitted for others to keep has the tiles that its parameters name."""
+    if (family == "layernorm" or family.startswith("fmha_") or (family.startswith("gemm_") and params.get("ALIGN", 0) >= 16)) and params.get("FILL", 1) == 1:
         return {**params, "FILL": 2}
     return params
 
