@@ -1493,9 +1493,8 @@ bool emitFmhaF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   const int64_t b = s.p["B"], h = s.p["H"], sl = s.p["S"], dh = s.p["D"];
   if (s.get("WAVEK", 0) > 0) return emitFmhaWavek(s, src, info, err, 0, s.get("QB", 1), s.get("WAVEK", 0));
   if (dh % 32 || dh > 256) { err = "fmha_f32: head dim must be a multiple of 32, at most 256"; return false; }
-  // (D2L = 0, no direct loads, is true of the split as well: a call gives the same bits with and without it, whichever form it takes)
-  bool own = s.get("D2L", 0) != 0;
-  for (const char* key : {"BR", "BC", "OCC", "PAIR"}) own = own || s.has(key);
+  bool own = false;
+  for (const char* key : {"BR", "BC", "D2L", "OCC", "PAIR"}) own = own || s.has(key);
   // queries per workgroup (32 per wavefront): four wavefronts, fewer for short sequences
   int64_t br = s.get("BR", 0);
   bool halved = false;
@@ -1544,7 +1543,8 @@ bool emitFmhaF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // instead of 40 at B1 H5 S1024 take 0.129 against 0.114 ms)
   const bool pair = s.get("PAIR", pairFits && (halved || (nq / 2) * b * h >= 512) ? 1 : 0) != 0;
   if (pair && !pairFits) { err = "fmha_f32: PAIR needs the causal mask and an even number of query tiles"; return false; }
-  if (!own) {
+  // (not where the direct loads are the default: with and without them the kernel gives the same bits, which a split would not)
+  if (!own && !d2l) {
     int64_t splitQb, splitWk;
     if (fmhaWavekAhead(s, 0, br, pair, (double)((pair ? nq / 2 : nq) * b * h), std::max<int64_t>(1, 4 * occ / (br / 32)), splitQb, splitWk))
       return emitFmhaWavek(s, src, info, err, 0, splitQb, splitWk);

@@ -15,9 +15,8 @@ def text_of(family, **params):
 def test_only_small_launches_without_wishes_split_the_keys(family):
     small = dict(B=1, H=8, S=333, D=64, SCALE=0.1, FILL=1)
     assert SPLIT in text_of(family, **small) and SPLIT in text_of(family, **dict(small, D=128, CAUSAL=1))
-    # fp32 at head dim 128 in whole tiles: the same bits with and without direct loads by default, so the same form
-    assert SPLIT in text_of(family, **dict(small, D=128, S=512)) and (family == "fmha_bf16" or SPLIT in text_of(family, **dict(small, D=128, S=512, D2L=0)))
-    assert SPLIT not in text_of(family, **dict(small, D=128, S=512, D2L=1))
+    # fp32 at head dim 128 in whole tiles: direct loads, which give the bits that the same kernel gives without them
+    assert (SPLIT in text_of(family, **dict(small, D=128, S=512))) == (family == "fmha_bf16")
     assert SPLIT not in R.emit_kernel(family, "kernel0", **small)[0]
     for other in (dict(FILL=0), dict(B=8, H=32, S=2048), dict(D=96), dict(D=32), dict(BR=64), dict(BC=32), dict(WAVEK=0)):
         assert SPLIT not in text_of(family, **dict(small, **other)), other

@@ -52,7 +52,7 @@ def test_forms(form, dtype, d, causal):
 
 
 @pytest.mark.parametrize("dtype,d,b,h,s,causal", [("bf16", 64, 1, 8, 333, False), ("f16", 128, 2, 16, 100, True), ("bf16", 128, 1, 8, 1024, True),
-                                                  ("f32", 64, 2, 16, 512, False), ("f32", 128, 1, 12, 77, True), ("f32", 128, 1, 8, 1024, False), ("f16", 64, 1, 8, 2048, False)])
+                                                  ("f32", 64, 2, 16, 512, False), ("f32", 128, 1, 12, 77, True), ("f16", 64, 1, 8, 2048, False)])
 def test_chosen(dtype, d, b, h, s, causal):
     """The same without asking for a form: the rule picks it for these launches."""
     from kernelcodegen_amd import runtime as R
@@ -78,4 +78,4 @@ def test_infinities_and_nan_stay_in_their_rows():
     ok = ~torch.isnan(want)
     assert float((got.double() - want)[ok].norm() / want[ok].norm()) < 4e-6
     k[0, 0, 9] = float("inf")
-    assert torch.isnan(ops.fmha(q, k, v, WAVEK=4)[0, 0]).all() and torch.isnan(ops.fmha(q, k, v, BR=128)[0, 0]).all()
+    assert torch.isnan(ops.fmha(q, k, v, WAVEK=4)[0, 0]).all() and torch.isnan(ops.fmha(q, k, v, D2L=0)[0, 0]).all()
