@@ -186,8 +186,8 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   const bool crowded = vpt > few || (tpr == 1024 && vpt * vw > 24);
   const bool wideGrid = f16 && ((vw == 8 && vpt <= 2) || (vw == 4 && n >= 1024 && n <= 4096));
   if (grid <= 0) grid = crowded ? groups : wideGrid ? 1024 : 512;      // rows too long to prefetch keep one workgroup per group
-  if (grid > groups) grid = groups;
-  if (grid > 0x7FFFFFFFLL) grid = 0x7FFFFFFFLL;
+  // (a launch takes fewer than 2^32 threads: 2^26 rows of 512, a wavefront each, are one workgroup too many; the rest is walked)
+  grid = std::min({grid, groups, (int64_t)(0xFFFFFFFFLL / (tpr * rpb))});
   s.p["GRID"] = grid;
   d.add("LN_GRID", grid);
   d.add("LN_STREAM", s.get("STREAM", 1) ? 1 : 0);

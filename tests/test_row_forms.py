@@ -81,3 +81,12 @@ def test_softmax_of_16_bit_rows_keeps_its_lanes_and_its_alignment_on_small_launc
         assert d["SM_VW"] == "4" and int(d["SM_TPR"]) == lanes_in_fours(n, 1024), n
     assert int(form(4096, 16384)["SM_TPR"]) == 128 and form(3892, 16384)["SM_VW"] == "8" and form(1500, 4000)["SM_VW"] == "4"
     assert int(form(3893, 1000)["SM_TPR"]) == lanes_in_fours(3893, 1024) and form(3893, 1000)["SM_VW"] == "8"
+
+
+@pytest.mark.parametrize("dtype", sorted(TYPES))
+@pytest.mark.parametrize("rows,n", [(1 << 26, 512), (1 << 25, 1024), (1 << 24, 5000), (1 << 28, 64), ((1 << 32) - 1, 8), (5000000, 32000)])
+def test_a_layernorm_of_very_many_rows_is_one_launch(rows, n, dtype):
+    """Fewer than 2^32 threads, the most that a launch takes; workgroups walk the rows that are left."""
+    text, info = R.emit_kernel("layernorm", "kernel0", ROWS=rows, N=n, NG=n, NB=n, EPS=1e-5, F16=TYPES[dtype])
+    assert info["grid"][0] * info["block"][0] < 1 << 32
+    assert "#define LN_GRID %d\n" % info["grid"][0] in text
