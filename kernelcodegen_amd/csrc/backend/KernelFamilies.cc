@@ -1287,6 +1287,10 @@ static int64_t fmhaWavekLds(int type, int64_t d, int64_t qb, int64_t wk) {
   return wk * (std::max(32 * (2 * row + 48), 32 * (d * 4 + 16)) + 32 * qb * 8);
 }
 
+// A launch takes fewer than 2^32 threads.  Wavefronts that split the keys are more of them than those that walk: 2^23 heads of 129 queries
+// under the mask are 2^32.3 in workgroups of two such wavefronts and 2^31 in pairs of 256 queries.
+static bool fmhaWavekLaunches(int64_t sl, double heads, int64_t qb, int64_t wk) { return (double)ceilDiv(sl, 32 * qb) * heads * (double)(64 * wk) < 4294967296.0; }
+
 // Wavefronts per SIMD that the registers of a form leave room for (130 to 190 of them in 16 bits, 174 to 361 in fp32).
 static int64_t fmhaWavekEu(int type, int64_t d, int64_t qb) { return type != 0 ? (d <= 64 && qb == 1 ? 4 : qb == 2 && d > 64 ? 1 : 2) : d <= 64 && qb == 1 ? 2 : 1; }
 
@@ -1294,8 +1298,8 @@ bool emitFmhaWavek(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   const int64_t b = s.p["B"], h = s.p["H"], sl = s.p["S"], dh = s.p["D"];
   const int64_t es = type == 0 ? 4 : 2;
   if ((dh != 32 && dh != 64 && dh != 128) || qb < 1 || qb > 2 || wk < 1 || wk > 16 || fmhaWavekLds(type, dh, qb, wk) > 160 * 1024 ||
-      (double)sl * (double)dh * (double)es >= 2147483648.0 || (double)ceilDiv(sl, 32 * qb) * (double)b * (double)h > 2147483647.0) {
-    err = s.family + ": WAVEK needs a head dim of 32, 64 or 128, QB 1 or 2, at most 16 wavefronts whose tiles fit 160 KiB of LDS, and heads below 2 GiB";
+      (double)sl * (double)dh * (double)es >= 2147483648.0 || !fmhaWavekLaunches(sl, (double)b * (double)h, qb, wk)) {
+    err = s.family + ": WAVEK needs a head dim of 32, 64 or 128, QB 1 or 2, at most 16 wavefronts whose tiles fit 160 KiB of LDS, heads below 2 GiB, and fewer than 2^32 threads";
     return false;
   }
   if (s.f.count("SCALE") && !(s.f["SCALE"] > 0.0)) { err = s.family + ": the softmax scale must be positive"; return false; }
@@ -1350,7 +1354,7 @@ static bool fmhaWavekAhead(const KernelSpec& s, int type, int64_t br, bool paire
   const int64_t row = dh * (type == 0 ? 4 : 2);
   for (int64_t q : {1, 2})
     for (int64_t w : {2, 4, 8}) {
-      if ((double)w > tiles || (q == 2 && (dh == 128 || (type == 0 && w != 4))) || fmhaWavekLds(type, dh, q, w) > 160 * 1024) continue;
+      if ((double)w > tiles || (q == 2 && (dh == 128 || (type == 0 && w != 4))) || fmhaWavekLds(type, dh, q, w) > 160 * 1024 || !fmhaWavekLaunches(sl, heads, q, w)) continue;
       const double groups = (double)ceilDiv(sl, 32 * q) * heads, per = std::ceil(groups / 256.0);
       const int64_t fit = std::max<int64_t>(1, std::min<int64_t>(160 * 1024 / fmhaWavekLds(type, dh, q, w), fmhaWavekEu(type, dh, q) * 4 / w));
       const double turns = std::ceil(groups / (256.0 * (double)fit));

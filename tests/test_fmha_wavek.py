@@ -28,6 +28,16 @@ def test_what_is_asked_for_and_does_not_fit_is_refused(bad):
         R.emit_kernel("fmha_bf16", "kernel0", **dict(dict(B=1, H=8, S=333, D=64, WAVEK=4), **bad))
 
 
+@pytest.mark.parametrize("heads,s", [(1 << 23, 129), (1 << 22, 333)])
+def test_a_launch_has_fewer_than_2_to_the_32_threads(heads, s):
+    """Very many heads: wavefronts that walk the keys, or 64 queries a workgroup, fit one launch where splitting over 32 does not."""
+    many = dict(B=1, H=heads, S=s, D=64, CAUSAL=1, SCALE=0.1)
+    _, info = R.emit_kernel("fmha_bf16", "kernel0", **R.launch_params("fmha_bf16", many))
+    assert info["grid"][0] * info["block"][0] < 1 << 32
+    with pytest.raises(_lib.KcgError):
+        R.emit_kernel("fmha_bf16", "kernel0", WAVEK=2, **many)
+
+
 @pytest.mark.parametrize("causal", [0, 1])
 @pytest.mark.parametrize("family,extra", [("fmha_bf16", dict()), ("fmha_bf16", dict(F16=1)), ("fmha_bf16", dict(OUT_BF16=0)), ("fmha_f32", dict())])
 def test_every_chosen_form_stays_in_registers(family, extra, causal):
