@@ -1315,7 +1315,11 @@ bool emitFmhaWavek(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
   d.add("FW_QB", qb); d.add("FW_WK", wk);
   d.add("FW_EU", std::max<int64_t>(1, s.get("EU", std::max(fmhaWavekEu(type, dh, qb), wk / 4))));
   d.add("FW_CAUSAL", causal ? 1 : 0);
-  d.add("FW_C", floatLiteral(scale * 1.4426950408889634));
+  // (a power of two down to 2^-126, the smallest normal number)
+  const double c = scale * 1.4426950408889634;
+  const int down = type == 2 || !(c < 1.0) ? 0 : std::max(-126, std::ilogb(c));
+  d.add("FW_QEXP", (int64_t)down);
+  d.add("FW_C", floatLiteral(std::ldexp(c, -down)));
   src = d.wrap(kTpl_fmha_wavek);
   info.name = s.name;
   info.grid[0] = (uint32_t)(ceilDiv(sl, 32 * qb) * b * h);

@@ -9,7 +9,9 @@
 //   FW_WK                  wavefronts per workgroup; wavefront w takes the key tiles w, w + FW_WK, ... of 32 keys
 //   FW_EU                  wavefronts per SIMD the register allocation has to leave room for
 //   FW_CAUSAL              1: key j contributes to query i only if j <= i
-//   FW_C                   softmax scale times log2(e), a float literal > 0
+//   FW_QEXP                the queries are scaled by 2^FW_QEXP, exactly: scores leave the fp32 range only where they do scaled (the kernels of
+//                          whole tiles scale the queries by all of it).  0 for IEEE half, whose products cannot overflow
+//   FW_C                   the rest of softmax scale times log2(e), a float literal > 0
 //
 // The kernels of whole tiles (fmha_bf16.hip, fmha_f32.hip) give a wavefront 32 queries and let it walk all keys, tile by tile
 // behind the workgroup's barriers.  Where heads x queries / 32 wavefronts do not fill the part, that walk is the launch's time
@@ -36,6 +38,7 @@ template <int TYPE> __device__ __forceinline__ kcg_f32x16 kcg_fw_mma(kcg_u32x4 a
 #define FW_PO (FW_D * 4 + 16)                    // of a result row
 #define FW_TILE (32 * (FW_PK + FW_PV))
 #define FW_PART (FW_TILE > 32 * FW_PO ? FW_TILE : 32 * FW_PO)        // LDS of one wavefront
+#define FW_QS __builtin_ldexpf(1.0f, FW_QEXP)
 #define FW_NQ ((FW_S + 32 * FW_QB - 1) / (32 * FW_QB))
 extern "C" __global__ __launch_bounds__(64 * FW_WK, FW_EU)
 void FW_NAME(const char* __restrict__ Q, const char* __restrict__ K, const char* __restrict__ V,
@@ -71,7 +74,20 @@ void FW_NAME(const char* __restrict__ Q, const char* __restrict__ K, const char*
     const int row = q0 + 32 * b + l32;
     const char* p = Q + base + (long)(row < FW_S ? row : FW_S - 1) * FW_ROW + 16 * lh;
 #pragma unroll
-    for (int s = 0; s < FW_ROW / 32; ++s) fq[b][s] = *(const kcg_u32x4*)(p + 32 * s);
+    for (int s = 0; s < FW_ROW / 32; ++s) {
+      fq[b][s] = *(const kcg_u32x4*)(p + 32 * s);
+#if FW_QEXP != 0
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned raw = fq[b][s][e];
+#if FW_TYPE == 0
+        fq[b][s][e] = __builtin_bit_cast(unsigned, __builtin_bit_cast(float, raw) * FW_QS);
+#else
+        fq[b][s][e] = kcg_pack_bf16x2(__builtin_bit_cast(float, raw << 16) * FW_QS, __builtin_bit_cast(float, raw & 0xffff0000u) * FW_QS);
+#endif
+      }
+#endif
+    }
   }
   kcg_f32x16 acc[FW_QB][DB];
   float m[FW_QB], l[FW_QB];
@@ -280,3 +296,4 @@ void FW_NAME(const char* __restrict__ Q, const char* __restrict__ K, const char*
 #undef FW_TILE
 #undef FW_PART
 #undef FW_NQ
+#undef FW_QS

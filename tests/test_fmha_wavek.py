@@ -52,3 +52,15 @@ def test_every_chosen_form_stays_in_registers(family, extra, causal):
                         seen.add(form)
                         assert scratch_bytes(R.compile_to_code(R.prelude() + text)) == 0, (heads, s, form)
     assert len(seen) >= 5, seen
+
+
+@pytest.mark.parametrize("scale", [64 ** -0.5, 1.0, 3.0, 2.0 ** -125, 2.0 ** -130, 1e30])
+@pytest.mark.parametrize("family,f16", [("fmha_f32", 0), ("fmha_bf16", 0), ("fmha_bf16", 1)])
+def test_queries_are_scaled_by_a_power_of_two(family, f16, scale):
+    """2^FW_QEXP, a normal number of at most 1, times FW_C is the scale; IEEE half, whose products stay in the fp32 range, is left alone."""
+    text = text_of(family, B=1, H=8, S=333, D=64, SCALE=scale, F16=f16, WAVEK=4)
+    define = {l.split()[1]: l.split()[2] for l in text.splitlines() if l.startswith(("#define FW_QEXP", "#define FW_C "))}
+    c, down = float.fromhex(define["FW_C"].rstrip("f")), int(define["FW_QEXP"])
+    want = scale * 1.4426950408889634
+    assert abs(c * 2.0 ** down / want - 1) < 2.0 ** -24 or (f16 and scale < 2.0 ** -126)
+    assert down == 0 if f16 or want >= 1 else (-126 <= down < 0 and (1 <= c < 2 or down == -126))

@@ -79,3 +79,19 @@ def test_infinities_and_nan_stay_in_their_rows():
     assert float((got.double() - want)[ok].norm() / want[ok].norm()) < 4e-6
     k[0, 0, 9] = float("inf")
     assert torch.isnan(ops.fmha(q, k, v, WAVEK=4)[0, 0]).all() and torch.isnan(ops.fmha(q, k, v, D2L=0)[0, 0]).all()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("form", [dict(WAVEK=4), dict()])
+def test_scores_leave_the_fp32_range_only_where_they_do_scaled(form, dtype):
+    """Products of queries and keys around 2^129, scaled back to 16 and at most 100; the kernels of whole tiles take them too.  A score of 100
+    is off by up to three roundings to 24 bits, 2e-5 of a probability in fp32; 16 bits as above (the walk rounds scaled queries)."""
+    from kernelcodegen_amd import ops
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(9)
+    q, k, v = (torch.randn(1, 8, 300, 64, generator=gen, device="cuda") for _ in range(3))
+    q, k, v = (q * 2.0 ** 63).to(DTYPE[dtype]), (k * 2.0 ** 63).to(DTYPE[dtype]), v.to(DTYPE[dtype])
+    got = ops.fmha(q, k, v, scale=2.0 ** -125, **form)
+    want = _reference(q, k, v, False, 2.0 ** -125)
+    assert float((got.double() - want).norm() / want.norm()) < (2e-5 if dtype == "f32" else TOL[dtype])
+    assert torch.isfinite(ops.fmha(q, k, v, scale=2.0 ** -125, WAVEK=0)).all()
