@@ -14,13 +14,14 @@ import hashlib
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 KDIR = os.path.join(CSRC, "backend", "kernels")
 LIB = os.path.join(PKG, "libkcg_hip.so")
-LAUNCH = os.path.join(PKG, "_launch.so")
+LAUNCH = os.path.join(PKG, "_launch" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))      # another Python does not find it
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 CXX = os.environ.get("CXX", "g++")
@@ -63,32 +64,44 @@ def _stamp():
 
 
 def build_launch(force=False, verbose=False):
-    """The bound launches of the Python operators (launch.cc), an extension module on torch's own libraries."""
-    import sysconfig
-    import torch
-    src = os.path.join(os.path.dirname(CSRC), "launch.cc")
-    base = os.path.join(os.path.dirname(torch.__file__))
-    inc = os.path.join(base, "include")
-    cmd = [CXX, "-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", inc, "-I", os.path.join(inc, "torch", "csrc", "api", "include"),
-           "-I", os.path.join(ROCM, "include"), "-I", sysconfig.get_paths()["include"], src, "-o", LAUNCH, "-L", os.path.join(base, "lib"),
-           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    """The bound launches of the Python operators (launch.cc), an extension module on torch's own libraries; None where there is no
+    torch to build it on or the compiler refuses it, whose messages are shown: ctypes launches take its place."""
     stamp_file = LAUNCH + ".stamp"
-    stamp = hashlib.sha256((open(src).read() + " ".join(cmd) + torch.__version__).encode()).hexdigest()
-    if not force and os.path.exists(LAUNCH) and os.path.exists(stamp_file) and open(stamp_file).read() == stamp:
-        return LAUNCH
-    if verbose:
-        print(" ".join(cmd))
-    subprocess.check_call(cmd, stderr=None if verbose else subprocess.DEVNULL)
+    try:
+        import torch
+        src = os.path.join(os.path.dirname(CSRC), "launch.cc")
+        base = os.path.dirname(torch.__file__)
+        inc = os.path.join(base, "include")
+        cmd = [CXX, "-std=c++17", "-O2", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+               "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, '-DKCG_TORCH_VERSION="%s"' % torch.__version__,
+               "-I", inc, "-I", os.path.join(inc, "torch", "csrc", "api", "include"),
+               "-I", os.path.join(ROCM, "include"), "-I", sysconfig.get_paths()["include"], src, "-o", LAUNCH, "-L", os.path.join(base, "lib"),
+               "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+        stamp = hashlib.sha256((open(src).read() + " ".join(cmd)).encode()).hexdigest()
+        if not force and os.path.exists(LAUNCH) and os.path.exists(stamp_file) and open(stamp_file).read() == stamp:
+            return LAUNCH
+        if verbose:
+            print(" ".join(cmd))
+        done = subprocess.run(cmd, stderr=subprocess.PIPE, text=True, errors="replace")
+        why = "%s\nstatus %d" % (done.stderr, done.returncode) if done.returncode else ""
+    except (ImportError, OSError) as e:
+        why = str(e)
+    if why:
+        for stale in (LAUNCH, stamp_file):
+            if os.path.exists(stale):
+                os.remove(stale)
+        print("%s\nthe native launches were not built: launches go through ctypes" % why, file=sys.stderr)
+        return None
     with open(stamp_file, "w") as f:
         f.write(stamp)
     return LAUNCH
 
 
 def build(force=False, verbose=False):
-    """libkcg_hip.so and the native launches; returns the library."""
+    """libkcg_hip.so, then the native launches where they can be built; returns the library."""
+    library = build_library(force, verbose)
     build_launch(force, verbose)
-    return build_library(force, verbose)
+    return library
 
 
 def build_library(force=False, verbose=False):

@@ -228,5 +228,10 @@ PyMODINIT_FUNC PyInit__launch(void) {
     Py_DECREF(m);
     return nullptr;
   }
+  // the version whose headers this was built on (torch.__version__), for the importer to compare
+  if (PyModule_AddStringConstant(m, "torch_version", KCG_TORCH_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
   return m;
 }

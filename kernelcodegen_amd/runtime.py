@@ -143,16 +143,27 @@ _launch_type = None
 
 
 def _native_launch():
-    """The type of native bound launches (launch.cc), None where it has not been built."""
+    """The type of native bound launches (launch.cc), None where it has not been built for this torch or does not load."""
     global _launch_type
     if _launch_type is None:
-        import torch  # noqa: F401  (the extension's libraries)
+        import importlib
+        import torch                    # (the extension's libraries)
+        _launch_type, why = False, None
         try:
-            from . import _launch
+            module = importlib.import_module(__package__ + "._launch")
         except ModuleNotFoundError:
-            _launch_type = False
+            pass
+        except ImportError as e:
+            why = str(e)
         else:
-            _launch_type = _launch.Launch
+            # objects of torch are laid out as in the headers of the build
+            if getattr(module, "torch_version", None) == torch.__version__:
+                _launch_type = module.Launch
+            else:
+                why = "built for torch %s, this is %s" % (getattr(module, "torch_version", "of another version"), torch.__version__)
+        if why:
+            import warnings
+            warnings.warn("the native launches are not used, ctypes takes their place: " + why, RuntimeWarning)
     return _launch_type or None
 
 

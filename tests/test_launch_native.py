@@ -66,6 +66,46 @@ def test_without_a_gpu_a_launch_is_an_error():
     assert not entry.calls
 
 
+@pytest.mark.parametrize("content", [None, b"no library", "other version"])
+def test_an_extension_that_is_missing_or_does_not_fit_gives_way_to_ctypes(tmp_path, monkeypatch, content):
+    """No file, one that does not load, and one that loads but was built for another torch."""
+    import sys
+    import types
+    import kernelcodegen_amd
+    from kernelcodegen_amd import build as B
+    name = "kernelcodegen_amd._launch"
+    monkeypatch.setattr(R, "_launch_type", None)
+    monkeypatch.setattr(kernelcodegen_amd, "__path__", [str(tmp_path)])
+    monkeypatch.delitem(sys.modules, name, raising=False)
+    if content == "other version":
+        monkeypatch.setitem(sys.modules, name, types.SimpleNamespace(torch_version="1.0", Launch=None))
+    elif content is not None:
+        (tmp_path / B.os.path.basename(B.LAUNCH)).write_bytes(content)
+    if content is None:
+        assert R._native_launch() is None
+    else:
+        with pytest.warns(RuntimeWarning, match="ctypes"):
+            assert R._native_launch() is None
+    kern = R.Kernel(None, C.c_void_p(5), dict(grid=(1, 1, 1), block=(64, 1, 1), lds_bytes=0, num_args=2, workspace_bytes=0))
+    monkeypatch.setattr(R, "_current_stream", lambda: lambda: 0)
+    assert not hasattr(kern.bind(), "result") and callable(kern.bind())
+
+
+def test_the_library_is_built_where_the_extension_cannot_be(tmp_path, monkeypatch, capfd):
+    from kernelcodegen_amd import build as B
+    compiler, launch = tmp_path / "cxx", tmp_path / "_launch.so"
+    compiler.write_text("#!/bin/sh\necho no such header >&2\nexit 1\n")
+    compiler.chmod(0o755)
+    launch.write_bytes(b"of an earlier build")
+    monkeypatch.setattr(B, "LAUNCH", str(launch))
+    monkeypatch.setattr(B, "CXX", str(compiler))
+    monkeypatch.setattr(B, "build_library", lambda force, verbose: "library")
+    assert B.build() == "library" and not launch.exists()
+    assert "no such header" in capfd.readouterr().err
+    monkeypatch.setitem(__import__("sys").modules, "torch", None)      # no torch at all
+    assert B.build() == "library"
+
+
 @pytest.mark.gpu
 def test_what_is_passed_on():
     entry = Entry()
