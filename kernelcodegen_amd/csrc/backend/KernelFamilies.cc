@@ -484,6 +484,14 @@ bool checkTile(const KernelSpec& s, int64_t bm, int64_t bn, int64_t bk, int64_t 
 // in 32 bits: where more than the whole tiles of the direct-load kernels is taken, longer ones keep the other kernels.
 static bool shortRows(int64_t n, int64_t k) { return n <= (1 << 23) && k <= (1 << 23); }
 
+// Whether a caller names nothing but the problem: a kernel that has no use for some other wish is not taken in its place.
+static bool namesOnly(const KernelSpec& s, std::initializer_list<const char*> problem) {
+  for (const auto& kv : s.p)
+    if (std::none_of(problem.begin(), problem.end(), [&](const char* key) { return kv.first == key; })) return false;
+  return true;
+}
+static bool namesOnlyProduct(const KernelSpec& s) { return namesOnly(s, {"M", "N", "K", "BATCH", "TA", "TB", "ALIGN", "FILL", "OUT_BF16", "F16", "RELU", "SCALE_PTR"}); }
+
 // GEMM whose wavefronts split k (kernels/gemm_wavek.hip).  type: 0 fp32, 1 bf16, 2 IEEE half, 3 fp8 e4m3.
 struct WavekForm { int64_t tm, tn, vw, wk, depth; };
 
@@ -570,7 +578,7 @@ static double wavekTime(int type, bool tb, bool out16, const WavekForm& f, int64
 
 // The form of least modelled time, if there is one and the caller asks for it (FILL = 2); `us`: that time.
 static bool chooseWavek(const KernelSpec& s, int type, int64_t m, int64_t n, int64_t k, int64_t batch, WavekForm& best, double& us) {
-  if (s.get("FILL", 0) < 2 || s.has("WAVEK") || !wavekFits(s, type, n, k)) return false;
+  if (s.get("FILL", 0) < 2 || !wavekFits(s, type, n, k)) return false;
   static const int64_t tiles[][2] = {{1, 1}, {1, 2}, {2, 1}, {2, 2}, {1, 4}, {2, 4}, {4, 2}, {4, 4}, {3, 4}, {4, 3}};
   const bool tb = s.get("TB", 0) != 0, out16 = s.get("OUT_BF16", 0) != 0;
   const int64_t es = type == 0 ? 4 : type == 3 ? 1 : 2, steps = ceilDiv(k * es, 128);
@@ -614,7 +622,7 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   bool own = false;
   for (const char* key : {"BM", "BN", "BK", "WM", "WN", "WK", "NBUF", "PAD"}) own = own || s.has(key);
   const bool direct = s.get("D2L", 1) != 0 && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !s.get("TA", 0) && k % 4 == 0 && (s.get("TB", 0) || n % 4 == 0);
-  const bool any = own;
+  const bool plain = namesOnlyProduct(s);
   const bool divides = m % tile == 0 && n % tile == 0 && k % (tile <= 128 ? 32 : 16) == 0;
   if (!own && (!divides || (direct && s.get("TB", 0))) && m >= 64 && n >= 64 && k >= 16) {
     static const struct { int64_t t; double weight; } sizes[] = {{256, 0.985}, {128, 1.0}, {64, 1.06}};
@@ -633,7 +641,7 @@ bool emitGemmF32(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // on average): rounds of tiles and the part of them in use, and on few 64 x 64 tiles a k-tile's way from memory.  us, this and
   // that: 256^3 6.6 and 2.5, 256 x 256 x 2048 36 and 7.1, 2 x 700 x 300 x 1500 47 and 20; 1500 x 400 x 1100 34 and 22; level at
   // 1024^3 (20); 4 x 1024^3 70 and 75.
-  if (!any && s.get("D2L", 1) != 0 && m >= 64 && n >= 64 && k >= 16) {
+  if (plain && m >= 64 && n >= 64 && k >= 16) {
     WavekForm form;
     double us;
     if (chooseWavek(s, 0, m, n, k, batch, form, us)) {
@@ -943,7 +951,7 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
     form = chooseGemm16Form(m, n, k, batch, &cost);
     WavekForm split;
     const int type = s.get("F16", 0) ? 2 : 1;
-    if (!s.get("FP8_PAIRS", 0) && wavekAhead(s, type, form, cost, m, n, k, batch, split)) return emitGemmWavek(s, src, info, err, type, split, m, n, k, batch);
+    if (namesOnlyProduct(s) && wavekAhead(s, type, form, cost, m, n, k, batch, split)) return emitGemmWavek(s, src, info, err, type, split, m, n, k, batch);
     if (!s.get("FP8_PAIRS", 0)) form = chooseThirds(form, m, n, k, batch);
   }
   if (form) {
@@ -1109,7 +1117,7 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
     double cost;
     const Gemm16Form* tiled = chooseGemm16Form(m, n, k / 2, batch, &cost);
     WavekForm split;
-    if (wavekAhead(s, 3, tiled, cost, m, n, k, batch, split)) return emitGemmWavek(s, src, info, err, 3, split, m, n, k, batch);
+    if (namesOnlyProduct(s) && wavekAhead(s, 3, tiled, cost, m, n, k, batch, split)) return emitGemmWavek(s, src, info, err, 3, split, m, n, k, batch);
   }
   if (!own && !whole && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !ta && k % 16 == 0 && n % 16 == 0 && s.get("SCALE_PTR", 0) == 0) {
     const Gemm16Form* form = chooseGemm16Form(m, n, k / 2, batch);
@@ -1341,7 +1349,7 @@ bool emitFmhaWavek(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
 static bool fmhaWavekAhead(const KernelSpec& s, int type, int64_t br, bool paired, double items, int64_t held, int64_t& qb, int64_t& wk) {
   const int64_t sl = s.get("S", 0), dh = s.get("D", 0);
   const double heads = (double)s.get("B", 0) * (double)s.get("H", 0);
-  if (s.get("FILL", 0) < 2 || s.has("WAVEK") || (dh != 64 && dh != 128) || (double)sl * (double)dh * 4.0 >= 2147483648.0) return false;
+  if (s.get("FILL", 0) < 2 || !namesOnly(s, {"B", "H", "S", "D", "CAUSAL", "OUT_BF16", "F16", "FILL"}) || (dh != 64 && dh != 128) || (double)sl * (double)dh * 4.0 >= 2147483648.0) return false;
   struct Rates { double fixed, walk, work, merge, l2, tiled, tiledWalk, tiledWork, ragged, margin; };
   static const Rates rates[2][2] = {      // 16 bits, fp32; head dim 64, 128
       {{1.94, 0.745, 0.415, 3.71, 0.0186, 2.90, 0.449, 0.104, 0.097, 0.85}, {1.87, 1.01, 0.714, 8.07, 0.0436, 3.93, 0.837, 0.179, 0.091, 0.78}},

@@ -392,7 +392,7 @@ _kernel_cache = {}
 def launch_params(family, params):
     """The parameters of a kernel that is compiled to be launched from here.  Attention, LayerNorm, and a product whose caller has
     looked at the operands' addresses (ALIGN = 16), may take the forms that fill the part, those whose wavefronts split k or the keys
-    included (FILL = 2), unless the caller names another FILL than 1.  Text that is emitted for others to keep has the tiles that its parameters name."""
+    included (FILL = 2), unless the caller names another FILL than 1.  WAVEK = 0 beside it leaves the split out: the forms of FILL = 1.  Text that is emitted for others to keep has the tiles that its parameters name."""
     if (family == "layernorm" or family.startswith("fmha_") or (family.startswith("gemm_") and params.get("ALIGN", 0) >= 16)) and params.get("FILL", 1) == 1:
         return {**params, "FILL": 2}
     return params

@@ -64,3 +64,9 @@ def test_queries_are_scaled_by_a_power_of_two(family, f16, scale):
     want = scale * 1.4426950408889634
     assert abs(c * 2.0 ** down / want - 1) < 2.0 ** -24 or (f16 and scale < 2.0 ** -126)
     assert down == 0 if f16 or want >= 1 else (-126 <= down < 0 and (1 <= c < 2 or down == -126))
+
+
+@pytest.mark.parametrize("family,wish", [("fmha_bf16", dict(VPAD=48)), ("fmha_bf16", dict(QW=1)), ("fmha_bf16", dict(OCC=1)), ("fmha_bf16", dict(STAGE_O=0)), ("fmha_bf16", dict(PERSIST=0)),
+                                         ("fmha_bf16", dict(PAIR=0)), ("fmha_bf16", dict(D2L=0)), ("fmha_f32", dict(OCC=1)), ("fmha_f32", dict(PAIR=0)), ("fmha_f32", dict(D2L=0))])
+def test_a_wish_that_the_split_has_no_use_for_is_not_dropped(family, wish):
+    assert SPLIT not in text_of(family, B=1, H=8, S=333, D=64, SCALE=0.1, **wish)

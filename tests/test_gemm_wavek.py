@@ -50,3 +50,26 @@ def test_every_chosen_form_stays_in_registers(family, extra, tb):
                 seen.add(form)
                 assert scratch_bytes(R.compile_to_code(R.prelude() + text)) == 0, (m, n, k, form)
     assert len(seen) >= 3, seen
+
+
+WISHES = {"gemm_bf16": dict(BM=64, BN=64, BK=64, WM=2, WN=2, GROUP_M=4, M16=1, D2L=1, BTR=0, BPAD=0, STAGES=1, NBUF=2, SK_UNITS=0, INTERLEAVE=1, SETPRIO=1,
+                            STAGE_C=0, KROT=1, STAGGER=1, M16_DEAL=1),
+          "gemm_fp8": dict(BM=64, BN=64, BK=128, WM=2, WN=2, GROUP_M=4, D2L=0, BTR=1, STAGES=1, PREFETCH=1, ROTATE=1, PINGPONG=1, PERSIST=0, STAGE_C=0, NT_STORE=1, STAGGER=1),
+          "gemm_f32": dict(BM=64, BN=64, BK=32, WM=2, WN=2, WK=1, NBUF=2, PAD=4, GROUP_M=4, D2L=1)}
+
+
+@pytest.mark.parametrize("family,key", [(f, k) for f in sorted(WISHES) for k in sorted(WISHES[f])])
+def test_a_wish_that_the_split_has_no_use_for_is_not_dropped(family, key):
+    """Each parameter of the kernels of whole tiles, by itself, keeps the product on them."""
+    small = dict(M=64, N=256, K=1024, TB=1, ALIGN=16)
+    assert SPLIT in text_of(family, **small)
+    try:
+        assert SPLIT not in text_of(family, **dict(small, **{key: WISHES[family][key]}))
+    except _lib.KcgError:
+        pass                              # (refused as it would be without the split)
+
+
+@pytest.mark.parametrize("family,problem", [("gemm_bf16", dict(M=64, N=256, K=1024, TB=1, ALIGN=16)), ("gemm_f32", dict(M=256, N=256, K=1024, ALIGN=16)),
+                                            ("gemm_fp8", dict(M=64, N=256, K=1024, TB=1, ALIGN=16)), ("fmha_bf16", dict(B=1, H=8, S=333, D=64)), ("fmha_f32", dict(B=1, H=8, S=333, D=64))])
+def test_without_the_split_a_launch_has_the_forms_of_whole_tiles(family, problem):
+    assert text_of(family, WAVEK=0, **problem) == R.emit_kernel(family, "kernel0", FILL=1, **problem)[0] != text_of(family, **problem)
