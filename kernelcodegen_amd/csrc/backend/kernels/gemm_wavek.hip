@@ -175,6 +175,8 @@ void GW_NAME(const char* __restrict__ A, const char* __restrict__ B,
   constexpr int TAIL = (int)(GW_KB % 128 / 16), REST = (int)(GW_KB % 16);
   constexpr bool CUT = GW_KB % 128 != 0;
 
+  // fp32 rows of no whole chunks start on any multiple of four bytes
+  typedef unsigned int Stored __attribute__((ext_vector_type(4), aligned(GW_KB % 16 == 0 ? 16 : 4)));
   kcg_wk_chunk ra[DEPTH][RA];
   BRaw rb[DEPTH][NB];
   // step n of this wavefront into slot d; the last one may be partial (K no whole steps) or not there
@@ -188,12 +190,12 @@ void GW_NAME(const char* __restrict__ A, const char* __restrict__ B,
     const char* pa = base_a + (long)s * 128 - (CUT && last ? 16 : 0);
 #pragma unroll
     for (int t = 0; t < RA; ++t)
-      if (GW_M % GW_BM == 0 || m0 + 8 * t < GW_M) ra[d][t] = *(const kcg_wk_chunk*)(pa + (off_a[t] + shift));
+      if (GW_M % GW_BM == 0 || m0 + 8 * t < GW_M) ra[d][t] = *(const Stored*)(pa + (off_a[t] + shift));
 #if GW_TB
     const char* pb = base_b + (long)s * 128 - (CUT && last ? 16 : 0);
 #pragma unroll
     for (int t = 0; t < RB; ++t)
-      if (GW_N % GW_BN == 0 || n0 + 8 * t < GW_N) rb[d][t] = *(const kcg_wk_chunk*)(pb + (off_b[t] + shift));
+      if (GW_N % GW_BN == 0 || n0 + 8 * t < GW_N) rb[d][t] = *(const Stored*)(pb + (off_b[t] + shift));
 #else
     const char* pb = base_b + (long)s * (128 / GW_ES) * PITCH_B;
 #pragma unroll

@@ -73,3 +73,16 @@ def test_a_wish_that_the_split_has_no_use_for_is_not_dropped(family, key):
                                             ("gemm_fp8", dict(M=64, N=256, K=1024, TB=1, ALIGN=16)), ("fmha_bf16", dict(B=1, H=8, S=333, D=64)), ("fmha_f32", dict(B=1, H=8, S=333, D=64))])
 def test_without_the_split_a_launch_has_the_forms_of_whole_tiles(family, problem):
     assert text_of(family, WAVEK=0, **problem) == R.emit_kernel(family, "kernel0", FILL=1, **problem)[0] != text_of(family, **problem)
+
+
+@pytest.mark.parametrize("k,tb", [(1001, 1), (1002, 0), (1024, 1)])
+def test_loads_declare_the_alignment_that_rows_have(k, tb, tmp_path):
+    """fp32 rows of no whole 16-byte chunks start on any multiple of four bytes: no load of the operands may promise more."""
+    import re
+    import subprocess
+    from kernelcodegen_amd import build as B
+    src, out = tmp_path / "k.hip", tmp_path / "k.ll"
+    src.write_text(R.prelude() + text_of("gemm_f32", M=256, N=256, K=k, TB=tb, ALIGN=16, WAVEK=4, TM=2, TN=2, **({} if tb else dict(VW=1))))
+    subprocess.run([B.HIPCC] + B.DEVICE_FLAGS + ["--cuda-device-only", "-S", "-emit-llvm", str(src), "-o", str(out)], check=True, stderr=subprocess.PIPE)
+    aligned = {int(a) for a in re.findall(r"load <4 x i32>, ptr addrspace\(1\) [^\n]*?, align (\d+)", out.read_text())}
+    assert aligned == ({16} if k % 4 == 0 else {4}), aligned
