@@ -576,6 +576,18 @@ static double wavekTime(int type, bool tb, bool out16, const WavekForm& f, int64
   return r.fixed + most + r.sums * per * f.tm * f.tn * f.wk / 16.0 + r.wait * wait;
 }
 
+// Whether a form's registers hold it.  Eight wavefronts leave 256 each; beside 128 of slots and sums the compiler still finds room for
+// fragments, addresses and the last steps that it unrolls, beside 160 not (up to 480 bytes a lane in scratch memory; 36 at 33 x 3840 x
+// 2816 fp8 row-major on 64 x 32 tiles, two steps in flight), nor beside 64 sums while it sorts a row-major B of 8 or 16 bits.  The next
+// best forms are 1.29 (fp8, 13 products whose form spilled) and 1.16 (fp32, 17) times as fast: 63 x 7072 x 3712 fp8 20.1 us and
+// 10.6, 320 x 901 x 3205 fp32 66.7 and 51.2; those that did not spill gain 3 % on average
+// and lose 9 % at worst (fp8 33 x 3856 x 2880 7.1 and 7.7).
+static bool wavekStaysInRegisters(int type, bool tb, const WavekForm& f) {
+  const int64_t es = type == 0 ? 4 : type == 3 ? 1 : 2;
+  const int64_t slotB = tb ? 8 * f.tn : 2 * f.tn / f.vw * (16 / es) * std::max<int64_t>(1, f.vw * es / 4);
+  return f.wk <= 4 || (f.depth * (8 * f.tm + slotB) + 4 * f.tm * f.tn <= 128 && (tb || type == 0 || f.tm * f.tn < 16));
+}
+
 // The form of least modelled time, if there is one and the caller asks for it (FILL = 2); `us`: that time.
 static bool chooseWavek(const KernelSpec& s, int type, int64_t m, int64_t n, int64_t k, int64_t batch, WavekForm& best, double& us) {
   if (s.get("FILL", 0) < 2 || !wavekFits(s, type, n, k)) return false;
@@ -593,6 +605,7 @@ static bool chooseWavek(const KernelSpec& s, int type, int64_t m, int64_t n, int
       for (int64_t depth : {1, 2}) {
         if (wk > steps || (depth > 1 && steps <= wk)) continue;
         const WavekForm f = {t[0], t[1], tb ? 1 : n % 4 || t[1] % 2 ? 1 : std::min<int64_t>(t[1], 4), wk, depth};
+        if (!wavekStaysInRegisters(type, tb, f)) continue;
         const double time = wavekTime(type, tb, out16, f, m, n, k, batch);
         if (us == 0.0 || time < us) { us = time; best = f; }
       }

@@ -75,6 +75,15 @@ def test_without_the_split_a_launch_has_the_forms_of_whole_tiles(family, problem
     assert text_of(family, WAVEK=0, **problem) == R.emit_kernel(family, "kernel0", FILL=1, **problem)[0] != text_of(family, **problem)
 
 
+@pytest.mark.parametrize("family,tb,sizes", [("gemm_fp8", 0, [(40, 4800, 3968), (33, 3840, 2816), (40, 5776, 3888), (37, 4096, 3072), (63, 7072, 3712), (545, 544, 4032)]),
+                                             ("gemm_f32", 1, [(664, 1111, 3520), (320, 901, 3205, 2), (1420, 475, 3560), (244, 174, 4052, 15)])])
+def test_products_of_the_largest_tiles_stay_in_registers(family, tb, sizes):
+    """Products for which eight wavefronts on the largest tiles, two steps in flight, would be the form of least modelled time."""
+    for m, n, k, *batch in sizes:
+        text = text_of(family, M=m, N=n, K=k, TB=tb, ALIGN=16, BATCH=batch[0] if batch else 1)
+        assert scratch_bytes(R.compile_to_code(R.prelude() + text)) == 0, (m, n, k, batch)
+
+
 @pytest.mark.parametrize("k,tb", [(1001, 1), (1002, 0), (1024, 1)])
 def test_loads_declare_the_alignment_that_rows_have(k, tb, tmp_path):
     """fp32 rows of no whole 16-byte chunks start on any multiple of four bytes: no load of the operands may promise more."""
