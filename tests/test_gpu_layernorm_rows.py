@@ -32,10 +32,29 @@ def _check(rows, n, dtype, gelu=False, **cfg):
     assert float(err) < TOL[dtype], (rows, n, dtype, cfg, float(err))
 
 
+ROWS = [1, 7, 256, 257, 1025, 2049]
+LENGTHS = [512, 513, 519, 1023, 1032, 1280, 2049, 3071, 3073, 4100, 5119, 5120, 6145, 7168, 8191, 8192]
+
+
+@pytest.fixture(scope="module")
+def compiled():
+    """The kernels of test_lengths, compiled side by side into the code-object cache: one after the other they are most of its time."""
+    from concurrent.futures import ThreadPoolExecutor
+    from kernelcodegen_amd import ops, runtime as R
+
+    def one(of):
+        n, rows, dtype = of
+        text, _ = R.emit_kernel("layernorm", "kernel0", **R.launch_params("layernorm", dict(
+            ROWS=rows, N=n, NG=n, NB=n, EPS=1e-5, GELU=n % 2, F16=ops._STORAGE[DTYPE[dtype]])))
+        R.compile_to_code(R.prelude() + text)
+    with ThreadPoolExecutor(16) as pool:
+        list(pool.map(one, [(n, rows, dtype) for n in LENGTHS for rows in ROWS for dtype in DTYPE]))
+
+
 @pytest.mark.parametrize("dtype", sorted(DTYPE))
-@pytest.mark.parametrize("rows", [1, 7, 256, 257, 1025, 2049])
-@pytest.mark.parametrize("n", [512, 513, 519, 1023, 1032, 1280, 2049, 3071, 3073, 4100, 5119, 5120, 6145, 7168, 8191, 8192])
-def test_lengths(n, rows, dtype):
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("n", LENGTHS)
+def test_lengths(n, rows, dtype, compiled):
     _check(rows, n, dtype, gelu=n % 2 == 1)
 
 
