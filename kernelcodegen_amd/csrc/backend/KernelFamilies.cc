@@ -1156,7 +1156,9 @@ bool emitGemmFp8(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::s
   // Tiles of 192 columns where they make less of the last round idle: rounds and the part of them in use, in us at K = 4096, fitted to
   // 81 products (us, 256 and 192 columns: 2000 x 11008 x 4096 99 and 89, 1500 x 11008 x 4096 94 and 77, 3000 x 11008 x 4096 147 and 129,
   // 1500 x 4096 x 4096 row-major 53 and 41; but 4096 x 11008 x 4096 162 and 167, 2407 x 5440 x 2048 34 and 46): 23 of the 29 products
-  // on 256 x 256 tiles gain 11 % on average, none loses more than 2 %.
+  // on 256 x 256 tiles gain 11 % on average, none loses more than 2 %.  Products of fewer than 192 columns take them too, on the guarded
+  // kernel (gemm_fp8.hip), which computes less past the edge with them: row-major, us, 256 and 192 columns, 131072 x 128 x 4096 590 and
+  // 167, 65536 x 176 x 512 20.8 and 18.0, 256 times 256 x 128 x 512 20.3 and 18.0, 65536 x 16 x 512 12.0 and 10.5, 512 x 176 x 1024 the same.
   if (!own && dm == 256 && dn == 256 && s.get("ALIGN", 0) >= 16 && shortRows(n, k) && !ta && n % 16 == 0 && k % 128 == 0 && m >= 256 && s.get("SCALE_PTR", 0) == 0 &&
       (shift256 || k <= 4096)) {
     auto time = [&](int64_t cols, double a, double b) {

@@ -56,3 +56,15 @@ def test_chosen(m, n, k, dtype, trans_b):
         t = torch.bfloat16 if dtype == "bf16" else torch.float16
         c = ops.batched_matmul(a.to(t), b.to(t), trans_b=trans_b, out_dtype=t)
     assert torch.equal(c, ref.float().to(c.dtype))
+
+
+@pytest.mark.parametrize("m,n,k,batch", [(70000, 176, 640, 1), (65793, 16, 128, 1), (65793, 48, 384, 1), (256, 128, 512, 256), (300, 144, 384, 150)])
+def test_fp8_of_fewer_columns(m, n, k, batch):
+    """Row-major weights of fewer than 192 columns: the same tiles on the guarded kernel."""
+    from kernelcodegen_amd import ops, runtime as R
+    text = R.emit_kernel("gemm_fp8", **R.launch_params("gemm_fp8", dict(M=m, N=n, K=k, TB=0, BATCH=batch, ALIGN=16, OUT_BF16=1)))[0]
+    assert "#define GF_BN 192\n" in text and "#define GF_EDGE 1\n" in text
+    a, b, ref = _operands(m, n, k, False, batch)
+    for out in (torch.float32, torch.bfloat16):
+        c = ops.matmul_fp8(a.to(torch.float8_e4m3fn), b.to(torch.float8_e4m3fn), 0.5, 4.0, trans_b=False, out_dtype=out)
+        assert torch.equal(c, (2 * ref).float().to(out)), out
