@@ -95,7 +95,11 @@ bool emitLayerNorm(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
     if (lanes * 6 * wide < n || (!f16 && rows > 256 && hold && n > 4096)) lanes = 512;
     s.p["VW"] = wide; s.p["TPR"] = lanes;
     s.p["LEAN"] = !hold;
-    s.p["GRID"] = hold && rows > 256 ? (n <= 1024 ? 768 : 512) : rows;       // (fp32 16384 x 832 19.5 us and 21.0, 9208 x 948 13.0 and 13.6)
+    // Held rows walk on 512 workgroups, up to 1024 elements on 768 (fp32 16384 x 832 19.5 us and 21.0, 9208 x 948 13.0 and 13.6), and so do
+    // fp32 rows that start off the vectors on teams of 128 and 256 while they are not many more than the caches hold: 512 and 768, 4926 x
+    // 2639 23.3 and 19.4, 8684 x 1497 21.3 and 19.7, 3241 x 4010 20.0 and 18.5; but 16004 x 3999 85 and 90.
+    const bool off = !f16 && n % wide != 0 && lanes >= 128 && lanes <= 256 && elements <= 32e6;
+    s.p["GRID"] = hold && rows > 256 ? (n <= 1024 || off ? 768 : 512) : rows;
   }
   // Else 16 bytes per access where all lengths divide into them (16-bit types fall back to fours), and on launches of at least a
   // million elements of any row length, scale and bias then being of that length; smaller odd launches and short rows, where most of

@@ -90,3 +90,11 @@ def test_a_layernorm_of_very_many_rows_is_one_launch(rows, n, dtype):
     text, info = R.emit_kernel("layernorm", "kernel0", ROWS=rows, N=n, NG=n, NB=n, EPS=1e-5, F16=TYPES[dtype])
     assert info["grid"][0] * info["block"][0] < 1 << 32
     assert "#define LN_GRID %d\n" % info["grid"][0] in text
+
+
+@pytest.mark.parametrize("rows,n,grid", [(5888, 2639, 768), (8814, 1497, 768), (4714, 3318, 768), (16004, 3999, 512), (4096, 4096, 512), (16384, 4096, 512), (5151, 5435, 512), (11807, 1101, 512),
+                                         (16384, 832, 768)])
+def test_held_layernorm_rows_walk_on_few_workgroups(rows, n, grid):
+    """fp32 rows that start off the vectors on somewhat more of them than whole ones, while they are not far beyond the caches."""
+    _, info = R.emit_kernel("layernorm", "kernel0", ROWS=rows, N=n, NG=n, NB=n, EPS=1e-5)
+    assert info["grid"][0] == grid
