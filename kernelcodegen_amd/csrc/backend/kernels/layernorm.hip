@@ -39,6 +39,7 @@
 //                LN_TPR * LN_VW); the emitter asks for it only then.
 #define LN_GROUPS ((LN_ROWS + LN_RPB - 1) / LN_RPB)
 #define LN_WALKS (LN_GRID < LN_GROUPS)
+#define LN_APART (LN_WALKS || LN_VW == 1)        // each vector is loaded behind a branch of its own
 #ifndef LN_F16
 #define LN_F16 0
 #define LN_F16_DEFAULTED
@@ -98,17 +99,18 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
 
   // Workgroups that walk the rows load each vector behind a branch of its own, which waits for the row before the next one is
   // reduced; without the branches a row's loads stay in flight over the reductions of the one before, and the time goes up (fp32
-  // 16384 x 8192 180 us and 190, 16384 x 4096 87.2 and 88.5): the memory is faster with fewer requests at a time.
+  // 16384 x 8192 180 us and 190, 16384 x 4096 87.2 and 88.5): the memory is faster with fewer requests at a time.  So do rows of
+  // single elements, 8 to 16 of them a lane (fp16 6631 x 10317 79.9 us without the branches and 74.2).
   auto load_row = [&](long row, io_vec_t (&dst)[LN_VPT]) __attribute__((always_inline)) {
     const bool live = row < LN_ROWS;
     const LN_IO* __restrict__ x = X + (live ? row : 0) * (long)LN_N;
 #pragma unroll
     for (int i = 0; i < LN_VPT; ++i)
-      if (LN_WALKS && !(live && begin(i) < LN_N)) {
+      if (LN_APART && !(live && begin(i) < LN_N)) {
 #pragma unroll
         for (int j = 0; j < LN_VW; ++j) dst[i][j] = (LN_IO)0.0f;
       } else {
-        dst[i] = kcg_stream_load<LN_STREAM != 0>((const io_vec_t*)(x + (LN_WALKS ? place(i) : column(i))));   // read once: 3-4 % faster from HBM with the hint, 10 % slower when the input is still in the last-level cache
+        dst[i] = kcg_stream_load<LN_STREAM != 0>((const io_vec_t*)(x + (LN_APART ? place(i) : column(i))));   // read once: 3-4 % faster from HBM with the hint, 10 % slower when the input is still in the last-level cache
       }
   };
 
@@ -189,7 +191,7 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
 #pragma unroll
     for (int i = 0; i < LN_VPT; ++i)
 #pragma unroll
-      for (int j = 0; j < LN_VW; ++j) s += (LN_WALKS && LN_N % LN_VW == 0) || counts(i, j) ? v[i][j] : 0.0f;
+      for (int j = 0; j < LN_VW; ++j) s += (LN_APART && LN_N % LN_VW == 0) || counts(i, j) ? v[i][j] : 0.0f;
     s = kcg_wave_sum(s);
 #if LN_TPR > KCG_WAVE
     if ((tr % KCG_WAVE) == 0) red[0][rb][wv] = s;
@@ -251,6 +253,7 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
 }
 #undef LN_GROUPS
 #undef LN_WALKS
+#undef LN_APART
 #undef LN_IO
 #ifdef LN_ONEPASS_DEFAULTED
 #undef LN_ONEPASS
