@@ -1029,7 +1029,7 @@ bool emitGemmBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::
   if (m16 && (!m16Fits || edge)) { err = "gemm_bf16: M16 needs full 64-deep tiles, TA = 0, one staging set and no tail split"; return false; }
   s.p["D2L"] = d2l;
   if (fewRows && !(shift && clamp && d2l)) { err = "gemm_bf16: tiles of 32 rows need aligned operands and direct loads"; return false; }
-  if (d2l && !d2lFits) { err = "gemm_bf16: D2L needs M16 and whole 1 KiB blocks per wavefront (row-major weights: BN = 64, 128 or 256)"; return false; }
+  if (d2l && !d2lFits) { err = "gemm_bf16: D2L needs M16 and whole 1 KiB blocks per wavefront (row-major weights: BN = 64, 128, 192 or 256)"; return false; }
   const int64_t nbuf = s.get("NBUF", 2);
   if (nbuf < 2 || nbuf > 6 || (nbuf > 2 && (!d2l || (nbuf - 1) * (bm / 8 + bn / 8) / waves > 63))) {
     err = "gemm_bf16: NBUF is 2 to 6, more than two with direct loads only";

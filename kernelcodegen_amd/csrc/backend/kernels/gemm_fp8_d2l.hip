@@ -1,9 +1,9 @@
 // ---- fp8 (e4m3) GEMM on v_mfma_f32_16x16x128_f8f6f4, operand tiles straight from global memory into LDS --------
 // C[b] = scale_a * scale_b * A[b] * B[b]: A is [M][K]; B is [N][K] (both contiguous along k) or, with G8_BTR, row-major
-// [K][N]; fp8 e4m3, one fp32 scale per tensor, fp32 accumulate, fp32 or bf16 out.  Full 256 x 256 x 128 tiles only (the emitter falls back to
-// gemm_fp8.hip for every other case).  Parameters:
+// [K][N]; fp8 e4m3, one fp32 scale per tensor, fp32 accumulate, fp32 or bf16 out.  Tiles of 256 x 256 or 256 x 192, k-tiles of 128, whole or moved back
+// from the edge (gemm_fp8.hip takes every other case).  Parameters:
 //   G8_NAME                      kernel symbol
-//   G8_M G8_N G8_K G8_BATCH      problem: multiples of 256, 256 and 128
+//   G8_M G8_N G8_K G8_BATCH      problem: multiples of 256, G8_BN and 128 (M and N: see G8_SHIFT)
 //   G8_BN                        columns of a tile, 256 (default) or 192 (results through LDS, one workgroup per tile)
 //   G8_SHIFT                     1: M and N are at least a tile and N a multiple of 16; the last tile of a row or column of tiles
 //                                is moved back to end at the edge and stores only what the tile before it does not own
@@ -23,9 +23,10 @@
 // Why this shape.  The part is power bound on 8-bit products, and v_mfma_f32_16x16x128 reads and writes the fp32
 // accumulators half as often per result as v_mfma_f32_32x32x64: a register-only loop on random e4m3 operands sustains
 // 4.8 against 4.0 PFLOP/s, 3.9 against 3.5 with the fragment reads from LDS.  One instruction takes a whole 128-byte
-// k-tile, so a tile is one k-step: eight wavefronts (4 x 2) of 64 x 128 results = 4 x 8 MFMA tiles, 32 MFMAs per tile.
+// k-tile, so a tile is one k-step: eight wavefronts (4 x 2) of 64 x 128 results = 4 x 8 MFMA tiles, 32 MFMAs
+// per tile (192 columns: 64 x 96, 4 x 6, 24).
 //
-// LDS.  Two buffers per operand of 256 rows x 128 bytes (A's two, then B's two), no padding; chunk c (16 bytes) of row r lies at position
+// LDS.  Two buffers per operand of 256 rows x 128 bytes (A's two, then B's two, which have G8_BN rows), no padding; chunk c (16 bytes) of row r lies at position
 // c ^ ((r / 2) % 8).  Lane l of a fragment holds row l % 16 and the chunks l / 16 and l / 16 + 4 of the row (the same
 // regrouping of k for A and B, so the products pair up): the sixteen lanes that a ds_read_b128 serves in one pass
 // (lanes 0-3, 12-15, 20-27 of a half-wave, then the rest) then read sixteen different groups of four banks.
@@ -38,11 +39,11 @@
 //
 // Pipeline.  The MFMAs of a tile go column by column; the B fragment of a column is read two columns ahead (four B
 // fragments in registers), the four A fragments of a tile have a second set.  One barrier per tile, in front of
-// column 6: by then a wavefront has received all its fragments of the tile (so the tile's buffer is free) and has
+// the last two columns, 6 and 7 (of 192: 4 and 5): by then a wavefront has received all its fragments of the tile (so the tile's buffer is free) and has
 // waited for its share of the next tile (so that tile is complete once everyone has arrived).  Behind the barrier,
-// under the MFMAs of columns 6 and 7, the next tile's A fragments and first two B fragments are read, and the loads
+// under those columns' MFMAs, the next tile's A fragments and first two B fragments are read, and the loads
 // of the tile after next start into the freed buffer (four instructions behind each of these two columns; spread over
-// four columns, two each, measured 1 to 4 % slower): they have until the next tile's column 6 to land.
+// four columns, two each, measured 1 to 4 % slower): they have until the next tile's barrier to land.
 #ifndef KCG_GEMM8D_HELPERS
 #define KCG_GEMM8D_HELPERS
 template <bool B> struct KcgBool8d { static constexpr bool v = B; };
@@ -167,7 +168,7 @@ void G8_NAME(const unsigned char* __restrict__ A, const unsigned char* __restric
   B += batch * (long)G8_K * G8_N;
   C += batch * (long)G8_M * G8_N;
 
-  // ---- loads: instruction t (0..3) of this wavefront moves rows (4 wave + t) * 8 .. + 7 of an operand tile ----
+  // ---- loads: instruction t (0..3) of this wavefront moves rows (4 wave + t) * 8 .. + 7 of an operand tile (of B (UB wave + t) * 8) ----
   const unsigned lds_base = (unsigned)(size_t)(__attribute__((address_space(3))) char*)kcg_smem;
   const unsigned lds_wave = __builtin_amdgcn_readfirstlane(lds_base + wave_u * 4096), lds_wave_b = __builtin_amdgcn_readfirstlane(lds_base + B_AT + wave_u * (UB * 1024));
   const unsigned dma_lane = (unsigned)(lane >> 3) * (unsigned)G8_K + (unsigned)(((lane & 7) ^ (lane >> 4)) * 16);
@@ -360,8 +361,8 @@ void G8_NAME(const unsigned char* __restrict__ A, const unsigned char* __restric
         acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fa[par][i], fb[(j + S) & 3], acc[i][j], 0, 0, 0, 0, 0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
-      // all eight loads of tile kt+2 go out in the two columns behind the barrier, four each: they then have six columns
-      // of MFMA work to land before the next barrier asks for them
+      // all 4 + UB loads of tile kt+2 go out in the two columns behind the barrier, A's four and B's UB half in each: they then have
+      // TN - 2 columns of MFMA work to land before the next barrier asks for them
       if (j >= LAST2 && fetch) {
         const int u = 2 * (j - LAST2);
         dma(u, kt + 2, par); dma(u + 1, kt + 2, par); dma(4 + u, kt + 2, par); dma(5 + u, kt + 2, par);
