@@ -1365,6 +1365,12 @@ bool emitFmhaWavek(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std:
 // and 1.47 (128) times as fast as walks alone and no more than 5 % slower on all but one of them.  us, walk and split, D 64: bf16
 // heads x S 8 x 333 7.8 and 4.7, 8 x 1024 14.5 and 7.8, 32 x 512 9.3 and 7.6; but 32 x 1024 15.8 and 17.2, 128 x 512 15.5 and 18.3; fp32
 // 8 x 1024 78 and 23, 32 x 512 44 and 23, 48 x 1024 133 and 113, but 128 x 512 76 and 84.
+// More workgroups than the part holds at a time take up to 1.6 times what is modelled.  Of 660 drawn launches (8 to 400 heads, S 40
+// to 1600) on which the split was taken, 35 % faster on average, 34 were more than 3 % slower, most of them these: at head dim 64 in
+// 16 bits 19 of 58, causal, 183 x 362 18.2 and 21.5, 371 x 1126 138 and 172.  There a walk in whole rounds is priced, its last one like the
+// others, and the split taken below 0.63 of it: no loser is left, and those that go gained 1 % on average (291 x 270, whose
+// walk has a second round of 35 workgroups, stays: 35.5 and 21.6).  fp32, head dim 128: not where a wavefront's second tile is the
+// exception (255 x 91 causal 22.9 and 30.5).
 static bool fmhaWavekAhead(const KernelSpec& s, int type, int64_t br, bool paired, double items, int64_t held, int64_t& qb, int64_t& wk) {
   const int64_t sl = s.get("S", 0), dh = s.get("D", 0);
   const double heads = (double)s.get("B", 0) * (double)s.get("H", 0);
@@ -1381,7 +1387,9 @@ static bool fmhaWavekAhead(const KernelSpec& s, int type, int64_t br, bool paire
   const double rounds = std::ceil(items / (256.0 * (double)held)), longest = causal && !paired ? tiles : each;
   const bool ragged = sl % br != 0 || sl % 64 != 0;
   const double walk = r.tiled + (1.0 + (ragged ? r.ragged : 0.0)) * longer(r.tiledWalk * rounds * longest, r.tiledWork * each * items / 256.0 * (br / 32), 0.0);
-  double least = 0.0;
+  const double busy = paired || !causal ? std::ceil(items / 256.0) : items / 256.0;
+  const double whole = r.tiled + (1.0 + (ragged ? r.ragged : 0.0)) * longer(r.tiledWalk * rounds * longest, r.tiledWork * each * busy * (br / 32), 0.0);
+  double least = 0.0, most = r.margin * walk;
   const int64_t row = dh * (type == 0 ? 4 : 2);
   for (int64_t q : {1, 2})
     for (int64_t w : {2, 4, 8}) {
@@ -1392,9 +1400,13 @@ static bool fmhaWavekAhead(const KernelSpec& s, int type, int64_t br, bool paire
       const double chain = turns * std::ceil((turns == 1.0 ? tiles : mean) / (double)w);
       const double work = (causal ? std::max(groups / 256.0, 1.0) * 1.15 : per) * mean * (double)q / 4.0;
       const double us = r.fixed + longer(r.walk * chain, r.work * work, r.l2 * groups * mean * (double)row * 64.0 / 1e6) + r.merge * (double)(w * q) * per / 16.0;
-      if (least == 0.0 || us < least) { least = us; qb = q; wk = w; }
+      if (least == 0.0 || us < least) {
+        least = us; qb = q; wk = w; most = r.margin * walk;
+        if (turns > 1.0 && type != 0 && dh == 64) most = std::min(most, 0.63 * whole);
+        if (turns > 1.0 && type == 0 && dh == 128 && tiles < 2.0 * (double)w) most = 0.0;
+      }
     }
-  return least > 0.0 && least < r.margin * walk;
+  return least > 0.0 && least < most;
 }
 
 bool emitFmhaBf16(KernelSpec& s, std::string& src, KernelLaunchInfo& info, std::string& err) {

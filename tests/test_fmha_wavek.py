@@ -70,3 +70,10 @@ def test_queries_are_scaled_by_a_power_of_two(family, f16, scale):
                                          ("fmha_bf16", dict(PAIR=0)), ("fmha_bf16", dict(D2L=0)), ("fmha_f32", dict(OCC=1)), ("fmha_f32", dict(PAIR=0)), ("fmha_f32", dict(D2L=0))])
 def test_a_wish_that_the_split_has_no_use_for_is_not_dropped(family, wish):
     assert SPLIT not in text_of(family, B=1, H=8, S=333, D=64, SCALE=0.1, **wish)
+
+
+@pytest.mark.parametrize("family,heads,s,d,split", [("fmha_bf16", 183, 362, 64, False), ("fmha_bf16", 371, 1126, 64, False), ("fmha_bf16", 234, 400, 64, False), ("fmha_bf16", 291, 270, 64, True),
+                                                    ("fmha_bf16", 8, 333, 64, True), ("fmha_f32", 255, 91, 128, False), ("fmha_f32", 225, 89, 128, False), ("fmha_f32", 97, 970, 64, True)])
+def test_more_workgroups_than_the_part_holds_rarely_split(family, heads, s, d, split):
+    """Under the mask, launches that were measured slower split than walked beside such as were faster."""
+    assert (SPLIT in text_of(family, B=1, H=heads, S=s, D=d, CAUSAL=1, SCALE=0.1)) == split
