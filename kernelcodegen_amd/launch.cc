@@ -84,7 +84,10 @@ PyObject* callLaunch(PyObject* me, PyObject* const* args, size_t nargsf, PyObjec
     if (THPVariable_Check(args[i])) {
       slots[i] = (uint64_t)(uintptr_t)THPVariable_Unpack(args[i]).data_ptr();
     } else {
-      slots[i] = PyLong_AsUnsignedLongLong(args[i]);
+      PyObject* whole = PyNumber_Index(args[i]);
+      if (!whole) return nullptr;
+      slots[i] = PyLong_AsUnsignedLongLong(whole);
+      Py_DECREF(whole);
       if (slots[i] == (uint64_t)-1 && PyErr_Occurred()) return nullptr;
     }
   }

@@ -55,6 +55,19 @@ def test_wrong_arguments_are_refused():
     assert not entry.calls
 
 
+def test_a_pointer_is_any_whole_number():
+    """What has __index__, as for the ctypes launches."""
+    numpy = pytest.importorskip("numpy")
+    entry = Entry()
+    run = make(entry, 2, 0)
+    if torch.cuda.is_available():
+        run(numpy.int64(16), numpy.uint64(1 << 63))
+        assert entry.calls[-1][3] == [16, 1 << 63]
+    else:
+        with pytest.raises(RuntimeError):         # (of the stream that is not there, behind the arguments)
+            run(numpy.int64(16), numpy.uint64(1 << 63))
+
+
 def test_without_a_gpu_a_launch_is_an_error():
     if torch.cuda.is_available():
         pytest.skip("there is one")
