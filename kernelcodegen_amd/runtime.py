@@ -148,7 +148,7 @@ def _native_launch():
     if _launch_type is None:
         import importlib
         import torch                    # (the extension's libraries)
-        _launch_type, why = False, None
+        found, why = False, None
         try:
             module = importlib.import_module(__package__ + "._launch")
         except ModuleNotFoundError:
@@ -158,12 +158,13 @@ def _native_launch():
         else:
             # objects of torch are laid out as in the headers of the build
             if getattr(module, "torch_version", None) == torch.__version__:
-                _launch_type = module.Launch
+                found = module.Launch
             else:
                 why = "built for torch %s, this is %s" % (getattr(module, "torch_version", "of another version"), torch.__version__)
         if why:
             import warnings
             warnings.warn("the native launches are not used, ctypes takes their place: " + why, RuntimeWarning)
+        _launch_type = found
     return _launch_type or None
 
 
@@ -392,7 +393,8 @@ _kernel_cache = {}
 def launch_params(family, params):
     """The parameters of a kernel that is compiled to be launched from here.  Attention, LayerNorm, and a product whose caller has
     looked at the operands' addresses (ALIGN = 16), may take the forms that fill the part, those whose wavefronts split k or the keys
-    included (FILL = 2), unless the caller names another FILL than 1.  WAVEK = 0 beside it leaves the split out: the forms of FILL = 1.  Text that is emitted for others to keep has the tiles that its parameters name."""
+    included (FILL = 2), unless the caller names another FILL than 1.  WAVEK = 0 beside it leaves the split out: the forms of FILL = 1.
+    Text that is emitted for others to keep has the tiles that its parameters name."""
     if (family == "layernorm" or family.startswith("fmha_") or (family.startswith("gemm_") and params.get("ALIGN", 0) >= 16)) and params.get("FILL", 1) == 1:
         return {**params, "FILL": 2}
     return params
