@@ -38,13 +38,35 @@ def _check(b, h, s, d, dtype, causal, cfg, out=None, spread=1.0):
 FORMS = [dict(WAVEK=2), dict(WAVEK=4), dict(WAVEK=8), dict(WAVEK=4, QB=2), dict(WAVEK=1)]
 
 
+TYPES = [("f32", 64), ("f32", 128), ("bf16", 64), ("f16", 64), ("bf16", 128), ("f16", 128), ("f16", 32), ("f32", 32)]
+SIZES = [(1, 3, 1), (1, 8, 32), (2, 4, 33), (1, 5, 97), (1, 8, 300)]
+
+
+@pytest.fixture(scope="module")
+def compiled():
+    """The kernels of test_forms: one after the other they are most of its time."""
+    from compile_ahead import compile_ahead
+    kernels = []
+    for dtype, d in TYPES:
+        for form in FORMS:
+            for causal in (0, 1):
+                for b, h, s in SIZES + [(1, 2, 130)]:
+                    problem = dict(B=b, H=h, S=s, D=d, CAUSAL=causal, SCALE=d ** -0.5, FILL=1, **form)
+                    if dtype == "f32":
+                        if d < 128 or form["WAVEK"] <= 4:
+                            kernels.append(("fmha_f32", problem))
+                    else:
+                        kernels += [("fmha_bf16", dict(problem, F16=int(dtype == "f16"), OUT_BF16=out)) for out in ((1, 0) if s == 130 else (1,))]
+    compile_ahead(kernels)
+
+
 @pytest.mark.parametrize("causal", [False, True])
-@pytest.mark.parametrize("dtype,d", [("f32", 64), ("f32", 128), ("bf16", 64), ("f16", 64), ("bf16", 128), ("f16", 128), ("f16", 32), ("f32", 32)])
+@pytest.mark.parametrize("dtype,d", TYPES)
 @pytest.mark.parametrize("form", FORMS)
-def test_forms(form, dtype, d, causal):
+def test_forms(form, dtype, d, causal, compiled):
     if dtype == "f32" and d == 128 and form["WAVEK"] > 4:
         pytest.skip("the wavefronts' tiles do not fit the LDS")
-    for b, h, s in [(1, 3, 1), (1, 8, 32), (2, 4, 33), (1, 5, 97), (1, 8, 300)]:
+    for b, h, s in SIZES:
         _check(b, h, s, d, dtype, causal, form)
     _check(1, 2, 130, d, dtype, causal, form, spread=40.0)
     if dtype != "f32":

@@ -38,17 +38,10 @@ LENGTHS = [512, 513, 519, 1023, 1032, 1280, 2049, 3071, 3073, 4100, 5119, 5120, 
 
 @pytest.fixture(scope="module")
 def compiled():
-    """The kernels of test_lengths, compiled side by side into the code-object cache: one after the other they are most of its time."""
-    from concurrent.futures import ThreadPoolExecutor
-    from kernelcodegen_amd import ops, runtime as R
-
-    def one(of):
-        n, rows, dtype = of
-        text, _ = R.emit_kernel("layernorm", "kernel0", **R.launch_params("layernorm", dict(
-            ROWS=rows, N=n, NG=n, NB=n, EPS=1e-5, GELU=n % 2, F16=ops._STORAGE[DTYPE[dtype]])))
-        R.compile_to_code(R.prelude() + text)
-    with ThreadPoolExecutor(16) as pool:
-        list(pool.map(one, [(n, rows, dtype) for n in LENGTHS for rows in ROWS for dtype in DTYPE]))
+    """The kernels of test_lengths: one after the other they are most of its time."""
+    from compile_ahead import compile_ahead
+    compile_ahead([("layernorm", dict(ROWS=rows, N=n, NG=n, NB=n, EPS=1e-5, GELU=n % 2, F16=["f32", "f16", "bf16"].index(dtype)))
+                   for n in LENGTHS for rows in ROWS for dtype in DTYPE])
 
 
 @pytest.mark.parametrize("dtype", sorted(DTYPE))

@@ -16,12 +16,31 @@ def _operands(m, n, k, trans_b, batch=1):
     return a, b, a.double() @ (b.double().transpose(-1, -2).contiguous() if trans_b else b.double())
 
 
+TILES = [(256, 192, 4, 2, 2), (192, 256, 2, 4, 2), (128, 192, 4, 2, 2), (128, 192, 4, 2, 3), (192, 128, 2, 4, 2), (192, 128, 2, 4, 3)]
+
+
+def _sizes(bm, bn):
+    return [(bm, bn, 64), (bm + 1, bn + 8, 192), (2 * bm - 3, 3 * bn - 16, 200), (bm + 100, 2 * bn, 1096), (700, 1000, 640)]
+
+
+def _tile(bm, bn, wm, wn, nbuf):
+    return dict(BM=bm, BN=bn, WM=wm, WN=wn, NBUF=nbuf, M16=1, D2L=1)
+
+
+@pytest.fixture(scope="module")
+def compiled():
+    """The kernels of test_16_bit: one after the other they are most of its time."""
+    from compile_ahead import compile_ahead
+    compile_ahead([("gemm_bf16", dict(M=m, N=n, K=k, BATCH=1, TA=0, TB=tb, OUT_BF16=out, ALIGN=16, **(dict(F16=1) if half else {}), **_tile(*tile)))
+                   for tile in TILES for m, n, k in _sizes(*tile[:2]) for tb in (0, 1) for half in (0, 1) for out in (0, 1)])
+
+
 @pytest.mark.parametrize("trans_b", [True, False])
-@pytest.mark.parametrize("bm,bn,wm,wn,nbuf", [(256, 192, 4, 2, 2), (192, 256, 2, 4, 2), (128, 192, 4, 2, 2), (128, 192, 4, 2, 3), (192, 128, 2, 4, 2), (192, 128, 2, 4, 3)])
-def test_16_bit(bm, bn, wm, wn, nbuf, trans_b):
+@pytest.mark.parametrize("bm,bn,wm,wn,nbuf", TILES)
+def test_16_bit(bm, bn, wm, wn, nbuf, trans_b, compiled):
     from kernelcodegen_amd import ops
-    cfg = dict(BM=bm, BN=bn, WM=wm, WN=wn, NBUF=nbuf, M16=1, D2L=1)
-    for m, n, k in [(bm, bn, 64), (bm + 1, bn + 8, 192), (2 * bm - 3, 3 * bn - 16, 200), (bm + 100, 2 * bn, 1096), (700, 1000, 640)]:
+    cfg = _tile(bm, bn, wm, wn, nbuf)
+    for m, n, k in _sizes(bm, bn):
         a, b, ref = _operands(m, n, k, trans_b)
         for dtype in (torch.bfloat16, torch.float16):
             for out in (torch.float32, dtype):
