@@ -24,7 +24,8 @@ _bound = {}
 
 def _into(run, shape=None, dtype=None):
     """A bound launch whose last pointer is the result: a function of the operand tensors (and numbers) that allocates the result,
-    of that shape and type on the first operand's device, or like the first operand, launches and returns it."""
+    of that shape and type on the first operand's device, or like the first operand, launches and returns it.  The result is a plain
+    tensor; where a subclass of the operand decides about it (torch.empty_like), the caller allocates."""
     native = getattr(run, "result", None)
     if native is not None:
         return native(shape, dtype)
@@ -54,7 +55,9 @@ def layernorm(x, gamma, beta, axis, eps=1e-5, gelu=False, out=None, **cfg):
         if not cfg:
             _bound[key] = hit
     if out is None:
-        return hit[1](x, gamma, beta)
+        if type(x) is torch.Tensor:
+            return hit[1](x, gamma, beta)
+        out = torch.empty_like(x)
     hit[0](x.data_ptr(), gamma.data_ptr(), beta.data_ptr(), out.data_ptr())
     return out
 
@@ -87,7 +90,7 @@ def elementwise(x, op, inplace=False, out_dtype=None, **cfg):
     if inplace:
         run(x.data_ptr())
         return x if out_dtype == x.dtype else x.view(out_dtype)
-    if into is not None:
+    if into is not None and type(x) is torch.Tensor:
         return into(x)
     y = torch.empty(x.shape, dtype=out_dtype, device=x.device)
     run(x.data_ptr(), y.data_ptr())
@@ -296,13 +299,17 @@ def softmax(x, inplace=False):
         raise ValueError("the softmax kernel takes fp32, IEEE half or bfloat16 operands")
     inplace = int(inplace)
     key = ("softmax", x.shape, x.dtype, inplace)
-    run = _bound.get(key)
-    if run is None:
+    hit = _bound.get(key)
+    if hit is None:
         n = x.shape[-1]
         run = R.get_kernel("softmax", ROWS=x.numel() // n, N=n, INPLACE=int(inplace), F16=_STORAGE[x.dtype]).bind()
-        _bound[key] = run = run if inplace else _into(run)
+        _bound[key] = hit = run, None if inplace else _into(run)
     if inplace:
-        run(x.data_ptr())
+        hit[0](x.data_ptr())
         return x
-    return run(x)
+    if type(x) is torch.Tensor:
+        return hit[1](x)
+    y = torch.empty_like(x)
+    hit[0](x.data_ptr(), y.data_ptr())
+    return y
 

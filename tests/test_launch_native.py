@@ -145,3 +145,20 @@ def test_a_failed_launch_raises():
     for call in (lambda: run(16, 32), lambda: run.result(None, None)(x)):
         with pytest.raises(ValueError, match="status 5"):
             call()
+
+
+class Marked(torch.Tensor):
+    pass
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("wrap,like", [(lambda x: x.as_subclass(Marked), Marked), (lambda x: torch.nn.Parameter(x, requires_grad=False), torch.Tensor)])
+def test_a_result_like_the_operand_is_of_its_subclass(wrap, like):
+    """What torch.empty_like gives; the other results are plain tensors."""
+    from kernelcodegen_amd import ops
+    x, one, zero = torch.randn(64, 512, device="cuda"), torch.ones(512, device="cuda"), torch.zeros(512, device="cuda")
+    for call, result in [(lambda x: ops.softmax(x), like), (lambda x: ops.layernorm(x, one, zero, 1), like),
+                         (lambda x: ops.elementwise(x, "Relu"), torch.Tensor), (lambda x: ops.matmul(x, x.t().contiguous()), torch.Tensor)]:
+        got = call(wrap(x))
+        assert type(got) is result
+        assert torch.equal(got.as_subclass(torch.Tensor), call(x))
