@@ -39,7 +39,7 @@
 //                LN_TPR * LN_VW); the emitter asks for it only then.
 #define LN_GROUPS ((LN_ROWS + LN_RPB - 1) / LN_RPB)
 #define LN_WALKS (LN_GRID < LN_GROUPS)
-#define LN_APART (LN_WALKS || LN_VW == 1)        // each vector is loaded behind a branch of its own
+#define LN_APART (LN_WALKS || (LN_VW == 1 && LN_VPT > 8))        // each vector is loaded behind a branch of its own
 #ifndef LN_F16
 #define LN_F16 0
 #define LN_F16_DEFAULTED
@@ -100,7 +100,8 @@ void LN_NAME(const LN_IO* __restrict__ X, const LN_IO* __restrict__ G,
   // Workgroups that walk the rows load each vector behind a branch of its own, which waits for the row before the next one is
   // reduced; without the branches a row's loads stay in flight over the reductions of the one before, and the time goes up (fp32
   // 16384 x 8192 180 us and 190, 16384 x 4096 87.2 and 88.5): the memory is faster with fewer requests at a time.  So do rows of
-  // single elements, 8 to 16 of them a lane (fp16 6631 x 10317 79.9 us without the branches and 74.2).
+  // single elements, 9 to 16 of them a lane (fp16 6631 x 10317 79.9 us without the branches and 74.2, bf16 547 x 10519 10.6 and 10.0); up
+  // to 8 of them, on rows of at most 4096, are slower behind branches (fp16 138 x 387 2.96 us without them and 3.24, 13 x 2723 2.88 and 3.18).
   auto load_row = [&](long row, io_vec_t (&dst)[LN_VPT]) __attribute__((always_inline)) {
     const bool live = row < LN_ROWS;
     const LN_IO* __restrict__ x = X + (live ? row : 0) * (long)LN_N;

@@ -98,3 +98,12 @@ def test_held_layernorm_rows_walk_on_few_workgroups(rows, n, grid):
     """fp32 rows that start off the vectors on somewhat more of them than whole ones, while they are not far beyond the caches."""
     _, info = R.emit_kernel("layernorm", "kernel0", ROWS=rows, N=n, NG=n, NB=n, EPS=1e-5)
     assert info["grid"][0] == grid
+
+
+@pytest.mark.parametrize("rows,n,ng,branches", [(138, 387, 387, 0), (13, 2723, 1, 0), (2, 3989, 1, 0), (445, 10115, 10115, 1), (12087, 8743, 8743, 1), (16384, 387, 387, 1), (4096, 1024, 1024, 0)])
+def test_layernorm_loads_behind_branches_where_they_are_faster(rows, n, ng, branches):
+    """Workgroups that walk, and rows of more than eight single elements a lane; not shorter ones with a workgroup each."""
+    text, _ = R.emit_kernel("layernorm", "kernel0", **R.launch_params("layernorm", dict(ROWS=rows, N=n, NG=ng, NB=ng, EPS=1e-5, F16=1)))
+    lines = [l for l in text.splitlines() if l.startswith("#define LN_")]
+    done = subprocess.run(["g++", "-E", "-P", "-x", "c", "-"], input="\n".join(lines) + "\n#if LN_APART\nbranches 1\n#else\nbranches 0\n#endif\n", capture_output=True, text=True, check=True)
+    assert done.stdout.split()[-2:] == ["branches", str(branches)]
